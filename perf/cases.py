@@ -195,3 +195,58 @@ def tolerance(case):
     if case["path"] in ("gemm", "matmul", "train"):
         return {"rel": {"bfloat16": 6.6e-3, "float16": 8.3e-4, "float32": 7.2e-8 * math.sqrt(case["k"])}[case["dtype"]]}
     return {"rel": 6.6e-3}
+
+
+_E2M1 = (0.0, 0.5, 1.0, 1.5, 2.0, 3.0, 4.0, 6.0, -0.0, -0.5, -1.0, -1.5, -2.0, -3.0, -4.0, -6.0)
+
+
+def _from_mxfp4(codes, scales):
+    """The values that packed e2m1 codes and their block scales stand for (scale byte 0 is 2**-127)."""
+    values = torch.tensor(_E2M1, dtype=torch.float64, device=codes.device)
+    c = codes.long()
+    v = values[torch.stack([c & 15, c >> 4], -1).reshape(codes.shape[0], -1)]
+    return v * torch.ldexp(torch.ones((), dtype=torch.float64, device=codes.device), scales.long() - 127).repeat_interleave(32, 1)
+
+
+def _rotate_and_quantise(x):
+    """Every 32 values of a row times H32 / sqrt(32) in single precision (butterflies of stride 1, 2, 4, 8, 16), their scale the power of two
+    two below the largest one's, a mantissa of 1.75 and above rounded up; values to the nearest e2m1, ties away from zero."""
+    y = x.float().reshape(-1, 32)
+    for h in (1, 2, 4, 8, 16):
+        y = y.reshape(-1, 16 // h, 2, h)
+        y = torch.stack([y[:, :, 0] + y[:, :, 1], y[:, :, 0] - y[:, :, 1]], 2)
+    y = y.reshape(-1, 32) * torch.tensor(0x3E3504F3, dtype=torch.int32, device=x.device).view(torch.float32)
+    top = ((y.abs().amax(1).view(torch.int32) + 0x200000) >> 23) - 129
+    scale = torch.ldexp(torch.ones((), dtype=torch.float64, device=x.device), top.clamp(-127, 127).unsqueeze(1))
+    q = y.double() / scale
+    mag, steps = q.abs(), torch.tensor((0.25, 0.75, 1.25, 1.75, 2.5, 3.5, 5.0), dtype=torch.float64, device=x.device)
+    v = torch.tensor(_E2M1[:8], dtype=torch.float64, device=x.device)[torch.bucketize(mag, steps, right=True)]
+    return (torch.copysign(v, q) * scale).reshape(x.shape)
+
+
+def exact(case, seed):
+    """The outputs of run() from plain torch operations in 64 bits.  Operands that the path rounds to 8 or 4 bits are rounded in the same
+    way first: what is measured is the product's own error."""
+    s, path = prepare(case, seed), case["path"]
+    if path in ("gemm", "matmul"):
+        return s["a"].double() @ s["b"].double()
+    if path == "train":
+        x, w, bias, g = (s[name].detach().double() for name in ("x", "w", "bias", "grad"))
+        kn = w.T if s["transposed"] else w
+        dw = x.T @ g
+        return x @ kn + bias, g @ kn.T, dw.T if s["transposed"] else dw, g.sum(0)
+    if path in ("a8w8", "linear8"):
+        if path == "a8w8":
+            q, scale = s["a"], s["a_scale"]
+        else:
+            x = s["x"].float()
+            top = 127.0 if s["dtype"] == torch.int8 else torch.finfo(s["dtype"]).max
+            scale = x.abs().amax(1).clamp(min=1e-8) / top
+            q = x * (1.0 / scale).unsqueeze(1)
+            q = (q.round().clamp(-top, top) if s["dtype"] == torch.int8 else q).to(s["dtype"])
+        return (q.double() @ s["w"].double()) * scale.double().reshape(-1, 1) * s["w_scale"].double().reshape(1, -1)
+    if path == "moe":
+        at = s["offsets"].tolist()
+        parts = [(s["a"][lo:hi].double() @ s["w"][e].double().T) * s["w_scale"][e].double().reshape(1, -1) for e, (lo, hi) in enumerate(zip(at, at[1:]))]
+        return torch.cat(parts) * s["a_scale"].double().reshape(-1, 1)
+    return _rotate_and_quantise(s["x"]) @ _from_mxfp4(s["w"], s["w_scale"]).T
