@@ -296,6 +296,23 @@ typedef struct tb_quant_desc {
 
 int tb_hadamard_mxfp4_quant(const tb_quant_desc* desc, void* stream);
 
+/* ---- 8-bit quantisation with one scale per row (replaces quantize_tensor_per_channel along the contiguous
+ *      axis, utils.py:340-377): scale = max(amax, min_scale) * (1 / top) with top = 448 (e4m3), 57344 (e5m2)
+ *      or 127 (int8), q = x * (1 / scale), int8 rounded to nearest even and clamped to [-127, 127] -------- */
+typedef struct tb_row_quant_desc {
+  uint32_t struct_bytes;
+  int32_t x_type;             /* TB_BF16, TB_F16 or TB_F32                                           */
+  int32_t q_type;             /* TB_FP8_E4M3, TB_FP8_E5M2 or TB_I8                                   */
+  float min_scale;            /* floor of amax                                                       */
+  int64_t m, n;
+  const void* x;
+  int64_t x_stride_m;         /* elements; unit stride along n                                       */
+  void* q;                    /* (m, n) bytes, contiguous                                            */
+  float* scale;               /* (m)                                                                 */
+} tb_row_quant_desc;
+
+int tb_quantize_rows(const tb_row_quant_desc* desc, void* stream);
+
 /* ---- tile order ------------------------------------------------------------------------------
  * Host-side evaluation of the kernels' tile id -> (row block, column block) map, for tests and tools.
  * With panel_n = 0 it is the reference's GROUP_M swizzle (kernels/stages/schedule.py:124-145); with

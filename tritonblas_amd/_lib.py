@@ -26,6 +26,7 @@ TB_WS_QUEUES, TB_WS_GLOBAL_ATOMIC, TB_WS_HIERARCHICAL = 0, 1, 2
 EXPORTED_SYMBOLS = [
     "tb_abi_version", "tb_status_string", "tb_device_info", "tb_select", "tb_list_tiles", "tb_gemm",
     "tb_workspace_bytes", "tb_gemm_fp4", "tb_grouped_gemm_fp8", "tb_grouped_workspace_bytes", "tb_streamk_tail_tiles", "tb_hadamard_mxfp4_quant",
+    "tb_quantize_rows",
     "tb_tile_coords", "tb_default_panel", "tb_ws_queue_tile", "tb_hierarchical_split",
     "tb_workspace_layout", "tb_debug_option", "tb_gemm_static_workspace", "tb_static_workspace_status", "tb_gemm_launch_info",
 ]
@@ -98,6 +99,12 @@ class tb_quant_desc(C.Structure):
                 ("scales", C.c_void_p), ("scales_stride_m", C.c_int64), ("hadamard", C.c_int32)]
 
 
+class tb_row_quant_desc(C.Structure):
+    _fields_ = [("struct_bytes", C.c_uint32), ("x_type", C.c_int32), ("q_type", C.c_int32), ("min_scale", C.c_float),
+                ("m", C.c_int64), ("n", C.c_int64), ("x", C.c_void_p), ("x_stride_m", C.c_int64), ("q", C.c_void_p),
+                ("scale", C.c_void_p)]
+
+
 _lib = None
 
 
@@ -127,6 +134,7 @@ def load():
     lib.tb_grouped_workspace_bytes.restype = C.c_size_t
     lib.tb_streamk_tail_tiles.argtypes = [C.c_int32] * 5
     lib.tb_hadamard_mxfp4_quant.argtypes = [C.POINTER(tb_quant_desc), C.c_void_p]
+    lib.tb_quantize_rows.argtypes = [C.POINTER(tb_row_quant_desc), C.c_void_p]
     lib.tb_tile_coords.argtypes = [C.c_int32] * 5 + [C.POINTER(C.c_int32), C.POINTER(C.c_int32)]
     lib.tb_default_panel.argtypes = [C.c_int32] * 3
     lib.tb_ws_queue_tile.argtypes = [C.c_int32] * 7 + [C.POINTER(C.c_int32)] * 2

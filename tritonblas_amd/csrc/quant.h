@@ -1,4 +1,4 @@
-// Host/device shared declarations of the MXFP4 quantisation kernel.
+// Host/device shared declarations of the quantisation kernels (MXFP4 blocks, 8-bit rows).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -22,5 +22,19 @@ struct QuantParams {
 };
 
 hipError_t launch_quant(const QuantParams& p, int x_type, bool hadamard, bool force_div64, hipStream_t stream);
+
+enum : int { RQ_E4M3 = 2, RQ_I8 = 5, RQ_E5M2 = 6 };  // same numbering as the public element types
+
+struct RowQuantParams {
+  const uint8_t* x;
+  uint8_t* q;             // (m, n) bytes, rows one after the other
+  float* scale;           // (m)
+  int64_t m, n;
+  int64_t x_stride;       // elements
+  float inv_top, min_scale;
+};
+
+// q_type: RQ_*
+hipError_t launch_row_quant(const RowQuantParams& p, int x_type, int q_type, hipStream_t stream);
 
 }  // namespace tb

@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <stdlib.h>
+#include <type_traits>
 #include "quant.h"
 
 namespace tb {
@@ -170,6 +171,243 @@ hipError_t launch_quant(const QuantParams& p, int x_type, bool hadamard, bool fo
   if (x_type == QT_BF16) return hadamard ? launch_t<QT_BF16, true>(p, force_div64, stream) : launch_t<QT_BF16, false>(p, force_div64, stream);
   if (x_type == QT_F16) return hadamard ? launch_t<QT_F16, true>(p, force_div64, stream) : launch_t<QT_F16, false>(p, force_div64, stream);
   return hadamard ? launch_t<QT_F32, true>(p, force_div64, stream) : launch_t<QT_F32, false>(p, force_div64, stream);
+}
+
+// ---- one 8-bit scale per row -----------------------------------------------------------------------
+// amax of a row -> scale = max(amax, min_scale) * (1 / top) -> q = x * (1 / scale) in fp32 -> e4m3 / e5m2 / int8.
+//
+// Bound by HBM: the row is read once and stays in registers between the two uses, so a row costs its own bytes, the codes and
+// one float.  Written as tensor operations (convert, abs, amax, clamp, two scalings, product, convert) the same values cost nine
+// launches and five passes over fp32 copies of x: quantising 512x14336 bf16 and multiplying by a 4096x14336 e4m3 weight took
+// 114 us as tensor operations + GEMM and takes 54 us with this kernel (49 us of it the GEMM).
+// RT threads share a row: a wave while 4096 values fit its registers, a workgroup of 256 up to 16384, 1024 threads beyond.
+// Few rows: more threads per row, so that the loads of a row are spread over the CU (launch_row_quant).  Rows longer than 65536
+// values are read twice (LOOP), the second time mostly from the caches.
+struct RowChunk16 { v4i a; };
+struct RowChunk32 { v4i a, b; };
+
+template <int XT> using row_chunk = typename std::conditional<XT == QT_F32, RowChunk32, RowChunk16>::type;
+
+// eight values of a row, zero past its end.  VEC: rows start on 16 bytes and hold whole chunks.
+template <int XT, bool VEC>
+__device__ __forceinline__ row_chunk<XT> row_load(const uint8_t* row, int64_t c, int64_t n) {
+  row_chunk<XT> r;
+  if constexpr (XT == QT_F32) { r.a = v4i{0, 0, 0, 0}; r.b = v4i{0, 0, 0, 0}; } else { r.a = v4i{0, 0, 0, 0}; }
+  const int64_t left = n - c * 8;
+  if (left <= 0) return r;
+  if constexpr (VEC) {
+    if constexpr (XT == QT_F32) { r.a = *(const v4i*)(row + c * 32); r.b = *(const v4i*)(row + c * 32 + 16); }
+    else r.a = *(const v4i*)(row + c * 16);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j < left) {
+        if constexpr (XT == QT_F32) {
+          const int v = *(const int*)(row + (c * 8 + j) * 4);
+          if (j < 4) r.a[j & 3] = v; else r.b[j & 3] = v;
+        } else {
+          r.a[j >> 1] |= (int)((uint32_t)*(const uint16_t*)(row + (c * 8 + j) * 2) << (16 * (j & 1)));
+        }
+      }
+    }
+  }
+  return r;
+}
+
+template <int XT>
+__device__ __forceinline__ void row_values(const row_chunk<XT>& r, float (&v)[8]) {
+  if constexpr (XT == QT_F32) {
+    const v4f a = __builtin_bit_cast(v4f, r.a), b = __builtin_bit_cast(v4f, r.b);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  } else {
+    const uint32_t w[4] = {(uint32_t)r.a.x, (uint32_t)r.a.y, (uint32_t)r.a.z, (uint32_t)r.a.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (XT == QT_BF16) {
+        v[2 * i] = __builtin_bit_cast(float, w[i] << 16);
+        v[2 * i + 1] = __builtin_bit_cast(float, w[i] & 0xffff0000u);
+      } else {
+        v[2 * i] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w[i] & 0xffffu));
+        v[2 * i + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w[i] >> 16));
+      }
+    }
+  }
+}
+
+// |x| as the integer its bits are: the order of the magnitudes, with NaN above everything (so that a NaN reaches the scale)
+template <int XT>
+__device__ __forceinline__ uint32_t row_amax(const row_chunk<XT>& r, uint32_t m) {
+  float v[8];
+  row_values<XT>(r, v);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, v[j]) & 0x7fffffffu;
+    m = b > m ? b : m;
+  }
+  return m;
+}
+
+// Eight codes of one chunk, lowest byte first.  |x / scale| is at most `top` but for one rounding, and a scale so small that its
+// reciprocal overflows; the converters' own overflow rule is not relied on: the float formats take what lies half a step above
+// the largest finite value to NaN (e4m3) or infinity (e5m2), as a conversion without saturation does.
+template <int XT, int OT>
+__device__ __forceinline__ uint64_t row_codes(const row_chunk<XT>& r, float inv) {
+  float v[8];
+  row_values<XT>(r, v);
+  uint32_t w[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    float q[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) q[j] = v[4 * h + j] * inv;
+    if constexpr (OT == RQ_I8) {
+      w[h] = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float t = __builtin_rintf(q[j]);
+        t = t != t ? 0.f : fminf(fmaxf(t, -127.f), 127.f);
+        w[h] |= ((uint32_t)(int)t & 0xffu) << (8 * j);
+      }
+    } else {
+      constexpr float over = OT == RQ_E4M3 ? 464.f : 61440.f;        // half a step above the largest finite value
+      constexpr float lim = OT == RQ_E4M3 ? 448.f : 57344.f;
+      constexpr uint32_t high = OT == RQ_E4M3 ? 0x7fu : 0x7cu;
+      float s[4];
+      bool any = false;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        s[j] = q[j] != q[j] ? 0.f : fminf(fmaxf(q[j], -lim), lim);
+        any |= !(fabsf(q[j]) < over) || (OT == RQ_E4M3 && fabsf(q[j]) == over);
+      }
+      int p = 0;
+      if constexpr (OT == RQ_E4M3) {
+        p = __builtin_amdgcn_cvt_pk_fp8_f32(s[0], s[1], p, false);
+        p = __builtin_amdgcn_cvt_pk_fp8_f32(s[2], s[3], p, true);
+      } else {
+        p = __builtin_amdgcn_cvt_pk_bf8_f32(s[0], s[1], p, false);
+        p = __builtin_amdgcn_cvt_pk_bf8_f32(s[2], s[3], p, true);
+      }
+      w[h] = (uint32_t)p;
+      if (any) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t sign = (__builtin_bit_cast(uint32_t, q[j]) >> 24) & 0x80u;
+          const bool nan = q[j] != q[j];
+          const bool big = OT == RQ_E4M3 ? fabsf(q[j]) > over : fabsf(q[j]) >= over;   // (464 is a tie: to even, 448)
+          if (nan || big) w[h] = (w[h] & ~(0xffu << (8 * j))) | ((sign | (nan ? 0x7fu : high)) << (8 * j));
+        }
+      }
+    }
+  }
+  return (uint64_t)w[0] | ((uint64_t)w[1] << 32);
+}
+
+template <int XT, int OT, int RT, int CH, bool VEC, bool LOOP>
+__global__ __launch_bounds__(RT < 256 ? 256 : RT) void row_quant_kernel(const RowQuantParams p) {
+  constexpr int ROWS = RT < 256 ? 256 / RT : 1;
+  constexpr int XB = XT == QT_F32 ? 4 : 2;
+  constexpr int WAVES = RT / 64;
+  __shared__ uint32_t part[WAVES > 1 ? WAVES : 1];
+  const int64_t row = (int64_t)blockIdx.x * ROWS + threadIdx.x / RT;
+  if (ROWS > 1 && row >= p.m) return;          // (a whole wave: its lanes share the row)
+  const int t = threadIdx.x % RT;
+  const uint8_t* xr = p.x + row * p.x_stride * XB;
+  const int64_t chunks = (p.n + 7) >> 3;
+
+  row_chunk<XT> r[CH];
+  uint32_t m = 0;
+  if constexpr (LOOP) {
+    for (int64_t c0 = 0; c0 < chunks; c0 += (int64_t)RT * CH) {
+#pragma unroll
+      for (int i = 0; i < CH; ++i) r[i] = row_load<XT, VEC>(xr, c0 + i * RT + t, p.n);
+#pragma unroll
+      for (int i = 0; i < CH; ++i) m = row_amax<XT>(r[i], m);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < CH; ++i) r[i] = row_load<XT, VEC>(xr, i * RT + t, p.n);
+#pragma unroll
+    for (int i = 0; i < CH; ++i) m = row_amax<XT>(r[i], m);
+  }
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    const uint32_t o = (uint32_t)__shfl_xor((int)m, d);
+    m = o > m ? o : m;
+  }
+  if constexpr (WAVES > 1) {
+    if ((t & 63) == 0) part[t >> 6] = m;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) m = part[w] > m ? part[w] : m;
+  }
+  const float amax = __builtin_bit_cast(float, m);
+  const float top = amax < p.min_scale ? p.min_scale : amax;     // (a NaN stays)
+  const float scale = top * p.inv_top;
+  const float inv = 1.0f / scale;
+  if (t == 0) p.scale[row] = scale;
+
+  uint8_t* qr = p.q + row * p.n;
+  auto put = [&](int64_t c, const row_chunk<XT>& x) {
+    const int64_t left = p.n - c * 8;
+    if (left <= 0) return;
+    const uint64_t w = row_codes<XT, OT>(x, inv);
+    if constexpr (VEC) {
+      *(uint64_t*)(qr + c * 8) = w;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) if (j < left) qr[c * 8 + j] = (uint8_t)(w >> (8 * j));
+    }
+  };
+  if constexpr (LOOP) {
+    for (int64_t c0 = 0; c0 < chunks; c0 += (int64_t)RT * CH) {
+#pragma unroll
+      for (int i = 0; i < CH; ++i) r[i] = row_load<XT, VEC>(xr, c0 + i * RT + t, p.n);
+#pragma unroll
+      for (int i = 0; i < CH; ++i) put(c0 + i * RT + t, r[i]);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < CH; ++i) put(i * RT + t, r[i]);
+  }
+}
+
+template <int XT, int OT, int RT, int CH, bool LOOP = false>
+static hipError_t row_quant_t(const RowQuantParams& p, hipStream_t stream) {
+  constexpr int ROWS = RT < 256 ? 256 / RT : 1;
+  constexpr int XB = XT == QT_F32 ? 4 : 2;
+  const int64_t grid = (p.m + ROWS - 1) / ROWS;
+  if (grid > INT32_MAX) return hipErrorInvalidValue;
+  const bool vec = p.n % 8 == 0 && ((uintptr_t)p.x & 15) == 0 && (p.x_stride * XB) % 16 == 0 && ((uintptr_t)p.q & 7) == 0;
+  const dim3 block(RT < 256 ? 256 : RT);
+  if (vec) hipLaunchKernelGGL((row_quant_kernel<XT, OT, RT, CH, true, LOOP>), dim3((unsigned)grid), block, 0, stream, p);
+  else hipLaunchKernelGGL((row_quant_kernel<XT, OT, RT, CH, false, LOOP>), dim3((unsigned)grid), block, 0, stream, p);
+  return hipGetLastError();
+}
+
+template <int XT, int OT>
+static hipError_t row_quant_o(const RowQuantParams& p, hipStream_t stream) {
+  const int64_t chunks = (p.n + 7) / 8;
+  // (a wave per row only where the rows alone fill the device: 256 CUs x 8 waves)
+  if (chunks <= 64 * 2 && p.m >= 2048) return row_quant_t<XT, OT, 64, 2>(p, stream);
+  if (chunks <= 64 * 8 && p.m >= 2048) return row_quant_t<XT, OT, 64, 8>(p, stream);
+  if (chunks <= 256 * 2) return row_quant_t<XT, OT, 256, 2>(p, stream);
+  if (chunks <= 256 * 8 && p.m >= 256) return row_quant_t<XT, OT, 256, 8>(p, stream);
+  if (chunks <= 1024 * 4) return row_quant_t<XT, OT, 1024, 4>(p, stream);
+  if (chunks <= 1024 * 8) return row_quant_t<XT, OT, 1024, 8>(p, stream);
+  return row_quant_t<XT, OT, 1024, 4, true>(p, stream);
+}
+
+template <int XT>
+static hipError_t row_quant_x(const RowQuantParams& p, int q_type, hipStream_t stream) {
+  if (q_type == RQ_E4M3) return row_quant_o<XT, RQ_E4M3>(p, stream);
+  if (q_type == RQ_E5M2) return row_quant_o<XT, RQ_E5M2>(p, stream);
+  return row_quant_o<XT, RQ_I8>(p, stream);
+}
+
+hipError_t launch_row_quant(const RowQuantParams& p, int x_type, int q_type, hipStream_t stream) {
+  if (x_type == QT_BF16) return row_quant_x<QT_BF16>(p, q_type, stream);
+  if (x_type == QT_F16) return row_quant_x<QT_F16>(p, q_type, stream);
+  return row_quant_x<QT_F32>(p, q_type, stream);
 }
 
 }  // namespace tb

@@ -1084,4 +1084,23 @@ int tb_hadamard_mxfp4_quant(const tb_quant_desc* d, void* stream) {
   return TB_OK;
 }
 
+int tb_quantize_rows(const tb_row_quant_desc* d, void* stream) {
+  if (!d) return TB_ERR_NULL_POINTER;
+  if (d->struct_bytes != sizeof(tb_row_quant_desc)) return TB_ERR_BAD_ARGUMENT;
+  if (!d->x || !d->q || !d->scale) return TB_ERR_NULL_POINTER;
+  if (d->m <= 0 || d->n <= 0) return TB_ERR_BAD_SHAPE;
+  if (d->x_type != TB_F16 && d->x_type != TB_BF16 && d->x_type != TB_F32) return TB_ERR_BAD_DTYPE;
+  float top;
+  if (d->q_type == TB_FP8_E4M3) top = 448.f;
+  else if (d->q_type == TB_FP8_E5M2) top = 57344.f;
+  else if (d->q_type == TB_I8) top = 127.f;
+  else return TB_ERR_BAD_DTYPE;
+  if (((uintptr_t)d->x & (d->x_type == TB_F32 ? 3 : 1)) || ((uintptr_t)d->scale & 3)) return TB_ERR_BAD_LAYOUT;
+  RowQuantParams p;
+  p.x = (const uint8_t*)d->x; p.q = (uint8_t*)d->q; p.scale = d->scale;
+  p.m = d->m; p.n = d->n; p.x_stride = d->x_stride_m; p.inv_top = 1.0f / top; p.min_scale = d->min_scale;
+  if (launch_row_quant(p, d->x_type, d->q_type, (hipStream_t)stream) != hipSuccess) { (void)hipGetLastError(); return TB_ERR_LAUNCH; }
+  return TB_OK;
+}
+
 }  // extern "C"

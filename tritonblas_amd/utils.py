@@ -16,13 +16,65 @@ def get_fp8_dtypes():
     return torch.float8_e4m3fn, torch.float8_e5m2
 
 
+def _plain(t: torch.Tensor) -> bool:
+    """True where a kernel may read the tensor's memory behind torch's back: a real GPU tensor that nothing is recording
+    (autograd in either direction, functorch transforms, torch.compile and jit tracing, dispatch or function modes)."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.layout == torch.strided and not t.is_neg()
+            and not (t.requires_grad and torch.is_grad_enabled())
+            and torch.autograd.forward_ad._current_level < 0
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing())
+
+
+def _rows(t: torch.Tensor, axis: int):
+    """(m, n, row stride) when ``axis`` runs along adjacent elements and the other axes are equally spaced rows, in order."""
+    axis = axis % t.ndim
+    n = t.shape[axis]
+    if t.ndim == 2:
+        m, stride = t.shape[1 - axis], t.stride(1 - axis)
+    else:
+        if axis != t.ndim - 1 or not t.is_contiguous():
+            return None
+        m, stride = t.numel() // n, n
+    if n > 1 and t.stride(axis) != 1:
+        return None
+    return (m, n, stride) if m == 1 or stride >= n else None
+
+
+def _quantize_rows(t, target_dtype, axis, min_scale, rows):
+    m, n, stride = rows
+    scale_shape = [d for i, d in enumerate(t.shape) if i != axis % t.ndim]
+    if axis % t.ndim == t.ndim - 1:
+        q = torch.empty(t.shape, dtype=target_dtype, device=t.device)
+    else:       # the columns of a matrix that is stored transposed: so are the codes
+        q = torch.empty((m, n), dtype=target_dtype, device=t.device).T
+    scale = torch.empty(scale_shape, dtype=torch.float32, device=t.device)
+    d = _lib.tb_row_quant_desc()
+    d.struct_bytes = C.sizeof(_lib.tb_row_quant_desc)
+    d.x_type, d.q_type, d.min_scale = _lib.tb_dtype(t.dtype), _lib.tb_dtype(target_dtype), min_scale
+    d.m, d.n, d.x, d.x_stride_m = m, n, t.data_ptr(), stride
+    d.q, d.scale = q.data_ptr(), scale.data_ptr()
+    with torch.cuda.device(t.device):
+        _lib.check(_lib.load().tb_quantize_rows(d, _lib.stream_handle(t.device)), "tb_quantize_rows")
+    return q, scale
+
+
 def quantize_tensor_per_channel(tensor: torch.Tensor, target_dtype: torch.dtype, axis: int, *,
                                 min_scale: float = 1e-8) -> Tuple[torch.Tensor, torch.Tensor]:
     """amax along ``axis`` -> scale = amax / dtype_max -> q = (x * (1/scale)).to(dtype); returns
     (q, scale squeezed along axis, fp32).  int8: dtype_max = 127, q rounded to nearest and clamped
-    to [-127, 127] first.  Reference utils.py:340-377."""
+    to [-127, 127] first.  Reference utils.py:340-377.
+
+    One kernel where ``axis`` is the contiguous one of a GPU tensor that nothing records; the tensor operations below give the
+    same codes and scales bit for bit everywhere else."""
     if target_dtype not in (torch.float8_e4m3fn, torch.float8_e5m2, torch.int8):
         raise ValueError(f"Unsupported quantized dtype: {target_dtype}")
+    if tensor.ndim >= 2 and -tensor.ndim <= axis < tensor.ndim and tensor.dtype in (torch.bfloat16, torch.float16, torch.float32) \
+            and tensor.numel() and _plain(tensor):
+        rows = _rows(tensor, axis)
+        if rows is not None:
+            return _quantize_rows(tensor, target_dtype, axis, min_scale, rows)
     base = tensor.to(torch.float32)
     max_abs = torch.clamp(base.abs().amax(dim=axis, keepdim=True), min=min_scale)
     dtype_max = 127.0 if target_dtype == torch.int8 else torch.finfo(target_dtype).max
