@@ -1,0 +1,41 @@
+"""The tile kernels on every storage order of their operands, against the product in 64 bits: sizes at the edges of the tiles and of
+the 16-byte copies, and few enough tiles or many enough for each depth of the copy pipeline.
+
+Tolerances: half a unit in the last place of the result's type per element bounds the rounding (in the 2-norm at most eps / 2), and
+single-precision sums of k terms add about sqrt(k) * 2**-24; twice that sum is allowed."""
+import math
+
+import pytest
+import torch
+
+import tritonblas_amd as tb
+
+pytestmark = pytest.mark.gpu
+
+
+def _stored(gen, rows, cols, order, dtype):
+    x = torch.randn((rows, cols) if order == "T" else (cols, rows), device="cuda", generator=gen).to(dtype)
+    return x if order == "T" else x.T
+
+
+def _check(c, a, b):
+    want = a.double() @ b.double()
+    tol = 2 * (torch.finfo(c.dtype).eps / 2 + math.sqrt(a.shape[1]) * 2.0 ** -24)
+    err = ((c.double() - want).norm() / want.norm()).item()
+    assert err <= tol, f"relative error {err:.3e} > {tol:.3e}"
+
+
+@pytest.mark.parametrize("ta,tb_", [("T", "T"), ("T", "N"), ("N", "T"), ("N", "N")])
+@pytest.mark.parametrize("dtype,tile", [(d, t) for d in (torch.bfloat16, torch.float16, torch.float32) for t in ((256, 256), (128, 128), (64, 64))] +
+                         [(torch.bfloat16, (32, 128)), (torch.float16, (32, 128))])
+def test_every_tile_and_storage_order(dtype, tile, ta, tb_):
+    bk = (256 if tile[0] == 32 else 128) // dtype.itemsize
+    gen = torch.Generator(device="cuda").manual_seed(tile[0])
+    # one K step, fewer than the pipeline is deep, more; one row chunk, a tile and a chunk, several tiles
+    for m, n, k in [(8, 8, bk), (tile[0] + 8, tile[1] - 8, 3 * bk), (2 * tile[0] - 16, 3 * tile[1] + 24, 7 * bk), (1544, 1536, 2 * bk)]:
+        a, b = _stored(gen, m, k, ta, dtype), _stored(gen, k, n, tb_, dtype)
+        c = torch.full((m, n), float("nan"), dtype=dtype, device="cuda")
+        sel = tb.OrigamiMatmulSelector(m, n, k, dtype, dtype, dtype, a.device)
+        sel._sel.block_m, sel._sel.block_n, sel._sel.block_k = tile[0], tile[1], bk
+        tb.matmul_lt(a, b, c, sel, tb.matmul_preamble(sel))
+        _check(c, a, b)

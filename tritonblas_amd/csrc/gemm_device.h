@@ -2,9 +2,10 @@
 // fused scale/bias/cast epilogue, and the four tile schedules (data-parallel, work-stealing queues,
 // Stream-K with partial-tile fixup, grouped expert table).
 //
-// One kernel template covers every element type: operands are moved as 16-byte "chunks" along K,
-// both operands sit K-major in LDS, and only the MFMA instruction and the chunk->lane assignment
-// depend on the type.
+// One kernel template covers every element type: operands are moved as 16-byte "chunks" along their
+// contiguous index and sit in LDS the way they sit in memory (rows of K, or for 16- and 32-bit types
+// K rows of the other index); only the MFMA instruction, the chunk->lane assignment and how a
+// fragment is read from LDS depend on type and layout.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -17,6 +18,7 @@ typedef int v8i __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef short s4 __attribute__((ext_vector_type(4)));
 
 enum : int { DT_F16 = 0, DT_BF16 = 1, DT_FP8 = 2, DT_FP4 = 3, DT_F32 = 4, DT_I8 = 5, DT_E5M2 = 6,
              DT_E4E5 = 7,    // A in e4m3, B in e5m2 (operand types only; never an output type)
@@ -113,7 +115,7 @@ struct TileCtx {
 };
 
 template <int DT_, int BM_, int BN_, int BKB_, int WM_, int WN_, int ALAY_, int BLAY_, int MINB_ = 1,
-          bool FAST_ = true, int STAGES_ = 2, bool USE_DMA_ = true>
+          bool FAST_ = true, int STAGES_ = 2>
 struct Tile {
   static constexpr int DT = DT_, BM = BM_, BN = BN_, BKB = BKB_, WM = WM_, WN = WN_;
   static constexpr int ALAY = ALAY_, BLAY = BLAY_, MINB = MINB_, STAGES = STAGES_;
@@ -121,7 +123,7 @@ struct Tile {
   // of the K step (and row counts of M-contiguous operands multiples of 8): loaders carry no
   // bounds handling besides clamping rows.  !FAST: element-wise gathers, any strides, any K.
   static constexpr bool FAST = FAST_;
-  static constexpr bool DMA = USE_DMA_ && FAST && ALAY == LAY_K && BLAY == LAY_K;  // global -> LDS without registers
+  static constexpr bool DMA = FAST;                                    // global -> LDS without registers
   static constexpr int THREADS = WM * WN * 64;
   static constexpr int USZ = (DT == DT_F16 || DT == DT_BF16) ? 2 : (DT == DT_F32 ? 4 : 1);  // bytes per storage unit
   static constexpr int UPC = 16 / USZ;                                 // units per 16-byte chunk
@@ -265,24 +267,42 @@ __device__ __forceinline__ v4i gather_units(const uint8_t* rowp, int64_t ku, int
   return out;
 }
 
-// LDS image of an operand tile: ROWS rows of CPR chunks; chunk c of row r sits at chunk slot
-// r*CPR + (c ^ swz(r)).  Slot q is filled by thread q % THREADS in round q / THREADS, so a wave
-// always fills 64 consecutive slots (what the LDS-direct load requires).
+// LDS image of an operand tile.
+//   LAY_K: ROWS rows of CPR chunks; chunk c of row r sits at chunk slot r*CPR + (c ^ swz(r)).
+//   LAY_M: UPS rows of one k each, MCPR chunks of consecutive tile rows; chunk c of k row k sits at slot
+//   k*MCPR + (c ^ mswz(k)).  The matrix is copied as it lies in memory and transposed where the fragments
+//   are read (ds_read_b64_tr_b16 for 16-bit types, one dword per value for fp32): the transpose costs no
+//   vector instruction and no register.  (The loader it replaces moved 8x8 blocks through registers and
+//   transposed them with vector instructions: 4096x14336x4096 bf16, B M-contiguous, 507 -> 350 us, 1024^3 fp16
+//   17.2 -> 9.5 us; fp32 had the element-wise gather kernel, 2048^3 304 -> 160 us.)
+// Slot q is filled by thread q % THREADS in round q / THREADS, so a wave always fills 64 consecutive
+// slots (what the LDS-direct load requires).
 template <class T, int ROWS, int LAY>
 struct Operand {
   static constexpr int CHUNKS = ROWS * T::CPR;
   static constexpr int NCH = (CHUNKS + T::THREADS - 1) / T::THREADS;  // slots per thread
-  static constexpr int RG = ROWS / 8;                                  // 8-row groups (LAY_M)
-  static constexpr int NBLK = RG * T::CPR;                             // 8x8 blocks (LAY_M)
-  static constexpr int NBT = (NBLK + T::THREADS - 1) / T::THREADS;
-  static constexpr bool TRANSPOSING = T::FAST && LAY == LAY_M;
-  static constexpr int NREG = TRANSPOSING ? NBT * 8 : NCH;
-  static constexpr int NOFF = TRANSPOSING ? NBT : NCH;
-  static_assert(!TRANSPOSING || T::USZ == 2, "transposing loader is for 16-bit operands");
+  static constexpr bool MROWS = T::FAST && LAY == LAY_M;
+  static constexpr int MCPR = ROWS * T::USZ / 16;                      // chunks per k row (LAY_M)
+  static constexpr int MPITCH = ROWS * T::USZ;                         // bytes per k row
+  static constexpr int KPL = T::USZ == 2 ? 8 : 4;                      // k values a lane takes per MFMA slice
+  static_assert(!MROWS || T::USZ == 2 || T::USZ == 4, "M-contiguous operands: 16- and 32-bit types");
+  static_assert(!MROWS || (MPITCH % 64 == 0 && (T::USZ == 2 || MPITCH >= 256)), "swizzle of the k rows");
+
+  // XOR mask on the chunk index of k row k.  One fragment read touches, per 16 lanes, 32 bytes of four
+  // adjacent k rows (16-bit types), or 64 bytes of one k row (fp32), and the four 16-lane groups sit
+  // KPL * KSUB k rows apart: the mask spreads the rows of a read over all banks.
+  __device__ static __forceinline__ int mswz(int k) {
+    const int g = k / (KPL * T::KSUB);            // the 16-lane group that reads this row
+    if constexpr (T::USZ == 4) return 4 * (g & 3);
+    const int gx = (g ^ (g >> 1)) & 1;
+    if constexpr (MPITCH >= 256) return 2 * ((k & 3) | (gx << 2));
+    else if constexpr (MPITCH == 128) return 2 * ((k & 3) ^ gx);
+    else return 2 * (((k >> 1) & 1) ^ gx);
+  }
 
   struct St {
     const uint8_t* base;     // FAST: tile origin; else matrix origin
-    uint32_t off[NOFF];      // FAST: per-slot byte offset from the K-step origin
+    uint32_t off[NCH];       // FAST: per-slot byte offset from the K-step origin
     int64_t s_row, s_k;      // storage units
     int row0, row_lim;
   };
@@ -304,13 +324,14 @@ struct Operand {
         st.off[i] = (uint32_t)(rowc * (int)(s_row * T::USZ) + c * 16);
       }
     } else {
-      st.base = mat + (int64_t)row0 * 2;
-      const int last = ((rows_valid - 1) / 8) * 8;
+      st.base = mat + (int64_t)row0 * T::USZ;
+      const int last = (rows_valid - 1) / T::UPC;      // (row counts are multiples of a chunk)
 #pragma unroll
-      for (int ib = 0; ib < NBT; ++ib) {
-        int b = ib * T::THREADS + tid;
-        int rg = b % RG, c = b / RG;
-        st.off[ib] = (uint32_t)(min(rg * 8, last) * 2 + c * 8 * (int)(s_k * 2));
+      for (int i = 0; i < NCH; ++i) {
+        int q = i * T::THREADS + tid;
+        int k = q / MCPR, pc = q % MCPR;
+        int c = pc ^ mswz(k);
+        st.off[i] = (uint32_t)(min(c, last) * 16 + k * (int)(s_k * T::USZ));
       }
     }
   }
@@ -319,7 +340,7 @@ struct Operand {
   __device__ static __forceinline__ const uint8_t* step_ptr(const St& st, int it) {
     if constexpr (!T::FAST) return st.base;
     else if constexpr (LAY == LAY_K) return st.base + (int64_t)it * T::BKB;
-    else return st.base + (int64_t)it * T::UPS * st.s_k * 2;
+    else return st.base + (int64_t)it * T::UPS * st.s_k * T::USZ;
   }
 
   // LDS-direct copy of K step `it` into `lds` (no registers involved).  Written as inline assembly
@@ -344,72 +365,25 @@ struct Operand {
     }
   }
 
-  __device__ static __forceinline__ void gload(v4i (&r)[NREG], const St& st, int it, int64_t KU, int tid) {
-    const uint8_t* gp = step_ptr(st, it);
-    if constexpr (!T::FAST) {
-      const int64_t ku0 = (int64_t)it * T::UPS;
+  __device__ static __forceinline__ void gload(v4i (&r)[NCH], const St& st, int it, int64_t KU, int tid) {
+    const int64_t ku0 = (int64_t)it * T::UPS;
 #pragma unroll
-      for (int i = 0; i < NCH; ++i) {
-        int q = i * T::THREADS + tid;
-        if (CHUNKS % T::THREADS != 0 && q >= CHUNKS) continue;
-        int row = q / T::CPR, pc = q % T::CPR;
-        int c = pc ^ T::swz(row);
-        int64_t grow = min(st.row0 + row, st.row_lim - 1);
-        r[i] = gather_units<T>(gp + grow * st.s_row * T::USZ, ku0 + (int64_t)c * T::UPC, st.s_k, KU);
-      }
-    } else if constexpr (LAY == LAY_K) {
-#pragma unroll
-      for (int i = 0; i < NCH; ++i) {
-        if (CHUNKS % T::THREADS != 0 && i * T::THREADS + tid >= CHUNKS) continue;
-        r[i] = *(const v4i*)(gp + st.off[i]);
-      }
-    } else {
-      const int64_t ldk = st.s_k * 2;
-#pragma unroll
-      for (int ib = 0; ib < NBT; ++ib) {
-        if (NBLK % T::THREADS != 0 && ib * T::THREADS + tid >= NBLK) continue;
-        uint32_t w[8][4];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          v4i v = *(const v4i*)(gp + st.off[ib] + j * ldk);
-          w[j][0] = v.x; w[j][1] = v.y; w[j][2] = v.z; w[j][3] = v.w;
-        }
-        // 8x8 transpose of 16-bit values: out row i, dword d holds k = 2d (low half) and 2d+1 (high).
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          uint32_t o[4];
-#pragma unroll
-          for (int d = 0; d < 4; ++d) {
-            uint32_t lo = w[2 * d][i >> 1], hi = w[2 * d + 1][i >> 1];
-            o[d] = (i & 1) ? ((lo >> 16) | (hi & 0xffff0000u)) : ((lo & 0xffffu) | (hi << 16));
-          }
-          v4i ov = {(int)o[0], (int)o[1], (int)o[2], (int)o[3]};
-          r[ib * 8 + i] = ov;
-        }
-      }
+    for (int i = 0; i < NCH; ++i) {
+      int q = i * T::THREADS + tid;
+      if (CHUNKS % T::THREADS != 0 && q >= CHUNKS) continue;
+      int row = q / T::CPR, pc = q % T::CPR;
+      int c = pc ^ T::swz(row);
+      int64_t grow = min(st.row0 + row, st.row_lim - 1);
+      r[i] = gather_units<T>(st.base + grow * st.s_row * T::USZ, ku0 + (int64_t)c * T::UPC, st.s_k, KU);
     }
   }
 
-  __device__ static __forceinline__ void sstore(uint8_t* lds, const v4i (&r)[NREG], int tid) {
-    if constexpr (!TRANSPOSING) {
+  __device__ static __forceinline__ void sstore(uint8_t* lds, const v4i (&r)[NCH], int tid) {
 #pragma unroll
-      for (int i = 0; i < NCH; ++i) {
-        int q = i * T::THREADS + tid;
-        if (CHUNKS % T::THREADS != 0 && q >= CHUNKS) continue;
-        *(v4i*)(lds + q * 16) = r[i];
-      }
-    } else {
-#pragma unroll
-      for (int ib = 0; ib < NBT; ++ib) {
-        int b = ib * T::THREADS + tid;
-        if (NBLK % T::THREADS != 0 && b >= NBLK) continue;
-        int rg = b % RG, c = b / RG;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          int row = rg * 8 + i;
-          *(v4i*)(lds + row * T::BKB + ((c ^ T::swz(row)) << 4)) = r[ib * 8 + i];
-        }
-      }
+    for (int i = 0; i < NCH; ++i) {
+      int q = i * T::THREADS + tid;
+      if (CHUNKS % T::THREADS != 0 && q >= CHUNKS) continue;
+      *(v4i*)(lds + q * 16) = r[i];
     }
   }
 };
@@ -420,6 +394,26 @@ struct Operand {
 template <class T>
 struct Frag {
   using type = typename std::conditional<is_f8(T::DT), v8i, v4i>::type;
+
+  // M-contiguous operand O: the 16 tile rows from row16 on, MFMA slice ks.  The same k values in the same
+  // places of the register as read() gives (lane group g owns KPL * KSUB consecutive k).  16-bit types: within 16
+  // lanes, lane i names the 8 bytes of tile rows 4 (i % 4) .. +3 of k row i / 4; after the transposing read it
+  // holds the four k values of tile row i.
+  template <class O>
+  __device__ static __forceinline__ type read_m(const uint8_t* lds, int row16, int ks, const LaneInfo& li) {
+    const int k0 = li.g * O::KPL * T::KSUB;
+    if constexpr (T::USZ == 2) {
+      const int k = k0 + (li.r >> 2);
+      const uint8_t* rp = lds + k * O::MPITCH + (((row16 / 8 + ((li.r >> 1) & 1)) ^ O::mswz(k)) << 4) + (li.r & 1) * 8 + ks * 8 * O::MPITCH;
+      typedef __attribute__((address_space(3))) s4* tr_ptr;
+      const s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)rp);
+      const s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr_ptr)(rp + 4 * O::MPITCH));
+      return __builtin_bit_cast(v4i, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    } else {
+      const uint8_t* rp = lds + (k0 + ks * 4) * O::MPITCH + (((row16 / 4 + (li.r >> 2)) ^ O::mswz(k0)) << 4) + (li.r & 3) * 4;
+      return v4i{*(const int*)rp, *(const int*)(rp + O::MPITCH), *(const int*)(rp + 2 * O::MPITCH), *(const int*)(rp + 3 * O::MPITCH)};
+    }
+  }
 
   // row: tile row of this lane (wave row base + 16*t + lane%16); g = lane/16; m = swizzle mask of row.
   __device__ static __forceinline__ type read(const uint8_t* lds, int row, int ks, int g, int m) {
@@ -660,9 +654,17 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
     // and the matrix pipe has that row block to chew on while they arrive.
     frag_t bf[T::TN];
     frag_t afn;
-    auto request_b = [&](const uint8_t* sB, int ks, int j) { bf[j] = Frag<T>::read(sB, li.wn0 + j * 16 + li.r, ks, li.g, swm); };
-    auto request_a = [&](const uint8_t* sA, int ks, int i) { return Frag<T>::read(sA, li.wm0 + i * 16 + li.r, ks, li.g, swm); };
-    constexpr int RPF = is_f8(T::DT) ? 2 : 1;  // LDS reads per fragment
+    auto request_b = [&](const uint8_t* sB, int ks, int j) {
+      if constexpr (OB::MROWS) bf[j] = Frag<T>::template read_m<OB>(sB, li.wn0 + j * 16, ks, li);
+      else bf[j] = Frag<T>::read(sB, li.wn0 + j * 16 + li.r, ks, li.g, swm);
+    };
+    auto request_a = [&](const uint8_t* sA, int ks, int i) {
+      if constexpr (OA::MROWS) return Frag<T>::template read_m<OA>(sA, li.wm0 + i * 16, ks, li);
+      else return Frag<T>::read(sA, li.wm0 + i * 16 + li.r, ks, li.g, swm);
+    };
+    constexpr int RPM = T::USZ == 2 ? 2 : 4;                               // LDS reads per fragment of an M-contiguous operand,
+    constexpr int RPFA = OA::MROWS ? RPM : (is_f8(T::DT) ? 2 : 1);         // of A
+    constexpr int RPFB = OB::MROWS ? RPM : (is_f8(T::DT) ? 2 : 1);         // and of B
 
     // one block: slice KSV of the K step in stage (sA, sB).  `boundary` runs before the last row block;
     // afterwards the fragments of slice nks of stage (nA, nB) are requested.  After the last step of
@@ -682,8 +684,8 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
           // a scheduling region): one fragment request (plus a scale read), then one row block of MFMAs
 #pragma unroll
           for (int q = 0; q + 1 < T::TM; ++q) {
-            if (LAST && q >= 1) __builtin_amdgcn_sched_group_barrier(0x100, RPF + 1, 0);
-            else __builtin_amdgcn_sched_group_barrier(0x100, RPF, 0);
+            if (LAST && q >= 1) __builtin_amdgcn_sched_group_barrier(0x100, RPFA + 1, 0);
+            else __builtin_amdgcn_sched_group_barrier(0x100, RPFA, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, T::TN, 0);
           }
           if constexpr (LAST) {
@@ -715,13 +717,13 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
         }
       }
       // last row block: the next A fragment, then MFMAs and B fragment (and scale) requests alternate
-      __builtin_amdgcn_sched_group_barrier(0x100, RPF, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, RPFA, 0);
 #pragma unroll
       for (int j = 0; j < T::TN; ++j) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (LAST && j == 0) __builtin_amdgcn_sched_group_barrier(0x100, RPF + 2, 0);
-        else if (LAST) __builtin_amdgcn_sched_group_barrier(0x100, RPF + 1, 0);
-        else __builtin_amdgcn_sched_group_barrier(0x100, RPF, 0);
+        if (LAST && j == 0) __builtin_amdgcn_sched_group_barrier(0x100, RPFB + 2, 0);
+        else if (LAST) __builtin_amdgcn_sched_group_barrier(0x100, RPFB + 1, 0);
+        else __builtin_amdgcn_sched_group_barrier(0x100, RPFB, 0);
       }
       if constexpr (MXG && !LAST) {
         // (same reason as above: keeps this slice's last row block in front of the next slice)
@@ -792,7 +794,7 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
     };
     for (int it = it0; it < it1; ++it) kstep(it);
   } else {
-    v4i ra[OA::NREG], rb[OB::NREG];
+    v4i ra[OA::NCH], rb[OB::NCH];
     uint8_t* sA0 = lds;
     uint8_t* sB0 = lds + T::A_BYTES;
     OA::gload(ra, sa, it0, p.KU, li.tid);

@@ -4,27 +4,24 @@
 
 namespace tb {
 
-#define TB_LAYOUTS(BM, BN, WM, WN, MINB)                                              \
-  make_variant<Tile<DT_BF16, BM, BN, 128, WM, WN, LAY_K, LAY_K, MINB, true, 2>>(),      \
-  make_variant<Tile<DT_BF16, BM, BN, 128, WM, WN, LAY_K, LAY_M, MINB, true, 2>>(),      \
-  make_variant<Tile<DT_BF16, BM, BN, 128, WM, WN, LAY_M, LAY_K, MINB, true, 2>>(),      \
-  make_variant<Tile<DT_BF16, BM, BN, 128, WM, WN, LAY_M, LAY_M, MINB, true, 2>>()
+#define TB_LAYOUTS(BM, BN, BK, WM, WN, MINB, STAGES)                                    \
+  make_variant<Tile<DT_BF16, BM, BN, BK, WM, WN, LAY_K, LAY_K, MINB, true, STAGES>>(),   \
+  make_variant<Tile<DT_BF16, BM, BN, BK, WM, WN, LAY_K, LAY_M, MINB, true, STAGES>>(),   \
+  make_variant<Tile<DT_BF16, BM, BN, BK, WM, WN, LAY_M, LAY_K, MINB, true, STAGES>>(),   \
+  make_variant<Tile<DT_BF16, BM, BN, BK, WM, WN, LAY_M, LAY_M, MINB, true, STAGES>>()
 
 const Variant g_variants_bf16[] = {
     // hand-scheduled 4-wave kernel (K-major operands): taken when K is a multiple of two K steps and no Stream-K tail is asked for
     make_variant_w4<W4Tile<DT_BF16>>(),
-    TB_LAYOUTS(256, 256, 2, 4, 1),
-    TB_LAYOUTS(128, 128, 2, 2, 2),
-    TB_LAYOUTS(64, 64, 2, 2, 4),
+    TB_LAYOUTS(256, 256, 128, 2, 4, 1, 2),
+    TB_LAYOUTS(128, 128, 128, 2, 2, 2, 2),
+    TB_LAYOUTS(64, 64, 128, 2, 2, 4, 2),
     // deeper copy pipelines of the small tile for problems with few tiles per CU (each K step then
     // waits less for its copy; fewer workgroups fit a CU)
-    make_variant<Tile<DT_BF16, 64, 64, 128, 2, 2, LAY_K, LAY_K, 3, true, 3>>(),
-    make_variant<Tile<DT_BF16, 64, 64, 128, 2, 2, LAY_K, LAY_K, 2, true, 4>>(),
+    TB_LAYOUTS(64, 64, 128, 2, 2, 3, 3),
+    TB_LAYOUTS(64, 64, 128, 2, 2, 2, 4),
     // a handful of rows against a long K: short, wide, deep tile with three copy stages
-    make_variant<Tile<DT_BF16, 32, 128, 256, 1, 4, LAY_K, LAY_K, 1, true, 3>>(),
-    make_variant<Tile<DT_BF16, 32, 128, 256, 1, 4, LAY_K, LAY_M, 1, true, 2>>(),
-    make_variant<Tile<DT_BF16, 32, 128, 256, 1, 4, LAY_M, LAY_K, 1, true, 2>>(),
-    make_variant<Tile<DT_BF16, 32, 128, 256, 1, 4, LAY_M, LAY_M, 1, true, 2>>(),
+    TB_LAYOUTS(32, 128, 256, 1, 4, 1, 3),
     make_variant<Tile<DT_BF16, 64, 64, 128, 2, 2, LAY_K, LAY_K, 2, false, 2>>(),
 };
 const int g_num_variants_bf16 = sizeof(g_variants_bf16) / sizeof(Variant);

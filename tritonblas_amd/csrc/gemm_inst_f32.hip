@@ -1,14 +1,20 @@
 // fp32 tile GEMM kernels (v_mfma_f32_16x16x4_f32: full fp32 products and sums; this target has no
-// reduced-precision fp32 matrix mode).  K-contiguous operands take the LDS-direct kernels; every
-// other layout goes through the element-wise-gather kernel.
+// reduced-precision fp32 matrix mode) for the four operand layout combinations, plus one
+// element-wise-gather kernel for operands the vector loaders cannot address.
 #include "gemm_variants.h"
 
 namespace tb {
 
+#define TB_LAYOUTS(BM, BN, WM, WN, MINB)                                       \
+  make_variant<Tile<DT_F32, BM, BN, 128, WM, WN, LAY_K, LAY_K, MINB, true, 2>>(),   \
+  make_variant<Tile<DT_F32, BM, BN, 128, WM, WN, LAY_K, LAY_M, MINB, true, 2>>(),   \
+  make_variant<Tile<DT_F32, BM, BN, 128, WM, WN, LAY_M, LAY_K, MINB, true, 2>>(),   \
+  make_variant<Tile<DT_F32, BM, BN, 128, WM, WN, LAY_M, LAY_M, MINB, true, 2>>()
+
 const Variant g_variants_f32[] = {
-    make_variant<Tile<DT_F32, 256, 256, 128, 2, 4, LAY_K, LAY_K, 1, true, 2>>(),
-    make_variant<Tile<DT_F32, 128, 128, 128, 2, 2, LAY_K, LAY_K, 2, true, 2>>(),
-    make_variant<Tile<DT_F32, 64, 64, 128, 2, 2, LAY_K, LAY_K, 4, true, 2>>(),
+    TB_LAYOUTS(256, 256, 2, 4, 1),
+    TB_LAYOUTS(128, 128, 2, 2, 2),
+    TB_LAYOUTS(64, 64, 2, 2, 4),
     make_variant<Tile<DT_F32, 64, 64, 128, 2, 2, LAY_K, LAY_K, 2, false, 2>>(),
 };
 const int g_num_variants_f32 = sizeof(g_variants_f32) / sizeof(Variant);
