@@ -39,3 +39,25 @@ def test_every_tile_and_storage_order(dtype, tile, ta, tb_):
         sel._sel.block_m, sel._sel.block_n, sel._sel.block_k = tile[0], tile[1], bk
         tb.matmul_lt(a, b, c, sel, tb.matmul_preamble(sel))
         _check(c, a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(64, 72, 80), (65, 72, 83), (40, 77, 64), (1, 8, 8)])
+@pytest.mark.parametrize("view", ["rows", "transposed", "offset", "strided"])
+def test_gradients_for_every_way_an_operand_is_stored(view, m, n, k, dtype):
+    gen = torch.Generator(device="cuda").manual_seed(m + n)
+
+    def operand(rows, cols):
+        if view == "transposed":
+            return _stored(gen, rows, cols, "N", dtype)
+        if view == "offset":
+            return _stored(gen, rows, cols + 3, "T", dtype)[:, 3:]
+        if view == "strided":
+            return _stored(gen, 2 * rows, 2 * cols, "T", dtype)[::2, ::2]
+        return _stored(gen, rows, cols, "T", dtype)
+
+    a, b, g = operand(m, k).requires_grad_(), operand(k, n).requires_grad_(), operand(m, n)
+    da, db = torch.autograd.grad(tb.matmul(a, b), (a, b), g)
+    assert da.shape == a.shape and db.shape == b.shape
+    _check(da, g, b.detach().T)
+    _check(db, a.detach().T, g)
