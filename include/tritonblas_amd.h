@@ -313,6 +313,23 @@ typedef struct tb_row_quant_desc {
 
 int tb_quantize_rows(const tb_row_quant_desc* desc, void* stream);
 
+/* ---- sums over the rows of a row-major matrix, formed in fp32 (a layer's bias gradient) ----------------------
+ *      partial: fp32 workspace of tb_column_sum_bytes(m, n) bytes (null when that is 0); contents need not be
+ *      set and are not kept                                                                                   */
+typedef struct tb_column_sum_desc {
+  uint32_t struct_bytes;
+  int32_t type;               /* TB_BF16, TB_F16 or TB_F32: of x and of out                          */
+  int64_t m, n;
+  const void* x;
+  int64_t x_stride_m;         /* elements; unit stride along n                                       */
+  void* out;                  /* (n)                                                                 */
+  float* partial;
+  size_t partial_bytes;
+} tb_column_sum_desc;
+
+size_t tb_column_sum_bytes(int64_t m, int64_t n);
+int tb_column_sum(const tb_column_sum_desc* desc, void* stream);
+
 /* ---- tile order ------------------------------------------------------------------------------
  * Host-side evaluation of the kernels' tile id -> (row block, column block) map, for tests and tools.
  * With panel_n = 0 it is the reference's GROUP_M swizzle (kernels/stages/schedule.py:124-145); with

@@ -27,6 +27,8 @@ EXPORTED_SYMBOLS = [
     "tb_abi_version", "tb_status_string", "tb_device_info", "tb_select", "tb_list_tiles", "tb_gemm",
     "tb_workspace_bytes", "tb_gemm_fp4", "tb_grouped_gemm_fp8", "tb_grouped_workspace_bytes", "tb_streamk_tail_tiles", "tb_hadamard_mxfp4_quant",
     "tb_quantize_rows",
+    "tb_column_sum",
+    "tb_column_sum_bytes",
     "tb_tile_coords", "tb_default_panel", "tb_ws_queue_tile", "tb_hierarchical_split",
     "tb_workspace_layout", "tb_debug_option", "tb_gemm_static_workspace", "tb_static_workspace_status", "tb_gemm_launch_info",
 ]
@@ -105,6 +107,11 @@ class tb_row_quant_desc(C.Structure):
                 ("scale", C.c_void_p)]
 
 
+class tb_column_sum_desc(C.Structure):
+    _fields_ = [("struct_bytes", C.c_uint32), ("type", C.c_int32), ("m", C.c_int64), ("n", C.c_int64), ("x", C.c_void_p),
+                ("x_stride_m", C.c_int64), ("out", C.c_void_p), ("partial", C.c_void_p), ("partial_bytes", C.c_size_t)]
+
+
 _lib = None
 
 
@@ -135,6 +142,9 @@ def load():
     lib.tb_streamk_tail_tiles.argtypes = [C.c_int32] * 5
     lib.tb_hadamard_mxfp4_quant.argtypes = [C.POINTER(tb_quant_desc), C.c_void_p]
     lib.tb_quantize_rows.argtypes = [C.POINTER(tb_row_quant_desc), C.c_void_p]
+    lib.tb_column_sum_bytes.argtypes = [C.c_int64, C.c_int64]
+    lib.tb_column_sum_bytes.restype = C.c_size_t
+    lib.tb_column_sum.argtypes = [C.POINTER(tb_column_sum_desc), C.c_void_p]
     lib.tb_tile_coords.argtypes = [C.c_int32] * 5 + [C.POINTER(C.c_int32), C.POINTER(C.c_int32)]
     lib.tb_default_panel.argtypes = [C.c_int32] * 3
     lib.tb_ws_queue_tile.argtypes = [C.c_int32] * 7 + [C.POINTER(C.c_int32)] * 2

@@ -11,6 +11,7 @@
 #include "gemm_variants.h"
 #include "quant.h"
 #include "skinny.h"
+#include "colsum.h"
 #include "selector.h"
 
 using namespace tb;
@@ -1100,6 +1101,34 @@ int tb_quantize_rows(const tb_row_quant_desc* d, void* stream) {
   p.x = (const uint8_t*)d->x; p.q = (uint8_t*)d->q; p.scale = d->scale;
   p.m = d->m; p.n = d->n; p.x_stride = d->x_stride_m; p.inv_top = 1.0f / top; p.min_scale = d->min_scale;
   if (launch_row_quant(p, d->x_type, d->q_type, (hipStream_t)stream) != hipSuccess) { (void)hipGetLastError(); return TB_ERR_LAUNCH; }
+  return TB_OK;
+}
+
+static int sum_parts(int64_t m, int64_t n) {
+  tb_hw hw;
+  if (current_hw(&hw) != TB_OK) default_hw(&hw);
+  return column_sum_parts(m, n, hw.n_cu);
+}
+
+size_t tb_column_sum_bytes(int64_t m, int64_t n) {
+  if (m <= 0 || n <= 0) return 0;
+  const int parts = sum_parts(m, n);
+  return parts > 1 ? (size_t)parts * (size_t)n * 4 : 0;
+}
+
+int tb_column_sum(const tb_column_sum_desc* d, void* stream) {
+  if (!d) return TB_ERR_NULL_POINTER;
+  if (d->struct_bytes != sizeof(tb_column_sum_desc)) return TB_ERR_BAD_ARGUMENT;
+  if (!d->x || !d->out) return TB_ERR_NULL_POINTER;
+  if (d->m <= 0 || d->n <= 0) return TB_ERR_BAD_SHAPE;
+  if (d->type != TB_F16 && d->type != TB_BF16 && d->type != TB_F32) return TB_ERR_BAD_DTYPE;
+  const uintptr_t esz = d->type == TB_F32 ? 4 : 2;
+  if ((uintptr_t)d->x % esz || (uintptr_t)d->out % esz) return TB_ERR_BAD_LAYOUT;
+  ColumnSumParams p;
+  p.x = (const uint8_t*)d->x; p.m = d->m; p.n = d->n; p.stride = d->x_stride_m; p.out = d->out; p.partial = d->partial;
+  p.parts = sum_parts(d->m, d->n);
+  if (p.parts > 1 && (!d->partial || d->partial_bytes < (size_t)p.parts * (size_t)d->n * 4 || ((uintptr_t)d->partial & 3))) return TB_ERR_WORKSPACE;
+  if (launch_column_sum(p, d->type, (hipStream_t)stream) != hipSuccess) { (void)hipGetLastError(); return TB_ERR_LAUNCH; }
   return TB_OK;
 }
 

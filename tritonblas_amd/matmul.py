@@ -300,6 +300,41 @@ def _(a, b, out, enable_streamk=False, sk_grid=None, work_stealing=False):
     return None
 
 
+@torch.library.custom_op("tritonblas_amd::_column_sum", mutates_args=())
+def _column_sum(x: torch.Tensor) -> torch.Tensor:
+    """``x.sum(dim=0)`` of a contiguous matrix, formed in fp32 (a bias gradient)."""
+    m, n = x.shape
+    if m == 0 or n == 0 or not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16, torch.float32):
+        return x.sum(dim=0)
+    out = x.new_empty(n)
+    lib = _lib.load()
+    with _on_device(x.device):
+        need = lib.tb_column_sum_bytes(m, n)
+        partial = torch.empty(need // 4, dtype=torch.float32, device=x.device)
+        d = _lib.tb_column_sum_desc()
+        d.struct_bytes = C.sizeof(_lib.tb_column_sum_desc)
+        d.type, d.m, d.n, d.x, d.x_stride_m = _lib.tb_dtype(x.dtype), m, n, x.data_ptr(), x.stride(0)
+        d.out, d.partial, d.partial_bytes = out.data_ptr(), partial.data_ptr() if need else None, need
+        _lib.check(lib.tb_column_sum(d, _lib.stream_handle(x.device)), "tb_column_sum")
+    return out
+
+
+@_column_sum.register_fake
+def _(x):
+    return x.new_empty(x.shape[1])
+
+
+def _column_sum_setup_context(ctx, inputs, output):
+    ctx.rows = inputs[0].shape[0]
+
+
+def _column_sum_backward(ctx, grad_output):
+    return grad_output.expand(ctx.rows, -1)
+
+
+_column_sum.register_autograd(_column_sum_backward, setup_context=_column_sum_setup_context)
+
+
 @torch.library.custom_op("tritonblas_amd::_addmm", mutates_args=())
 def _addmm(bias: torch.Tensor, a: torch.Tensor, b: torch.Tensor, enable_streamk: Optional[bool] = False,
            sk_grid: Optional[int] = None, work_stealing: Optional[bool] = False) -> torch.Tensor:
@@ -325,7 +360,7 @@ def _addmm_backward(ctx, grad_output):
     a, b = ctx.saved_tensors
     g = grad_output.contiguous()
     grad_a, grad_b = _product_gradients(a, b, g, ctx.opts)
-    return grad_output.sum(dim=0).reshape(ctx.bias_shape), grad_a, grad_b, None, None, None
+    return _column_sum(g).reshape(ctx.bias_shape), grad_a, grad_b, None, None, None
 
 
 _addmm.register_autograd(_addmm_backward, setup_context=_addmm_setup_context)
