@@ -61,3 +61,37 @@ def test_gradients_for_every_way_an_operand_is_stored(view, m, n, k, dtype):
     assert da.shape == a.shape and db.shape == b.shape
     _check(da, g, b.detach().T)
     _check(db, a.detach().T, g)
+
+
+def _poisoned(gen, rows, cols, order, dtype, pad):
+    """An operand whose rows (as stored) are followed by ``pad`` NaNs, for int8 by its largest value."""
+    r, c = (rows, cols) if order == "T" else (cols, rows)
+    x = torch.randint(-9, 9, (r, c + pad), device="cuda", generator=gen).float()
+    x[:, c:] = float("nan") if dtype != torch.int8 else 127
+    x = x.to(dtype)[:, :c]
+    return x if order == "T" else x.T
+
+
+@pytest.mark.parametrize("dtype,ta,tb_", [(d, "T", "N") for d in (torch.float8_e4m3fn, torch.float8_e5m2, torch.int8)] +
+                         [(d, x, y) for d in (torch.bfloat16, torch.float32) for x in "TN" for y in "TN"])
+@pytest.mark.parametrize("tile", [(256, 256), (128, 128), (64, 64)])
+@pytest.mark.parametrize("schedule", ["persistent", "streamk"])
+def test_k_that_is_no_multiple_of_the_k_step(schedule, tile, dtype, ta, tb_):
+    chunk = 16 // dtype.itemsize
+    out = torch.bfloat16 if dtype.itemsize == 1 else dtype
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    for m, n, k in [(16, 16, chunk), (tile[0] + 16, 2 * tile[1], 8 * chunk + chunk), (272, 304, 37 * chunk), (520, 512, 63 * chunk)]:
+        if (ta, tb_) == ("N", "T"):
+            k -= 1                     # K along neither operand's rows: any K
+        a, b = _poisoned(gen, m, k, ta, dtype, chunk), _poisoned(gen, k, n, tb_, dtype, chunk)
+        c = torch.full((m, n), float("nan"), dtype=out, device="cuda")
+        sel = tb.OrigamiMatmulSelector(m, n, k, dtype, dtype, out, a.device, streamk=schedule == "streamk")
+        sel._sel.block_m, sel._sel.block_n, sel._sel.block_k = tile[0], tile[1], 128 // dtype.itemsize
+        config = tb.matmul_preamble(sel)
+        if dtype.itemsize == 1:
+            one_m, one_n = torch.ones(m, device="cuda"), torch.ones(n, device="cuda")
+            tb.matmul_a8w8_lt(a, b, one_m, one_n, c, sel, config, enable_streamk=schedule == "streamk")
+        else:
+            tb.matmul_lt(a, b, c, sel, config, enable_streamk=schedule == "streamk")
+        # (whole numbers below 2**24: the sums are exact and only the result is rounded)
+        assert torch.equal(c, (a.double() @ b.double()).float().to(out)), (m, n, k)

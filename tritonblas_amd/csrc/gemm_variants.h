@@ -9,7 +9,7 @@ struct Variant {
   int dt, bm, bn, bk;     // element type and tile in elements
   int alay, blay;         // operand loaders (LAY_K / LAY_M)
   int wm, wn, threads, lds_bytes, minb;
-  int fast, stages;       // fast: vector/LDS-direct loaders (alignment + K multiple required)
+  int fast, stages;       // fast: vector/LDS-direct loaders (alignment required, whole 16-byte chunks)
   const void* kernel;     // __global__ void (*)(const GemmParams), whole-tile schedules
   const void* kernel_sk;  // same tile with the Stream-K tail (null: this variant has none)
   int k_step_pairs;       // 1: hand-scheduled 4-wave kernel -- K must be an even number of K steps, at least four; with a

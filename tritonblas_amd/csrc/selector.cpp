@@ -170,7 +170,7 @@ static double score(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bo
   const int area = v.bm * v.bn;
 
   const double ideal_step_us = 2.0 * v.bm * v.bn * v.bk / mfma_flops_per_clk(pr.a_type) / clk * 1e6;
-  const bool w4 = v.threads == 256 && area >= 256 * 256 && k_iters >= 4 && k_iters % 2 == 0;
+  const bool w4 = v.threads == 256 && area >= 256 * 256 && k_iters >= 4 && k_iters % 2 == 0 && pr.k % v.bk == 0;
   const double t_thru = ideal_step_us / family_efficiency(pr.a_type, v, w4);   // CU time per tile K step, saturated
   double t_lat = 0.30 + (v.bm + v.bn) * (v.bk * esz) / 1.0e5;                // floor per K step of one workgroup: round trip + its own copy at ~100 GB/s
   // the 64x64 tile of the 8- and 16-bit float types runs with four (three) copy stages while no more

@@ -297,7 +297,9 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
     bm = sel.block_m; bn = sel.block_n; bk = sel.block_k;
   }
   const Variant* v = nullptr;
-  bool fast = alay >= 0 && blay >= 0 && (KU % (bk / epu) == 0);
+  // a K-contiguous operand is copied in 16-byte chunks along K; the kernels fill up the last K step themselves, except
+  // for fp4, whose scales would have to be filled up too
+  bool fast = alay >= 0 && blay >= 0 && (j.dt == TB_FP4_E2M1 ? KU % (bk / epu) == 0 : (alay == LAY_M && blay == LAY_M) || KU % (16 / usz) == 0);
   if (j.dt == TB_FP4_E2M1) {
     // the fast fp4 kernels stage 16 scale bytes per row at a time through LDS with 16-byte copies
     const bool mx_ok = j.mxa_sk == 1 && j.mxb_sk == 1 && (j.K / 32) % 16 == 0 && j.mxa_sr % 16 == 0 && j.mxb_sr % 16 == 0 &&
