@@ -1,0 +1,44 @@
+"""Operands whose rows start anywhere (16-byte loads through registers): every storage order and tile at sizes around the tiles, the 16-byte
+chunks and the K steps, inside buffers whose other values are NaN.  Values are small whole numbers: the sums are exact."""
+import pytest
+import torch
+
+import tritonblas_amd as tb
+
+pytestmark = pytest.mark.gpu
+
+
+def _inside_nans(gen, rows, cols, order, dtype, pad, lead):
+    r, c = (rows, cols) if order == "T" else (cols, rows)
+    base = torch.full((r * (c + pad) + lead + 8,), float("nan"), device="cuda", dtype=dtype)
+    x = base[lead:lead + r * (c + pad)].view(r, c + pad)[:, :c]
+    x.copy_(torch.randint(-9, 9, (r, c), device="cuda", generator=gen))
+    return x if order == "T" else x.T
+
+
+SIZES = [(8, 8, 8), (9, 11, 13), (64, 65, 63), (129, 127, 65), (130, 70, 131), (71, 257, 200), (1187, 301, 153)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("ta,tb_", [("T", "T"), ("T", "N"), ("N", "T"), ("N", "N")])
+@pytest.mark.parametrize("pad,lead", [(0, 0), (3, 1), (8, 5)])
+def test_any_alignment(pad, lead, ta, tb_, dtype):
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    for m, n, k in SIZES:
+        a, b = _inside_nans(gen, m, k, ta, dtype, pad, lead), _inside_nans(gen, k, n, tb_, dtype, pad, lead)
+        want = (a.double() @ b.double()).float().to(dtype)
+        assert torch.equal(tb.matmul(a, b), want), (m, n, k)
+        assert torch.equal(tb.matmul(a, b, enable_streamk=True), want), (m, n, k, "stream-k")
+        assert torch.equal(tb.matmul(a, b, work_stealing=True), want), (m, n, k, "work stealing")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (3, 5, 100), (100, 5, 3), (100, 3, 100), (7, 100, 7)])
+def test_indices_shorter_than_a_chunk_and_other_strides(m, n, k, dtype):
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    for ta in "TN":
+        for tb_ in "TN":
+            a, b = _inside_nans(gen, m, k, ta, dtype, 1, 1), _inside_nans(gen, k, n, tb_, dtype, 1, 1)
+            assert torch.equal(tb.matmul(a, b), (a.double() @ b.double()).float().to(dtype))
+    a, b = torch.ones(m, 2 * k, device="cuda", dtype=dtype)[:, ::2], torch.ones(1, n, device="cuda", dtype=dtype).expand(k, n)
+    assert (tb.matmul(a, b) == k).all()

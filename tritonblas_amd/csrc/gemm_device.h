@@ -31,6 +31,7 @@ constexpr int f8_fmt_b(int dt) { return (dt == DT_E5M2 || dt == DT_E4E5) ? 1 : 0
 enum : int { MODE_STATIC = 0, MODE_WS = 1, MODE_SK = 2, MODE_GROUPED = 3 };
 enum : int { WS_QUEUES = 0, WS_GLOBAL = 1, WS_HIERARCHICAL = 2 };   // how work-stealing workgroups find tiles
 enum : int { LAY_K = 0, LAY_M = 1 };  // which index is contiguous in global memory for an operand
+enum : int { LOAD_GATHER = 0, LOAD_DIRECT = 1, LOAD_REGS = 2 };   // how operands get to LDS, see Tile
 
 // Word offsets inside the control block at the head of a workspace.
 enum : int { CTL_STATUS = 0, CTL_DONE = 1, CTL_EPOCH = 2, CTL_WORDS = 64 };
@@ -115,14 +116,17 @@ struct TileCtx {
 };
 
 template <int DT_, int BM_, int BN_, int BKB_, int WM_, int WN_, int ALAY_, int BLAY_, int MINB_ = 1,
-          bool FAST_ = true, int STAGES_ = 2>
+          int LOADER_ = LOAD_DIRECT, int STAGES_ = 2>
 struct Tile {
   static constexpr int DT = DT_, BM = BM_, BN = BN_, BKB = BKB_, WM = WM_, WN = WN_;
   static constexpr int ALAY = ALAY_, BLAY = BLAY_, MINB = MINB_, STAGES = STAGES_;
-  // FAST: operands are 16-byte aligned, unit stride along their contiguous index, which has a whole
-  // number of 16-byte chunks; K need not be a multiple of the K step (fp4: it is): the last step's
-  // copies take zeros for what lies beyond it.  !FAST: element-wise gathers, any strides, any K.
-  static constexpr bool FAST = FAST_;
+  // LOAD_DIRECT (FAST): operands are 16-byte aligned, unit stride along their contiguous index, which
+  // has a whole number of 16-byte chunks; K need not be a multiple of the K step (fp4: it is): the last
+  // step's copies take zeros for what lies beyond it.  LOAD_REGS: unit stride along one index, any
+  // alignment of rows and any sizes of at least one chunk: 16-byte loads through registers.
+  // LOAD_GATHER: element-wise, any strides, any K.
+  static constexpr bool FAST = LOADER_ == LOAD_DIRECT, REGS = LOADER_ == LOAD_REGS;
+  static constexpr int LOADER = LOADER_;
   static constexpr bool DMA = FAST;                                    // global -> LDS without registers
   static constexpr int THREADS = WM * WN * 64;
   static constexpr int USZ = (DT == DT_F16 || DT == DT_BF16) ? 2 : (DT == DT_F32 ? 4 : 1);  // bytes per storage unit
@@ -284,7 +288,7 @@ template <class T, int ROWS, int LAY>
 struct Operand {
   static constexpr int CHUNKS = ROWS * T::CPR;
   static constexpr int NCH = (CHUNKS + T::THREADS - 1) / T::THREADS;  // slots per thread
-  static constexpr bool MROWS = T::FAST && LAY == LAY_M;
+  static constexpr bool MROWS = T::LOADER != LOAD_GATHER && LAY == LAY_M;
   static constexpr int MCPR = ROWS * T::USZ / 16;                      // chunks per k row (LAY_M)
   static constexpr int MPITCH = ROWS * T::USZ;                         // bytes per k row
   static constexpr int KPL = T::USZ == 2 ? 8 : 4;                      // k values a lane takes per MFMA slice
@@ -304,8 +308,8 @@ struct Operand {
   }
 
   struct St {
-    const uint8_t* base;     // FAST: tile origin; else matrix origin
-    uint32_t off[NCH];       // FAST: per-slot byte offset from the K-step origin
+    const uint8_t* base;     // tile origin; gather: matrix origin
+    uint32_t off[NCH];       // per-slot byte offset from the K-step origin (LOAD_REGS: signed)
     int64_t s_row, s_k;      // storage units
     int row0, row_lim;
     int whole_steps, tail;   // K steps without a remainder, storage units in the one behind them
@@ -316,7 +320,7 @@ struct Operand {
     st.s_row = s_row; st.s_k = s_k; st.row0 = row0; st.row_lim = row_lim;
     st.whole_steps = (int)(KU / T::UPS); st.tail = (int)(KU % T::UPS);
     const int rows_valid = row_lim - row0;
-    if constexpr (!T::FAST) {
+    if constexpr (T::LOADER == LOAD_GATHER) {
       st.base = mat;
     } else if constexpr (LAY == LAY_K) {
       st.base = mat + (int64_t)row0 * s_row * T::USZ;
@@ -330,21 +334,22 @@ struct Operand {
       }
     } else {
       st.base = mat + (int64_t)row0 * T::USZ;
-      const int last = (rows_valid - 1) / T::UPC;      // (row counts are multiples of a chunk)
+      // the last chunk of the matrix; where its rows are no whole number of chunks (LOAD_REGS) a chunk that
+      // reaches beyond them is loaded from the last UPC rows and put in its place by settle()
+      const int last = T::FAST ? (rows_valid - 1) / T::UPC * T::UPC : rows_valid - T::UPC;
 #pragma unroll
       for (int i = 0; i < NCH; ++i) {
         int q = i * T::THREADS + tid;
         int k = q / MCPR, pc = q % MCPR;
         int c = pc ^ mswz(k);
-        st.off[i] = (uint32_t)(min(c, last) * 16 + k * (int)(s_k * T::USZ));
+        st.off[i] = (uint32_t)(min(c * T::UPC, last) * T::USZ + k * (int)(s_k * T::USZ));
       }
     }
   }
 
   // K-step origin for iteration `it`
   __device__ static __forceinline__ const uint8_t* step_ptr(const St& st, int it) {
-    if constexpr (!T::FAST) return st.base;
-    else if constexpr (LAY == LAY_K) return st.base + (int64_t)it * T::BKB;
+    if constexpr (LAY == LAY_K) return st.base + (int64_t)it * T::BKB;
     else return st.base + (int64_t)it * T::UPS * st.s_k * T::USZ;
   }
 
@@ -381,15 +386,31 @@ struct Operand {
     for (int i = 0; i < NCH; ++i) {
       if (CHUNKS % T::THREADS != 0 && i * T::THREADS + wave_slot >= CHUNKS) continue;
       const uint32_t dst = lds0 + (uint32_t)((i * T::THREADS + wave_slot) * 16);
-      const int q = i * T::THREADS + tid;
-      const int unit = LAY == LAY_K ? ((q % T::CPR) ^ T::swz(q / T::CPR)) * T::UPC : q / MCPR;
-      const uint8_t* src = unit < st.tail ? gp + st.off[i] : (const uint8_t*)&g_zero_chunk;
+      const uint8_t* src = slot_k(i * T::THREADS + tid) < st.tail ? gp + st.off[i] : (const uint8_t*)&g_zero_chunk;
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(dst), "v"(src) : "memory", "m0");
     }
   }
 
   __device__ static __forceinline__ void gload(v4i (&r)[NCH], const St& st, int it, int64_t KU, int tid) {
     const int64_t ku0 = (int64_t)it * T::UPS;
+    if constexpr (T::REGS) {
+      // every load stays inside the matrix: in the step behind the last whole one a chunk that reaches beyond K is
+      // loaded from the last UPC k (the last k row) instead
+      const uint8_t* gp = step_ptr(st, it);
+      const bool part = it >= st.whole_steps;
+#pragma unroll
+      for (int i = 0; i < NCH; ++i) {
+        if (CHUNKS % T::THREADS != 0 && i * T::THREADS + tid >= CHUNKS) continue;
+        int64_t at = (int)st.off[i];
+        if (part) {
+          const int unit = slot_k(i * T::THREADS + tid);
+          if constexpr (LAY == LAY_K) at += (min(unit, st.tail - T::UPC) - unit) * T::USZ;
+          else at += (int64_t)(min(unit, st.tail - 1) - unit) * st.s_k * T::USZ;
+        }
+        __builtin_memcpy(&r[i], gp + at, 16);      // (one load: global memory takes any alignment)
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       int q = i * T::THREADS + tid;
@@ -399,6 +420,39 @@ struct Operand {
       int64_t grow = min(st.row0 + row, st.row_lim - 1);
       r[i] = gather_units<T>(st.base + grow * st.s_row * T::USZ, ku0 + (int64_t)c * T::UPC, st.s_k, KU);
     }
+  }
+
+  // LOAD_REGS: what gload() took from a shifted place goes where it belongs, zeros beyond the end of K
+  __device__ static __forceinline__ void settle(v4i (&r)[NCH], const St& st, int it, int tid) {
+    const bool part = it >= st.whole_steps;
+    const int rows_valid = st.row_lim - st.row0;
+    if (!part && !(LAY == LAY_M && rows_valid < ROWS && rows_valid % T::UPC != 0)) return;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int q = i * T::THREADS + tid, unit = slot_k(q);
+      int shift = 0;      // units
+      if constexpr (LAY == LAY_K) {
+        shift = part ? unit - min(unit, st.tail - T::UPC) : 0;
+      } else {
+        const int row = ((q % MCPR) ^ mswz(unit)) * T::UPC;
+        shift = row - min(row, rows_valid - T::UPC);
+        if (shift >= T::UPC) shift = 0;             // (rows that nobody stores)
+        if (part && unit >= st.tail) shift = T::UPC;
+      }
+      v4i v = r[i];
+      const int d = shift * T::USZ / 4;
+      if (d & 1) v = v4i{v[1], v[2], v[3], 0};
+      if (d & 2) v = v4i{v[2], v[3], 0, 0};
+      if (T::USZ == 2 && (shift & 1)) {
+        v = v4i{(int)__builtin_amdgcn_alignbit((uint32_t)v[1], (uint32_t)v[0], 16u), (int)__builtin_amdgcn_alignbit((uint32_t)v[2], (uint32_t)v[1], 16u),
+                (int)__builtin_amdgcn_alignbit((uint32_t)v[3], (uint32_t)v[2], 16u), (int)((uint32_t)v[3] >> 16)};
+      }
+      r[i] = shift >= T::UPC ? v4i{0, 0, 0, 0} : v;
+    }
+  }
+  // the k (storage units from the step's origin) that slot q's chunk starts at
+  __device__ static __forceinline__ int slot_k(int q) {
+    return LAY == LAY_K ? ((q % T::CPR) ^ T::swz(q / T::CPR)) * T::UPC : q / MCPR;
   }
 
   __device__ static __forceinline__ void sstore(uint8_t* lds, const v4i (&r)[NCH], int tid) {
@@ -551,6 +605,19 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
 
   constexpr bool MXG = (T::DT == DT_FP4) && T::DMA;   // MX scales staged through LDS
 
+  // the fragment of row block i (j) of this wave for slice ks, and how many LDS reads that is
+  auto read_b = [&](const uint8_t* sB, int ks, int j) {
+    if constexpr (OB::MROWS) return Frag<T>::template read_m<OB>(sB, li.wn0 + j * 16, ks, li);
+    else return Frag<T>::read(sB, li.wn0 + j * 16 + li.r, ks, li.g, swm);
+  };
+  auto read_a = [&](const uint8_t* sA, int ks, int i) {
+    if constexpr (OA::MROWS) return Frag<T>::template read_m<OA>(sA, li.wm0 + i * 16, ks, li);
+    else return Frag<T>::read(sA, li.wm0 + i * 16 + li.r, ks, li.g, swm);
+  };
+  constexpr int RPM = T::USZ == 2 ? 2 : 4;
+  constexpr int RPFA = OA::MROWS ? RPM : (is_f8(T::DT) ? 2 : 1);
+  constexpr int RPFB = OB::MROWS ? RPM : (is_f8(T::DT) ? 2 : 1);
+
   // One K step of MFMAs from an LDS stage.  The A-side fragment of row block i+1 is requested before
   // the MFMAs of row block i are issued, so an LDS read is always in flight under the matrix pipe.
   auto compute = [&](const uint8_t* sA, const uint8_t* sB) {
@@ -558,12 +625,12 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
     for (int ks = 0; ks < T::KSUB; ++ks) {
       frag_t bf[T::TN];
 #pragma unroll
-      for (int j = 0; j < T::TN; ++j) bf[j] = Frag<T>::read(sB, li.wn0 + j * 16 + li.r, ks, li.g, swm);
+      for (int j = 0; j < T::TN; ++j) bf[j] = read_b(sB, ks, j);
       frag_t af[2];
-      af[0] = Frag<T>::read(sA, li.wm0 + li.r, ks, li.g, swm);
+      af[0] = read_a(sA, ks, 0);
 #pragma unroll
       for (int i = 0; i < T::TM; ++i) {
-        if (i + 1 < T::TM) af[(i + 1) & 1] = Frag<T>::read(sA, li.wm0 + (i + 1) * 16 + li.r, ks, li.g, swm);
+        if (i + 1 < T::TM) af[(i + 1) & 1] = read_a(sA, ks, i + 1);
 #pragma unroll
         for (int j = 0; j < T::TN; ++j) {
           // output rows follow the first MFMA operand: feed B there so that one lane owns four
@@ -576,11 +643,10 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
       }
       // pin the issue order for the machine scheduler: B fragments and the first A fragment, then
       // alternately the next A fragment's reads and one row block of MFMAs
-      constexpr int RPF = is_f8(T::DT) ? 2 : 1;  // LDS reads per fragment
-      __builtin_amdgcn_sched_group_barrier(0x100, RPF * (T::TN + 1), 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, RPFB * T::TN + RPFA, 0);
 #pragma unroll
       for (int i = 0; i + 1 < T::TM; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x100, RPF, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, RPFA, 0);
         __builtin_amdgcn_sched_group_barrier(0x008, T::TN, 0);
       }
       __builtin_amdgcn_sched_group_barrier(0x008, T::TN, 0);
@@ -687,17 +753,8 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
     // and the matrix pipe has that row block to chew on while they arrive.
     frag_t bf[T::TN];
     frag_t afn;
-    auto request_b = [&](const uint8_t* sB, int ks, int j) {
-      if constexpr (OB::MROWS) bf[j] = Frag<T>::template read_m<OB>(sB, li.wn0 + j * 16, ks, li);
-      else bf[j] = Frag<T>::read(sB, li.wn0 + j * 16 + li.r, ks, li.g, swm);
-    };
-    auto request_a = [&](const uint8_t* sA, int ks, int i) {
-      if constexpr (OA::MROWS) return Frag<T>::template read_m<OA>(sA, li.wm0 + i * 16, ks, li);
-      else return Frag<T>::read(sA, li.wm0 + i * 16 + li.r, ks, li.g, swm);
-    };
-    constexpr int RPM = T::USZ == 2 ? 2 : 4;                               // LDS reads per fragment of an M-contiguous operand,
-    constexpr int RPFA = OA::MROWS ? RPM : (is_f8(T::DT) ? 2 : 1);         // of A
-    constexpr int RPFB = OB::MROWS ? RPM : (is_f8(T::DT) ? 2 : 1);         // and of B
+    auto request_b = [&](const uint8_t* sB, int ks, int j) { bf[j] = read_b(sB, ks, j); };
+    auto request_a = [&](const uint8_t* sA, int ks, int i) { return read_a(sA, ks, i); };
 
     // one block: slice KSV of the K step in stage (sA, sB).  `boundary` runs before the last row block;
     // afterwards the fragments of slice nks of stage (nA, nB) are requested.  After the last step of
@@ -830,6 +887,7 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
     OA::gload(ra, sa, it0, p.KU, li.tid);
     OB::gload(rb, sb, it0, p.KU, li.tid);
     load_scales(it0, sca, scb);
+    if constexpr (T::REGS) { OA::settle(ra, sa, it0, li.tid); OB::settle(rb, sb, it0, li.tid); }
     OA::sstore(sA0, ra, li.tid);
     OB::sstore(sB0, rb, li.tid);
     __syncthreads();
@@ -843,6 +901,7 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
       }
       if (!TB_LAB(p, 2)) compute(sA0 + cur * T::STAGE_BYTES, sB0 + cur * T::STAGE_BYTES);
       if (has_next) {
+        if constexpr (T::REGS) { OA::settle(ra, sa, it + 1, li.tid); OB::settle(rb, sb, it + 1, li.tid); }
         OA::sstore(sA0 + (cur ^ 1) * T::STAGE_BYTES, ra, li.tid);
         OB::sstore(sB0 + (cur ^ 1) * T::STAGE_BYTES, rb, li.tid);
 #pragma unroll

@@ -10,6 +10,12 @@ namespace tb {
   make_variant<Tile<DT_F16, BM, BN, BK, WM, WN, LAY_M, LAY_K, MINB, true, STAGES>>(),   \
   make_variant<Tile<DT_F16, BM, BN, BK, WM, WN, LAY_M, LAY_M, MINB, true, STAGES>>()
 
+#define TB_REGS_LAYOUTS(BM, BN, MINB)                                          \
+  make_variant<Tile<DT_F16, BM, BN, 128, 2, 2, LAY_K, LAY_K, MINB, LOAD_REGS, 2>>(),   \
+  make_variant<Tile<DT_F16, BM, BN, 128, 2, 2, LAY_K, LAY_M, MINB, LOAD_REGS, 2>>(),   \
+  make_variant<Tile<DT_F16, BM, BN, 128, 2, 2, LAY_M, LAY_K, MINB, LOAD_REGS, 2>>(),   \
+  make_variant<Tile<DT_F16, BM, BN, 128, 2, 2, LAY_M, LAY_M, MINB, LOAD_REGS, 2>>()
+
 const Variant g_variants_f16[] = {
     // hand-scheduled 4-wave kernel (K-major operands): taken when K is a multiple of two K steps and no Stream-K tail is asked for
     make_variant_w4<W4Tile<DT_F16>>(),
@@ -22,6 +28,9 @@ const Variant g_variants_f16[] = {
     TB_LAYOUTS(64, 64, 128, 2, 2, 2, 4),
     // a handful of rows against a long K: short, wide, deep tile with three copy stages
     TB_LAYOUTS(32, 128, 256, 1, 4, 1, 3),
+    // unit stride, any alignment of the rows
+    TB_REGS_LAYOUTS(128, 128, 2),
+    TB_REGS_LAYOUTS(64, 64, 4),
     make_variant<Tile<DT_F16, 64, 64, 128, 2, 2, LAY_K, LAY_K, 2, false, 2>>(),
 };
 const int g_num_variants_f16 = sizeof(g_variants_f16) / sizeof(Variant);

@@ -9,7 +9,7 @@ struct Variant {
   int dt, bm, bn, bk;     // element type and tile in elements
   int alay, blay;         // operand loaders (LAY_K / LAY_M)
   int wm, wn, threads, lds_bytes, minb;
-  int fast, stages;       // fast: vector/LDS-direct loaders (alignment required, whole 16-byte chunks)
+  int fast, stages;       // fast: LOAD_*; the tile selector chooses among the LOAD_DIRECT ones
   const void* kernel;     // __global__ void (*)(const GemmParams), whole-tile schedules
   const void* kernel_sk;  // same tile with the Stream-K tail (null: this variant has none)
   int k_step_pairs;       // 1: hand-scheduled 4-wave kernel -- K must be an even number of K steps, at least four; with a
@@ -19,7 +19,7 @@ struct Variant {
 template <class T>
 constexpr Variant make_variant() {
   return Variant{T::DT, T::BM, T::BN, T::BK, T::ALAY, T::BLAY, T::WM, T::WN, T::THREADS, T::LDS_ALLOC, T::MINB,
-                 T::FAST ? 1 : 0, T::STAGES, (const void*)&gemm_kernel<T, false>, (const void*)&gemm_kernel<T, true>, 0};
+                 T::LOADER, T::STAGES, (const void*)&gemm_kernel<T, false>, (const void*)&gemm_kernel<T, true>, 0};
 }
 
 // The hand-scheduled 4-wave kernels of gemm_w4.h (256x256 tile, 128-byte K steps) are compiled in a

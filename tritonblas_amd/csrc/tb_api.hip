@@ -138,6 +138,7 @@ std::vector<TileInfo> tile_infos(int dt) {
   variant_table(dt, &v, &n);
   std::vector<TileInfo> out;
   for (int i = 0; i < n; ++i) {
+    if (v[i].fast == LOAD_REGS) continue;      // (stands in for a tile of its shape where the operands' alignment asks for it)
     bool seen = false;
     for (auto& t : out) seen |= (t.bm == v[i].bm && t.bn == v[i].bn && t.bk == v[i].bk && t.fast == v[i].fast);
     if (!seen) out.push_back(TileInfo{v[i].dt, v[i].bm, v[i].bn, v[i].bk, v[i].threads, v[i].lds_bytes, v[i].minb, v[i].fast, v[i].stages});
@@ -297,6 +298,14 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
     bm = sel.block_m; bn = sel.block_n; bk = sel.block_k;
   }
   const Variant* v = nullptr;
+  // Unit stride along one index, but rows off 16 bytes or with a partial chunk: 16-byte loads through registers, in the
+  // tile that was chosen up to 128x128 (1187x3001x1531 bf16: 248 us in the gather kernel, 42 in this one).  Each contiguous index has a chunk at least.
+  auto any_alignment = [&](int64_t s_row, int64_t s_k, int64_t rows) {
+    if (usz < 2 || j.num_groups > 0) return -1;
+    if (s_k == 1 && s_row >= 0 && KU >= 16 / usz) return (int)LAY_K;
+    return s_row == 1 && s_k >= 0 && rows >= 16 / usz ? (int)LAY_M : -1;
+  };
+  const int ralay = any_alignment(j.a_sr, j.a_sk, j.M), rblay = any_alignment(j.b_sr, j.b_sk, j.N);
   // a K-contiguous operand is copied in 16-byte chunks along K; the kernels fill up the last K step themselves, except
   // for fp4, whose scales would have to be filled up too
   bool fast = alay >= 0 && blay >= 0 && (j.dt == TB_FP4_E2M1 ? KU % (bk / epu) == 0 : (alay == LAY_M && blay == LAY_M) || KU % (16 / usz) == 0);
@@ -328,7 +337,12 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
       for (auto& t : tile_infos(j.dt)) known |= (t.bm == bm && t.bn == bn && t.bk == bk);
       if (!known) return TB_ERR_BAD_TILE;
     }
-    v = find_variant(j.dt, 0, 0, 0, LAY_K, LAY_K, 0);
+    if (ralay >= 0 && rblay >= 0) {
+      const int side = bm >= 128 ? 128 : 64, k_step = 128 / usz;
+      const bool near = (ralay == LAY_K ? side * j.a_sr : k_step * j.a_sk) * usz < (1ll << 31) && (rblay == LAY_K ? side * j.b_sr : k_step * j.b_sk) * usz < (1ll << 31);
+      if (near) v = find_variant(j.dt, side, side, k_step, ralay, rblay, LOAD_REGS);
+    }
+    if (!v) v = find_variant(j.dt, 0, 0, 0, LAY_K, LAY_K, LOAD_GATHER);
     if (!v) return TB_ERR_BAD_LAYOUT;
   }
   if (j.dt == TB_FP4_E2M1 && (j.a_sk != 1 || j.b_sk != 1)) return TB_ERR_BAD_LAYOUT;
@@ -486,7 +500,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
         whole.grid = 0;
         return make_plan(whole, hw, need_device, plan);
       }
-      if (v->fast && j.c_type != TB_I8) {
+      if (v->fast == LOAD_DIRECT && j.c_type != TB_I8) {
         const Variant* w = find_variant(j.dt, v->bm, v->bn, v->bk, v->alay, v->blay, 1, 0, &hw, false, j.K, is_f8_type(j.c_type) ? 1 : 0);
         if (w && w->k_step_pairs && w->bm == v->bm && w->bn == v->bn && w->bk == v->bk &&
             std::max(1, std::min(w->minb, hw.lds_bytes / w->lds_bytes)) == occ)
@@ -634,7 +648,7 @@ int g_splits_used = 0;
 int64_t column_split_point(const Job& j, const tb_hw& hw, const Plan& whole) {
   const Variant* v = whole.v;
   const int64_t total = whole.p.total_tiles, G = whole.grid, tiles_m = whole.p.tiles_m, tiles_n = whole.p.tiles_n;
-  if (whole.skinny || whole.p.mode != MODE_STATIC || !v->fast || total <= G || total % G == 0) return 0;
+  if (whole.skinny || whole.p.mode != MODE_STATIC || v->fast != LOAD_DIRECT || total <= G || total % G == 0) return 0;
   const int64_t tn1 = (total / G) * G / tiles_m;
   if (tn1 <= 0 || tn1 >= tiles_n) return 0;
   const int64_t n1 = tn1 * v->bn, n2 = j.N - n1;
