@@ -72,8 +72,10 @@ class Problem:
     def __init__(self, kind, m, n, ksteps, tiles, pad=0, scales=True):
         self.kind, self.m, self.n, self.ksteps, self.tiles = kind, m, n, ksteps, tiles
         kb = ksteps * 128                           # bytes of K per operand row
-        self.A = Space("A", 0x10_0000_0000, m, kb + pad, kb)
-        self.B = Space("B", 0x20_0000_0000, n, kb + pad, kb)
+        # M-contiguous operands of 16-bit types (the kind's ending): a row of the space is one k
+        self.am, self.bm = (x == "m" for x in (kind.partition("_")[2] or "kk"))
+        self.A = Space("A", 0x10_0000_0000, ksteps * 64, m * 2 + pad, m * 2) if self.am else Space("A", 0x10_0000_0000, m, kb + pad, kb)
+        self.B = Space("B", 0x20_0000_0000, ksteps * 64, n * 2 + pad, n * 2) if self.bm else Space("B", 0x20_0000_0000, n, kb + pad, kb)
         self.C = Space("C", 0x30_0000_0000, m, n * 2 + 2 * pad, n * 2)
         self.fp4 = kind == "fp4"
         self.scaled = kind in ("fp8", "e5m2", "i8") and scales
@@ -104,6 +106,7 @@ class Wave:
         self.srb = np.array([b_tile_row(int(x)) for x in self.sra])
         self.S = {}          # scalar registers by name ("s70", "m0", "scc") and bound operands ("%[A]")
         self.V = {}          # vector registers that hold addresses: number -> uint32[64]
+        self.quarter = {}    # vector register written by a transposing read -> which four k of its half
         self.meta = {}       # vector register -> what an LDS read put there
         self.lds = group.lds  # LDS byte offset (4-byte granularity) -> dict(what=..., vm=entry, pub=bool), shared
         self.vmq = []        # vector memory operations in issue order: dict(done=bool, lds=[offsets])
@@ -115,19 +118,33 @@ class Wave:
         self.step = None     # (tile index, K step) the MFMAs in flight belong to
         self.log = []
 
+    # chunk masks of the K rows of M-contiguous operands
+    @staticmethod
+    def mask_a(k):
+        return 2 * ((k & 3) ^ (((k >> 4) ^ (k >> 5)) & 1))
+
+    @staticmethod
+    def mask_b(k):
+        return 4 * ((k >> 1) & 1)
+
     # ---- operand restatement of gemm_w4.h ------------------------------------------------------------------
     def tile_args(self, t):
         p = self.prob
         m0, n0 = t[:2]
         it0 = t[2] if len(t) > 2 else 0          # a Stream-K piece starts at K step it0 of its tile
         rva, rvb = min(256, p.m - m0), min(256, p.n - n0)
-        a = {"A": p.A.base + m0 * p.A.stride + it0 * 128, "B": p.B.base + n0 * p.B.stride + it0 * 128,
+        a_at = 2 * m0 + it0 * 64 * p.A.stride if p.am else m0 * p.A.stride + it0 * 128
+        b_at = 2 * n0 + it0 * 64 * p.B.stride if p.bm else n0 * p.B.stride + it0 * 128
+        a = {"A": p.A.base + a_at, "B": p.B.base + b_at,
              "mxa": p.mxa.base + m0 * p.mxa.stride + it0 * 8, "mxb": p.mxb.base + n0 * p.mxb.stride + it0 * 8, "rva": rva, "rvb": rvb}
         off = []
-        for i in range(8):
-            off.append(np.minimum(i * 32 + self.pa, rva - 1) * p.A.stride + self.c16)
-        for i in range(8):
-            off.append(np.minimum(i * 32 + self.pb, rvb - 1) * p.B.stride + self.c16)
+        for transposed, space, valid, rows, mask in ((p.am, p.A, rva, self.pa, self.mask_a), (p.bm, p.B, rvb, self.pb, self.mask_b)):
+            for i in range(8):
+                if transposed:
+                    k = (i & 1) * 32 + self.wave * 8 + (self.lane >> 3)
+                    off.append(k * space.stride + np.minimum((i >> 1) * 8 + ((self.lane & 7) ^ mask(k)), (valid - 1) // 8) * 16)
+                else:
+                    off.append(np.minimum(i * 32 + rows, valid - 1) * space.stride + self.c16)
         a["off"] = off
         a["sca"] = np.minimum(self.sra, rva - 1) * p.mxa.stride
         a["scb"] = np.minimum(self.srb, rvb - 1) * p.mxb.stride
@@ -159,6 +176,17 @@ class Wave:
         b0 = LDS0 + 32768 + (self.wn0 + self.r) * 128 + lo
         for i, v in enumerate((a0, a0 ^ 16, b0, b0 ^ 16, a0 + 65536, (a0 ^ 16) + 65536, b0 + 65536, (b0 ^ 16) + 65536)):
             V[224 + i] = v
+        k = 16 * self.g + (self.r >> 2)
+        if p.am:
+            S["%[astep]"] = 64 * p.A.stride
+            for t in range(4):
+                V[160 + t] = LDS0 + self.wm0 * 128 + k * 128 + (((2 * t + ((self.r >> 1) & 1)) ^ self.mask_a(k)) << 4) + (self.r & 1) * 8
+                V[164 + t] = V[160 + t] + 65536
+        if p.bm:
+            S["%[bstep]"] = 64 * p.B.stride
+            for u in range(2):
+                V[226 + u] = LDS0 + 32768 + self.wn0 * 128 + k * 128 + (((4 * u + (self.r & 3)) ^ self.mask_b(k)) << 4)
+                V[230 + u] = V[226 + u] + 65536
         coff = (self.r * p.C.stride + 16 * self.g) & MASK32      # ((r * c_sm + 8 g) * 2 with c_sm in elements)
         if p.fp4:
             V[232] = LDS0 + SC0 + (self.wm0 + self.r) * 16 + self.g * 2
@@ -271,9 +299,13 @@ class Wave:
     def expect_rows(self, space, t, tile):
         m0, n0 = self.prob.tiles[tile][:2]
         if space in ("A", "mxa"):
-            return np.minimum(m0 + self.wm0 + 16 * t + self.r, self.prob.m - 1)
-        rows = np.array([b_tile_row(int(x)) for x in (self.wn0 + 16 * t + self.r)])
-        return np.minimum(n0 + rows, self.prob.n - 1)
+            rows, lim, chunked = m0 + self.wm0 + 16 * t + self.r, self.prob.m, space == "A" and self.prob.am
+        else:
+            rows, lim = n0 + np.array([b_tile_row(int(x)) for x in (self.wn0 + 16 * t + self.r)]), self.prob.n
+            chunked = space == "B" and self.prob.bm
+        if chunked:      # (rows beyond the matrix: the last chunk of eight again)
+            return np.minimum(rows // 8, (lim - 1) // 8) * 8 + rows % 8
+        return np.minimum(rows, lim - 1)
 
     def note_fragment(self, dst, got):
         """ds_read_b128 of half a fragment: which operand, K step and half the lanes agree on, and each lane's row"""
@@ -296,6 +328,32 @@ class Wave:
         rows = np.array([got[l][0][0][1] for l in range(64)])
         for r in self.gen.Gen._vregs(dst):
             self.meta[r] = ("frag", sp, kstep, half, rows)
+
+    def note_transposed(self, dst, got):
+        """ds_read_b64_tr_b16: within 16 lanes, lane i ends up with element i % 4 of what lanes 4 j + i / 4 named, j = 0..3: the four
+        K rows 16 g + 8 half + 4 h + j of one tile row"""
+        keys, rows = set(), []
+        for l in range(64):
+            i, row = l & 15, set()
+            for j in range(4):
+                lane, sub = got[(l & ~15) + 4 * j + i // 4]
+                if sub != 0 or lane[1] != (lane[0][0], lane[0][1], lane[0][2] + 4):
+                    raise Fail("a transposing read names bytes of two copies")
+                sp, k, col = lane[0]
+                kk = k % 64 - 16 * int(self.g[l]) - j
+                if kk not in (0, 4, 8, 12):
+                    raise Fail(f"lane {l} of a transposing read got K row {k % 64} in place {j}")
+                keys.add((sp, k // 64, kk))
+                row.add(col // 2 + i % 4)
+            if len(row) != 1:
+                raise Fail(f"lane {l} of a transposing read got several tile rows: {row}")
+            rows.append(row.pop())
+        if len(keys) != 1:
+            raise Fail(f"lanes of a transposing read disagree: {keys}")
+        sp, kstep, kk = keys.pop()
+        for r in self.gen.Gen._vregs(dst):
+            self.meta[r] = ("frag", sp, kstep, kk // 8, np.array(rows))
+            self.quarter[r] = kk // 4 % 2
 
     def note_scale(self, dst, got):
         regs = self.gen.Gen._vregs(dst)
@@ -321,6 +379,8 @@ class Wave:
                 if md is None or md[0] != "frag":
                     raise Fail(f"{text}: v{r} holds no fragment")
                 _, sp, ks, hf, rows = md
+                if r in self.quarter and self.quarter[r] != (r - first) // 2 % 2:
+                    raise Fail(f"{text}: v{r} holds the other four k of its half")
                 if sp != space or ks != kstep or not np.array_equal(rows, want_rows):
                     raise Fail(f"MFMA for accumulator ({i}, {j}) of tile {tile} step {kstep} reads v{r} = {sp} step {ks} rows {rows[:3]}.. (wanted {space} rows {want_rows[:3]}..)")
             if last - first == 7:
@@ -436,12 +496,15 @@ class Wave:
         elif op.startswith("ds_read"):
             areg, _, tail = a[1].partition(" ")
             imm = int(tail.split("offset:")[1]) if "offset:" in tail else 0
-            size = {"ds_read_b128": 16, "ds_read_b32": 4, "ds_read_u16": 2}[op]
+            size = {"ds_read_b128": 16, "ds_read_b32": 4, "ds_read_u16": 2, "ds_read_b64_tr_b16": 8}[op]
             got = self.read(a[0], areg, imm, size)
             area = self.lds_area(int(self.vval(areg)[0]) + imm - LDS0)
             for r in self.gen.Gen._vregs(a[0]):
                 self.meta.pop(r, None)
-            if area[0] in "AB" and size == 16:
+                self.quarter.pop(r, None)
+            if op == "ds_read_b64_tr_b16":
+                self.note_transposed(a[0], got)
+            elif area[0] in "AB" and size == 16:
                 self.note_fragment(a[0], got)
             elif area == "scale":
                 self.note_scale(a[0], got)

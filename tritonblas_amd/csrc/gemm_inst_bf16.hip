@@ -17,8 +17,11 @@ namespace tb {
   make_variant<Tile<DT_BF16, BM, BN, 128, 2, 2, LAY_M, LAY_M, MINB, LOAD_REGS, 2>>()
 
 const Variant g_variants_bf16[] = {
-    // hand-scheduled 4-wave kernel (K-major operands): taken when K is a multiple of two K steps and no Stream-K tail is asked for
+    // hand-scheduled 4-wave kernel: taken when K is a multiple of two K steps and no Stream-K tail is asked for (with one: K-major operands only)
     make_variant_w4<W4Tile<DT_BF16>>(),
+    make_variant_w4<W4Tile<DT_BF16, LAY_K, LAY_M>>(),
+    make_variant_w4<W4Tile<DT_BF16, LAY_M, LAY_K>>(),
+    make_variant_w4<W4Tile<DT_BF16, LAY_M, LAY_M>>(),
     TB_LAYOUTS(256, 256, 128, 2, 4, 1, 2),
     TB_LAYOUTS(128, 128, 128, 2, 2, 2, 2),
     TB_LAYOUTS(64, 64, 128, 2, 2, 4, 2),

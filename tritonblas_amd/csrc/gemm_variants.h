@@ -24,10 +24,12 @@ constexpr Variant make_variant() {
 
 // The hand-scheduled 4-wave kernels of gemm_w4.h (256x256 tile, 128-byte K steps) are compiled in a
 // translation unit of their own (gemm_inst_w4.hip), which hands out their addresses.
+// (the ones with an M-contiguous operand in gemm_inst_w4m.hip)
 const void* w4_kernel(int dt);
+const void* w4_kernel_m(int dt, int alay, int blay);
 const void* w4_kernel_sk(int dt);
-template <int DT>
-using W4Tile = Tile<DT, 256, 256, 128, 2, 2, LAY_K, LAY_K, 1, true, 2>;
+template <int DT, int ALAY = LAY_K, int BLAY = LAY_K>
+using W4Tile = Tile<DT, 256, 256, 128, 2, 2, ALAY, BLAY, 1, LOAD_DIRECT, 2>;
 // LDS of these kernels: two 64 KB stages, 16 KB of FP4 scale buffers, 1 KB per wave of epilogue scales,
 // the schedule's broadcast word
 constexpr int W4_EPS_OFFSET = 131072 + 16384;
@@ -35,7 +37,8 @@ constexpr int W4_LDS_BYTES = W4_EPS_OFFSET + 4096 + 16;
 template <class T>
 Variant make_variant_w4() {
   return Variant{T::DT, T::BM, T::BN, T::BK, T::ALAY, T::BLAY, T::WM, T::WN, T::THREADS, W4_LDS_BYTES, 1,
-                 1, T::STAGES, w4_kernel(T::DT), w4_kernel_sk(T::DT), 1};
+                 1, T::STAGES, T::ALAY == LAY_M || T::BLAY == LAY_M ? w4_kernel_m(T::DT, T::ALAY, T::BLAY) : w4_kernel(T::DT),
+                 T::ALAY == LAY_M || T::BLAY == LAY_M ? nullptr : w4_kernel_sk(T::DT), 1};
 }
 
 // defined one per translation unit

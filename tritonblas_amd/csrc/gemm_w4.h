@@ -19,6 +19,14 @@
 // values a lane holds for MFMA tiles 2q and 2q+1 eight consecutive columns: the epilogue stores them
 // as one 16-byte write per lane straight from registers (64 contiguous bytes per row and instruction),
 // with no LDS staging -- the LDS already belongs to the next tile's first K steps by then.
+//
+// M-contiguous operands (16-bit types) are copied as they lie in memory and transposed by the fragment reads,
+// with the same fragments in the same registers: block b of an operand's half stage (8 KB) is tile rows 64 b .. +63,
+// K row k of it 128 bytes at 128 k, chunk c of those at slot c ^ mask(k).  A: mask 2 ((k % 4) ^ x), x the parity of
+// the bits of k / 16 (a fragment read takes 32 bytes of four K rows per 16 lanes, and 16 lanes after 16 lanes sit 16 K
+// rows apart); B, whose column order makes that 8 bytes of each of four chunks: mask 4 ((k / 2) % 2).
+// (Three rounds of tiles of 4096x12288x4096 bf16, B M-contiguous, 350 -> 326 us; 14336x4096x4096, both M-contiguous, 332 -> 305 us,
+// both K-contiguous 315: the eight-wave kernel's figure is the first one of each pair.)
 #pragma once
 #include <utility>
 #include "gemm_variants.h"
@@ -66,19 +74,32 @@ struct W4Lane {
   uint32_t c16;          // swizzled chunk (byte offset) this lane copies in every row it copies
   int pa, pb;            // tile row this lane copies with copy instruction 0 (instruction i: + 32 i)
   int sra, srb;          // FP4: tile rows whose scales this lane copies
+  int k8, cm;            // M-contiguous operands: K row (copy instruction i: + 32 (i % 2)), chunk slot this lane copies
 };
+
+__device__ __forceinline__ int w4_mask_a(int k) {
+  const int g = k >> 4;
+  return 2 * ((k & 3) ^ ((g ^ (g >> 1)) & 1));
+}
+__device__ __forceinline__ int w4_mask_b(int k) { return 4 * ((k >> 1) & 1); }
 
 // it0: first K step of the work item (a Stream-K piece starts inside the tile's K range)
 template <class T>
 __device__ __forceinline__ void w4_tile_args(const GemmParams& p, const TileCtx& tc, int it0, const W4Lane& ln, W4TileArgs& t) {
   const int rva = tc.m_lim - tc.m0, rvb = tc.n_lim - tc.n0;
   const uint32_t sra = (uint32_t)p.a_sr * T::USZ, srb = (uint32_t)p.b_sr * T::USZ;   // row strides in bytes
-  t.A = p.A + (int64_t)tc.m0 * p.a_sr * T::USZ + (int64_t)it0 * 128;
-  t.B = tc.B + (int64_t)tc.n0 * p.b_sr * T::USZ + (int64_t)it0 * 128;
+  t.A = p.A + (int64_t)tc.m0 * p.a_sr * T::USZ + (T::ALAY == LAY_M ? (int64_t)it0 * T::UPS * p.a_sk * T::USZ : (int64_t)it0 * 128);
+  t.B = tc.B + (int64_t)tc.n0 * p.b_sr * T::USZ + (T::BLAY == LAY_M ? (int64_t)it0 * T::UPS * p.b_sk * T::USZ : (int64_t)it0 * 128);
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    t.off[i] = (int)((uint32_t)min(i * 32 + ln.pa, rva - 1) * sra + ln.c16);
-    t.off[8 + i] = (int)((uint32_t)min(i * 32 + ln.pb, rvb - 1) * srb + ln.c16);
+    const int k = (i & 1) * 32 + ln.k8;
+    // (row counts of M-contiguous operands are multiples of a chunk)
+    if constexpr (T::ALAY == LAY_M)
+      t.off[i] = (int)((uint32_t)k * (uint32_t)p.a_sk * T::USZ + (uint32_t)min((i >> 1) * 8 + (ln.cm ^ w4_mask_a(k)), (rva - 1) / 8) * 16u);
+    else t.off[i] = (int)((uint32_t)min(i * 32 + ln.pa, rva - 1) * sra + ln.c16);
+    if constexpr (T::BLAY == LAY_M)
+      t.off[8 + i] = (int)((uint32_t)k * (uint32_t)p.b_sk * T::USZ + (uint32_t)min((i >> 1) * 8 + (ln.cm ^ w4_mask_b(k)), (rvb - 1) / 8) * 16u);
+    else t.off[8 + i] = (int)((uint32_t)min(i * 32 + ln.pb, rvb - 1) * srb + ln.c16);
   }
   if constexpr (T::DT == DT_FP4) {
     t.mxa = p.mxa + (int64_t)tc.m0 * p.mxa_sr + it0 * 8;      // (eight E8M0 bytes per row and K step)
@@ -354,6 +375,7 @@ template <class T, bool SK = false>
 __global__ __launch_bounds__(256, 1) void gemm_kernel_w4(const GemmParams p) {
   static_assert(T::BM == 256 && T::BN == 256 && T::BKB == 128 && T::WM == 2 && T::WN == 2 && T::STAGES == 2, "fixed shape");
   static_assert(is_f8(T::DT) || T::DT == DT_FP4 || T::DT == DT_BF16 || T::DT == DT_F16 || T::DT == DT_I8, "element types with a generated K loop");
+  static_assert((T::ALAY == LAY_K && T::BLAY == LAY_K) || (T::USZ == 2 && !SK), "M-contiguous operands: 16-bit types, whole tiles");
   // two stages, the FP4 scale buffers (16 KB), 1 KB per wave for epilogue scales, the schedule's broadcast word
   __shared__ __attribute__((aligned(16))) uint8_t lds[W4_LDS_BYTES];
   int& s_bcast = *(int*)(lds + W4_LDS_BYTES - 16);
@@ -374,6 +396,8 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel_w4(const GemmParams p) {
   ln.pa = wave * 8 + l8;
   // B: LDS row rho = 16j + 4g' + e (within a wave's 128 rows) takes tile row 32(j/2) + 8g' + 4(j%2) + e
   ln.pb = ((wave & 1) * 2 + (l8 >> 2)) * 8 + (wave >> 1) * 4 + (l8 & 3);
+  ln.k8 = wave * 8 + l8;
+  ln.cm = lane & 7;
   ln.sra = wave * 64 + lane;
   {
     const int rho = ln.sra & 127, j = rho >> 4, gg = (rho >> 2) & 3, e = rho & 3;
@@ -389,6 +413,26 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel_w4(const GemmParams p) {
     fa[0] = (int)a0; fa[1] = (int)(a0 ^ 16u); fa[2] = (int)b0; fa[3] = (int)(b0 ^ 16u);
     fa[4] = (int)(a0 + 65536u); fa[5] = (int)((a0 ^ 16u) + 65536u); fa[6] = (int)(b0 + 65536u); fa[7] = (int)((b0 ^ 16u) + 65536u);
   }
+  // M-contiguous operands: lane (g, r) names 8 bytes of K row 16 g + r / 4 (and, by offset, of 4, 8 and 12 rows further)
+  v8i fm = {0, 0, 0, 0, 0, 0, 0, 0};
+  {
+    const int k = 16 * ln.g + (ln.r >> 2);
+    if constexpr (T::ALAY == LAY_M) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int a = (int)(lds0 + (uint32_t)ln.wm0 * 128u) + k * 128 + (((2 * t + ((ln.r >> 1) & 1)) ^ w4_mask_a(k)) << 4) + (ln.r & 1) * 8;
+        fm[t] = a; fm[4 + t] = a + 65536;
+      }
+    }
+    if constexpr (T::BLAY == LAY_M) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int b = (int)(lds0 + 32768u + (uint32_t)ln.wn0 * 128u) + k * 128 + (((4 * u + (ln.r & 3)) ^ w4_mask_b(k)) << 4);
+        fa[2 + u] = b; fa[6 + u] = b + 65536;
+      }
+    }
+  }
+  const uint32_t s_astep = uniform((uint32_t)p.a_sk * 128u), s_bstep = uniform((uint32_t)p.b_sk * 128u);   // (64 K rows of 2-byte values)
   const uint32_t wl = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + (uint32_t)wave * 1024u));
 
   Sched<T, SK> sched;
@@ -496,6 +540,54 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel_w4(const GemmParams p) {
 #include "w4_clobbers_i8.inc"
         );
       }
+    } else if constexpr (T::DT == DT_BF16 && T::ALAY == LAY_K && T::BLAY == LAY_M) {
+      asm volatile(
+#include "w4_kloop_bf16_km.inc"
+          : [scbuf] "+s"(scbuf)
+          : W4_COMMON_OPERANDS, [eo] "{v[240:243]}"(eo), [bstep] "s"(s_bstep)
+          :
+#include "w4_clobbers_bf16_km.inc"
+      );
+    } else if constexpr (T::DT == DT_BF16 && T::ALAY == LAY_M && T::BLAY == LAY_K) {
+      asm volatile(
+#include "w4_kloop_bf16_mk.inc"
+          : [scbuf] "+s"(scbuf)
+          : W4_COMMON_OPERANDS, [eo] "{v[240:243]}"(eo), [fm] "{v[160:167]}"(fm), [astep] "s"(s_astep)
+          :
+#include "w4_clobbers_bf16_mk.inc"
+      );
+    } else if constexpr (T::DT == DT_BF16 && T::ALAY == LAY_M && T::BLAY == LAY_M) {
+      asm volatile(
+#include "w4_kloop_bf16_mm.inc"
+          : [scbuf] "+s"(scbuf)
+          : W4_COMMON_OPERANDS, [eo] "{v[240:243]}"(eo), [fm] "{v[160:167]}"(fm), [astep] "s"(s_astep), [bstep] "s"(s_bstep)
+          :
+#include "w4_clobbers_bf16_mm.inc"
+      );
+    } else if constexpr (T::DT == DT_F16 && T::ALAY == LAY_K && T::BLAY == LAY_M) {
+      asm volatile(
+#include "w4_kloop_f16_km.inc"
+          : [scbuf] "+s"(scbuf)
+          : W4_COMMON_OPERANDS, [eo] "{v[240:243]}"(eo), [bstep] "s"(s_bstep)
+          :
+#include "w4_clobbers_f16_km.inc"
+      );
+    } else if constexpr (T::DT == DT_F16 && T::ALAY == LAY_M && T::BLAY == LAY_K) {
+      asm volatile(
+#include "w4_kloop_f16_mk.inc"
+          : [scbuf] "+s"(scbuf)
+          : W4_COMMON_OPERANDS, [eo] "{v[240:243]}"(eo), [fm] "{v[160:167]}"(fm), [astep] "s"(s_astep)
+          :
+#include "w4_clobbers_f16_mk.inc"
+      );
+    } else if constexpr (T::DT == DT_F16 && T::ALAY == LAY_M && T::BLAY == LAY_M) {
+      asm volatile(
+#include "w4_kloop_f16_mm.inc"
+          : [scbuf] "+s"(scbuf)
+          : W4_COMMON_OPERANDS, [eo] "{v[240:243]}"(eo), [fm] "{v[160:167]}"(fm), [astep] "s"(s_astep), [bstep] "s"(s_bstep)
+          :
+#include "w4_clobbers_f16_mm.inc"
+      );
     } else if constexpr (T::DT == DT_BF16) {
       asm volatile(
 #include "w4_kloop_bf16.inc"

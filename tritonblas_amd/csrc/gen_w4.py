@@ -1,7 +1,8 @@
 #!/usr/bin/env python3
 """Writes the hand-scheduled K loop of the 4-wave 256x256 tile kernels (gemm_w4.h) as inline-assembly text.
 
-    python3 gen_w4.py fp8 > w4_kloop_fp8.inc        (also: e5m2, e4e5, e5e4, fp4, bf16, f16, i8)
+    python3 gen_w4.py fp8 > w4_kloop_fp8.inc        (also: e5m2, e4e5, e5e4, fp4, bf16, f16, i8, and bf16_km, bf16_mk,
+                                                     bf16_mm, f16_km, ...)
     python3 gen_w4.py clobbers fp8 > w4_clobbers_fp8.inc
     python3 gen_w4.py check                          (walks every kind through the wait-count checker)
 
@@ -10,7 +11,11 @@ tile: 8x8 MFMA tiles of 16x16, i.e. 256 accumulator registers a[0:255]; acc(i, j
 B row block j sits in a[(8i+j)*4 .. +3].  A K step is 128 bytes of every operand row (128 FP8 values,
 256 FP4 values or 64 16-bit values); LDS holds two stages of 64 KB: stage s at s*65536, A rows at +0,
 B rows at +32768, row r at r*128 with its eight 16-byte chunks XOR-swizzled (the layout the 8-wave
-kernels use).  FP4 adds two 8 KB buffers of E8M0 scales behind the stages (16 scale bytes per row =
+kernels use).  The kinds of a 16-bit type with an ending (bf16_km: A K-contiguous, B M-contiguous; _mk, _mm) copy
+an M-contiguous operand as it lies in memory: four blocks of 64 tile rows, each 64 K rows of 128 bytes, whose
+eight 16-byte chunks are XOR-swizzled by the K row.  Copy instructions 2b and 2b+1 fill block b, so the copies
+fall into the same groups (A lo, A hi) by the row blocks they hold, and a fragment is four transposing 8-byte
+reads instead of two 16-byte ones.  FP4 adds two 8 KB buffers of E8M0 scales behind the stages (16 scale bytes per row =
 two K steps).
 
 The text is the code of ONE asm statement that runs the whole K loop of one output tile (at least four
@@ -47,11 +52,13 @@ as needed.
 
 Register map (VGPR):  0..127   B fragment sets 0/1 (8 fragments x 8 registers each)
                       128..159 A fragment buffers 0..3
+                      160..167 A M-contiguous, in: its fragment read addresses, 4 * stage + (row block % 4)
                       160..191 FP4: E8M0 scale registers (set p: A rows 160+16p+i, B rows 168+16p+j);
                                FP8: epilogue column scales sb (in/out)
                       192..207 in: byte offsets of this tile's copies (A 192+i, B 200+i, i = copy instruction)
                       208..223 in: the same for the next tile
                       224..231 in: fragment read addresses (A lo, A hi, B lo, B hi) for stage 0, then stage 1
+                               (B M-contiguous: for fragments with (j / 2) % 2 = 0, 1)
                       FP4:  232..237 in: scale read addresses (A, B), scale copy offsets (A, B) now and next;
                             238 in: C offset of this lane; 240, 241 scale read addresses of the current buffer
                       else: 240 in: C offset of this lane; FP8: 241 in: lane * 4, 242 in / 243 in: LDS
@@ -98,7 +105,11 @@ F8_KINDS = ("fp8", "e5m2", "e4e5", "e5e4")
 
 class Gen:
     def __init__(self, kind, lab=()):
-        self.kind = kind                # "fp8" | "e5m2" | "e4e5" | "e5e4" | "fp4" | "bf16" | "f16" | "i8"
+        # "fp8" | "e5m2" | "e4e5" | "e5e4" | "fp4" | "bf16" | "f16" | "i8", the 16-bit ones also with the operands' layouts
+        kind, _, lay = kind.partition("_")
+        self.kind = kind
+        self.mrows = tuple(x == "m" for x in (lay or "kk"))     # A, B: the rows of the tile, not K, are contiguous in memory
+        assert lay in ("", "km", "mk", "mm") and (not lay or kind in ("bf16", "f16"))
         # 8-bit floats: one MFMA of K = 128 per fragment pair; the kinds differ in its format fields (e4e5: A in e4m3, B in
         # e5m2; e5e4 the other way round)
         self.f8 = kind in F8_KINDS
@@ -122,6 +133,7 @@ class Gen:
         self.earlyb = os.environ.get("W4GEN_EARLYB", "1" if kind == "fp4" else "0") == "1"
         self.earlysc = os.environ.get("W4GEN_EARLYSC", "0") == "1"
         self.v_coff = 238 if self.fp4 else 240
+        self.v_am = 160
         self.v_lane4, self.v_sa_rd, self.v_sb_rd = 241, 242, 243
         self.v_sb, self.v_sa, self.epi_tmp = 64, 96, 104
 
@@ -149,6 +161,15 @@ class Gen:
     # ---- building blocks --------------------------------------------------------------------------
     def frag_read(self, dst, op, stage, t):
         """both 16-byte halves of fragment t (16 rows x 128 bytes of K) of operand op"""
+        if self.mrows[op]:
+            # half ks, registers 2h and 2h+1: K rows 16 g + 8 ks + 4 h + 0..3.  The swizzle moves A's fragments about within a
+            # block of 64 rows (an address for each of four); B's are 8 bytes of every 16 (see gemm_w4.h for the column order)
+            if op == 0:
+                reg, off = self.v_am + 4 * stage + t % 4, t // 4 * 8192
+            else:
+                reg, off = self.fa(1, (t >> 1) & 1, stage), t // 4 * 8192 + t % 2 * 8
+            return [Op(f"ds_read_b64_tr_b16 v[{dst + 4 * ks + 2 * h}:{dst + 4 * ks + 2 * h + 1}], v{reg} offset:{off + ks * 1024 + h * 512}")
+                    for ks in range(2) for h in range(2)]
         return [Op(f"ds_read_b128 v[{dst}:{dst + 3}], v{self.fa(op, 0, stage)} offset:{t * 2048}"),
                 Op(f"ds_read_b128 v[{dst + 4}:{dst + 7}], v{self.fa(op, 1, stage)} offset:{t * 2048}")]
 
@@ -173,8 +194,9 @@ class Gen:
         return ops
 
     def dma_advance(self):
-        return [Op(f"s_add_u32 s{S_CA}, s{S_CA}, 128"), Op(f"s_addc_u32 s{S_CA + 1}, s{S_CA + 1}, 0"),
-                Op(f"s_add_u32 s{S_CB}, s{S_CB}, 128"), Op(f"s_addc_u32 s{S_CB + 1}, s{S_CB + 1}, 0")]
+        sa, sb = ("%[astep]" if self.mrows[0] else "128"), ("%[bstep]" if self.mrows[1] else "128")
+        return [Op(f"s_add_u32 s{S_CA}, s{S_CA}, {sa}"), Op(f"s_addc_u32 s{S_CA + 1}, s{S_CA + 1}, 0"),
+                Op(f"s_add_u32 s{S_CB}, s{S_CB}, {sb}"), Op(f"s_addc_u32 s{S_CB + 1}, s{S_CB + 1}, 0")]
 
     def scale_dma(self, nxt, tag):
         """copy of one scale group (16 bytes per row, A rows then B rows) into the buffer s79 names, then toggle it"""
@@ -409,8 +431,7 @@ class Gen:
         older = set(range(self.vB(p, 0), self.vB(p, 0) + 64)) | set(range(self.vA(0), self.vA(0) + 8))
         if self.fp4:
             older |= set(range(self.scA(p, 0), self.scA(p, 0) + 16))
-        a1, a2 = self.vA(1), self.vA(2)
-        return [older, set(range(a1, a1 + 4)), set(range(a1 + 4, a1 + 8)), set(range(a2, a2 + 4)), set(range(a2 + 4, a2 + 8))]
+        return [older] + self.read_dests(self.frag_read(self.vA(1), 0, p, 1) + self.frag_read(self.vA(2), 0, p, 2))
 
     @classmethod
     def read_dests(cls, ops):
@@ -489,8 +510,7 @@ class Gen:
         P["setup"] = setup
         P["prologue"] = self.prologue()
         # later tiles: steps 0 and 1 (and scale group 0) were requested during the previous tile
-        resume = [Op(f"s_add_u32 s{S_CA}, s{S_CA}, 256"), Op(f"s_addc_u32 s{S_CA + 1}, s{S_CA + 1}, 0"),
-                  Op(f"s_add_u32 s{S_CB}, s{S_CB}, 256"), Op(f"s_addc_u32 s{S_CB + 1}, s{S_CB + 1}, 0")]
+        resume = self.dma_advance() + self.dma_advance()
         if fp4:
             resume += [Op(f"s_add_u32 s{S_CSA}, s{S_CSA}, 16"), Op(f"s_addc_u32 s{S_CSA + 1}, s{S_CSA + 1}, 0"),
                        Op(f"s_add_u32 s{S_CSB}, s{S_CSB}, 16"), Op(f"s_addc_u32 s{S_CSB + 1}, s{S_CSB + 1}, 0"),
@@ -692,7 +712,7 @@ def main():
         sys.stdout.write(clobbers(sys.argv[2]))
         return
     if what == "check":
-        for kind in F8_KINDS + ("fp4", "bf16", "f16", "i8"):
+        for kind in F8_KINDS + ("fp4", "bf16", "f16", "i8", "bf16_km", "bf16_mk", "bf16_mm"):
             w = Gen(kind).check()
             print(kind, "ok; smallest slack per wait site:", min(w.values()), "largest:", max(w.values()))
         return
