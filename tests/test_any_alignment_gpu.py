@@ -42,3 +42,25 @@ def test_indices_shorter_than_a_chunk_and_other_strides(m, n, k, dtype):
             assert torch.equal(tb.matmul(a, b), (a.double() @ b.double()).float().to(dtype))
     a, b = torch.ones(m, 2 * k, device="cuda", dtype=dtype)[:, ::2], torch.ones(1, n, device="cuda", dtype=dtype).expand(k, n)
     assert (tb.matmul(a, b) == k).all()
+
+
+@pytest.mark.parametrize("pad,lead", [(0, 0), (3, 5)])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 32), (65, 63, 96), (128, 130, 480), (200, 70, 544), (33, 257, 1056), (300, 260, 4128)])
+def test_mxfp4_rows_and_scales_at_any_alignment(m, n, k, pad, lead):
+    from tritonblas_amd.utils import e8m0_to_f32, mxfp4_to_f32
+    gen = torch.Generator(device="cuda").manual_seed(k)
+
+    def rows(count, width, lo, hi, fill):
+        base = torch.full((count * (width + pad) + lead,), fill, device="cuda", dtype=torch.uint8)
+        x = base[lead:].view(count, width + pad)[:, :width]
+        x.copy_(torch.randint(lo, hi, (count, width), device="cuda", generator=gen))
+        return x
+
+    # (what lies between the rows: scale byte 255 is NaN)
+    a, b = rows(m, k // 2, 0, 256, 0x77), rows(n, k // 2, 0, 256, 0x77)
+    sa, sb = rows(m, k // 32, 126, 129, 255), rows(n, k // 32, 126, 129, 255)
+    c = torch.full((m, n), float("nan"), device="cuda", dtype=torch.bfloat16)
+    tb.matmul_fp4(a, b, c, sa, sb)
+    full = [mxfp4_to_f32(x.contiguous()).double() * e8m0_to_f32(s.contiguous()).double().repeat_interleave(32, 1) for x, s in ((a, sa), (b, sb))]
+    # (multiples of 1/16 below 2**16 * 144: the sums are exact)
+    assert torch.equal(c, (full[0] @ full[1].T).float().to(torch.bfloat16))

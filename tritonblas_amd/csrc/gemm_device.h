@@ -67,7 +67,7 @@ struct GemmParams {
   int32_t c_line;                // C rows are 16-byte aligned with unit column stride: full-line store path
   int32_t c_nt;                  // C is larger than the L2s together: store it non-temporal so that it
                                  // does not push operand strips out of them
-  int32_t mx_vec;                // scale rows can be read KSUB bytes at a time
+  int32_t mx_vec;                // a row's scales are consecutive bytes
   int32_t mx_lds;                // scale rows are 16-byte aligned and K/32 is a multiple of 32: stage scales in LDS
   int32_t tiles_m, tiles_n, total_tiles, k_iters;
   int32_t group_m, num_xcds, chunk;
@@ -545,9 +545,9 @@ __device__ __forceinline__ v4f mma(typename Frag<T>::type x, typename Frag<T>::t
 template <class T>
 __device__ __forceinline__ uint32_t load_mx(const uint8_t* rowp, int64_t s_k, int64_t kb, int64_t kb_total, bool vec) {
   if (vec && kb + T::KSUB <= kb_total) {
-    if constexpr (T::KSUB == 4) return *(const uint32_t*)(rowp + kb);
-    if constexpr (T::KSUB == 2) return *(const uint16_t*)(rowp + kb);
-    if constexpr (T::KSUB == 1) return *(rowp + kb);
+    uint32_t v = 0;
+    __builtin_memcpy(&v, rowp + kb, T::KSUB);      // (one load: global memory takes any alignment)
+    return v;
   }
   uint32_t w = 0;
 #pragma unroll

@@ -11,6 +11,9 @@ const Variant g_variants_fp4[] = {
     make_variant<Tile<DT_FP4, 128, 128, 64, 2, 2, LAY_K, LAY_K, 2, true, 2>>(),
     make_variant<Tile<DT_FP4, 64, 64, 128, 2, 2, LAY_K, LAY_K, 4, true, 2>>(),
     make_variant<Tile<DT_FP4, 64, 64, 128, 2, 2, LAY_K, LAY_K, 2, false, 2>>(),
+    // any alignment of the rows, any multiple of 32 values: the scales go straight to registers
+    make_variant<Tile<DT_FP4, 128, 128, 128, 2, 2, LAY_K, LAY_K, 2, LOAD_REGS, 2>>(),
+    make_variant<Tile<DT_FP4, 64, 64, 128, 2, 2, LAY_K, LAY_K, 4, LOAD_REGS, 2>>(),
 };
 const int g_num_variants_fp4 = sizeof(g_variants_fp4) / sizeof(Variant);
 

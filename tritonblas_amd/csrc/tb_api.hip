@@ -301,7 +301,9 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
   // Unit stride along one index, but rows off 16 bytes or with a partial chunk: 16-byte loads through registers, in the
   // tile that was chosen up to 128x128 (1187x3001x1531 bf16: 248 us in the gather kernel, 42 in this one).  Each contiguous index has a chunk at least.
   auto any_alignment = [&](int64_t s_row, int64_t s_k, int64_t rows) {
-    if (usz < 2 || j.num_groups > 0) return -1;
+    if (j.num_groups > 0) return -1;
+    // (one-byte units: whole chunks only.  fp4 1000x4096x4128, whose scale rows cannot be staged: 397 us in the gather kernel, 71 in this one)
+    if (usz == 1) return j.dt == TB_FP4_E2M1 && s_k == 1 && s_row >= 0 && KU % 16 == 0 ? (int)LAY_K : -1;
     if (s_k == 1 && s_row >= 0 && KU >= 16 / usz) return (int)LAY_K;
     return s_row == 1 && s_k >= 0 && rows >= 16 / usz ? (int)LAY_M : -1;
   };
@@ -338,7 +340,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
       if (!known) return TB_ERR_BAD_TILE;
     }
     if (ralay >= 0 && rblay >= 0) {
-      const int side = bm >= 128 ? 128 : 64, k_step = 128 / usz;
+      const int side = bm >= 128 ? 128 : 64, k_step = 128 / usz * epu;
       const bool near = (ralay == LAY_K ? side * j.a_sr : k_step * j.a_sk) * usz < (1ll << 31) && (rblay == LAY_K ? side * j.b_sr : k_step * j.b_sk) * usz < (1ll << 31);
       if (near) v = find_variant(j.dt, side, side, k_step, ralay, rblay, LOAD_REGS);
     }
@@ -365,9 +367,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
   // (8192x28672x8192 FP8 +0.6 %, 8192^3 bf16 +1.6 %; a small C stays cacheable for whoever reads it next)
   p.c_nt = ((int64_t)j.M * j.N * cb > (int64_t)hw.num_xcd * std::max(hw.l2_bytes, 1 << 20)) ? 1 : 0;
   if (j.dt == TB_FP4_E2M1) {
-    const int ksub = v->bk / 128;
-    p.mx_vec = (j.mxa_sk == 1 && j.mxb_sk == 1 && j.mxa_sr % ksub == 0 && j.mxb_sr % ksub == 0 &&
-                ((uintptr_t)j.mxa % ksub) == 0 && ((uintptr_t)j.mxb % ksub) == 0) ? 1 : 0;
+    p.mx_vec = (j.mxa_sk == 1 && j.mxb_sk == 1) ? 1 : 0;
     p.mx_lds = v->fast;
   }
   p.tiles_m = (int32_t)((j.M + v->bm - 1) / v->bm);
