@@ -65,6 +65,26 @@ def test_static_workspace_rejects_what_does_not_fit():
     assert lib.tb_gemm_static_workspace(d, _lib.stream_handle()) == _lib.TB_ERR_WORKSPACE
 
 
+@pytest.mark.parametrize("dtype,m,n,k,grid,tile,b_rows", [
+    (torch.bfloat16, 4352, 4096, 1032, 256, (256, 256, 64), False),    # K is no multiple of the K step
+    (torch.bfloat16, 2176, 2047, 1001, 400, (128, 128, 64), False),    # rows off 16 bytes
+    (torch.float32, 4352, 4096, 1024, 256, (256, 256, 32), True),      # N-contiguous weight
+])
+def test_static_workspace_takes_smaller_tiles(dtype, m, n, k, grid, tile, b_rows):
+    """Operands that the 64x64 gather kernel takes too run there when the chosen tile's partial tiles do not fit.  Whole numbers, exact sums."""
+    from tritonblas_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a = torch.randint(-3, 4, (m, k), device="cuda", generator=g).to(dtype)
+    b = torch.randint(-3, 4, (k, n), device="cuda", generator=g).to(dtype) if b_rows else torch.randint(-3, 4, (n, k), device="cuda", generator=g).to(dtype).T
+    c = torch.empty(m, n, dtype=dtype, device="cuda")
+    d = _desc(_lib, a, b, c, _lib.TB_SCHED_STREAMK, grid)
+    d.block_m, d.block_n, d.block_k = tile
+    assert lib.tb_workspace_bytes(d) > 16 << 20, "the case must not fit"
+    assert lib.tb_gemm_static_workspace(d, _lib.stream_handle()) == _lib.TB_OK
+    assert torch.equal(c, (a.double() @ b.double()).float().to(dtype))
+
+
 def test_static_workspace_status_word():
     """tb_static_workspace_status reads (and clears) the status word a poll-bound Stream-K launch sets in the
     library's own array.  The bound is forced from the host (one poll); every kernel still ends normally."""

@@ -220,6 +220,7 @@ struct Job {
   int bm = 0, bn = 0, bk = 0, group_m = 0, num_xcds = 0;
   int schedule = TB_SCHED_PERSISTENT, grid = 0, counters_per_xcd = 0;
   void* workspace = nullptr; size_t workspace_bytes = 0;
+  bool element_wise = false;      // the gather kernel, whatever the operands allow (see run_plan)
   uint32_t epoch = 1, spin_limit = 0;
   const int32_t* cu_mask = nullptr; int cu_mask_len = 0, ws_mode = 0, ws_local = 0, ws_global = 0;
   // grouped
@@ -317,6 +318,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
                        ((uintptr_t)j.mxa % 16) == 0 && ((uintptr_t)j.mxb % 16) == 0;
     if (!mx_ok || hooks().no_mxlds) fast = false;
   }
+  if (j.element_wise) fast = false;
   if (fast) {
     // 32-bit offsets inside a tile
     if ((alay == LAY_K && (int64_t)bm * j.a_sr * usz >= (1ll << 31)) || (blay == LAY_K && (int64_t)bn * j.b_sr * usz >= (1ll << 31)) ||
@@ -339,7 +341,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
       for (auto& t : tile_infos(j.dt)) known |= (t.bm == bm && t.bn == bn && t.bk == bk);
       if (!known) return TB_ERR_BAD_TILE;
     }
-    if (ralay >= 0 && rblay >= 0) {
+    if (ralay >= 0 && rblay >= 0 && !j.element_wise) {
       const int side = bm >= 128 ? 128 : 64, k_step = 128 / usz * epu;
       const bool near = (ralay == LAY_K ? side * j.a_sr : k_step * j.a_sk) * usz < (1ll << 31) && (rblay == LAY_K ? side * j.b_sr : k_step * j.b_sk) * usz < (1ll << 31);
       if (near) v = find_variant(j.dt, side, side, k_step, ralay, rblay, LOAD_REGS);
@@ -617,6 +619,20 @@ int run_plan(const Job& j, Plan& plan, hipStream_t stream) {
   if (plan.skinny) {
     if (launch_skinny(p, j.dt, stream) != hipSuccess) { (void)hipGetLastError(); return TB_ERR_LAUNCH; }
     return TB_OK;
+  }
+  if (plan.p.mode == MODE_SK && j.num_groups == 0 && j.workspace && j.workspace_bytes < plan.ws_need &&
+      (plan.v->fast == LOAD_REGS || j.K % plan.v->bk != 0 || (j.dt == TB_F32 && (plan.v->alay == LAY_M || plan.v->blay == LAY_M)))) {
+    // Partial tiles of the vector loaders' larger tiles that do not fit the workspace, for operands that the gather kernel
+    // takes just as well: its 64x64 tiles need 16 KB per workgroup instead of up to 256 (bf16 4352x4096x4104 on 256
+    // workgroups: 4 MiB instead of 64, against the 16 MiB of the static workspace).
+    Job small = j;
+    small.element_wise = true;
+    tb_hw hw;
+    int st = current_hw(&hw);
+    Plan gather;
+    if (st == TB_OK) st = make_plan(small, hw, true, &gather);
+    if (st != TB_OK) return st;
+    plan = gather;
   }
   if (plan.ws_need) {
     if (!j.workspace || j.workspace_bytes < plan.ws_need || ((uintptr_t)j.workspace & 255)) return TB_ERR_WORKSPACE;
