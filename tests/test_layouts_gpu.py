@@ -9,6 +9,7 @@ import pytest
 import torch
 
 import tritonblas_amd as tb
+from tritonblas_amd.matmul import streamk_matmul_lt
 
 pytestmark = pytest.mark.gpu
 
@@ -95,3 +96,47 @@ def test_k_that_is_no_multiple_of_the_k_step(schedule, tile, dtype, ta, tb_):
             tb.matmul_lt(a, b, c, sel, config, enable_streamk=schedule == "streamk")
         # (whole numbers below 2**24: the sums are exact and only the result is rounded)
         assert torch.equal(c, (a.double() @ b.double()).float().to(out)), (m, n, k)
+
+
+@pytest.mark.parametrize("types", [(torch.float8_e4m3fn, torch.float8_e5m2), (torch.float8_e5m2, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("tile", [(256, 256), (128, 128), (64, 64)])
+@pytest.mark.parametrize("schedule", ["persistent", "streamk"])
+def test_k_remainder_of_mixed_formats(schedule, tile, types):
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    for m, n, k in [(16, 16, 16), (tile[0] + 16, 2 * tile[1], 144), (272, 304, 592), (520, 512, 1008)]:
+        a, b = _poisoned(gen, m, k, "T", types[0], 16), _poisoned(gen, k, n, "N", types[1], 16)
+        c = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda")
+        sel = tb.OrigamiMatmulSelector(m, n, k, *types, c.dtype, a.device, streamk=schedule == "streamk")
+        sel._sel.block_m, sel._sel.block_n, sel._sel.block_k = tile[0], tile[1], 128
+        tb.matmul_a8w8_lt(a, b, torch.ones(m, device="cuda"), torch.ones(n, device="cuda"), c, sel, tb.matmul_preamble(sel), enable_streamk=schedule == "streamk")
+        assert torch.equal(c, (a.double() @ b.double()).float()), (m, n, k)
+
+
+@pytest.mark.parametrize("k", [16, 144, 1040, 2064])
+@pytest.mark.parametrize("tile", [(None, None, None), (256, 256, 128), (128, 128, 128), (64, 64, 128)])
+def test_grouped_k_remainder(tile, k):
+    """Experts without rows, with one, with ragged last blocks; behind every row of both operands lie NaNs."""
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    counts, n = [70, 0, 1, 257, 300], 200
+    offsets = torch.tensor([0] + counts).cumsum(0)
+    a = _poisoned(gen, sum(counts), k, "T", torch.float8_e4m3fn, 16)
+    w = _poisoned(gen, len(counts) * n, k, "T", torch.float8_e4m3fn, 16).unflatten(0, (len(counts), n))
+    c = torch.full((sum(counts), n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    tb.grouped_matmul_a8w8(a, w, None, None, c, offsets.int().cuda(), *tile)
+    for e, (lo, hi) in enumerate(zip(offsets.tolist(), offsets.tolist()[1:])):
+        assert torch.equal(c[lo:hi], (a[lo:hi].double() @ w[e].double().T).float().to(torch.bfloat16)), e
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_k_remainder_in_more_stream_k_pieces_than_stages(dtype):
+    """A tile cut into pieces of one to three K steps: the remainder lies in one piece only, the first copy stages of the others are whole."""
+    chunk = 16 // dtype.itemsize
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    for grid in (5, 17, 64):
+        m, n, k = 64, 64, 17 * 8 * chunk + 3 * chunk
+        a, b = _poisoned(gen, m, k, "T", dtype, chunk), _poisoned(gen, k, n, "N", dtype, chunk)
+        c = torch.full((m, n), float("nan"), dtype=dtype, device="cuda")
+        sel = tb.OrigamiMatmulSelector(m, n, k, dtype, dtype, dtype, a.device, streamk=True)
+        sel._sel.block_m, sel._sel.block_n, sel._sel.block_k = 64, 64, 8 * chunk
+        streamk_matmul_lt(a, b, c, sel, tb.matmul_preamble(sel), sk_grid=grid)
+        assert torch.equal(c, (a.double() @ b.double()).float().to(dtype)), grid

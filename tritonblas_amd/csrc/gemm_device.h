@@ -63,12 +63,13 @@ struct GemmParams {
   int64_t mxa_sr, mxa_sk, mxb_sr, mxb_sk;  // bytes
   int64_t bias_stride;
   int32_t c_type, bias_type;
-  int32_t a_vec, b_vec, c_vec;   // 16-byte vector access is legal for this operand (c_vec: 4-element rows)
+  int32_t k_tail;                // LOAD_DIRECT: storage units of a last, partial K step, which the kernel takes as step 0; A and B
+                                 // are then one K step in front of the operands, so that step `it` of the whole ones lies at `it` steps
+  int32_t c_vec;                 // C rows hold whole groups of 4 elements
   int32_t c_line;                // C rows are 16-byte aligned with unit column stride: full-line store path
   int32_t c_nt;                  // C is larger than the L2s together: store it non-temporal so that it
                                  // does not push operand strips out of them
   int32_t mx_vec;                // a row's scales are consecutive bytes
-  int32_t mx_lds;                // scale rows are 16-byte aligned and K/32 is a multiple of 32: stage scales in LDS
   int32_t tiles_m, tiles_n, total_tiles, k_iters;
   int32_t group_m, num_xcds, chunk;
   int32_t panel_n;               // tile order: column panels of this many tiles, swept top to bottom (0: one panel)
@@ -312,13 +313,13 @@ struct Operand {
     uint32_t off[NCH];       // per-slot byte offset from the K-step origin (LOAD_REGS: signed)
     int64_t s_row, s_k;      // storage units
     int row0, row_lim;
-    int whole_steps, tail;   // K steps without a remainder, storage units in the one behind them
+    int whole_steps, tail;   // LOAD_REGS: K steps without a remainder, storage units in the one behind them
   };
 
   __device__ static __forceinline__ void init(St& st, const uint8_t* mat, int64_t s_row, int64_t s_k, int row0,
                                               int row_lim, int64_t KU, int tid) {
     st.s_row = s_row; st.s_k = s_k; st.row0 = row0; st.row_lim = row_lim;
-    st.whole_steps = (int)(KU / T::UPS); st.tail = (int)(KU % T::UPS);
+    if constexpr (T::REGS) { st.whole_steps = (int)(KU / T::UPS); st.tail = (int)(KU % T::UPS); }
     const int rows_valid = row_lim - row0;
     if constexpr (T::LOADER == LOAD_GATHER) {
       st.base = mat;
@@ -375,18 +376,20 @@ struct Operand {
     }
   }
 
-  // The step behind the last whole one: chunks beyond K come from a chunk of zeros, so the lanes need 64-bit
-  // addresses; as many copies as in a whole step, so the waits stay the same.  (4096x4096x14352 FP8: 6160 us with
-  // the gather kernel, 234 here; 2048x2048x2056 bf16 364 and 34 us.)
-  __device__ static __forceinline__ void dma_tail(const St& st, int it, uint8_t* lds, int tid) {
-    const uint8_t* gp = step_ptr(st, it);
+  // The remainder of K, k_tail storage units behind the K steps in front of step `end`: chunks beyond K come from a chunk of
+  // zeros, so the lanes need 64-bit addresses; as many copies as in a whole step, so the waits stay the same.  It is taken as
+  // step 0, whose copy stands in front of the K loop: as the last step it put a second form of the copies into the loop, and calls
+  // without a remainder paid for it (2048^3 bf16 26.0 -> 27.0 us, 100x4096x4096 FP8 11.3 -> 12.6; 26.1 and 11.6 this way).
+  // (4096x4096x14352 FP8: 6250 us with the gather kernel, 226 here; 2048x2048x2056 bf16 255 and 33 us.)
+  __device__ static __forceinline__ void dma_tail(const St& st, int end, int k_tail, uint8_t* lds, int tid) {
+    const uint8_t* gp = step_ptr(st, end);
     const int wave_slot = __builtin_amdgcn_readfirstlane(tid & ~63);
     const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) uint8_t*)lds);
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       if (CHUNKS % T::THREADS != 0 && i * T::THREADS + wave_slot >= CHUNKS) continue;
       const uint32_t dst = lds0 + (uint32_t)((i * T::THREADS + wave_slot) * 16);
-      const uint8_t* src = slot_k(i * T::THREADS + tid) < st.tail ? gp + st.off[i] : (const uint8_t*)&g_zero_chunk;
+      const uint8_t* src = slot_k(i * T::THREADS + tid) < k_tail ? gp + st.off[i] : (const uint8_t*)&g_zero_chunk;
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(dst), "v"(src) : "memory", "m0");
     }
   }
@@ -716,22 +719,22 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
       sc_dma(g0);
       if ((g0 + 1) * T::SCG < it1) sc_dma(g0 + 1);
     }
-    // both operands' copies of K step `it` into stage s (the one test keeps the loop's copies in line)
+    // both operands' copies of K step `it` into stage s
     auto copy_step = [&](int it, int s) {
       uint8_t* to = lds + s * T::STAGE_BYTES;
-      if (T::DT == DT_FP4 || __builtin_expect(it < sa.whole_steps, 1)) {
-        OA::dma(sa, it, to, li.tid);
-        OB::dma(sb, it, to + T::A_BYTES, li.tid);
-      } else {
-        OA::dma_tail(sa, it, to, li.tid);
-        OB::dma_tail(sb, it, to + T::A_BYTES, li.tid);
-      }
+      OA::dma(sa, it, to, li.tid);
+      OB::dma(sb, it, to + T::A_BYTES, li.tid);
     };
     int issued = 0;
 #pragma unroll
     for (int s = 0; s < S; ++s) {
       if (it0 + s < it1) {
-        copy_step(it0 + s, s);
+        if (T::DT != DT_FP4 && s == 0 && it0 == 0 && __builtin_expect(p.k_tail != 0, 0)) {
+          OA::dma_tail(sa, p.k_iters, p.k_tail, lds, li.tid);
+          OB::dma_tail(sb, p.k_iters, p.k_tail, lds + T::A_BYTES, li.tid);
+        } else {
+          copy_step(it0 + s, s);
+        }
         ++issued;
       }
     }

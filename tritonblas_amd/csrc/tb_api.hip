@@ -361,7 +361,6 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
   p.c_sm = j.c_sm; p.c_sn = j.c_sn;
   p.mxa_sr = j.mxa_sr; p.mxa_sk = j.mxa_sk; p.mxb_sr = j.mxb_sr; p.mxb_sk = j.mxb_sk;
   p.bias_stride = j.bias_stride; p.c_type = j.c_type; p.bias_type = j.bias_type;
-  p.a_vec = p.b_vec = v->fast;
   const int cb = c_bytes(j.c_type);
   p.c_vec = (j.c_sn == 1 && (j.c_sm % 4 == 0 || j.M == 1) && ((uintptr_t)j.C % (4 * cb)) == 0) ? 1 : 0;
   p.c_line = (j.c_type != TB_I8 && !is_f8_type(j.c_type) && j.c_sn == 1 && ((j.c_sm * cb) % 16 == 0 || j.M == 1) && ((uintptr_t)j.C % 16) == 0) ? 1 : 0;
@@ -370,7 +369,6 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
   p.c_nt = ((int64_t)j.M * j.N * cb > (int64_t)hw.num_xcd * std::max(hw.l2_bytes, 1 << 20)) ? 1 : 0;
   if (j.dt == TB_FP4_E2M1) {
     p.mx_vec = (j.mxa_sk == 1 && j.mxb_sk == 1) ? 1 : 0;
-    p.mx_lds = v->fast;
   }
   p.tiles_m = (int32_t)((j.M + v->bm - 1) / v->bm);
   p.tiles_n = (int32_t)((j.N + v->bn - 1) / v->bn);
@@ -643,6 +641,14 @@ int run_plan(const Job& j, Plan& plan, hipStream_t stream) {
     p.ctl = (uint32_t*)ws;
     if (p.mode == MODE_WS || p.sk_ws) p.counters = (int32_t*)(ws + plan.ws_counters_off);
     if (p.mode == MODE_SK || p.grp_sk) { p.flags = (uint32_t*)(ws + plan.ws_flags_off); p.P = (float*)(ws + plan.ws_p_off); }
+  }
+  const Variant* v = plan.v;
+  p.A = (const uint8_t*)j.A; p.B = (const uint8_t*)j.B;
+  p.k_tail = v->fast == LOAD_DIRECT && j.dt != TB_FP4_E2M1 ? (int32_t)(j.K % v->bk) : 0;
+  if (p.k_tail) {
+    const int64_t step = (int64_t)v->bk * unit_bytes(j.dt);
+    p.A -= v->alay == LAY_K ? step : step * j.a_sk;
+    p.B -= v->blay == LAY_K ? step : step * j.b_sk;
   }
   void* args[] = {(void*)&p};
   const void* kern = (p.mode == MODE_SK || p.grp_sk) ? plan.v->kernel_sk : plan.v->kernel;
