@@ -81,3 +81,14 @@ def test_which_rows_the_kernel_takes(shape, axis, want):
         assert U._rows(x.T, 0) == want
         assert U._rows(x[:, ::2], 1) is None
         assert U._rows(x[:1].expand(4, 8), 1) is None
+
+
+@pytest.mark.gpu
+def test_more_rows_than_one_launch_has_threads_for():
+    """2**26 rows: HIP refuses launches of 2**32 threads and more."""
+    x = torch.randn(2 ** 26 + 3, 8, device="cuda", dtype=torch.bfloat16)
+    q, s = U.quantize_tensor_per_channel(x, torch.int8, 1)
+    for rows in (slice(0, 4096), slice(2 ** 25 - 5, 2 ** 25 + 4096), slice(2 ** 26 - 4096, None)):
+        wq, ws = _by_tensor_operations(x[rows], torch.int8, 1)
+        assert torch.equal(q[rows], wq) and torch.equal(s[rows], ws)
+    assert bool((s > 0).all())

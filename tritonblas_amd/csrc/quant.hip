@@ -308,66 +308,68 @@ __global__ __launch_bounds__(RT < 256 ? 256 : RT) void row_quant_kernel(const Ro
   constexpr int XB = XT == QT_F32 ? 4 : 2;
   constexpr int WAVES = RT / 64;
   __shared__ uint32_t part[WAVES > 1 ? WAVES : 1];
-  const int64_t row = (int64_t)blockIdx.x * ROWS + threadIdx.x / RT;
-  if (ROWS > 1 && row >= p.m) return;          // (a whole wave: its lanes share the row)
   const int t = threadIdx.x % RT;
-  const uint8_t* xr = p.x + row * p.x_stride * XB;
-  const int64_t chunks = (p.n + 7) >> 3;
+  const int64_t stride = (int64_t)gridDim.x * ROWS;
+  for (int64_t row = (int64_t)blockIdx.x * ROWS + threadIdx.x / RT; row < p.m; row += stride) {
+    const uint8_t* xr = p.x + row * p.x_stride * XB;
+    const int64_t chunks = (p.n + 7) >> 3;
 
-  row_chunk<XT> r[CH];
-  uint32_t m = 0;
-  if constexpr (LOOP) {
-    for (int64_t c0 = 0; c0 < chunks; c0 += (int64_t)RT * CH) {
+    row_chunk<XT> r[CH];
+    uint32_t m = 0;
+    if constexpr (LOOP) {
+      for (int64_t c0 = 0; c0 < chunks; c0 += (int64_t)RT * CH) {
 #pragma unroll
-      for (int i = 0; i < CH; ++i) r[i] = row_load<XT, VEC>(xr, c0 + i * RT + t, p.n);
+        for (int i = 0; i < CH; ++i) r[i] = row_load<XT, VEC>(xr, c0 + i * RT + t, p.n);
+#pragma unroll
+        for (int i = 0; i < CH; ++i) m = row_amax<XT>(r[i], m);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < CH; ++i) r[i] = row_load<XT, VEC>(xr, i * RT + t, p.n);
 #pragma unroll
       for (int i = 0; i < CH; ++i) m = row_amax<XT>(r[i], m);
     }
-  } else {
 #pragma unroll
-    for (int i = 0; i < CH; ++i) r[i] = row_load<XT, VEC>(xr, i * RT + t, p.n);
+    for (int d = 32; d > 0; d >>= 1) {
+      const uint32_t o = (uint32_t)__shfl_xor((int)m, d);
+      m = o > m ? o : m;
+    }
+    if constexpr (WAVES > 1) {
+      if ((t & 63) == 0) part[t >> 6] = m;
+      __syncthreads();
 #pragma unroll
-    for (int i = 0; i < CH; ++i) m = row_amax<XT>(r[i], m);
-  }
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) {
-    const uint32_t o = (uint32_t)__shfl_xor((int)m, d);
-    m = o > m ? o : m;
-  }
-  if constexpr (WAVES > 1) {
-    if ((t & 63) == 0) part[t >> 6] = m;
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) m = part[w] > m ? part[w] : m;
-  }
-  const float amax = __builtin_bit_cast(float, m);
-  const float top = amax < p.min_scale ? p.min_scale : amax;     // (a NaN stays)
-  const float scale = top * p.inv_top;
-  const float inv = 1.0f / scale;
-  if (t == 0) p.scale[row] = scale;
+      for (int w = 0; w < WAVES; ++w) m = part[w] > m ? part[w] : m;
+    }
+    const float amax = __builtin_bit_cast(float, m);
+    const float top = amax < p.min_scale ? p.min_scale : amax;     // (a NaN stays)
+    const float scale = top * p.inv_top;
+    const float inv = 1.0f / scale;
+    if (t == 0) p.scale[row] = scale;
 
-  uint8_t* qr = p.q + row * p.n;
-  auto put = [&](int64_t c, const row_chunk<XT>& x) {
-    const int64_t left = p.n - c * 8;
-    if (left <= 0) return;
-    const uint64_t w = row_codes<XT, OT>(x, inv);
-    if constexpr (VEC) {
-      *(uint64_t*)(qr + c * 8) = w;
+    uint8_t* qr = p.q + row * p.n;
+    auto put = [&](int64_t c, const row_chunk<XT>& x) {
+      const int64_t left = p.n - c * 8;
+      if (left <= 0) return;
+      const uint64_t w = row_codes<XT, OT>(x, inv);
+      if constexpr (VEC) {
+        *(uint64_t*)(qr + c * 8) = w;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) if (j < left) qr[c * 8 + j] = (uint8_t)(w >> (8 * j));
+      }
+    };
+    if constexpr (LOOP) {
+      for (int64_t c0 = 0; c0 < chunks; c0 += (int64_t)RT * CH) {
+#pragma unroll
+        for (int i = 0; i < CH; ++i) r[i] = row_load<XT, VEC>(xr, c0 + i * RT + t, p.n);
+#pragma unroll
+        for (int i = 0; i < CH; ++i) put(c0 + i * RT + t, r[i]);
+      }
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) if (j < left) qr[c * 8 + j] = (uint8_t)(w >> (8 * j));
+      for (int i = 0; i < CH; ++i) put(i * RT + t, r[i]);
     }
-  };
-  if constexpr (LOOP) {
-    for (int64_t c0 = 0; c0 < chunks; c0 += (int64_t)RT * CH) {
-#pragma unroll
-      for (int i = 0; i < CH; ++i) r[i] = row_load<XT, VEC>(xr, c0 + i * RT + t, p.n);
-#pragma unroll
-      for (int i = 0; i < CH; ++i) put(c0 + i * RT + t, r[i]);
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < CH; ++i) put(i * RT + t, r[i]);
+    if constexpr (WAVES > 1) { if (row + stride < p.m) __syncthreads(); }      // (`part` is read before it is written again)
   }
 }
 
@@ -375,8 +377,8 @@ template <int XT, int OT, int RT, int CH, bool LOOP = false>
 static hipError_t row_quant_t(const RowQuantParams& p, hipStream_t stream) {
   constexpr int ROWS = RT < 256 ? 256 / RT : 1;
   constexpr int XB = XT == QT_F32 ? 4 : 2;
-  const int64_t grid = (p.m + ROWS - 1) / ROWS;
-  if (grid > INT32_MAX) return hipErrorInvalidValue;
+  // (a launch takes less than 2^32 threads; a workgroup goes on to further rows)
+  const int64_t blocks = (p.m + ROWS - 1) / ROWS, most = (1ll << 31) / (RT < 256 ? 256 : RT), grid = blocks < most ? blocks : most;
   const bool vec = p.n % 8 == 0 && ((uintptr_t)p.x & 15) == 0 && (p.x_stride * XB) % 16 == 0 && ((uintptr_t)p.q & 7) == 0;
   const dim3 block(RT < 256 ? 256 : RT);
   if (vec) hipLaunchKernelGGL((row_quant_kernel<XT, OT, RT, CH, true, LOOP>), dim3((unsigned)grid), block, 0, stream, p);
