@@ -32,7 +32,7 @@ def _same(x, dtype, axis, **kw):
 @pytest.mark.parametrize("dtype", DTYPES8)
 @pytest.mark.parametrize("src", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("shape", [(1, 1), (3, 7), (5, 4096), (2049, 1024), (2050, 4096), (300, 4104), (257, 16384), (2, 16392), (3, 32776),
-                                   (2, 65536), (2, 65544), (700, 999)])
+                                   (2, 65536), (2, 65544), (700, 999), (1, 8), (70001, 1), (5000, 8), (4099, 9), (3001, 64), (2050, 65), (40, 5)])
 def test_rows_match_the_tensor_operations(shape, src, dtype):
     g = torch.Generator(device="cuda").manual_seed(shape[0] * 7 + shape[1])
     x = (torch.randn(shape, device="cuda", generator=g) * torch.logspace(-4, 3, shape[0], device="cuda").unsqueeze(1)).to(src)

@@ -180,8 +180,10 @@ hipError_t launch_quant(const QuantParams& p, int x_type, bool hadamard, bool fo
 // one float.  Written as tensor operations (convert, abs, amax, clamp, two scalings, product, convert) the same values cost nine
 // launches and five passes over fp32 copies of x: quantising 512x14336 bf16 and multiplying by a 4096x14336 e4m3 weight took
 // 114 us as tensor operations + GEMM and takes 54 us with this kernel (49 us of it the GEMM).
-// RT threads share a row: a wave while 4096 values fit its registers, a workgroup of 256 up to 16384, 1024 threads beyond.
-// Few rows: more threads per row, so that the loads of a row are spread over the CU (launch_row_quant).  Rows longer than 65536
+// RT threads share a row: one while a chunk of eight values holds it, eight up to 64 values, a wave while 4096 values fit its
+// registers, a workgroup of 256 up to 16384, 1024 threads beyond.  Few rows: more threads per row, so that the loads of a row are
+// spread over the CU (launch_row_quant).  Short rows are bound by wavefronts, not by bytes: 2^24 rows of 8 bf16 take
+// 81 us with a thread each, 4360 with a wave each and 1273 as tensor operations; 2^20 rows of 64 take 39, 286 and 640.  Rows longer than 65536
 // values are read twice (LOOP), the second time mostly from the caches.
 struct RowChunk16 { v4i a; };
 struct RowChunk32 { v4i a, b; };
@@ -330,7 +332,7 @@ __global__ __launch_bounds__(RT < 256 ? 256 : RT) void row_quant_kernel(const Ro
       for (int i = 0; i < CH; ++i) m = row_amax<XT>(r[i], m);
     }
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
+    for (int d = (RT < 64 ? RT : 64) / 2; d > 0; d >>= 1) {
       const uint32_t o = (uint32_t)__shfl_xor((int)m, d);
       m = o > m ? o : m;
     }
@@ -389,6 +391,8 @@ static hipError_t row_quant_t(const RowQuantParams& p, hipStream_t stream) {
 template <int XT, int OT>
 static hipError_t row_quant_o(const RowQuantParams& p, hipStream_t stream) {
   const int64_t chunks = (p.n + 7) / 8;
+  if (chunks <= 1) return row_quant_t<XT, OT, 1, 1>(p, stream);
+  if (chunks <= 8) return row_quant_t<XT, OT, 8, 1>(p, stream);
   // (a wave per row only where the rows alone fill the device: 256 CUs x 8 waves)
   if (chunks <= 64 * 2 && p.m >= 2048) return row_quant_t<XT, OT, 64, 2>(p, stream);
   if (chunks <= 64 * 8 && p.m >= 2048) return row_quant_t<XT, OT, 64, 8>(p, stream);
