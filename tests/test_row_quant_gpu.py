@@ -92,3 +92,17 @@ def test_more_rows_than_one_launch_has_threads_for():
         wq, ws = _by_tensor_operations(x[rows], torch.int8, 1)
         assert torch.equal(q[rows], wq) and torch.equal(s[rows], ws)
     assert bool((s > 0).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES8)
+@pytest.mark.parametrize("shape", [(3, 131073), (2, 131080), (255, 147456), (256, 147456), (2, 200003), (1, (1 << 22) + 5), (1, 1 << 22)])
+def test_rows_in_parts(shape, dtype):
+    """Several workgroups to a row: their maxima, one scale, their codes."""
+    x = torch.randn(shape, device="cuda").bfloat16()
+    x[0, -1] = 9.0
+    if shape[0] > 1:
+        x[1, 16383], x[-1, 65536:] = float("nan") if shape[0] == 3 else -7.0, 0
+    _same(x, dtype, 1)
+    _same(x[:, 1:], dtype, 1)
+    _same(x.float(), dtype, 1, min_scale=20.0)

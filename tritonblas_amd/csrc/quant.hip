@@ -183,8 +183,8 @@ hipError_t launch_quant(const QuantParams& p, int x_type, bool hadamard, bool fo
 // RT threads share a row: one while a chunk of eight values holds it, eight up to 64 values, a wave while 4096 values fit its
 // registers, a workgroup of 256 up to 16384, 1024 threads beyond.  Few rows: more threads per row, so that the loads of a row are
 // spread over the CU (launch_row_quant).  Short rows are bound by wavefronts, not by bytes: 2^24 rows of 8 bf16 take
-// 81 us with a thread each, 4360 with a wave each and 1273 as tensor operations; 2^20 rows of 64 take 39, 286 and 640.  Rows longer than 65536
-// values are read twice (LOOP), the second time mostly from the caches.
+// 81 us with a thread each, 4360 with a wave each and 1273 as tensor operations; 2^20 rows of 64 take 39, 286 and 640.
+// Rows longer than 65536 values are read twice (LOOP), the second time mostly from the caches, or cut into parts, see below.
 struct RowChunk16 { v4i a; };
 struct RowChunk32 { v4i a, b; };
 
@@ -304,87 +304,151 @@ __device__ __forceinline__ uint64_t row_codes(const row_chunk<XT>& r, float inv)
   return (uint64_t)w[0] | ((uint64_t)w[1] << 32);
 }
 
+// the largest m of the RT threads (a power of two) that share a row; `part`: one word per wave of the workgroup
+template <int RT>
+__device__ __forceinline__ uint32_t row_max(uint32_t m, uint32_t* part) {
+#pragma unroll
+  for (int d = (RT < 64 ? RT : 64) / 2; d > 0; d >>= 1) {
+    const uint32_t o = (uint32_t)__shfl_xor((int)m, d);
+    m = o > m ? o : m;
+  }
+  if constexpr (RT > 64) {
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < RT / 64; ++w) m = part[w] > m ? part[w] : m;
+  }
+  return m;
+}
+
+__device__ __forceinline__ float row_scale(const RowQuantParams& p, uint32_t m) {
+  const float amax = __builtin_bit_cast(float, m);
+  return (amax < p.min_scale ? p.min_scale : amax) * p.inv_top;     // (a NaN stays)
+}
+
+// codes of chunk c of a row to where they belong
+template <int XT, int OT, bool VEC>
+__device__ __forceinline__ void row_store(uint8_t* qr, int64_t c, int64_t n, const row_chunk<XT>& x, float inv) {
+  const int64_t left = n - c * 8;
+  if (left <= 0) return;
+  const uint64_t w = row_codes<XT, OT>(x, inv);
+  if constexpr (VEC) {
+    *(uint64_t*)(qr + c * 8) = w;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) if (j < left) qr[c * 8 + j] = (uint8_t)(w >> (8 * j));
+  }
+}
+
 template <int XT, int OT, int RT, int CH, bool VEC, bool LOOP>
 __global__ __launch_bounds__(RT < 256 ? 256 : RT) void row_quant_kernel(const RowQuantParams p) {
   constexpr int ROWS = RT < 256 ? 256 / RT : 1;
   constexpr int XB = XT == QT_F32 ? 4 : 2;
-  constexpr int WAVES = RT / 64;
-  __shared__ uint32_t part[WAVES > 1 ? WAVES : 1];
+  __shared__ uint32_t part[RT > 64 ? RT / 64 : 1];
   const int t = threadIdx.x % RT;
   const int64_t stride = (int64_t)gridDim.x * ROWS;
   for (int64_t row = (int64_t)blockIdx.x * ROWS + threadIdx.x / RT; row < p.m; row += stride) {
     const uint8_t* xr = p.x + row * p.x_stride * XB;
-    const int64_t chunks = (p.n + 7) >> 3;
-
     row_chunk<XT> r[CH];
     uint32_t m = 0;
-    if constexpr (LOOP) {
-      for (int64_t c0 = 0; c0 < chunks; c0 += (int64_t)RT * CH) {
+    const int64_t chunks = LOOP ? (p.n + 7) >> 3 : 1;
+    for (int64_t c0 = 0; c0 < chunks; c0 += (int64_t)RT * CH) {
 #pragma unroll
-        for (int i = 0; i < CH; ++i) r[i] = row_load<XT, VEC>(xr, c0 + i * RT + t, p.n);
-#pragma unroll
-        for (int i = 0; i < CH; ++i) m = row_amax<XT>(r[i], m);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < CH; ++i) r[i] = row_load<XT, VEC>(xr, i * RT + t, p.n);
+      for (int i = 0; i < CH; ++i) r[i] = row_load<XT, VEC>(xr, c0 + i * RT + t, p.n);
 #pragma unroll
       for (int i = 0; i < CH; ++i) m = row_amax<XT>(r[i], m);
     }
-#pragma unroll
-    for (int d = (RT < 64 ? RT : 64) / 2; d > 0; d >>= 1) {
-      const uint32_t o = (uint32_t)__shfl_xor((int)m, d);
-      m = o > m ? o : m;
-    }
-    if constexpr (WAVES > 1) {
-      if ((t & 63) == 0) part[t >> 6] = m;
-      __syncthreads();
-#pragma unroll
-      for (int w = 0; w < WAVES; ++w) m = part[w] > m ? part[w] : m;
-    }
-    const float amax = __builtin_bit_cast(float, m);
-    const float top = amax < p.min_scale ? p.min_scale : amax;     // (a NaN stays)
-    const float scale = top * p.inv_top;
-    const float inv = 1.0f / scale;
+    m = row_max<RT>(m, part);
+    const float scale = row_scale(p, m), inv = 1.0f / scale;
     if (t == 0) p.scale[row] = scale;
-
-    uint8_t* qr = p.q + row * p.n;
-    auto put = [&](int64_t c, const row_chunk<XT>& x) {
-      const int64_t left = p.n - c * 8;
-      if (left <= 0) return;
-      const uint64_t w = row_codes<XT, OT>(x, inv);
-      if constexpr (VEC) {
-        *(uint64_t*)(qr + c * 8) = w;
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) if (j < left) qr[c * 8 + j] = (uint8_t)(w >> (8 * j));
-      }
-    };
-    if constexpr (LOOP) {
-      for (int64_t c0 = 0; c0 < chunks; c0 += (int64_t)RT * CH) {
+    for (int64_t c0 = 0; c0 < chunks; c0 += (int64_t)RT * CH) {
+      if constexpr (LOOP) {
 #pragma unroll
         for (int i = 0; i < CH; ++i) r[i] = row_load<XT, VEC>(xr, c0 + i * RT + t, p.n);
-#pragma unroll
-        for (int i = 0; i < CH; ++i) put(c0 + i * RT + t, r[i]);
       }
-    } else {
 #pragma unroll
-      for (int i = 0; i < CH; ++i) put(i * RT + t, r[i]);
+      for (int i = 0; i < CH; ++i) row_store<XT, OT, VEC>(p.q + row * p.n, c0 + i * RT + t, p.n, r[i], inv);
     }
-    if constexpr (WAVES > 1) { if (row + stride < p.m) __syncthreads(); }      // (`part` is read before it is written again)
+    if constexpr (RT > 64) { if (row + stride < p.m) __syncthreads(); }      // (`part` is read before it is written again)
   }
+}
+
+// Few very long rows, in parts of 16384 values with a workgroup each and three launches: amax of the parts, scale of the row, codes
+// of the parts.  The parts' amax wait where the row's first codes will be, which the third launch writes.  One workgroup for a row
+// reads 40 GB/s: a row of 2^22 bf16 418 us, 21 in parts, 49 as tensor operations; of 2^24 1650, 21 and 99.
+constexpr int ROW_PART_T = 256, ROW_PART_CH = 8;
+constexpr int64_t ROW_PART_CHUNKS = ROW_PART_T * ROW_PART_CH;
+
+template <int XT, bool VEC>
+__global__ __launch_bounds__(ROW_PART_T) void row_part_amax_kernel(const RowQuantParams p, int parts) {
+  constexpr int XB = XT == QT_F32 ? 4 : 2;
+  __shared__ uint32_t lds[ROW_PART_T / 64];
+  const int64_t row = blockIdx.x / (unsigned)parts, part = blockIdx.x % (unsigned)parts;
+  const uint8_t* xr = p.x + row * p.x_stride * XB;
+  row_chunk<XT> r[ROW_PART_CH];
+  uint32_t m = 0;
+#pragma unroll
+  for (int i = 0; i < ROW_PART_CH; ++i) r[i] = row_load<XT, VEC>(xr, part * ROW_PART_CHUNKS + i * ROW_PART_T + threadIdx.x, p.n);
+#pragma unroll
+  for (int i = 0; i < ROW_PART_CH; ++i) m = row_amax<XT>(r[i], m);
+  m = row_max<ROW_PART_T>(m, lds);
+  if (threadIdx.x == 0) __builtin_memcpy(p.q + row * p.n + part * 4, &m, 4);
+}
+
+__global__ __launch_bounds__(64) void row_part_scale_kernel(const RowQuantParams p, int parts) {
+  const int64_t row = blockIdx.x;
+  uint32_t m = 0;
+  for (int i = threadIdx.x; i < parts; i += 64) {
+    uint32_t v;
+    __builtin_memcpy(&v, p.q + row * p.n + (int64_t)i * 4, 4);
+    m = v > m ? v : m;
+  }
+  m = row_max<64>(m, nullptr);
+  if (threadIdx.x == 0) p.scale[row] = row_scale(p, m);
+}
+
+template <int XT, int OT, bool VEC>
+__global__ __launch_bounds__(ROW_PART_T) void row_part_codes_kernel(const RowQuantParams p, int parts) {
+  constexpr int XB = XT == QT_F32 ? 4 : 2;
+  const int64_t row = blockIdx.x / (unsigned)parts, part = blockIdx.x % (unsigned)parts;
+  const uint8_t* xr = p.x + row * p.x_stride * XB;
+  const float inv = 1.0f / p.scale[row];
+  row_chunk<XT> r[ROW_PART_CH];
+#pragma unroll
+  for (int i = 0; i < ROW_PART_CH; ++i) r[i] = row_load<XT, VEC>(xr, part * ROW_PART_CHUNKS + i * ROW_PART_T + threadIdx.x, p.n);
+#pragma unroll
+  for (int i = 0; i < ROW_PART_CH; ++i)
+    row_store<XT, OT, VEC>(p.q + row * p.n, part * ROW_PART_CHUNKS + i * ROW_PART_T + threadIdx.x, p.n, r[i], inv);
+}
+
+template <int XT>
+static bool row_vec(const RowQuantParams& p) {
+  constexpr int XB = XT == QT_F32 ? 4 : 2;
+  return p.n % 8 == 0 && ((uintptr_t)p.x & 15) == 0 && (p.x_stride * XB) % 16 == 0 && ((uintptr_t)p.q & 7) == 0;
 }
 
 template <int XT, int OT, int RT, int CH, bool LOOP = false>
 static hipError_t row_quant_t(const RowQuantParams& p, hipStream_t stream) {
-  constexpr int ROWS = RT < 256 ? 256 / RT : 1;
-  constexpr int XB = XT == QT_F32 ? 4 : 2;
+  constexpr int ROWS = RT < 256 ? 256 / RT : 1, THREADS = RT < 256 ? 256 : RT;
   // (a launch takes less than 2^32 threads; a workgroup goes on to further rows)
-  const int64_t blocks = (p.m + ROWS - 1) / ROWS, most = (1ll << 31) / (RT < 256 ? 256 : RT), grid = blocks < most ? blocks : most;
-  const bool vec = p.n % 8 == 0 && ((uintptr_t)p.x & 15) == 0 && (p.x_stride * XB) % 16 == 0 && ((uintptr_t)p.q & 7) == 0;
-  const dim3 block(RT < 256 ? 256 : RT);
-  if (vec) hipLaunchKernelGGL((row_quant_kernel<XT, OT, RT, CH, true, LOOP>), dim3((unsigned)grid), block, 0, stream, p);
-  else hipLaunchKernelGGL((row_quant_kernel<XT, OT, RT, CH, false, LOOP>), dim3((unsigned)grid), block, 0, stream, p);
+  const int64_t blocks = (p.m + ROWS - 1) / ROWS, most = (1ll << 31) / THREADS;
+  const dim3 grid((unsigned)(blocks < most ? blocks : most));
+  if (row_vec<XT>(p)) hipLaunchKernelGGL((row_quant_kernel<XT, OT, RT, CH, true, LOOP>), grid, dim3(THREADS), 0, stream, p);
+  else hipLaunchKernelGGL((row_quant_kernel<XT, OT, RT, CH, false, LOOP>), grid, dim3(THREADS), 0, stream, p);
+  return hipGetLastError();
+}
+
+template <int XT, int OT>
+static hipError_t row_quant_parts(const RowQuantParams& p, hipStream_t stream) {
+  const int64_t parts = ((p.n + 7) / 8 + ROW_PART_CHUNKS - 1) / ROW_PART_CHUNKS;
+  if (parts * p.m >= (1ll << 32) / ROW_PART_T) return hipErrorInvalidValue;      // (2^38 values)
+  const dim3 grid((unsigned)(parts * p.m));
+  const bool vec = row_vec<XT>(p);
+  if (vec) hipLaunchKernelGGL((row_part_amax_kernel<XT, true>), grid, dim3(ROW_PART_T), 0, stream, p, (int)parts);
+  else hipLaunchKernelGGL((row_part_amax_kernel<XT, false>), grid, dim3(ROW_PART_T), 0, stream, p, (int)parts);
+  hipLaunchKernelGGL(row_part_scale_kernel, dim3((unsigned)p.m), dim3(64), 0, stream, p, (int)parts);
+  if (vec) hipLaunchKernelGGL((row_part_codes_kernel<XT, OT, true>), grid, dim3(ROW_PART_T), 0, stream, p, (int)parts);
+  else hipLaunchKernelGGL((row_part_codes_kernel<XT, OT, false>), grid, dim3(ROW_PART_T), 0, stream, p, (int)parts);
   return hipGetLastError();
 }
 
@@ -400,7 +464,10 @@ static hipError_t row_quant_o(const RowQuantParams& p, hipStream_t stream) {
   if (chunks <= 256 * 8 && p.m >= 256) return row_quant_t<XT, OT, 256, 8>(p, stream);
   if (chunks <= 1024 * 4) return row_quant_t<XT, OT, 1024, 4>(p, stream);
   if (chunks <= 1024 * 8) return row_quant_t<XT, OT, 1024, 8>(p, stream);
-  return row_quant_t<XT, OT, 1024, 4, true>(p, stream);
+  // (a row of up to 2^17 values takes one workgroup less time than two more launches; 256 rows keep every CU reading, and read the
+  // second time from the caches: 512x131072 bf16 55 us, in parts 62)
+  if (chunks <= 1 << 14 || p.m >= 256) return row_quant_t<XT, OT, 1024, 4, true>(p, stream);
+  return row_quant_parts<XT, OT>(p, stream);
 }
 
 template <int XT>
