@@ -175,14 +175,18 @@ typedef struct tb_gemm_desc {
  * Replaces persistent_matmul_lt / streamk_matmul_lt (matmul.py:69-366). */
 int tb_gemm(const tb_gemm_desc* desc, void* stream);
 
-/* Bytes of workspace tb_gemm needs for this descriptor (0 for the persistent schedule). */
+/* Bytes of workspace tb_gemm needs for this descriptor (0 for the persistent schedule).  With fewer a launch is
+ * refused with TB_ERR_WORKSPACE; a Stream-K launch whose operands have rows off 16 bytes, a K that is no
+ * multiple of the K step, or fp32 values that are not K-contiguous runs on 64x64 tiles first, whose partial
+ * tiles take 16 KB per workgroup, and is refused if those do not fit either. */
 size_t tb_workspace_bytes(const tb_gemm_desc* desc);
 
 /* tb_gemm without a workspace from the caller and without any allocation: the queue counters, Stream-K
  * flags and partial tiles live in a buffer of TB_STATIC_WORKSPACE_BYTES that is part of the library's
  * device image (every GPU the library runs on holds it until the process ends).  desc->workspace,
  * workspace_bytes and epoch are ignored (the buffer counts its own launches, TB_EPOCH_ON_DEVICE); a launch that
- * needs more than TB_STATIC_WORKSPACE_BYTES is refused with TB_ERR_WORKSPACE.  No counterpart in the
+ * needs more than TB_STATIC_WORKSPACE_BYTES is refused with TB_ERR_WORKSPACE, but for the operands that go
+ * back to 64x64 tiles (see tb_workspace_bytes).  No counterpart in the
  * reference: it is for callers that cannot allocate device memory where they launch -- code under HIP
  * graph capture, tight serving loops, harnesses that forbid it.  All calls on one GPU share the buffer:
  * calls that may overlap in time (different streams) race; calls on one stream do not. */
@@ -193,7 +197,8 @@ int tb_gemm_static_workspace(const tb_gemm_desc* desc, void* stream);
 /* What a tb_gemm call with this descriptor would launch (nothing is launched): the tile, the kernel family
  * (waves per workgroup; four_wave: the hand-scheduled 256x256 kernel), the grid, how many tiles form the Stream-K
  * tail and in units of how many K steps their ranges are cut, whether the whole tiles come from the work-stealing
- * queues, whether the small-M streaming kernel runs instead of a tile kernel.  For tests and for callers that log
+ * queues, whether the small-M streaming kernel runs instead of a tile kernel.  Without a workspace in the
+ * descriptor: what runs with one of tb_workspace_bytes() bytes.  For tests and for callers that log
  * their launches; no counterpart in the reference (its launchers print the same facts when asked to be verbose). */
 typedef struct tb_launch_info {
   int32_t block_m, block_n, block_k, waves, four_wave, mode, grid, total_tiles, sk_tiles, sk_unit, sk_ws, skinny;

@@ -192,6 +192,33 @@ def test_grouped_descriptor_validation_and_workspace_size_without_a_gpu():
     assert lib.tb_grouped_workspace_bytes(g) == 0
 
 
+@pytest.mark.parametrize("a_type,m,n,k,a_pitch,n_major,tile,grid,small", [
+    (1, 4352, 4096, 4104, 4104, False, (256, 256, 64), 200, True),       # bf16, a remainder of K
+    (1, 4352, 4096, 4097, 4097, False, (256, 256, 64), 200, True),       # rows off 16 bytes
+    (4, 4352, 4096, 4096, 4096, True, (256, 256, 32), 200, True),        # fp32, N-contiguous weight
+    (1, 4352, 4096, 4096, 4096, False, (256, 256, 64), 200, False),      # whole K steps: refused by tb_gemm
+])
+def test_launch_info_of_stream_k_in_a_workspace_that_is_too_small(a_type, m, n, k, a_pitch, n_major, tile, grid, small):
+    from tritonblas_amd import _lib
+    lib = _lib.load()
+    d = _lib.tb_gemm_desc()
+    d.struct_bytes = C.sizeof(_lib.tb_gemm_desc)
+    d.a_type = d.b_type = d.c_type = a_type
+    d.m, d.n, d.k = m, n, k
+    d.a_stride_m, d.a_stride_k = a_pitch, 1
+    d.b_stride_k, d.b_stride_n = (n, 1) if n_major else (1, a_pitch)
+    d.c_stride_m, d.c_stride_n = n, 1
+    d.a = d.b = d.c = 1 << 20
+    d.block_m, d.block_n, d.block_k = tile
+    d.schedule, d.grid = _lib.TB_SCHED_STREAMK, grid
+    info = _lib.tb_launch_info()
+    assert lib.tb_gemm_launch_info(d, C.byref(info)) == _lib.TB_OK
+    assert info.mode == 2 and info.block_m >= 128 and lib.tb_workspace_bytes(d) > 8 << 20
+    d.workspace, d.workspace_bytes = 1 << 20, 8 << 20
+    assert lib.tb_gemm_launch_info(d, C.byref(info)) == _lib.TB_OK
+    assert info.mode == 2 and info.grid == grid and (info.block_m, info.block_n) == ((64, 64) if small else tile[:2])
+
+
 def test_python_api_refuses_cpu_tensors():
     import tritonblas_amd as tb
     a = torch.zeros(16, 16, dtype=torch.float16)

@@ -71,7 +71,7 @@ def test_static_workspace_rejects_what_does_not_fit():
     (torch.float32, 4352, 4096, 1024, 256, (256, 256, 32), True),      # N-contiguous weight
 ])
 def test_static_workspace_takes_smaller_tiles(dtype, m, n, k, grid, tile, b_rows):
-    """Operands that the 64x64 gather kernel takes too run there when the chosen tile's partial tiles do not fit.  Whole numbers, exact sums."""
+    """Operands that used to run on 64x64 tiles go back to them when the chosen tile's partial tiles do not fit.  Whole numbers, exact sums."""
     from tritonblas_amd import _lib
     lib = _lib.load()
     g = torch.Generator(device="cuda").manual_seed(3)
@@ -83,6 +83,21 @@ def test_static_workspace_takes_smaller_tiles(dtype, m, n, k, grid, tile, b_rows
     assert lib.tb_workspace_bytes(d) > 16 << 20, "the case must not fit"
     assert lib.tb_gemm_static_workspace(d, _lib.stream_handle()) == _lib.TB_OK
     assert torch.equal(c, (a.double() @ b.double()).float().to(dtype))
+
+
+def test_stream_k_without_a_workspace_on_tiles_that_need_none():
+    """16 tiles of 256x256 on 64 workgroups are shared, 256 tiles of 64x64 are not: K with a remainder, no workspace."""
+    from tritonblas_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(4)
+    a = torch.randint(-3, 4, (1024, 1032), device="cuda", generator=g).bfloat16()
+    b = torch.randint(-3, 4, (1024, 1032), device="cuda", generator=g).bfloat16().T
+    c = torch.empty(1024, 1024, dtype=torch.bfloat16, device="cuda")
+    d = _desc(_lib, a, b, c, _lib.TB_SCHED_STREAMK, 64)
+    d.block_m, d.block_n, d.block_k = 256, 256, 64
+    assert lib.tb_workspace_bytes(d) > 0
+    assert lib.tb_gemm(d, _lib.stream_handle()) == _lib.TB_OK
+    assert torch.equal(c, (a.double() @ b.double()).float().bfloat16())
 
 
 def test_static_workspace_status_word():

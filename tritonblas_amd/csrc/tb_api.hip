@@ -220,7 +220,7 @@ struct Job {
   int bm = 0, bn = 0, bk = 0, group_m = 0, num_xcds = 0;
   int schedule = TB_SCHED_PERSISTENT, grid = 0, counters_per_xcd = 0;
   void* workspace = nullptr; size_t workspace_bytes = 0;
-  bool element_wise = false;      // the gather kernel, whatever the operands allow (see run_plan)
+  int retreat = 0;                // 1: the 64x64 tile of the operands' loader, 2: the gather kernel (see fitting_plan)
   uint32_t epoch = 1, spin_limit = 0;
   const int32_t* cu_mask = nullptr; int cu_mask_len = 0, ws_mode = 0, ws_local = 0, ws_global = 0;
   // grouped
@@ -298,6 +298,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
     if (st != TB_OK) return st;
     bm = sel.block_m; bn = sel.block_n; bk = sel.block_k;
   }
+  if (j.retreat == 1) { bm = bn = 64; bk = 128 / usz * epu; }
   const Variant* v = nullptr;
   // Unit stride along one index, but rows off 16 bytes or with a partial chunk: 16-byte loads through registers, in the
   // tile that was chosen up to 128x128 (1187x3001x1531 bf16: 248 us in the gather kernel, 42 in this one).  Each contiguous index has a chunk at least.
@@ -318,7 +319,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
                        ((uintptr_t)j.mxa % 16) == 0 && ((uintptr_t)j.mxb % 16) == 0;
     if (!mx_ok || hooks().no_mxlds) fast = false;
   }
-  if (j.element_wise) fast = false;
+  if (j.retreat == 2) fast = false;
   if (fast) {
     // 32-bit offsets inside a tile
     if ((alay == LAY_K && (int64_t)bm * j.a_sr * usz >= (1ll << 31)) || (blay == LAY_K && (int64_t)bn * j.b_sr * usz >= (1ll << 31)) ||
@@ -341,7 +342,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
       for (auto& t : tile_infos(j.dt)) known |= (t.bm == bm && t.bn == bn && t.bk == bk);
       if (!known) return TB_ERR_BAD_TILE;
     }
-    if (ralay >= 0 && rblay >= 0 && !j.element_wise) {
+    if (ralay >= 0 && rblay >= 0 && j.retreat != 2) {
       const int side = bm >= 128 ? 128 : 64, k_step = 128 / usz * epu;
       const bool near = (ralay == LAY_K ? side * j.a_sr : k_step * j.a_sk) * usz < (1ll << 31) && (rblay == LAY_K ? side * j.b_sr : k_step * j.b_sk) * usz < (1ll << 31);
       if (near) v = find_variant(j.dt, side, side, k_step, ralay, rblay, LOAD_REGS);
@@ -554,7 +555,7 @@ PlanKey plan_key(const Job& j, int dev) {
       j.mxa_sr, j.mxa_sk, j.mxb_sr, j.mxb_sk, j.bias_stride, j.bm, j.bn, j.bk, j.group_m, j.num_xcds, j.grid,
       j.counters_per_xcd, j.ws_mode, j.ws_local, j.cu_mask_len, j.ws_global, j.num_groups, j.grp_phase, j.grp_big,
       j.grp_thr, j.grp_auto, j.grp_sk, j.b_group_stride, j.sb_group_stride, al(j.A), al(j.B), al(j.C), al(j.mxa), al(j.mxb),
-      al(j.bias), j.sa ? 1 : 0, j.sb ? 1 : 0, j.cu_mask ? 1 : 0, j.group_offsets ? 1 : 0, j.column_split,
+      al(j.bias), j.sa ? 1 : 0, j.sb ? 1 : 0, j.cu_mask ? 1 : 0, j.group_offsets ? 1 : 0, j.column_split, j.retreat,
       (int64_t)g_hooks_version};
   static_assert(sizeof(f) <= sizeof(k.v), "PlanKey too small");
   for (int64_t x : f) k.v[i++] = x;
@@ -602,12 +603,35 @@ int cached_plan(const Job& j, const tb_hw& hw, Plan* out) {
   return st;
 }
 
+// The plan of a job that brings a workspace.  A Stream-K launch whose partial tiles outgrow it is refused, but for operands that
+// ran on 64x64 tiles before the larger ones could take them (rows off 16 bytes, a remainder of K, M-contiguous fp32): their callers
+// sized the workspace for 16 KB per workgroup instead of up to 256 (bf16 4352x4096x4104 on 256 workgroups: 4 MiB instead of 64, against
+// the 16 MiB of the static workspace).  These go back to the 64x64 tile of the loader they have, and to the gather kernel, whose
+// grid is the smallest, if that one's grid does not fit either.  make: job -> plan.
+template <class F>
+int fitting_plan(const Job& j, F&& make, Plan* out) {
+  const int st = make(j, out);
+  if (st != TB_OK || j.num_groups > 0) return st;
+  const size_t room = j.workspace ? j.workspace_bytes : 0;
+  const bool small_before = out->v->fast == LOAD_REGS || j.K % out->v->bk != 0 || (j.dt == TB_F32 && (out->v->alay == LAY_M || out->v->blay == LAY_M));
+  for (int retreat = 1; small_before && retreat <= 2 && out->p.mode == MODE_SK && out->ws_need > room; ++retreat) {
+    Job small = j;
+    small.retreat = retreat;
+    Plan plan;
+    if (make(small, &plan) == TB_OK) *out = plan;
+  }
+  return TB_OK;
+}
+int launch_plan(const Job& j, const tb_hw& hw, Plan* out) {
+  return fitting_plan(j, [&](const Job& x, Plan* p) { return cached_plan(x, hw, p); }, out);
+}
+
 int launch(const Job& j, hipStream_t stream) {
   tb_hw hw;
   int st = current_hw(&hw);
   if (st != TB_OK) return st;
   Plan plan;
-  st = cached_plan(j, hw, &plan);
+  st = launch_plan(j, hw, &plan);
   if (st != TB_OK) return st;
   return run_plan(j, plan, stream);
 }
@@ -617,20 +641,6 @@ int run_plan(const Job& j, Plan& plan, hipStream_t stream) {
   if (plan.skinny) {
     if (launch_skinny(p, j.dt, stream) != hipSuccess) { (void)hipGetLastError(); return TB_ERR_LAUNCH; }
     return TB_OK;
-  }
-  if (plan.p.mode == MODE_SK && j.num_groups == 0 && j.workspace && j.workspace_bytes < plan.ws_need &&
-      (plan.v->fast == LOAD_REGS || j.K % plan.v->bk != 0 || (j.dt == TB_F32 && (plan.v->alay == LAY_M || plan.v->blay == LAY_M)))) {
-    // Partial tiles of the vector loaders' larger tiles that do not fit the workspace, for operands that the gather kernel
-    // takes just as well: its 64x64 tiles need 16 KB per workgroup instead of up to 256 (bf16 4352x4096x4104 on 256
-    // workgroups: 4 MiB instead of 64, against the 16 MiB of the static workspace).
-    Job small = j;
-    small.element_wise = true;
-    tb_hw hw;
-    int st = current_hw(&hw);
-    Plan gather;
-    if (st == TB_OK) st = make_plan(small, hw, true, &gather);
-    if (st != TB_OK) return st;
-    plan = gather;
   }
   if (plan.ws_need) {
     if (!j.workspace || j.workspace_bytes < plan.ws_need || ((uintptr_t)j.workspace & 255)) return TB_ERR_WORKSPACE;
@@ -699,7 +709,7 @@ int launch_columns(const Job& j, hipStream_t stream) {
     int st = current_hw(&hw);
     if (st != TB_OK) return st;
     Plan plan;
-    st = cached_plan(j, hw, &plan);
+    st = launch_plan(j, hw, &plan);
     if (st != TB_OK) return st;
     if (plan.skinny || plan.p.mode != MODE_STATIC) return run_plan(j, plan, stream);
     Job whole = j;
@@ -980,7 +990,8 @@ int tb_gemm_launch_info(const tb_gemm_desc* desc, tb_launch_info* out) {
   const bool have_dev = current_hw(&hw) == TB_OK;
   if (!have_dev) default_hw(&hw);
   Plan plan;
-  st = make_plan(j, hw, have_dev, &plan);
+  auto make = [&](const Job& x, Plan* p) { return make_plan(x, hw, have_dev, p); };
+  st = j.workspace ? fitting_plan(j, make, &plan) : make(j, &plan);
   if (st != TB_OK) return st;
   std::memset(out, 0, sizeof(*out));
   out->block_m = plan.v->bm; out->block_n = plan.v->bn; out->block_k = plan.v->bk;
