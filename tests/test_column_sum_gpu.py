@@ -40,3 +40,12 @@ def test_bias_gradient_can_be_differentiated_again():
     v = torch.randn(40, device="cuda")
     dg, = torch.autograd.grad(db, g, v)
     assert torch.equal(dg, v.expand(24, 40))
+
+
+@pytest.mark.gpu
+def test_more_columns_than_one_launch_has_threads_for():
+    """2**28 columns and a few, 16 to a workgroup of 256 threads: HIP refuses launches of 2**32 threads and more."""
+    x = torch.rand((1, 2 ** 28 + 3), device="cuda", dtype=torch.bfloat16)
+    assert torch.equal(_column_sum(x), x[0])
+    x = torch.rand((2, 2 ** 27 + 64), device="cuda", dtype=torch.bfloat16)
+    assert torch.equal(_column_sum(x), (x[0].float() + x[1].float()).bfloat16())

@@ -88,7 +88,6 @@ hipError_t launch_typed(const ColumnSumParams& p, hipStream_t stream) {
   constexpr int ESZ = DT == DT_F32 ? 4 : 2, VEC = 16 / ESZ;
   const bool vec = p.n % VEC == 0 && (p.stride * ESZ) % 16 == 0 && ((uintptr_t)p.x & 15) == 0;
   const int64_t cols = CS_TX * (vec ? VEC : 1), blocks = (p.n + cols - 1) / cols;
-  if (blocks > INT32_MAX) return hipErrorInvalidValue;
   const dim3 grid((unsigned)blocks, (unsigned)p.parts);
   if (vec) hipLaunchKernelGGL((column_sum_kernel<DT, VEC>), grid, dim3(CS_TX * CS_TY), 0, stream, p);
   else hipLaunchKernelGGL((column_sum_kernel<DT, 1>), grid, dim3(CS_TX * CS_TY), 0, stream, p);
@@ -99,8 +98,19 @@ hipError_t launch_typed(const ColumnSumParams& p, hipStream_t stream) {
 }
 
 hipError_t launch_column_sum(const ColumnSumParams& p, int x_type, hipStream_t stream) {
-  if (x_type == DT_F32) return launch_typed<DT_F32>(p, stream);
-  return x_type == DT_F16 ? launch_typed<DT_F16>(p, stream) : launch_typed<DT_BF16>(p, stream);
+  // (a launch takes less than 2^32 threads, and a workgroup of 256 may have as few as 16 columns)
+  constexpr int64_t MOST = 1ll << 27;
+  const int64_t esz = x_type == DT_F32 ? 4 : 2;
+  for (int64_t c = 0; c < p.n; c += MOST) {
+    ColumnSumParams part = p;
+    part.x += c * esz;
+    part.out = (uint8_t*)p.out + c * esz;
+    part.n = p.n - c < MOST ? p.n - c : MOST;
+    const hipError_t e = x_type == DT_F32 ? launch_typed<DT_F32>(part, stream)
+                         : x_type == DT_F16 ? launch_typed<DT_F16>(part, stream) : launch_typed<DT_BF16>(part, stream);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace tb
