@@ -49,3 +49,10 @@ def test_more_columns_than_one_launch_has_threads_for():
     assert torch.equal(_column_sum(x), x[0])
     x = torch.rand((2, 2 ** 27 + 64), device="cuda", dtype=torch.bfloat16)
     assert torch.equal(_column_sum(x), (x[0].float() + x[1].float()).bfloat16())
+
+
+@pytest.mark.gpu
+def test_column_sum_of_every_way_a_matrix_is_stored():
+    base = torch.randint(-9, 9, (96, 80), device="cuda").bfloat16()        # (whole numbers: exact sums)
+    for x in (base.T, base[:, ::2], base[::3, 8:72], base[:1].expand(50, 80), base[:, :1].expand(96, 33), base.T[:, :1], base[:, 5:6]):
+        assert torch.equal(_column_sum(x), x.double().sum(0).bfloat16())

@@ -302,10 +302,10 @@ def _(a, b, out, enable_streamk=False, sk_grid=None, work_stealing=False):
 
 @torch.library.custom_op("tritonblas_amd::_column_sum", mutates_args=())
 def _column_sum(x: torch.Tensor) -> torch.Tensor:
-    """``x.sum(dim=0)`` of a contiguous matrix, formed in fp32 (a bias gradient)."""
+    """``x.sum(dim=0)`` of a matrix, formed in fp32 (a bias gradient)."""
     m, n = x.shape
-    if m == 0 or n == 0 or not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16, torch.float32):
-        return x.sum(dim=0)
+    if m == 0 or n == 0 or not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16, torch.float32) or (n > 1 and x.stride(1) != 1):
+        return x.sum(dim=0)         # (the kernel reads rows of adjacent values)
     out = x.new_empty(n)
     lib = _lib.load()
     with _on_device(x.device):
