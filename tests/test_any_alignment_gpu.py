@@ -64,3 +64,25 @@ def test_mxfp4_rows_and_scales_at_any_alignment(m, n, k, pad, lead):
     full = [mxfp4_to_f32(x.contiguous()).double() * e8m0_to_f32(s.contiguous()).double().repeat_interleave(32, 1) for x, s in ((a, sa), (b, sb))]
     # (multiples of 1/16 below 2**16 * 144: the sums are exact)
     assert torch.equal(c, (full[0] @ full[1].T).float().to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_operands_stored_backwards(dtype):
+    """Negative strides, which the C interface takes (torch has none): the operands' K runs from the last stored row to the first."""
+    import ctypes as C
+    from tritonblas_amd import _lib
+    m, n, k = 136, 72, 96
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    a, b = (torch.randint(-9, 9, (k, s), device="cuda", generator=gen).to(dtype) for s in (m, n))
+    c = torch.empty(m, n, device="cuda", dtype=dtype)
+    d = _lib.tb_gemm_desc()
+    d.struct_bytes = C.sizeof(_lib.tb_gemm_desc)
+    d.a_type = d.b_type = d.c_type = _lib.tb_dtype(dtype)
+    d.m, d.n, d.k = m, n, k
+    d.a_stride_m, d.a_stride_k, d.b_stride_k, d.b_stride_n, d.c_stride_m, d.c_stride_n = 1, -m, n, 1, n, 1
+    d.a, d.b, d.c = a[-1].data_ptr(), b.data_ptr(), c.data_ptr()
+    assert _lib.load().tb_gemm(d, _lib.stream_handle()) == _lib.TB_OK
+    assert torch.equal(c, (a.flip(0).double().T @ b.double()).float().to(dtype))
+    d.a_stride_k, d.a, d.b_stride_k, d.b = m, a.data_ptr(), -n, b[-1].data_ptr()
+    assert _lib.load().tb_gemm(d, _lib.stream_handle()) == _lib.TB_OK
+    assert torch.equal(c, (a.double().T @ b.flip(0).double()).float().to(dtype))

@@ -219,6 +219,25 @@ def test_launch_info_of_stream_k_in_a_workspace_that_is_too_small(a_type, m, n, 
     assert info.mode == 2 and info.grid == grid and (info.block_m, info.block_n) == ((64, 64) if small else tile[:2])
 
 
+@pytest.mark.parametrize("dtype", [0, 1, 4])
+def test_operands_stored_backwards_are_planned_for_the_gather_kernel(dtype):
+    """The vector loaders' lane offsets are unsigned: a negative stride belongs to the element-wise kernel (64x64), whichever operand
+    and index has it."""
+    from tritonblas_amd import _lib
+    lib, n = _load(), 4096
+    for strides in [(1, -n, 1, n), (1, n, -n, 1), (n, 1, -n, 1), (-n, 1, 1, n), (n, -1, 1, n), (-1, n, n, 1)]:
+        d = _lib.tb_gemm_desc()
+        d.struct_bytes = C.sizeof(_lib.tb_gemm_desc)
+        d.a_type = d.b_type = d.c_type = dtype
+        d.m = d.n = d.k = n
+        d.a_stride_m, d.a_stride_k, d.b_stride_k, d.b_stride_n = strides
+        d.c_stride_m, d.c_stride_n = n, 1
+        d.a = d.b = d.c = 1 << 40
+        info = _lib.tb_launch_info()
+        assert lib.tb_gemm_launch_info(d, C.byref(info)) == _lib.TB_OK
+        assert (info.block_m, info.block_n) == (64, 64), strides
+
+
 def test_python_api_refuses_cpu_tensors():
     import tritonblas_amd as tb
     a = torch.zeros(16, 16, dtype=torch.float16)

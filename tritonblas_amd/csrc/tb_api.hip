@@ -277,7 +277,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
     return s_k == 1 && aligned16(ptr) && (rows == 1 || (s_row * usz) % 16 == 0) && s_row >= 0;
   };
   auto m_major_ok = [&](const void* ptr, int64_t s_row, int64_t s_k, int64_t rows) {
-    return usz >= 2 && s_row == 1 && aligned16(ptr) && (s_k * usz) % 16 == 0 && rows % (16 / usz) == 0 && j.num_groups == 0;
+    return usz >= 2 && s_row == 1 && s_k >= 0 && aligned16(ptr) && (s_k * usz) % 16 == 0 && rows % (16 / usz) == 0 && j.num_groups == 0;
   };
   int alay = -1, blay = -1;
   if (k_major_ok(j.A, j.a_sr, j.a_sk, j.M)) alay = LAY_K; else if (m_major_ok(j.A, j.a_sr, j.a_sk, j.M)) alay = LAY_M;
