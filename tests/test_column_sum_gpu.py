@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import tritonblas_amd as tb
-from tritonblas_amd.matmul import _column_sum
+from tritonblas_amd.matmul import _bias_gradient, _column_sum
 
 
 @pytest.mark.gpu
@@ -56,3 +56,14 @@ def test_column_sum_of_every_way_a_matrix_is_stored():
     base = torch.randint(-9, 9, (96, 80), device="cuda").bfloat16()        # (whole numbers: exact sums)
     for x in (base.T, base[:, ::2], base[::3, 8:72], base[:1].expand(50, 80), base[:, :1].expand(96, 33), base.T[:, :1], base[:, 5:6]):
         assert torch.equal(_column_sum(x), x.double().sum(0).bfloat16())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n", [(64, 128), (2048, 2040), (2048, 2056)])
+def test_bias_gradient_on_both_sides_of_its_rule(m, n):
+    """Sums of whole numbers below 2**24: exact on either way."""
+    g = torch.randint(-9, 9, (m, n), device="cuda").float()
+    assert torch.equal(_bias_gradient(g), g.double().sum(0).float())
+    bias = torch.zeros(n, device="cuda", requires_grad=True)
+    db, = torch.autograd.grad(tb.addmm(bias, torch.ones(m, 8, device="cuda"), torch.ones(8, n, device="cuda")), bias, g)
+    assert torch.equal(db, g.double().sum(0).float())
