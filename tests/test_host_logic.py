@@ -249,6 +249,20 @@ def test_python_api_refuses_cpu_tensors():
         tb.matmul(a.requires_grad_(), a, out=torch.zeros(16, 16, dtype=torch.float16))
 
 
+@pytest.mark.parametrize("rows,cols,pitch,g_cols,copied", [
+    (64, 72, 72, 40, False), (64, 72, 72, 41, False),      # rows on 16 bytes
+    (64, 73, 73, 40, True), (64, 72, 73, 40, True),        # off them, the copy's on them, the gradient's too
+    (64, 73, 73, 41, False), (65, 73, 73, 40, False),      # the gradient's or the copy's off them as well
+])
+def test_which_operands_of_the_backward_pass_are_copied(rows, cols, pitch, g_cols, copied):
+    from tritonblas_amd.matmul import _transposed
+    g = torch.zeros(3, g_cols, dtype=torch.bfloat16)
+    t = torch.zeros(rows, pitch, dtype=torch.bfloat16)[:, :cols]
+    assert (_transposed(t, g).data_ptr() != t.data_ptr()) == copied and torch.equal(_transposed(t, g), t.T)
+    t = torch.zeros(2 * rows, 2 * pitch, dtype=torch.bfloat16)[::2, ::2]
+    assert _transposed(t, g).is_contiguous()               # (no unit stride: the element-wise kernel otherwise)
+
+
 # ---- tile order of the kernels (host evaluation through the C ABI) -------------------------------
 import itertools
 

@@ -258,23 +258,28 @@ def _matmul_setup_context(ctx, inputs, output):
     ctx.opts = (enable_streamk, sk_grid, work_stealing)
 
 
-def _transposed(t):
-    """``t.T``, as it is stored where the tile kernels can load it that way, else copied.
+def _transposed(t, g):
+    """``t.T`` for a product with the contiguous gradient ``g``: as it is stored, or copied where the copy pays.
 
-    The kernels take either index of a 16- or 32-bit operand as the contiguous one at the same rate, so the copy
-    only costs (4096x14336x4096 bf16: two copies, 0.32 of 1.6 ms); it pays where a row of ``t`` does not start on 16 bytes."""
-    chunk = 16 // t.element_size()
+    The kernels take either index of a 16- or 32-bit operand as the contiguous one, so a copy of rows that start on 16 bytes only
+    costs (4096x14336x4096 bf16: two copies, 0.32 of 1.6 ms).  Rows that do not are loaded through registers; a copy whose rows do start
+    there saves that if the rows of ``g`` do too (a.T @ g of a 4096x4096x4099 bf16 product: 237 us as stored, 189 with the copy;
+    1184x3000x1531 39 and 35) and is lost otherwise (1187x3001x1531: 47 and 58; g @ b.T 42 and 83)."""
+    size = t.element_size()
+    chunk = 16 // size
     for inner, outer in ((1, 0), (0, 1)):
-        if t.element_size() > 1 and t.stride(inner) == 1 and t.shape[inner] % chunk == 0 and t.stride(outer) % chunk == 0 and t.storage_offset() % chunk == 0:
+        if size > 1 and t.stride(inner) == 1 and t.shape[inner] % chunk == 0 and t.stride(outer) % chunk == 0 and t.storage_offset() % chunk == 0:
             return t.T
+    if size > 1 and 1 in t.stride() and (t.shape[0] % chunk or g.shape[1] % chunk):
+        return t.T
     return t.T.contiguous()
 
 
 def _product_gradients(a, b, g, opts):
     # two more library GEMMs: grad_a = g @ b^T, grad_b = a^T @ g
     sk, grid, ws = opts
-    return (matmul(g, _transposed(b), enable_streamk=sk, sk_grid=grid, work_stealing=ws),
-            matmul(_transposed(a), g, enable_streamk=sk, sk_grid=grid, work_stealing=ws))
+    return (matmul(g, _transposed(b, g), enable_streamk=sk, sk_grid=grid, work_stealing=ws),
+            matmul(_transposed(a, g), g, enable_streamk=sk, sk_grid=grid, work_stealing=ws))
 
 
 def _matmul_backward(ctx, grad_output):
