@@ -86,3 +86,25 @@ def test_operands_stored_backwards(dtype):
     d.a_stride_k, d.a, d.b_stride_k, d.b = m, a.data_ptr(), -n, b[-1].data_ptr()
     assert _lib.load().tb_gemm(d, _lib.stream_handle()) == _lib.TB_OK
     assert torch.equal(c, (a.double().T @ b.flip(0).double()).float().to(dtype))
+
+
+def test_rows_further_apart_than_32_bit_offsets_reach():
+    """64 rows of 32 MiB and more: the gather kernel, for bf16 and for MXFP4 (whose other operands all take 16-byte loads)."""
+    from tritonblas_amd.utils import e8m0_to_f32, mxfp4_to_f32
+    m, n, pitch = 66, 40, (1 << 25) + 64
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    base = torch.empty(m * pitch, device="cuda", dtype=torch.uint8)
+    k = 136
+    a = base.view(torch.bfloat16).as_strided((m, k), (pitch // 2, 1))
+    a.copy_(torch.randint(-9, 9, (m, k), device="cuda", generator=gen))
+    b = torch.randint(-9, 9, (n, k), device="cuda", generator=gen).bfloat16().T
+    assert torch.equal(tb.matmul(a, b), (a.double() @ b.double()).float().bfloat16())
+    k = 544
+    codes = base.as_strided((m, k // 2), (pitch, 1))
+    codes.copy_(torch.randint(0, 256, (m, k // 2), device="cuda", generator=gen))
+    w = torch.randint(0, 256, (n, k // 2), device="cuda", generator=gen).to(torch.uint8)
+    sa, sw = (torch.randint(126, 129, (r, k // 32), device="cuda", generator=gen).to(torch.uint8) for r in (m, n))
+    c = torch.full((m, n), float("nan"), device="cuda", dtype=torch.bfloat16)
+    tb.matmul_fp4(codes, w, c, sa, sw)
+    full = [mxfp4_to_f32(x.contiguous()).double() * e8m0_to_f32(s).double().repeat_interleave(32, 1) for x, s in ((codes, sa), (w, sw))]
+    assert torch.equal(c, (full[0] @ full[1].T).float().to(torch.bfloat16))      # (exact sums, as above)

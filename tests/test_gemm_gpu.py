@@ -434,8 +434,8 @@ def _ref64(a_cpu, b_cpu, bias=None):
                                    (2048, 64, 4096), (1, 1, 1)])
 @pytest.mark.parametrize("transA,transB", [("T", "T"), ("N", "N"), ("T", "N"), ("N", "T")])
 def test_matmul_fp32(m, n, k, transA, transB):
-    """float32 in, float32 out (reference tests/test_matmul.py:23): K-contiguous operands run the
-    LDS-direct kernels, every other layout the gather kernel."""
+    """float32 in, float32 out (reference tests/test_matmul.py:23): every storage order, rows on 16 bytes (LDS-direct kernels),
+    off them (register-loading kernels) and too short for either (gather kernel)."""
     import tritonblas_amd as tb
     _say(f"matmul fp32 {m}x{n}x{k} {transA}{transB}")
     a_cpu, b_cpu = _rand((m, k), torch.float32, 40, 0.5), _rand((k, n), torch.float32, 41, 0.5)
@@ -496,20 +496,37 @@ def test_addmm_fp32(out_dtype):
 
 
 def test_streamk_grid_sized_for_another_tile():
-    """The selector sizes its Stream-K grid for the tile it picked; operands that need the gather kernel
-    run another tile with fewer co-resident workgroups.  The library then chooses the grid itself
-    instead of refusing the launch."""
+    """A Stream-K grid sized for the tile the selector picked, larger than what is co-resident of the kernel that runs: operands
+    without unit stride take the gather kernel, two workgroups to a CU.  The library then chooses the grid itself instead of
+    refusing the launch."""
+    import ctypes as C
     import tritonblas_amd as tb
+    from tritonblas_amd import _lib
     m, n, k = 1261, 670, 2688
     a_cpu, b_cpu = _rand((m, k), torch.float32, 70, 0.5), _rand((k, n), torch.float32, 71, 0.5)
-    a, b = a_cpu.cuda(), b_cpu.cuda()          # B is N-contiguous: no LDS-direct fp32 kernel for it
+    a, b = (torch.stack([x, x], 2).cuda().reshape(x.shape[0], -1)[:, ::2] for x in (a_cpu, b_cpu))
+    assert a.stride(1) == 2 and b.stride(1) == 2
     sel = tb.OrigamiMatmulSelector(m, n, k, a.dtype, b.dtype, torch.float32, a.device, streamk=True)
     cfg = tb.matmul_preamble(sel)
     c = torch.full((m, n), float("nan"), dtype=torch.float32, device="cuda")
+    d = _lib.tb_gemm_desc()
+    d.struct_bytes = C.sizeof(_lib.tb_gemm_desc)
+    d.a_type = d.b_type = d.c_type = _lib.tb_dtype(torch.float32)
+    d.m, d.n, d.k = m, n, k
+    (d.a_stride_m, d.a_stride_k), (d.b_stride_k, d.b_stride_n), (d.c_stride_m, d.c_stride_n) = a.stride(), b.stride(), c.stride()
+    d.a, d.b, d.c = a.data_ptr(), b.data_ptr(), c.data_ptr()
+    d.block_m, d.block_n, d.block_k = sel.block_m, sel.block_n, sel.block_k
+    d.schedule, d.grid = _lib.TB_SCHED_STREAMK, 1000
+    info = _lib.tb_launch_info()
+    assert _lib.load().tb_gemm_launch_info(d, C.byref(info)) == _lib.TB_OK
+    assert (info.block_m, info.block_n) == (64, 64) and 0 < info.grid < 1000
     tb.matmul_lt(a, b, c, sel, cfg, enable_streamk=True)
-    err = OG.rel_fro_error(c.cpu().double(), _ref64(a_cpu, b_cpu))
-    assert err <= TOL_32, f"{err:.3e}"
-    assert cfg.status() == 0
+    want = _ref64(a_cpu, b_cpu)
+    assert OG.rel_fro_error(c.cpu().double(), want) <= TOL_32 and cfg.status() == 0
+    from tritonblas_amd.matmul import streamk_matmul_lt
+    c.fill_(float("nan"))
+    streamk_matmul_lt(a, b, c, sel, cfg, sk_grid=1000)
+    assert OG.rel_fro_error(c.cpu().double(), want) <= TOL_32 and cfg.status() == 0
 
 
 # ---- int8 operands -------------------------------------------------------------------------------

@@ -74,15 +74,16 @@ def test_struct_sizes_match_the_header():
     import subprocess
     import tempfile
     from tritonblas_amd import _lib
-    src = '#include <stdio.h>\n#include "tritonblas_amd.h"\nint main(){printf("%zu %zu %zu %zu %zu %zu %zu\\n",' \
+    src = '#include <stdio.h>\n#include "tritonblas_amd.h"\nint main(){printf("%zu %zu %zu %zu %zu %zu %zu %zu %zu %zu\\n",' \
           'sizeof(tb_hw),sizeof(tb_problem),sizeof(tb_selection),sizeof(tb_gemm_desc),sizeof(tb_gemm_fp4_desc),' \
-          'sizeof(tb_grouped_gemm_desc),sizeof(tb_quant_desc));return 0;}'
+          'sizeof(tb_grouped_gemm_desc),sizeof(tb_quant_desc),sizeof(tb_row_quant_desc),sizeof(tb_column_sum_desc),' \
+          'sizeof(tb_launch_info));return 0;}'
     with tempfile.TemporaryDirectory() as td:
         open(os.path.join(td, "s.c"), "w").write(src)
         subprocess.check_call(["gcc", "-I", os.path.join(ROOT, "include"), "-o", os.path.join(td, "s"), os.path.join(td, "s.c")])
         sizes = [int(v) for v in subprocess.check_output([os.path.join(td, "s")]).split()]
     mine = [C.sizeof(t) for t in (_lib.tb_hw, _lib.tb_problem, _lib.tb_selection, _lib.tb_gemm_desc, _lib.tb_gemm_fp4_desc,
-                                  _lib.tb_grouped_gemm_desc, _lib.tb_quant_desc)]
+                                  _lib.tb_grouped_gemm_desc, _lib.tb_quant_desc, _lib.tb_row_quant_desc, _lib.tb_column_sum_desc, _lib.tb_launch_info)]
     assert mine == sizes
 
 

@@ -108,7 +108,7 @@ def _fp4_cases(n, seed):
                          ids=lambda c: f"{c['idx']}-{c['m']}x{c['n']}x{c['k']}-{c['tile']}")
 def test_random_fp4_case(case):
     """MXFP4: random codes and random, widely varying E8M0 scales; K any multiple of 32 (multiples of 512
-    take the LDS-direct kernels, the rest the gather kernel), forced or selected tiles, three output types."""
+    take the LDS-direct kernels, the rest the register-loading ones), forced or selected tiles, three output types."""
     import numpy as np
     import tritonblas_amd as tb
     print("random fp4 case", case, flush=True)

@@ -8,8 +8,8 @@
 // it -- tile schedule, per-tile addresses, epilogue -- stays C++.  The wave tile is a quarter of the
 // 8-wave kernels' K-step LDS traffic less (128 KB instead of 196 KB of fragment reads per 64 KB copied).
 //
-// Differences from the 8-wave kernels that matter to callers: K must be a multiple of two K steps and
-// there is no Stream-K variant (whole tiles only: data-parallel, work-stealing and grouped schedules).
+// Differences from the 8-wave kernels that matter to callers: K must be a multiple of two K steps; with a
+// Stream-K tail of four, both operands K-contiguous, and no 8-bit result.
 // Sums are formed in the same order (same MFMA instruction, same K grouping, K steps in ascending
 // order), so results are bit-identical to the 8-wave kernels'.
 //

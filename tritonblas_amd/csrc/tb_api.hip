@@ -75,7 +75,7 @@ int current_hw(tb_hw* out) {
 // launch path calls getenv.
 struct Hooks {
   int waves = 0;                // TB_WAVES=<wm><wn>[<stages>]: picks among variants that share a tile shape
-  int no_mxlds = 0;             // TB_NO_MXLDS=1: fp4 scales straight from global memory (gather kernel)
+  int no_mxlds = 0;             // TB_NO_MXLDS=1: fp4 scales straight from global memory (register-loading kernels)
   int no_cline = 0;             // TB_NO_CLINE=1: element-wise C stores
   int no_skinny = 0, skinny = 0;  // TB_NO_SKINNY / TB_SKINNY: force the small-M kernel choice
   int grid = 0;                 // TB_GRID=<n>: workgroups of a persistent / grouped launch
@@ -302,6 +302,9 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
   const Variant* v = nullptr;
   // Unit stride along one index, but rows off 16 bytes or with a partial chunk: 16-byte loads through registers, in the
   // tile that was chosen up to 128x128 (1187x3001x1531 bf16: 248 us in the gather kernel, 42 in this one).  Each contiguous index has a chunk at least.
+  // The choice is the LDS-direct kernels': of 13 odd sizes in bf16 and fp32, B in both orders, it is within 5 % of the faster side in 48
+  // of 52 (1187x3001x1531 bf16 43 us in 64x64 and 42 in 128x128, 1000x1001x999 18 and 30, 4001^3 341 and 214) and loses 20 % in
+  // 1501x1501x4097 bf16 (88 and 104) and 4097x4097x1023 fp32 (367 and 433).
   auto any_alignment = [&](int64_t s_row, int64_t s_k, int64_t rows) {
     if (j.num_groups > 0) return -1;
     // (one-byte units: whole chunks only.  fp4 1000x4096x4128, whose scale rows cannot be staged: 397 us in the gather kernel, 71 in this one)
