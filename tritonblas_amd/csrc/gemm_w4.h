@@ -25,6 +25,8 @@
 // K row k of it 128 bytes at 128 k, chunk c of those at slot c ^ mask(k).  A: mask 2 ((k % 4) ^ x), x the parity of
 // the bits of k / 16 (a fragment read takes 32 bytes of four K rows per 16 lanes, and 16 lanes after 16 lanes sit 16 K
 // rows apart); B, whose column order makes that 8 bytes of each of four chunks: mask 4 ((k / 2) % 2).
+// A's reads are free of bank conflicts; each of B's takes two cycles more (4096^3 bf16: 4.2e6 conflict cycles in 2.1e6 reads, and the
+// waves wait for LDS in 11 % of their time, 6 % where A is the M-contiguous one).
 // (Three rounds of tiles of 4096x12288x4096 bf16, B M-contiguous, 350 -> 326 us; 14336x4096x4096, both M-contiguous, 332 -> 305 us,
 // both K-contiguous 315: the eight-wave kernel's figure is the first one of each pair.)
 #pragma once
