@@ -137,7 +137,8 @@ typedef struct tb_gemm_desc {
   int32_t block_m, block_n, block_k;  /* tile variant, from tb_select; 0 = let the library select    */
   int32_t group_m, num_xcds;
   int32_t schedule;           /* TB_SCHED_*                                                         */
-  int32_t grid;               /* workgroups to launch; 0 = default (what is co-resident).  A Stream-K
+  int32_t grid;               /* workgroups to launch; 0 = default (persistent: one per tile, or what is
+                                 co-resident; else what is co-resident).  A Stream-K
                                  grid beyond what is co-resident is replaced by the default.  Few rows go
                                  to the streaming kernel, whose grid is its own (tb_launch_info.skinny),
                                  unless this one is smaller than what the device holds of the tile; at

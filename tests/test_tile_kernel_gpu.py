@@ -1,0 +1,58 @@
+"""The persistent schedule with one tile to a workgroup (a launch that names no grid) against the looping kernel (a launch with one): the same K loop and
+the same store, so the results are the same bit for bit, and within the rounding of their type of the product in 64 bits."""
+import ctypes as C
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TYPES = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32, "fp8": torch.float8_e4m3fn, "i8": torch.int8}
+# the rounding of a result to its type; fp32: sums of up to 1100 products of whole numbers up to 9 are exact
+REL = {"bf16": 2.0 ** -8, "f16": 2.0 ** -11, "f32": 0.0, "fp8": 2.0 ** -8, "i8": 2.0 ** -8}
+
+
+def _product(a, b, c, tile, grid):
+    from tritonblas_amd import _lib
+    d = _lib.tb_gemm_desc()
+    d.struct_bytes = C.sizeof(_lib.tb_gemm_desc)
+    d.a_type = d.b_type = _lib.tb_dtype(a.dtype)
+    d.c_type = _lib.tb_dtype(c.dtype)
+    d.m, d.k = a.shape
+    d.n = b.shape[1]
+    d.a_stride_m, d.a_stride_k = a.stride()
+    d.b_stride_k, d.b_stride_n = b.stride()
+    d.c_stride_m, d.c_stride_n = c.stride()
+    d.a, d.b, d.c = a.data_ptr(), b.data_ptr(), c.data_ptr()
+    d.block_m, d.block_n, d.block_k = tile
+    d.grid, d.column_split = grid, -1
+    assert _lib.load().tb_gemm(d, _lib.stream_handle()) == _lib.TB_OK
+    return c
+
+
+@pytest.mark.parametrize("kind,m,n,k,order", [
+    ("bf16", 1, 1, 8, "kk"), ("bf16", 129, 191, 64, "kn"), ("bf16", 640, 1000, 1096, "mn"),      # a corner of a tile; edges; a remainder of K
+    ("bf16", 131, 203, 1031, "kk"), ("f16", 257, 333, 777, "mn"),                                # rows off 16 bytes
+    ("f32", 65, 72, 36, "kk"), ("f32", 300, 520, 1092, "kn"), ("f32", 127, 131, 1001, "mk"),
+    ("fp8", 64, 64, 128, "kk"), ("fp8", 300, 1040, 1104, "kk"), ("i8", 33, 272, 1040, "kk"), ("i8", 100, 90, 1001, "kk"),
+    ("bf16", 5000, 4000, 128, "kk"),                                                             # more tiles than the device holds at once
+])
+def test_one_tile_per_workgroup_matches_the_loop(kind, m, n, k, order):
+    from tritonblas_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+
+    def stored(rows, cols, contiguous):
+        x = torch.randint(-3, 4, (rows, cols) if contiguous else (cols, rows), device="cuda", generator=g).to(TYPES[kind])
+        return x if contiguous else x.T
+
+    a, b = stored(m, k, order[0] == "k"), stored(k, n, order[1] == "n")
+    out = TYPES[kind] if kind in ("bf16", "f16", "f32") else torch.bfloat16
+    want = a.double() @ b.double()
+    buf = (C.c_int32 * 60)()
+    count = _lib.load().tb_list_tiles(_lib.tb_dtype(TYPES[kind]), buf, 20)
+    for i in range(count):
+        tile = tuple(buf[3 * i:3 * i + 3])
+        got = _product(a, b, torch.full((m, n), float("nan"), device="cuda", dtype=out), tile, 0)
+        loop = _product(a, b, torch.full((m, n), float("nan"), device="cuda", dtype=out), tile, 48)
+        assert torch.equal(got, loop), tile
+        assert ((got.double() - want).abs() <= REL[kind] * want.abs()).all(), tile

@@ -597,8 +597,7 @@ __device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70);
 // ------------------------------------------------------------------------------------------------
 // K loop: accumulates k iterations [it0, it1) of one output tile
 // ------------------------------------------------------------------------------------------------
-// WHOLE: the caller only ever passes complete tiles (it0 = 0, it1 = k_iters).
-template <class T, bool WHOLE>
+template <class T>
 __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc, int it0, int it1,
                                          v4f (&acc)[T::TM][T::TN], uint8_t* lds, const LaneInfo& li) {
   using OA = Operand<T, T::BM, T::ALAY>;
@@ -1010,8 +1009,12 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
       __syncthreads();
     }
   }
+}
+
+// int8 operands: int32 sums -> fp32 once per K range (exact below 2^24; Stream-K partials and the epilogue work in fp32)
+template <class T>
+__device__ __forceinline__ void sums_to_f32(v4f (&acc)[T::TM][T::TN]) {
   if constexpr (T::DT == DT_I8) {
-    // int32 sums -> fp32 once per K range (exact below 2^24; Stream-K partials and the epilogue work in fp32)
 #pragma unroll
     for (int i = 0; i < T::TM; ++i)
 #pragma unroll
@@ -1704,7 +1707,8 @@ __global__ __launch_bounds__(T::THREADS, T::MINB) void gemm_kernel(const GemmPar
   }
   while (sched.next(p, w, &s_bcast, li.tid)) {
     __syncthreads();  // the previous item's store staging may still be read by slower waves
-    mainloop<T, !SK>(p, w.tc, w.it0, w.it1, acc, lds, li);
+    mainloop<T>(p, w.tc, w.it0, w.it1, acc, lds, li);
+    sums_to_f32<T>(acc);
     if constexpr (SK) {
     if (w.kind == WK_FULL) {
       // whole tiles get their own copy of the epilogue: sharing the one behind the fixup code makes
@@ -1777,6 +1781,33 @@ __global__ __launch_bounds__(T::THREADS, T::MINB) void gemm_kernel(const GemmPar
       __hip_atomic_store(p.ctl + CTL_DONE, 0u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
+}
+
+// One tile to a workgroup, as many workgroups as tiles: the persistent schedule of a launch that names no grid.  The work loop of gemm_kernel costs
+// a launch 1.0 to 1.9 us in front of its first copy: what the other schedules carry from tile to tile fills the scalar registers (86 spilled, and
+// scratch memory with them; none here).  Back to back, gemm_kernel and this: bf16 512^3 6.0 and 4.9 us, 1024^3 8.7 and 7.7, 2048^3 25.3 and 23.5;
+// FP8 1024x1024x2048 8.2 and 6.9, 512x4096x14336 43.8 and 41.6.  More tiles than fit at once start as others end, which is as fast as a
+// resident grid that loops (FP8 1581x7488x1280 in 128x128 30.1 and 25.0, 2504x6272x1088 32.2 and 31.7; bf16 3200x5248x760 50.0 and 51.7).
+template <class T>
+__global__ __launch_bounds__(T::THREADS, T::MINB) void gemm_tile_kernel(const GemmParams p) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[T::LDS_ALLOC];
+  LaneInfo li;
+  li.tid = threadIdx.x;
+  li.lane = li.tid & 63;
+  li.r = li.lane & 15;
+  li.g = li.lane >> 4;
+  const int wave = li.tid >> 6;
+  li.wm0 = (wave / T::WN) * T::WTM;
+  li.wn0 = (wave % T::WN) * T::WTN;
+  int tile = blockIdx.x;
+  if (p.num_xcds > 1) tile = chiplet_transform_chunked(tile, p.total_tiles, p.num_xcds, p.chunk);
+  TileCtx tc;
+  plain_tile(p, tile, T::BM, T::BN, tc);
+  tc.m0 = uniform(tc.m0); tc.n0 = uniform(tc.n0);
+  v4f acc[T::TM][T::TN];
+  mainloop<T>(p, tc, 0, p.k_iters, acc, lds, li);
+  sums_to_f32<T>(acc);
+  epilogue<T>(p, tc, acc, li, lds);
 }
 
 }  // namespace tb

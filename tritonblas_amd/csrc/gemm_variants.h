@@ -11,6 +11,7 @@ struct Variant {
   int wm, wn, threads, lds_bytes, minb;
   int fast, stages;       // fast: LOAD_*; the tile selector chooses among the LOAD_DIRECT ones
   const void* kernel;     // __global__ void (*)(const GemmParams), whole-tile schedules
+  const void* kernel_one; // one tile to a workgroup (null: this variant has none)
   const void* kernel_sk;  // same tile with the Stream-K tail (null: this variant has none)
   int k_step_pairs;       // 1: hand-scheduled 4-wave kernel -- K must hold four K steps at least (MXFP4, M-contiguous operands, results whose rows are off
                           // 16 bytes: be an even number of them); with a
@@ -20,7 +21,7 @@ struct Variant {
 template <class T>
 constexpr Variant make_variant() {
   return Variant{T::DT, T::BM, T::BN, T::BK, T::ALAY, T::BLAY, T::WM, T::WN, T::THREADS, T::LDS_ALLOC, T::MINB,
-                 T::LOADER, T::STAGES, (const void*)&gemm_kernel<T, false>, (const void*)&gemm_kernel<T, true>, 0};
+                 T::LOADER, T::STAGES, (const void*)&gemm_kernel<T, false>, (const void*)&gemm_tile_kernel<T>, (const void*)&gemm_kernel<T, true>, 0};
 }
 
 // The hand-scheduled 4-wave kernels of gemm_w4.h (256x256 tile, 128-byte K steps) are compiled in a
@@ -38,7 +39,7 @@ constexpr int W4_LDS_BYTES = W4_EPS_OFFSET + 4096 + 16;
 template <class T>
 Variant make_variant_w4() {
   return Variant{T::DT, T::BM, T::BN, T::BK, T::ALAY, T::BLAY, T::WM, T::WN, T::THREADS, W4_LDS_BYTES, 1,
-                 1, T::STAGES, T::ALAY == LAY_M || T::BLAY == LAY_M ? w4_kernel_m(T::DT, T::ALAY, T::BLAY) : w4_kernel(T::DT),
+                 1, T::STAGES, T::ALAY == LAY_M || T::BLAY == LAY_M ? w4_kernel_m(T::DT, T::ALAY, T::BLAY) : w4_kernel(T::DT), nullptr,
                  T::ALAY == LAY_M || T::BLAY == LAY_M ? nullptr : w4_kernel_sk(T::DT), 1};
 }
 

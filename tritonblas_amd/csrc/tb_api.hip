@@ -282,6 +282,8 @@ struct Plan {
   const Variant* v = nullptr;
   GemmParams p;
   int grid = 0;
+  int resident = 0;      // workgroups that the device holds at once, at most the tiles
+  bool one = false;      // one tile to a workgroup (Variant::kernel_one)
   bool skinny = false;   // decode shapes: streaming kernel without tiles or workspace
   bool kept = false;     // the caller keeps the launch to a part of the device (a grid, a mask)
   int n_cu = 0;
@@ -450,6 +452,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
 
   GemmParams& p = plan->p;
   std::memset(&p, 0, sizeof(p));
+  plan->one = false;
   p.A = (const uint8_t*)j.A; p.B = (const uint8_t*)j.B; p.C = (uint8_t*)j.C;
   p.sa = j.sa; p.sb = j.sb; p.bias = (const uint8_t*)j.bias;
   p.mxa = (const uint8_t*)j.mxa; p.mxb = (const uint8_t*)j.mxb;
@@ -560,9 +563,15 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
     }
   } else if (j.schedule == TB_SCHED_PERSISTENT) {
     // a resident grid that loops over the tiles (matmul.py:160-198: for tile_id in range(pid, total, NUM_SMS))
+    // (one tile to a workgroup where the grid is the library's)
     p.mode = MODE_STATIC;
     grid = (int)std::min<int64_t>(total, j.grid > 0 ? j.grid : resident);
     if (hooks().grid > 0) grid = (int)std::min<int64_t>(total, hooks().grid);
+    // (but for two cases of the register-loading kernels, whose loop is ahead where every CU has a second tile: fp32 in 64x64, 2231x843x1377 55.2 us and
+    // 58.2, 1505x1280x951 41.5 and 42.0; MXFP4 128x128 tiles in more than one round, 5942x1328x4256 92.9 and 96.7.  The others of 42 odd sizes 0.99 to 1.49 times as fast.)
+    const bool loop = v->fast == LOAD_REGS && ((j.dt == TB_F32 && v->bm == 64 && total > hw.n_cu && total <= resident) ||
+                                               (j.dt == TB_FP4_E2M1 && v->bm == 128 && total > resident));
+    plan->one = v->kernel_one && j.grid <= 0 && hooks().grid <= 0 && !loop;
   } else if (j.schedule == TB_SCHED_WORK_STEALING) {
     p.mode = MODE_WS;
     grid = j.grid > 0 ? j.grid : (j.cu_mask ? j.cu_mask_len : resident);
@@ -647,7 +656,8 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
   p.chunk = std::min(p.group_m * p.group_m, std::max(1, grid / p.num_xcds));
   p.panel_n = default_panel_n(grid, p.chunk, p.group_m);
   if (hooks().panel >= 0) p.panel_n = hooks().panel;
-  plan->grid = grid;
+  plan->resident = grid;
+  plan->grid = plan->one ? (int)total : grid;
   plan->v = v;
   return TB_OK;
 }
@@ -790,7 +800,7 @@ int run_plan(const Job& j, Plan& plan, hipStream_t stream) {
     p.B -= v->blay == LAY_K ? step : step * j.b_sk;
   }
   void* args[] = {(void*)&p};
-  const void* kern = (p.mode == MODE_SK || p.grp_sk) ? plan.v->kernel_sk : p.k_rest ? w4_kernel_rest(j.dt) : plan.v->kernel;
+  const void* kern = (p.mode == MODE_SK || p.grp_sk) ? plan.v->kernel_sk : p.k_rest ? w4_kernel_rest(j.dt) : plan.one ? plan.v->kernel_one : plan.v->kernel;
   hipError_t e = hipLaunchKernel(kern, dim3((unsigned)plan.grid), dim3((unsigned)plan.v->threads), args, 0, stream);
   if (e != hipSuccess) { (void)hipGetLastError(); return TB_ERR_LAUNCH; }
   return TB_OK;
@@ -808,7 +818,7 @@ int g_splits_used = 0;
 // columns [0, n1) keep the planned tile, the rest becomes a problem of its own; 0 = do not split
 int64_t column_split_point(const Job& j, const tb_hw& hw, const Plan& whole) {
   const Variant* v = whole.v;
-  const int64_t total = whole.p.total_tiles, G = whole.grid, tiles_m = whole.p.tiles_m, tiles_n = whole.p.tiles_n;
+  const int64_t total = whole.p.total_tiles, G = whole.resident, tiles_m = whole.p.tiles_m, tiles_n = whole.p.tiles_n;
   if (whole.skinny || whole.p.mode != MODE_STATIC || v->fast != LOAD_DIRECT || total <= G || total % G == 0) return 0;
   const int64_t tn1 = (total / G) * G / tiles_m;
   if (tn1 <= 0 || tn1 >= tiles_n) return 0;
