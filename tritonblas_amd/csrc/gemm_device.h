@@ -597,7 +597,8 @@ __device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70);
 // ------------------------------------------------------------------------------------------------
 // K loop: accumulates k iterations [it0, it1) of one output tile
 // ------------------------------------------------------------------------------------------------
-template <class T>
+// WHOLE_STEP: the fragments of a whole K step are in registers when its MFMAs begin.
+template <class T, bool WHOLE_STEP = false>
 __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc, int it0, int it1,
                                          v4f (&acc)[T::TM][T::TN], uint8_t* lds, const LaneInfo& li) {
   using OA = Operand<T, T::BM, T::ALAY>;
@@ -690,7 +691,78 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
     }
   };
 
-  if constexpr (T::DMA) {
+  if constexpr (WHOLE_STEP) {
+    // Two sets of registers hold the fragments of the step that is computed and of the next one, so one barrier per step is enough and no MFMA
+    // waits for LDS: behind the barrier of step `it` its stage is free (everybody's reads of it have returned) and step it + 1 is there.  Against the loop
+    // below, 128x128 with eight waves: bf16 2048^3 23.5 -> 22.1 us, 584x4624x3688 38.3 -> 37.0, FP8 512x4096x14336 53.3 -> 49.7; 256x128
+    // FP8 2504x6272x1088 31.5 -> 28.7.
+    static_assert(T::FAST && T::DT != DT_FP4, "LDS-direct operands without block scales");
+    constexpr int S = T::STAGES;
+    constexpr int NG = OA::NCH + OB::NCH;
+    static_assert((S - 1) * NG <= 63, "vmcnt range");
+    auto copy_step = [&](int it, int s) {
+      uint8_t* to = lds + s * T::STAGE_BYTES;
+      OA::dma(sa, it, to, li.tid);
+      OB::dma(sb, it, to + T::A_BYTES, li.tid);
+    };
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      if (it0 + s < it1) {
+        if (s == 0 && it0 == 0 && __builtin_expect(p.k_tail != 0, 0)) {
+          OA::dma_tail(sa, p.k_iters, p.k_tail, lds, li.tid);
+          OB::dma_tail(sb, p.k_iters, p.k_tail, lds + T::A_BYTES, li.tid);
+        } else {
+          copy_step(it0 + s, s);
+        }
+      }
+    }
+    if (it1 - it0 >= S) __builtin_amdgcn_s_waitcnt(0x0F70 | (((S - 1) * NG) & 0xF) | ((((S - 1) * NG) >> 4) << 14));
+    else wait_vm0();
+    __syncthreads();
+    frag_t fa[2][T::KSUB][T::TM], fb[2][T::KSUB][T::TN];
+    auto request = [&](int u, const uint8_t* sA) {
+      const uint8_t* sB = sA + T::A_BYTES;
+#pragma unroll
+      for (int ks = 0; ks < T::KSUB; ++ks) {
+#pragma unroll
+        for (int j = 0; j < T::TN; ++j) fb[u][ks][j] = read_b(sB, ks, j);
+#pragma unroll
+        for (int i = 0; i < T::TM; ++i) fa[u][ks][i] = read_a(sA, ks, i);
+      }
+    };
+    request(0, lds);
+    int stage = 0;
+    constexpr int READS = T::KSUB * (RPFA * T::TM + RPFB * T::TN), MFMAS = T::KSUB * T::TM * T::TN;
+    auto step = [&](int u, int it) {
+      const int nstage = stage + 1 == S ? 0 : stage + 1;
+      // step it + 1 has landed (the S - 2 younger copies may stay in flight while they all exist) and this wave's fragments of step `it` are there
+      if (S > 2 && it + S - 1 < it1) {
+        constexpr int ALLOWED = (S - 2) * NG;
+        __builtin_amdgcn_s_waitcnt(0x0070 | (ALLOWED & 0xF) | ((ALLOWED >> 4) << 14));
+      } else {
+        __builtin_amdgcn_s_waitcnt(0x0070);
+      }
+      __syncthreads();
+      if (it + S < it1) copy_step(it + S, stage);
+      request(u ^ 1, lds + nstage * T::STAGE_BYTES);      // (after the last step: whatever the stage holds, nobody uses it)
+#pragma unroll
+      for (int ks = 0; ks < T::KSUB; ++ks)
+#pragma unroll
+        for (int i = 0; i < T::TM; ++i)
+#pragma unroll
+          for (int j = 0; j < T::TN; ++j) acc[i][j] = mma<T, 0>(fb[u][ks][j], fa[u][ks][i], acc[i][j], 0, 0);
+      // one read, then its share of the MFMAs
+#pragma unroll
+      for (int q = 0; q < READS; ++q) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, (MFMAS + READS - 1) / READS, 0);
+      }
+      stage = nstage;
+    };
+    int it = it0;
+    for (; it + 1 < it1; it += 2) { step(0, it); step(1, it + 1); }
+    if (it < it1) step(0, it);
+  } else if constexpr (T::DMA) {
     constexpr int S = T::STAGES;
     // Stage (it - it0) % S holds K step `it`.  One "group" is what a wave issues per K step: its share
     // of both operand copies.  All S stages are filled up front; afterwards the copy of step it+S is
@@ -1783,12 +1855,24 @@ __global__ __launch_bounds__(T::THREADS, T::MINB) void gemm_kernel(const GemmPar
   }
 }
 
+// Which tiles take the K loop with a whole step's fragments in registers, and their copy stages: the eight-wave ones of the 16- and 8-bit types, and 128x128 with
+// four waves in 16 bits (3200x5248x760 51.7 -> 51.1 us; FP8 1581x7488x1280 25.0 -> 25.4, which keeps the other loop).  128x64 gains least (bf16 2048^3
+// 30.3 -> 29.6, FP8 512x4096x14336 45.6 -> 44.6); 64x64 is level.  In 16 bits three stages are ahead of four here (2048^3 22.8 -> 22.1).
+template <class T>
+struct OneTile {
+  static constexpr bool HALF = T::DT == DT_F16 || T::DT == DT_BF16, BYTE = T::DT == DT_FP8 || T::DT == DT_E5M2 || T::DT == DT_I8;
+  static constexpr bool WHOLE_STEP = T::FAST && T::BKB == 128 && T::BN <= 128 &&
+                                     ((T::THREADS == 512 && (HALF || BYTE)) || (T::BM == 128 && T::BN == 128 && HALF));
+  static constexpr int STAGES = WHOLE_STEP && HALF && T::BM == 128 && T::BN == 128 && T::STAGES > 3 ? 3 : T::STAGES;
+  using tile = Tile<T::DT, T::BM, T::BN, T::BKB, T::WM, T::WN, T::ALAY, T::BLAY, T::MINB, T::LOADER, STAGES>;
+};
+
 // One tile to a workgroup, as many workgroups as tiles: the persistent schedule of a launch that names no grid.  The work loop of gemm_kernel costs
 // a launch 1.0 to 1.9 us in front of its first copy: what the other schedules carry from tile to tile fills the scalar registers (86 spilled, and
 // scratch memory with them; none here).  Back to back, gemm_kernel and this: bf16 512^3 6.0 and 4.9 us, 1024^3 8.7 and 7.7, 2048^3 25.3 and 23.5;
 // FP8 1024x1024x2048 8.2 and 6.9, 512x4096x14336 43.8 and 41.6.  More tiles than fit at once start as others end, which is as fast as a
 // resident grid that loops (FP8 1581x7488x1280 in 128x128 30.1 and 25.0, 2504x6272x1088 32.2 and 31.7; bf16 3200x5248x760 50.0 and 51.7).
-template <class T>
+template <class T, bool WHOLE_STEP>
 __global__ __launch_bounds__(T::THREADS, T::MINB) void gemm_tile_kernel(const GemmParams p) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[T::LDS_ALLOC];
   LaneInfo li;
@@ -1805,7 +1889,7 @@ __global__ __launch_bounds__(T::THREADS, T::MINB) void gemm_tile_kernel(const Ge
   plain_tile(p, tile, T::BM, T::BN, tc);
   tc.m0 = uniform(tc.m0); tc.n0 = uniform(tc.n0);
   v4f acc[T::TM][T::TN];
-  mainloop<T>(p, tc, 0, p.k_iters, acc, lds, li);
+  mainloop<T, WHOLE_STEP>(p, tc, 0, p.k_iters, acc, lds, li);
   sums_to_f32<T>(acc);
   epilogue<T>(p, tc, acc, li, lds);
 }
