@@ -106,3 +106,21 @@ def test_rows_in_parts(shape, dtype):
     _same(x, dtype, 1)
     _same(x[:, 1:], dtype, 1)
     _same(x.float(), dtype, 1, min_scale=20.0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES8)
+@pytest.mark.parametrize("n", [64, 1000, 4096, 16384])
+def test_rows_at_the_edge_of_plain_rounding(n, dtype):
+    """Rows whose values cannot leave the code's range are rounded without a look at it.  At that line: magnitudes up to the largest finite float beside an infinity
+    and a NaN, scales around the smallest normal number, rows of nothing but the largest magnitude."""
+    top = 127.0 if dtype == torch.int8 else torch.finfo(dtype).max
+    huge, tiny = torch.finfo(torch.float32).max, torch.finfo(torch.float32).tiny
+    peaks = [huge, float("inf"), float("nan"), tiny * top, tiny * top * 0.999, tiny * top * 1.001, tiny * 0.5, 1.0, 0.0]
+    x = torch.rand(len(peaks), n, device="cuda") * 2 - 1
+    for row, peak in enumerate(peaks):
+        x[row] *= min(peak, huge) if peak == peak else 1.0
+        x[row, n // 3] = peak
+    x[7] = torch.where(x[7] < 0, -1.0, 1.0)
+    _same(x, dtype, 1, min_scale=0.0)
+    _same(x, dtype, 1)
