@@ -264,10 +264,7 @@ typedef struct tb_grouped_gemm_desc {
   int32_t group_m, num_xcds;
   int32_t small_rows;         /* > 0: an expert's last, partial row block of at most this many rows is
                                  left to a second launch with a short (32-row) tile instead of costing
-                                 a whole tall tile per column block.  0: library default — threshold 64,
-                                 and the kernels price both plans from the row counts on the device
-                                 (rounds of tall tiles against rounds of short ones) and split only
-                                 when that is cheaper; off when block_m is forced.  -1: one launch.
+                                 a whole tall tile per column block.  0 and -1: one launch.
                                  The split needs k % 256 == 0 and a tall (>= 128-row) tile.            */
   int32_t streamk;            /* 1: the tiles that do not fill whole rounds of the grid are cut into K ranges
                                  (Stream-K, as kernels/streamk_gemm.py:160-384 does for one matrix) whenever the

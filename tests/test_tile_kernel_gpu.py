@@ -56,3 +56,30 @@ def test_one_tile_per_workgroup_matches_the_loop(kind, m, n, k, order):
         loop = _product(a, b, torch.full((m, n), float("nan"), device="cuda", dtype=out), tile, 48)
         assert torch.equal(got, loop), tile
         assert ((got.double() - want).abs() <= REL[kind] * want.abs()).all(), tile
+
+
+GROUPED_TILES = [((256, 128, 128), 423), ((128, 128, 128), 222), ((128, 128, 128), 424), ((128, 64, 128), 424), ((64, 64, 128), 222), ((64, 64, 128), 223),
+                 ((64, 64, 128), 224), ((32, 128, 256), 143), ((256, 256, 128), 22), (None, 0)]
+
+
+@pytest.mark.parametrize("counts,n,k", [
+    ([1], 1, 16), ([0, 33, 0, 31, 1, 0], 130, 272), ([127, 128, 129, 0, 255, 257], 200, 1040),      # corners, empty experts, edges of the tiles, remainders of K
+    ([3 * (e % 5) for e in range(131)], 96, 512),                                                   # more experts than a wave has lanes
+    ([5000, 1, 700], 1100, 640),                                                                    # more tiles than the device holds at once
+])
+def test_grouped_one_tile_per_workgroup(counts, n, k, tb_option):
+    import tritonblas_amd as tb
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    rows, experts = sum(counts), len(counts)
+    a = torch.randint(-2, 3, (rows, k), device="cuda", generator=g).to(torch.float8_e4m3fn)
+    w = torch.randint(-2, 3, (experts, n, k), device="cuda", generator=g).to(torch.float8_e4m3fn)
+    at = [0]
+    for c in counts:
+        at.append(at[-1] + c)
+    offsets = torch.tensor(at, dtype=torch.int32, device="cuda")
+    want = torch.cat([a[lo:hi].double() @ w[e].double().T for e, (lo, hi) in enumerate(zip(at, at[1:]))])     # (whole numbers below 2**24: exact in fp32)
+    for tile, waves in GROUPED_TILES:
+        tb_option("waves", waves)
+        got = torch.full((rows, n), float("nan"), device="cuda", dtype=torch.bfloat16)
+        tb.grouped_matmul_a8w8(a, w, None, None, got, offsets, *(tile or (None, None, None)))
+        assert ((got.double() - want).abs() <= REL["fp8"] * want.abs()).all(), (tile, waves)

@@ -100,12 +100,7 @@ struct GemmParams {
   // grouped, two launches: phase 1 tiles every expert's rows with grp_big-row blocks but leaves a last
   // partial block of at most grp_thr rows to phase 2, which tiles just those rows with a short tile
   // (a handful of rows would otherwise cost a whole tall tile per column block).  Phase 0: one launch.
-  // With grp_auto every workgroup of both launches first prices the two plans from the row counts
-  // (rounds of tall tiles cost 4, rounds of short tiles 3) and both launches act on the same verdict:
-  // either the first runs the one-launch table and the second does nothing, or they split the rows.
   int32_t grp_phase, grp_big, grp_thr;
-  int32_t grp_auto, grp_small_bm;
-  int32_t grp_other_tn, grp_other_grid;   // column tiles and grid of the other launch
   // grouped with a Stream-K tail (4-wave kernels): the tiles that do not fill whole rounds of the grid are cut into
   // K ranges as in MODE_SK; how many that is follows from the row counts, so every workgroup works it out
   // itself (sk_tail_tiles).  grp_sk_fix: what one extra piece of a tile costs its owner, in K steps.
@@ -1427,27 +1422,6 @@ __device__ __forceinline__ void plain_tile(const GemmParams& p, int tile, int BM
 }
 
 // Grouped table: experts in order, expert e owns (its row blocks in this phase) * tiles_n tiles, m-block fastest.
-// The phase this launch runs: 0 one-launch table, 1 / 2 the split tables, -1 nothing.
-__device__ __forceinline__ int grouped_phase(const GemmParams& p, int grid) {
-  if (p.grp_phase == 0 || !p.grp_auto) return p.grp_phase;
-  int b0 = 0, b1 = 0, b2 = 0;
-  for (int e = 0; e < p.num_groups; ++e) {
-    const int rows = max(p.group_offsets[e + 1] - p.group_offsets[e], 0);
-    const int full = rows / p.grp_big, rem = rows - full * p.grp_big;
-    const bool small = rem > 0 && rem <= p.grp_thr;
-    b0 += full + (rem > 0 ? 1 : 0);
-    b1 += full + ((rem > 0 && !small) ? 1 : 0);
-    b2 += small ? (rem + p.grp_small_bm - 1) / p.grp_small_bm : 0;
-  }
-  const int tn_big = p.grp_phase == 1 ? p.tiles_n : p.grp_other_tn, tn_small = p.grp_phase == 1 ? p.grp_other_tn : p.tiles_n;
-  const int g_big = p.grp_phase == 1 ? grid : p.grp_other_grid, g_small = p.grp_phase == 1 ? p.grp_other_grid : grid;
-  const int64_t one = 4 * (((int64_t)b0 * tn_big + g_big - 1) / g_big);
-  const int64_t two = 4 * (((int64_t)b1 * tn_big + g_big - 1) / g_big) + 3 * (((int64_t)b2 * tn_small + g_small - 1) / g_small);
-  const bool split = b2 > 0 && two < one;
-  if (p.grp_phase == 1) return split ? 1 : 0;
-  return split ? 2 : -1;
-}
-
 // the row blocks of expert e in the table of a phase: their number, the first row and the row limit
 __device__ __forceinline__ int grouped_rows(const GemmParams& p, int phase, int e, int BM, int& base, int& lim) {
   const int lo = p.group_offsets[e], hi = p.group_offsets[e + 1];
@@ -1530,13 +1504,11 @@ struct Sched {
   int step;               // work stealing: queue visit index
   int64_t start, last, q, rem;  // Stream-K iteration range of this workgroup
   int dp_tiles;
-  int gphase;             // grouped: which tile table this launch runs
   int gtotal;             // grouped with a Stream-K tail: entries of that table
   bool ws_phase;          // Stream-K with work stealing: still drawing whole tiles from the queues
 
   __device__ __forceinline__ void init(const GemmParams& p) {
     G = gridDim.x;
-    gphase = p.mode == MODE_GROUPED ? grouped_phase(p, G) : 0;
     gtotal = 0;
     pid = blockIdx.x;
     sk_id = blockIdx.x;
@@ -1559,11 +1531,11 @@ struct Sched {
       last = (int64_t)dp_tiles * ipt + (sk_id + 1) * q + min((int64_t)sk_id + 1, rem);
     }
     if constexpr (SK) {
-      if (p.mode == MODE_GROUPED && p.grp_sk && gphase >= 0) {
+      if (p.mode == MODE_GROUPED && p.grp_sk) {
         // the table's real length is only known here; whole rounds first, the rest in K ranges (ordered as in MODE_SK)
         const int unit = max(1, p.sk_unit);
         const int64_t ipt = p.k_iters / unit;
-        gtotal = grouped_total(p, gphase, T::BM);
+        gtotal = grouped_total(p, p.grp_phase, T::BM);
         const int skt = sk_tail_tiles(gtotal, G, (int)ipt, unit, p.grp_sk_fix);
         dp_tiles = gtotal - skt;
         const int64_t total_sk = (int64_t)skt * ipt;
@@ -1640,14 +1612,13 @@ struct Sched {
       bool tail = false;
       if constexpr (SK) tail = p.grp_sk != 0;
       if (!tail) {
-        if (gphase < 0 || next_tile >= p.total_tiles) return false;
-        bool ok = grouped_tile(p, gphase, next_tile, T::BM, T::BN, T::USZ, w.tc);
+        if (next_tile >= p.total_tiles) return false;
+        bool ok = grouped_tile(p, p.grp_phase, next_tile, T::BM, T::BN, T::USZ, w.tc);
         next_tile = ok ? next_tile + G : p.total_tiles;
         return ok;
       }
-      if (gphase < 0) return false;
       if (next_tile < dp_tiles) {
-        grouped_tile(p, gphase, next_tile, T::BM, T::BN, T::USZ, w.tc);
+        grouped_tile(p, p.grp_phase, next_tile, T::BM, T::BN, T::USZ, w.tc);
         next_tile += G;
         return true;
       }
@@ -1725,7 +1696,7 @@ struct Sched {
     const int64_t tile_first = (int64_t)tile * ipt;
     const int64_t tile_end = tile_first + ipt;
     const int64_t begin = max(tile_first, start);
-    if (grouped) grouped_tile(p, gphase, tile, T::BM, T::BN, T::USZ, w.tc);
+    if (grouped) grouped_tile(p, p.grp_phase, tile, T::BM, T::BN, T::USZ, w.tc);
     else plain_tile(p, tile, T::BM, T::BN, w.tc);
     w.it0 = (int)(begin - tile_first) * unit;
     w.it1 = (int)(last - tile_first) * unit;
@@ -1888,6 +1859,61 @@ __global__ __launch_bounds__(T::THREADS, T::MINB) void gemm_tile_kernel(const Ge
   TileCtx tc;
   plain_tile(p, tile, T::BM, T::BN, tc);
   tc.m0 = uniform(tc.m0); tc.n0 = uniform(tc.n0);
+  v4f acc[T::TM][T::TN];
+  mainloop<T, WHOLE_STEP>(p, tc, 0, p.k_iters, acc, lds, li);
+  sums_to_f32<T>(acc);
+  epilogue<T>(p, tc, acc, li, lds);
+}
+
+// The entry `tile` of the grouped table of one launch (see grouped_rows, phase 0), looked up by a whole wave: a lane takes an expert, the tiles in front of each
+// are a prefix sum over the lanes.  A scan expert by expert waits for two scalar loads and divides for each.
+template <class T>
+__device__ __forceinline__ bool grouped_tile_by_wave(const GemmParams& p, int tile, int lane, TileCtx& tc) {
+  for (int e0 = 0; e0 < p.num_groups; e0 += 64) {
+    const int e = e0 + lane;
+    int lo = 0, hi = 0;
+    if (e < p.num_groups) { lo = p.group_offsets[e]; hi = p.group_offsets[e + 1]; }
+    const int mb = (max(hi - lo, 0) + T::BM - 1) / T::BM, count = mb * p.tiles_n;
+    int upto = count;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(upto, d);
+      if (lane >= d) upto += v;
+    }
+    const uint64_t past = __ballot(tile < upto);
+    if (past) {
+      const int at = __ffsll((unsigned long long)past) - 1;
+      const int blocks = __builtin_amdgcn_readlane(mb, at), local = tile - (__builtin_amdgcn_readlane(upto, at) - __builtin_amdgcn_readlane(count, at));
+      tc.m0 = uniform(__builtin_amdgcn_readlane(lo, at) + (local % blocks) * T::BM);
+      tc.n0 = uniform((local / blocks) * T::BN);
+      tc.m_lim = __builtin_amdgcn_readlane(hi, at); tc.n_lim = p.N;
+      tc.B = uniform(p.B + (int64_t)(e0 + at) * p.b_group_stride * T::USZ);
+      tc.sb = p.sb ? uniform(p.sb + (int64_t)(e0 + at) * p.sb_group_stride) : nullptr;
+      return true;
+    }
+    tile -= __builtin_amdgcn_readlane(upto, 63);
+  }
+  return false;
+}
+
+// The grouped schedule, one tile to a workgroup: as many workgroups as the table can have entries (the row counts are on the device), those past its end leave.
+// gemm_kernel and this, same tile, us: 128x128 with four waves, 16 experts of 4096x2048, 4096 rows 83.8 and 67.0; 64x64, 64 rows 37.3 and 26.5; 8 experts of 14336x4096,
+// 64 rows 113.8 and 106.0; 256x128, 8 experts of 2048x1024, 3000 rows 19.6 and 17.2.  (The hand-scheduled 256x256 kernel stays with its loop.)
+template <class T, bool WHOLE_STEP>
+__global__ __launch_bounds__(T::THREADS, T::MINB) void gemm_group_kernel(const GemmParams p) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[T::LDS_ALLOC];
+  LaneInfo li;
+  li.tid = threadIdx.x;
+  li.lane = li.tid & 63;
+  li.r = li.lane & 15;
+  li.g = li.lane >> 4;
+  const int wave = li.tid >> 6;
+  li.wm0 = (wave / T::WN) * T::WTM;
+  li.wn0 = (wave % T::WN) * T::WTN;
+  int tile = blockIdx.x;
+  if (p.num_xcds > 1) tile = chiplet_transform_chunked(tile, gridDim.x, p.num_xcds, p.chunk);
+  TileCtx tc;
+  if (!grouped_tile_by_wave<T>(p, tile, li.lane, tc)) return;
   v4f acc[T::TM][T::TN];
   mainloop<T, WHOLE_STEP>(p, tc, 0, p.k_iters, acc, lds, li);
   sums_to_f32<T>(acc);

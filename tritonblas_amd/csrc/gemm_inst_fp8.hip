@@ -23,4 +23,23 @@ const Variant g_variants_fp8[] = {
 };
 const int g_num_variants_fp8 = sizeof(g_variants_fp8) / sizeof(Variant);
 
+template <class T>
+static bool group_kernel_of(const Variant& v, const void** out) {
+  if (v.dt != T::DT || v.bm != T::BM || v.bn != T::BN || v.bk != T::BK || v.threads != T::THREADS || v.stages != T::STAGES || v.fast != LOAD_DIRECT || v.k_step_pairs) return false;
+  *out = (const void*)&gemm_group_kernel<typename OneTile<T>::tile, OneTile<T>::WHOLE_STEP>;
+  return true;
+}
+template <class... T>
+static const void* group_kernel_among(const Variant& v) {
+  const void* k = nullptr;
+  (void)(group_kernel_of<T>(v, &k) || ...);
+  return k;
+}
+const void* group_kernel(const Variant& v) {
+  return group_kernel_among<Tile<DT_FP8, 256, 128, 128, 4, 2, LAY_K, LAY_K, 1, LOAD_DIRECT, 3>, Tile<DT_FP8, 128, 128, 128, 2, 2, LAY_K, LAY_K, 2, LOAD_DIRECT, 2>,
+                            Tile<DT_FP8, 128, 128, 128, 4, 2, LAY_K, LAY_K, 1, LOAD_DIRECT, 4>, Tile<DT_FP8, 128, 64, 128, 4, 2, LAY_K, LAY_K, 1, LOAD_DIRECT, 4>,
+                            Tile<DT_FP8, 64, 64, 128, 2, 2, LAY_K, LAY_K, 4, LOAD_DIRECT, 2>, Tile<DT_FP8, 64, 64, 128, 2, 2, LAY_K, LAY_K, 3, LOAD_DIRECT, 3>,
+                            Tile<DT_FP8, 64, 64, 128, 2, 2, LAY_K, LAY_K, 2, LOAD_DIRECT, 4>, Tile<DT_FP8, 32, 128, 256, 1, 4, LAY_K, LAY_K, 1, LOAD_DIRECT, 3>>(v);
+}
+
 }  // namespace tb

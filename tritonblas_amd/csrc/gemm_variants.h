@@ -43,6 +43,9 @@ Variant make_variant_w4() {
                  T::ALAY == LAY_M || T::BLAY == LAY_M ? nullptr : w4_kernel_sk(T::DT), 1};
 }
 
+// the grouped kernel of a tile, one tile to a workgroup (null: the tile has none; gemm_inst_fp8.hip)
+const void* group_kernel(const Variant& v);
+
 // defined one per translation unit
 extern const Variant g_variants_f16[];
 extern const int g_num_variants_f16;

@@ -22,6 +22,8 @@ int variant_occupancy(const TileInfo& v, const tb_hw& hw);
 int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, int ntiles, tb_selection* out);
 // model time (us) of one tile variant on a problem, and of the streaming small-M kernel
 double estimate_tile_us(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bool streamk);
+// ... of a grouped launch whose row counts only the device knows (FP8; 0: no figures for this variant)
+double estimate_grouped_us(const tb_problem& pr, const tb_hw& hw, const TileInfo& v);
 double estimate_streaming_us(const tb_problem& pr, const tb_hw& hw, int cols);
 double streaming_bound_us(const tb_problem& pr, const tb_hw& hw);   // ... and what it takes at most
 

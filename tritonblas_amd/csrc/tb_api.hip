@@ -263,7 +263,7 @@ struct Job {
   // grouped
   const int32_t* group_offsets = nullptr; int num_groups = 0;
   int64_t b_group_stride = 0, sb_group_stride = 0;
-  int grp_phase = 0, grp_big = 0, grp_thr = 0, grp_auto = 0;   // see GemmParams
+  int grp_phase = 0, grp_big = 0, grp_thr = 0;   // see GemmParams
   int grp_sk = 0;          // grouped: cut the tiles that do not fill whole rounds of the grid into K ranges (needs a workspace)
   int column_split = 0;
   int tiles_only = 0;      // 1: never the streaming kernel
@@ -324,6 +324,24 @@ bool grid_keeps(const Job& j, const tb_hw& hw, int bm, int bn, int bk) {
 // The grid of the whole-tile launch that a Stream-K launch without shared tiles becomes: what is resident, unless its
 // caller keeps it to fewer workgroups than there are CUs.
 int whole_tile_grid(const Job& j, const tb_hw& hw, const Plan& plan, int grid) { return plan.kept && j.grid < hw.n_cu ? grid : 0; }
+
+// The variant that the model has ahead for a grouped launch whose caller names no tile (operands that the LDS-direct loaders take).  tall: what stands for the
+// 256x256 tile, which has a kernel for whole K steps and one for the rest.
+const Variant* grouped_variant(const Job& j, const tb_hw& hw, const Variant* tall) {
+  tb_problem pr;
+  std::memset(&pr, 0, sizeof(pr));
+  pr.m = j.M; pr.n = j.N; pr.k = j.K; pr.a_type = pr.b_type = model_type(j.dt); pr.c_type = j.c_type; pr.num_groups = j.num_groups;
+  const Variant* best = nullptr;
+  double best_us = 0.0;
+  for (auto& x : variants_of(j.dt)) {
+    if (x.fast != LOAD_DIRECT || x.alay != LAY_K || x.blay != LAY_K) continue;
+    if (x.bm == 256 && x.bn == 256 ? &x != tall : !group_kernel(x)) continue;
+    if (x.bm * j.a_sr >= (1ll << 31) || x.bn * j.b_sr >= (1ll << 31)) continue;      // (32-bit offsets inside a tile)
+    const double us = estimate_grouped_us(pr, hw, TileInfo{x.dt, x.bm, x.bn, x.bk, x.threads, x.lds_bytes, x.minb, x.fast, x.stages});
+    if (us > 0.0 && (!best || us < best_us)) { best = &x; best_us = us; }
+  }
+  return best;
+}
 
 int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
   if (j.M <= 0 || j.N <= 0 || j.K <= 0) return TB_ERR_BAD_SHAPE;
@@ -419,8 +437,11 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
     int64_t at_once = ((j.M + bm - 1) / bm) * ((j.N + bn - 1) / bn);
     if (is_streamk(j.schedule)) at_once = j.grid > 0 ? std::max<int64_t>(at_once, j.grid) : 0;
     if (j.num_groups > 0) at_once = 0;
+    const bool by_model = j.num_groups > 0 && j.bm == 0 && !j.grp_sk && j.grp_phase == 0;
+    if (by_model) { bm = bn = 256; bk = 128; }
     v = find_variant(j.dt, bm, bn, bk, alay, blay, 1, at_once, &hw, is_streamk(j.schedule) && j.num_groups == 0, j.K,
                      j.c_type == TB_I8 ? 2 : (is_f8_type(j.c_type) ? 1 : 0), rest_pays());
+    if (by_model) v = grouped_variant(j, hw, v);
     if (!v) return TB_ERR_BAD_TILE;
   } else {
     if (j.bm != 0) {
@@ -533,7 +554,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
     // the tile table has at most this many entries (every expert may end in a partial row block);
     // a resident grid loops over it
     p.mode = MODE_GROUPED;
-    p.grp_phase = j.grp_phase; p.grp_big = j.grp_big; p.grp_thr = j.grp_thr; p.grp_auto = j.grp_auto;
+    p.grp_phase = j.grp_phase; p.grp_big = j.grp_big; p.grp_thr = j.grp_thr;
     if (p.grp_phase == 1) {
       // only a tall fast tile leaves its short last blocks to a second launch
       if (v->fast && v->bm >= 128 && j.grp_thr > 0 && j.grp_thr < v->bm) p.grp_big = v->bm;
@@ -542,11 +563,12 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
     if (p.grp_phase == 2 && (p.grp_big <= 0 || p.grp_thr <= 0)) return TB_ERR_BAD_ARGUMENT;
     const int64_t bound = p.grp_phase == 2
         ? (int64_t)j.num_groups * ((j.grp_thr + v->bm - 1) / v->bm) * p.tiles_n
-        : ((j.M + v->bm - 1) / v->bm + j.num_groups) * p.tiles_n;
+        : std::min<int64_t>(j.M, (j.M + (int64_t)j.num_groups * (v->bm - 1)) / v->bm) * p.tiles_n;
     if (bound > INT32_MAX) return TB_ERR_BAD_SHAPE;
     p.total_tiles = (int32_t)bound;
     grid = (int)std::min<int64_t>(bound, resident);
     if (hooks().grid > 0) grid = (int)std::min<int64_t>(bound, hooks().grid);
+    plan->one = p.grp_phase == 0 && hooks().grid <= 0 && group_kernel(*v) != nullptr;
     // Stream-K tail: only the hand-scheduled 4-wave kernel has the cheap exchange of partial tiles that makes
     // it pay (K ranges in blocks of four steps), and only the launch of the tall tiles
     if (j.grp_sk && p.grp_phase != 2 && v->k_step_pairs && v->kernel_sk && p.k_rest == 0 && p.k_iters % 4 == 0 && p.k_iters >= 8 && occ == 1) {
@@ -657,7 +679,9 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
   p.panel_n = default_panel_n(grid, p.chunk, p.group_m);
   if (hooks().panel >= 0) p.panel_n = hooks().panel;
   plan->resident = grid;
-  plan->grid = plan->one ? (int)total : grid;
+  // (a launch takes less than 2^32 threads)
+  plan->one = plan->one && (int64_t)p.total_tiles * v->threads < (1ll << 32);
+  plan->grid = plan->one ? p.total_tiles : grid;
   plan->v = v;
   return TB_OK;
 }
@@ -685,7 +709,7 @@ PlanKey plan_key(const Job& j, int dev) {
       j.dt, j.c_type, j.bias_type, j.schedule, dev, j.M, j.N, j.K, j.a_sr, j.a_sk, j.b_sr, j.b_sk, j.c_sm, j.c_sn,
       j.mxa_sr, j.mxa_sk, j.mxb_sr, j.mxb_sk, j.bias_stride, j.bm, j.bn, j.bk, j.group_m, j.num_xcds, j.grid,
       j.counters_per_xcd, j.ws_mode, j.ws_local, j.cu_mask_len, j.ws_global, j.num_groups, j.grp_phase, j.grp_big,
-      j.grp_thr, j.grp_auto, j.grp_sk, j.b_group_stride, j.sb_group_stride, al(j.A), al(j.B), al(j.C), al(j.mxa), al(j.mxb),
+      j.grp_thr, j.grp_sk, j.b_group_stride, j.sb_group_stride, al(j.A), al(j.B), al(j.C), al(j.mxa), al(j.mxb),
       al(j.bias), j.sa ? 1 : 0, j.sb ? 1 : 0, j.cu_mask ? 1 : 0, j.group_offsets ? 1 : 0, j.column_split, j.retreat, j.tiles_only, (int64_t)j.room,
       (int64_t)g_hooks_version};
   static_assert(sizeof(f) <= sizeof(k.v), "PlanKey too small");
@@ -800,7 +824,7 @@ int run_plan(const Job& j, Plan& plan, hipStream_t stream) {
     p.B -= v->blay == LAY_K ? step : step * j.b_sk;
   }
   void* args[] = {(void*)&p};
-  const void* kern = (p.mode == MODE_SK || p.grp_sk) ? plan.v->kernel_sk : p.k_rest ? w4_kernel_rest(j.dt) : plan.one ? plan.v->kernel_one : plan.v->kernel;
+  const void* kern = (p.mode == MODE_SK || p.grp_sk) ? plan.v->kernel_sk : p.k_rest ? w4_kernel_rest(j.dt) : !plan.one ? v->kernel : p.mode == MODE_GROUPED ? group_kernel(*v) : v->kernel_one;
   hipError_t e = hipLaunchKernel(kern, dim3((unsigned)plan.grid), dim3((unsigned)plan.v->threads), args, 0, stream);
   if (e != hipSuccess) { (void)hipGetLastError(); return TB_ERR_LAUNCH; }
   return TB_OK;
@@ -1199,14 +1223,11 @@ static int job_from_grouped(const tb_grouped_gemm_desc* d, Job* out, bool* two) 
     j.workspace = d->workspace; j.workspace_bytes = d->workspace_bytes;
     j.epoch = d->epoch; j.spin_limit = d->spin_limit;
   }
-  // Two launches unless switched off or a tile is forced: tall tiles for whole row blocks and long
-  // remainders, then a short streaming tile for the experts whose last block holds few rows (the row
-  // counts live on the device, so both tile tables are evaluated there; an empty second table costs
-  // one empty launch).
+  // Two launches where asked for: tall tiles for whole row blocks and long remainders, then a short streaming tile for the experts whose last
+  // block holds few rows.  (Never by itself: a short tile costs 3/4 of a tall one and covers half its columns, and an empty second launch takes 7 us.)
   if (d->small_rows < -1) return TB_ERR_BAD_ARGUMENT;
-  const int thr = d->small_rows > 0 ? d->small_rows : 64;
-  *two = (d->small_rows > 0 || (d->small_rows == 0 && d->block_m == 0)) && d->k % kGroupedSmallBK == 0;
-  if (*two) { j.grp_phase = 1; j.grp_thr = thr; j.grp_auto = d->small_rows == 0; }
+  *two = d->small_rows > 0 && d->k % kGroupedSmallBK == 0;
+  if (*two) { j.grp_phase = 1; j.grp_thr = d->small_rows; }
   *out = j;
   return TB_OK;
 }
@@ -1250,9 +1271,6 @@ int tb_grouped_gemm_fp8(const tb_grouped_gemm_desc* d, void* stream) {
   j2.grp_sk = 0; j2.workspace = nullptr; j2.workspace_bytes = 0;
   st = cached_plan(j2, hw, &second);
   if (st != TB_OK) return st;
-  first.p.grp_small_bm = second.p.grp_small_bm = second.v->bm;
-  first.p.grp_other_tn = second.p.tiles_n; first.p.grp_other_grid = second.grid;
-  second.p.grp_other_tn = first.p.tiles_n; second.p.grp_other_grid = first.grid;
   st = run_plan(j, first, (hipStream_t)stream);
   if (st != TB_OK) return st;
   return run_plan(j2, second, (hipStream_t)stream);
