@@ -367,17 +367,16 @@ struct Operand {
   // the compiler may just have written with a vector instruction and the load that reads it.
   __device__ static __forceinline__ void dma(const St& st, int it, uint8_t* lds, int tid) {
     const uint8_t* gp = step_ptr(st, it);
-    const int wave_slot = __builtin_amdgcn_readfirstlane(tid & ~63);
-    const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) uint8_t*)lds);
 #pragma unroll
-    for (int i = 0; i < NCH; ++i) {
-      if (CHUNKS % T::THREADS != 0 && i * T::THREADS + wave_slot >= CHUNKS) continue;
-      const uint32_t dst = lds0 + (uint32_t)((i * T::THREADS + wave_slot) * 16);
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2"
-                   :
-                   : "s"(dst), "v"(st.off[i]), "s"(gp)
-                   : "memory", "m0");
-    }
+    for (int i = 0; i < NCH; ++i) dma_one(st, i, gp, lds, tid);
+  }
+
+  // the i-th of a step's NCH copies, from the step's origin
+  __device__ static __forceinline__ void dma_one(const St& st, int i, const uint8_t* gp, uint8_t* lds, int tid) {
+    const int wave_slot = __builtin_amdgcn_readfirstlane(tid & ~63);
+    if (CHUNKS % T::THREADS != 0 && i * T::THREADS + wave_slot >= CHUNKS) return;
+    const uint32_t dst = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) uint8_t*)lds) + (uint32_t)((i * T::THREADS + wave_slot) * 16);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(dst), "v"(st.off[i]), "s"(gp) : "memory", "m0");
   }
 
   // The remainder of K, k_tail storage units behind the K steps in front of step `end`: chunks beyond K come from a chunk of
@@ -728,35 +727,68 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
     request(0, lds);
     int stage = 0;
     constexpr int READS = T::KSUB * (RPFA * T::TM + RPFB * T::TN), MFMAS = T::KSUB * T::TM * T::TN;
-    auto step = [&](int u, int it) {
+    // AMONG: the copies of step it + S between shares of the reads and MFMAs.  Issued in one go behind the barrier they hold every wave up together, a copy
+    // keeps the address path of the CU for 16 cycles, and only then its MFMAs begin.  Each in front of its share; behind it they start too late where the copies
+    // bound the step (128x128 below 46.6 -> 47.5, 47.8 -> 52).  In one go and among, 128x128, us: bf16 512x1024x4096 32.7 and 26.0, 2048^3 23.7 and 23.1,
+    // 1871x1728x12544 105.5 and 101.5, 2048x4096x4096 81.7 and 74.8, 584x4624x3688 46.0 and 46.6, 584x4608x3688 51.3 and 47.8; FP8 512x1024x4096 18.1 and 15.7, 2048^3 14.4 and
+    // 13.6; 128x64: bf16 512x1024x4096 23.0 and 19.4, 1536x1536x4096 48.9 and 45.3, 512x4096x14336 96.2 and 95.7; 256x128: bf16 2048x4096x4096 62.1
+    // and 60.6.  With four waves (one to a SIMD) up to twice the time: eight only.
+    constexpr bool EIGHT = T::THREADS == 512;
+    auto step = [&](auto AMONG, int u, int it) {
       const int nstage = stage + 1 == S ? 0 : stage + 1;
       // step it + 1 has landed (the S - 2 younger copies may stay in flight while they all exist) and this wave's fragments of step `it` are there
-      if (S > 2 && it + S - 1 < it1) {
-        constexpr int ALLOWED = (S - 2) * NG;
-        __builtin_amdgcn_s_waitcnt(0x0070 | (ALLOWED & 0xF) | ((ALLOWED >> 4) << 14));
-      } else {
-        __builtin_amdgcn_s_waitcnt(0x0070);
-      }
+      if (S > 2 && it + S - 1 < it1) __builtin_amdgcn_s_waitcnt(0x0070 | (((S - 2) * NG) & 0xF) | ((((S - 2) * NG) >> 4) << 14));
+      else __builtin_amdgcn_s_waitcnt(0x0070);
       __syncthreads();
-      if (it + S < it1) copy_step(it + S, stage);
-      request(u ^ 1, lds + nstage * T::STAGE_BYTES);      // (after the last step: whatever the stage holds, nobody uses it)
+      const uint8_t* nA = lds + nstage * T::STAGE_BYTES;
+      if constexpr (decltype(AMONG)::value) {
+        uint8_t* to = lds + stage * T::STAGE_BYTES;
+        const uint8_t *ga = OA::step_ptr(sa, it + S), *gb = OB::step_ptr(sb, it + S), *nB = nA + T::A_BYTES;
+        constexpr int FRAGS = T::KSUB * (T::TM + T::TN);
 #pragma unroll
-      for (int ks = 0; ks < T::KSUB; ++ks)
+        for (int q = 0; q < NG; ++q) {
+          if (q < OA::NCH) OA::dma_one(sa, q, ga, to, li.tid);
+          else OB::dma_one(sb, q - OA::NCH, gb, to + T::A_BYTES, li.tid);
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < T::TM; ++i)
+          for (int f = 0; f < FRAGS; ++f) {
+            if (f * NG / FRAGS != q) continue;
+            const int ks = f / (T::TM + T::TN), x = f % (T::TM + T::TN);
+            if (x < T::TN) fb[u ^ 1][ks][x] = read_b(nB, ks, x);
+            else fa[u ^ 1][ks][x - T::TN] = read_a(nA, ks, x - T::TN);
+          }
 #pragma unroll
-          for (int j = 0; j < T::TN; ++j) acc[i][j] = mma<T, 0>(fb[u][ks][j], fa[u][ks][i], acc[i][j], 0, 0);
-      // one read, then its share of the MFMAs
+          for (int m = 0; m < MFMAS; ++m) {
+            if (m * NG / MFMAS != q) continue;
+            const int ks = m / (T::TM * T::TN), i = m / T::TN % T::TM, j = m % T::TN;
+            acc[i][j] = mma<T, 0>(fb[u][ks][j], fa[u][ks][i], acc[i][j], 0, 0);
+            asm volatile("" : "+v"(acc[i][j]));      // (side-effect-free: without a use here it could go behind the next copy)
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+        if (it + S < it1) copy_step(it + S, stage);
+        request(u ^ 1, nA);      // (after the last step: whatever the stage holds, nobody uses it)
 #pragma unroll
-      for (int q = 0; q < READS; ++q) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, (MFMAS + READS - 1) / READS, 0);
+        for (int ks = 0; ks < T::KSUB; ++ks)
+#pragma unroll
+          for (int i = 0; i < T::TM; ++i)
+#pragma unroll
+            for (int j = 0; j < T::TN; ++j) acc[i][j] = mma<T, 0>(fb[u][ks][j], fa[u][ks][i], acc[i][j], 0, 0);
+        // one read, then its share of the MFMAs
+#pragma unroll
+        for (int q = 0; q < READS; ++q) {
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, (MFMAS + READS - 1) / READS, 0);
+        }
       }
       stage = nstage;
     };
     int it = it0;
-    for (; it + 1 < it1; it += 2) { step(0, it); step(1, it + 1); }
-    if (it < it1) step(0, it);
+    if constexpr (EIGHT)
+      for (; it + 1 + S < it1; it += 2) { step(std::true_type{}, 0, it); step(std::true_type{}, 1, it + 1); }
+    for (; it + 1 < it1; it += 2) { step(std::false_type{}, 0, it); step(std::false_type{}, 1, it + 1); }
+    if (it < it1) step(std::false_type{}, 0, it);
   } else if constexpr (T::DMA) {
     constexpr int S = T::STAGES;
     // Stage (it - it0) % S holds K step `it`.  One "group" is what a wave issues per K step: its share
@@ -1826,16 +1858,14 @@ __global__ __launch_bounds__(T::THREADS, T::MINB) void gemm_kernel(const GemmPar
   }
 }
 
-// Which tiles take the K loop with a whole step's fragments in registers, and their copy stages: the eight-wave ones of the 16- and 8-bit types, and 128x128 with
+// Which tiles take the K loop with a whole step's fragments in registers: the eight-wave ones of the 16- and 8-bit types, and 128x128 with
 // four waves in 16 bits (3200x5248x760 51.7 -> 51.1 us; FP8 1581x7488x1280 25.0 -> 25.4, which keeps the other loop).  128x64 gains least (bf16 2048^3
-// 30.3 -> 29.6, FP8 512x4096x14336 45.6 -> 44.6); 64x64 is level.  In 16 bits three stages are ahead of four here (2048^3 22.8 -> 22.1).
+// 30.3 -> 29.6, FP8 512x4096x14336 45.6 -> 44.6); 64x64 is level.
 template <class T>
 struct OneTile {
   static constexpr bool HALF = T::DT == DT_F16 || T::DT == DT_BF16, BYTE = T::DT == DT_FP8 || T::DT == DT_E5M2 || T::DT == DT_I8;
   static constexpr bool WHOLE_STEP = T::FAST && T::BKB == 128 && T::BN <= 128 &&
                                      ((T::THREADS == 512 && (HALF || BYTE)) || (T::BM == 128 && T::BN == 128 && HALF));
-  static constexpr int STAGES = WHOLE_STEP && HALF && T::BM == 128 && T::BN == 128 && T::STAGES > 3 ? 3 : T::STAGES;
-  using tile = Tile<T::DT, T::BM, T::BN, T::BKB, T::WM, T::WN, T::ALAY, T::BLAY, T::MINB, T::LOADER, STAGES>;
 };
 
 // One tile to a workgroup, as many workgroups as tiles: the persistent schedule of a launch that names no grid.  The work loop of gemm_kernel costs

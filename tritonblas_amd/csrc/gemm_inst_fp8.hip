@@ -26,7 +26,7 @@ const int g_num_variants_fp8 = sizeof(g_variants_fp8) / sizeof(Variant);
 template <class T>
 static bool group_kernel_of(const Variant& v, const void** out) {
   if (v.dt != T::DT || v.bm != T::BM || v.bn != T::BN || v.bk != T::BK || v.threads != T::THREADS || v.stages != T::STAGES || v.fast != LOAD_DIRECT || v.k_step_pairs) return false;
-  *out = (const void*)&gemm_group_kernel<typename OneTile<T>::tile, OneTile<T>::WHOLE_STEP>;
+  *out = (const void*)&gemm_group_kernel<T, OneTile<T>::WHOLE_STEP>;
   return true;
 }
 template <class... T>

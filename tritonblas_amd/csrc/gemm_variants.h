@@ -21,7 +21,7 @@ struct Variant {
 template <class T>
 constexpr Variant make_variant() {
   return Variant{T::DT, T::BM, T::BN, T::BK, T::ALAY, T::BLAY, T::WM, T::WN, T::THREADS, T::LDS_ALLOC, T::MINB,
-                 T::LOADER, T::STAGES, (const void*)&gemm_kernel<T, false>, (const void*)&gemm_tile_kernel<typename OneTile<T>::tile, OneTile<T>::WHOLE_STEP>, (const void*)&gemm_kernel<T, true>, 0};
+                 T::LOADER, T::STAGES, (const void*)&gemm_kernel<T, false>, (const void*)&gemm_tile_kernel<T, OneTile<T>::WHOLE_STEP>, (const void*)&gemm_kernel<T, true>, 0};
 }
 
 // The hand-scheduled 4-wave kernels of gemm_w4.h (256x256 tile, 128-byte K steps) are compiled in a
