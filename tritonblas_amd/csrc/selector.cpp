@@ -101,22 +101,25 @@ struct Family {
 };
 // lat: the deeper variants of the 64x64 tile run while at most two (three) tiles per CU exist, the eight-wave 128x128 tile while every tile has
 // a CU of its own (find_variant)
-static Family family(int dt, const TileInfo& v, bool w4, int64_t tiles, int n_cu, bool grouped) {
+static Family family(int dt, const TileInfo& v, bool w4, int64_t tiles, int n_cu, bool grouped, bool streamk) {
   const int area = v.bm * v.bn;
   const int cls = (v.bm < 64 || v.bn < 64) ? 5 : area >= 256 * 256 ? 0 : area >= 256 * 128 ? 1 : area >= 128 * 128 ? 2 : area >= 128 * 64 ? 3 : 4;
   if (dt == TB_FP4_E2M1 || dt == TB_F32) {
     static const double f4[6] = {0.50, 0.36, 0.36, 0.22, 0.22, 0.10};   // (256x256: 8192x8192x16384 in 0.43-0.47 ms)
     // (the fp32 matrix pipe is slow enough to hide everything else; four 64x64 workgroups to a CU hide more of it than two of 128x128:
-    // 2048^3 130 us against 147, 1000x3000x1504 79 and 108)
-    static const double f32[6] = {0.92, 0.77, 0.77, 0.86, 0.86, 0.65};
+    // 2048^3 130 us against 147, 1000x3000x1504 79 and 108.  One 64x64 workgroup to a CU hides nothing, its step takes twice the MFMAs' time: 32x32 tiles
+    // fill the CUs better there, 1664x480x5568 164 us and 105, 512x2048x2848 86 and 59, 240x3552x4672 140 and 91.  Of 894 problems, 100..8192 a side, four orders, the tile
+    // taken was 1.029 times the best one's time in the geometric mean, 1.57 at most; with these three figures 1.003 and 1.19.  Stream-K launches cut such tiles
+    // instead and keep their own.)
+    static const double f32[6] = {0.92, 0.77, 0.77, 0.86, 0.82, 0.70}, f32_sk[6] = {0.92, 0.77, 0.77, 0.86, 0.86, 0.65};
     const double tile_us = cls == 0 ? (w4 ? 8.0 : 12.0) : (cls <= 2 ? 4.0 : 3.0);
-    double lat = dt == TB_F32 && cls == 5 ? 0.6 : 1.0;
+    double lat = dt != TB_F32 ? 1.0 : cls == 5 ? (streamk ? 0.6 : 0.4) : cls == 4 && !streamk ? 1.7 : 1.0;
     if (dt == TB_FP4_E2M1 && !grouped) {      // (three copy stages: see find_variant)
       if (cls == 2 && tiles <= n_cu && v.bk == 256) lat = 0.88;
       if (cls == 3) lat = 0.85;
       if (cls == 4 && tiles <= 2 * (int64_t)n_cu) lat = 0.66;
     }
-    return {dt == TB_F32 ? f32[cls] : (w4 && cls == 0 ? 0.56 : f4[cls]), tile_us, lat};
+    return {dt == TB_F32 ? (streamk ? f32_sk : f32)[cls] : (w4 && cls == 0 ? 0.56 : f4[cls]), tile_us, lat};
   }
   //                                     256x256  256x128 128x128 128x64 64x64  32x128
   static const double eff16[6] = {0.69, 0.506, 0.388, 0.357, 0.246, 0.12}, us16[6] = {9.5, 5.0, 3.8, 2.8, 3.0, 3.0};
@@ -223,7 +226,7 @@ static double score(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bo
     k_steps = whole_k & ~1ll;
     rest_us = 2.0 + 3.5 * (double)(k_iters - k_steps);
   }
-  const Family fam = family(pr.a_type, v, w4, cdiv(pr.m, v.bm) * cdiv(pr.n, v.bn), hw.n_cu, pr.num_groups > 0);
+  const Family fam = family(pr.a_type, v, w4, cdiv(pr.m, v.bm) * cdiv(pr.n, v.bn), hw.n_cu, pr.num_groups > 0, streamk);
   const double t_thru = ideal_step_us / fam.eff;   // CU time per tile K step, saturated
   const double t_lat = (0.30 + (v.bm + v.bn) * (v.bk * esz) / 1.0e5) * fam.lat;   // floor per K step of one workgroup
   const double t_tile = fam.tile_us + rest_us;
