@@ -27,18 +27,23 @@ def _launch(entry, desc, index, what):
         _lib.check(status, what)
 
 
+# (by their own names: each dot on the way to one of them costs a call that takes five us a tenth of a us)
+_TENSORS, _STRIDED, _forward_ad = (torch.Tensor, torch.nn.Parameter), torch.strided, torch.autograd.forward_ad
+_grad_enabled, _functorch_wrapped, _jit_tracing = torch.is_grad_enabled, torch._C._functorch.is_functorch_wrapped_tensor, torch.jit.is_tracing
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+
+
 def _plain(*tensors) -> bool:
     """True where a kernel may read the tensors' memory behind torch's back: real GPU tensors that nothing is recording
     (autograd in either direction, functorch transforms, torch.compile and jit tracing, dispatch or function modes)."""
     if torch.compiler.is_compiling():       # (first: the tracer follows Python code up to here)
         return False
-    recording = torch.is_grad_enabled()
+    recording = _grad_enabled()
     for t in tensors:
-        if not (type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.layout == torch.strided and not t.is_neg()
-                and not (recording and t.requires_grad) and not torch._C._functorch.is_functorch_wrapped_tensor(t)):
+        if (type(t) not in _TENSORS or not t.is_cuda or t.layout is not _STRIDED or t.is_neg()
+                or (recording and t.requires_grad) or _functorch_wrapped(t)):
             return False
-    return (torch.autograd.forward_ad._current_level < 0 and torch._C._len_torch_dispatch_stack() == 0
-            and torch._C._len_torch_function_stack() == 0 and not torch.jit.is_tracing())
+    return _forward_ad._current_level < 0 and _dispatch_modes() == 0 and _function_modes() == 0 and not _jit_tracing()
 
 
 def _rows(t: torch.Tensor, axis: int):
@@ -58,12 +63,12 @@ def _rows(t: torch.Tensor, axis: int):
 
 def _quantize_rows(t, target_dtype, axis, min_scale, rows):
     m, n, stride = rows
-    scale_shape = [d for i, d in enumerate(t.shape) if i != axis % t.ndim]
-    if axis % t.ndim == t.ndim - 1:
-        q = torch.empty(t.shape, dtype=target_dtype, device=t.device)
+    last = axis % t.ndim == t.ndim - 1
+    if last:
+        q = t.new_empty(t.shape, dtype=target_dtype)
     else:       # the columns of a matrix that is stored transposed: so are the codes
-        q = torch.empty((m, n), dtype=target_dtype, device=t.device).T
-    scale = torch.empty(scale_shape, dtype=torch.float32, device=t.device)
+        q = t.new_empty((m, n), dtype=target_dtype).T
+    scale = t.new_empty(t.shape[:-1] if last else (m,), dtype=torch.float32)
     _lib.load()
     desc = _lib.pack_quant_rows(_lib.ROW_QUANT_BYTES, _lib.tb_dtype(t.dtype), _lib.tb_dtype(target_dtype), C.c_float(min_scale).value, m, n, t.data_ptr(), stride,
                                 q.data_ptr(), scale.data_ptr())
@@ -127,8 +132,8 @@ def _quant(x: torch.Tensor, hadamard: bool, out=None):
         # boundary needs a real copy: .contiguous() would hand the same memory back)
         x = x.clone(memory_format=torch.contiguous_format)
     if out is None:
-        codes = torch.empty((M, N // 2), dtype=torch.uint8, device=x.device)
-        scales = torch.empty((M, N // 32), dtype=torch.uint8, device=x.device)
+        codes = x.new_empty((M, N // 2), dtype=torch.uint8)
+        scales = x.new_empty((M, N // 32), dtype=torch.uint8)
     else:
         codes, scales = out
         for t, cols in ((codes, N // 2), (scales, N // 32)):
