@@ -83,3 +83,18 @@ def test_grouped_one_tile_per_workgroup(counts, n, k, tb_option):
         got = torch.full((rows, n), float("nan"), device="cuda", dtype=torch.bfloat16)
         tb.grouped_matmul_a8w8(a, w, None, None, got, offsets, *(tile or (None, None, None)))
         assert ((got.double() - want).abs() <= REL["fp8"] * want.abs()).all(), (tile, waves)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "f16", "fp8", "i8"])
+@pytest.mark.parametrize("m,n,k", [(65, 1024, 256), (64, 1024, 512), (64, 1000, 528), (33, 40, 4096), (200, 1000, 2000), (256, 256, 7904), (31, 33, 272), (1, 1000, 1040)])
+def test_few_tiles(m, n, k, kind):
+    """Both sides of the rule for the 32x32 and 64x32 tiles: the library's own choice, and the two named."""
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randint(-2, 3, (m, k), device="cuda", generator=g).to(TYPES[kind])
+    b = torch.randint(-2, 3, (n, k), device="cuda", generator=g).to(TYPES[kind]).T
+    want = a.double() @ b.double()
+    out = TYPES[kind] if kind in ("bf16", "f16") else torch.bfloat16
+    step = 128 if kind in ("bf16", "f16") else 256
+    for tile in ((0, 0, 0), (32, 32, step), (64, 32, step)):
+        got = _product(a, b, torch.full((m, n), float("nan"), device="cuda", dtype=out), tile, 0)
+        assert ((got.double() - want).abs() <= REL[kind] * want.abs()).all(), tile       # (whole numbers below 2**24: the sums are exact)

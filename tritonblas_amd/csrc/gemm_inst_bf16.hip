@@ -32,6 +32,9 @@ const Variant g_variants_bf16[] = {
     TB_LAYOUTS(64, 64, 128, 2, 2, 2, 4),
     // a handful of rows against a long K: short, wide, deep tile with three copy stages
     TB_LAYOUTS(32, 128, 256, 1, 4, 1, 3),
+    // few tiles: what a CU copies for a K step is what the step takes, so tiles of a quarter and half of 64x64 on the CUs that would be idle, with half the steps
+    TB_LAYOUTS(32, 32, 256, 2, 2, 2, 4),
+    TB_LAYOUTS(64, 32, 256, 2, 2, 1, 4),
     // unit stride, any alignment of the rows
     TB_REGS_LAYOUTS(128, 128, 2, 2, 2, 2),
     // (eight waves and a K step more in flight while every tile has a CU of its own)

@@ -11,6 +11,9 @@ const Variant g_variants_fp8[] = {
     make_variant<Tile<DT_FP8, 128, 128, 128, 2, 2, LAY_K, LAY_K, 2, true, 2>>(),
     make_variant<Tile<DT_FP8, 64, 64, 128, 2, 2, LAY_K, LAY_K, 4, true, 2>>(),
     make_variant<Tile<DT_FP8, 32, 128, 256, 1, 4, LAY_K, LAY_K, 1, true, 3>>(),
+    // few tiles: what a CU copies for a K step is what the step takes, so tiles of a quarter and half of 64x64 on the CUs that would be idle, with half the steps
+    make_variant<Tile<DT_FP8, 32, 32, 256, 2, 2, LAY_K, LAY_K, 2, true, 4>>(),
+    make_variant<Tile<DT_FP8, 64, 32, 256, 2, 2, LAY_K, LAY_K, 1, true, 4>>(),
     // deeper copy pipelines of the small tile for problems with few tiles per CU (each K step then
     // waits less for its copy; fewer workgroups fit a CU)
     make_variant<Tile<DT_FP8, 64, 64, 128, 2, 2, LAY_K, LAY_K, 3, true, 3>>(),

@@ -129,6 +129,11 @@ static Family family(int dt, const TileInfo& v, bool w4, int64_t tiles, int n_cu
   static const double effi[6] = {0.665, 0.46, 0.367, 0.293, 0.159, 0.15}, usi[6] = {6.3, 5.8, 4.4, 2.6, 1.8, 3.0};
   static const double effi_sk[6] = {0.705, 0.368, 0.367, 0.293, 0.211, 0.15}, usi_sk[6] = {7.0, 5.8, 3.5, 2.3, 2.4, 3.0};
   const bool half = dt == TB_F16 || dt == TB_BF16;
+  // 32x32 and 64x32, 256-byte K steps: where 64x64 tiles leave CUs idle.  A step takes what its CU copies for it, about 26 bytes a cycle however deep the
+  // pipeline; a quarter of the bytes on four times the CUs.  bf16, 64x64 and 32x32, us: 256x256x7904 32.2 and 17.8, 128x1024x14336 65.3 and 33.1, 96x1280x5120 22.0 and 12.6,
+  // 200x1000x2000 11.4 and 6.9; FP8 256x256x7904 19.9 and 9.9, 130x520x3008 8.6 and 5.7.  64x32: bf16 128x4096x4096 21.6 and 16.6.  On 1500 problems of at most 768 tiles of 64x64 each in
+  // bf16 and FP8 the choice among the three takes 1.003 and 1.015 times the best one's time, 1/1.35 and 1/1.26 of what 64x64 takes.
+  if (v.bn == 32) return half ? (v.bm == 32 ? Family{0.10, 1.2, 0.33} : Family{0.12, 1.2, 0.36}) : v.bm == 32 ? Family{0.10, 1.2, 0.36} : Family{0.15, 1.5, 0.55};
   Family f = half ? Family{eff16[cls], us16[cls], 1.0} : dt == TB_I8 ? (streamk ? Family{effi_sk[cls], usi_sk[cls], 1.0} : Family{effi[cls], usi[cls], 1.0}) : Family{eff8[cls], us8[cls], 1.0};
   // (the eight-wave 256x256 kernel.  16-bit, M-contiguous operands and a rest of K, 44 problems of 256..8192 in three orders: the model's tile 1.013 times the
   // fastest one's time; 1.021 with 0.89 and 4 us more a tile, which kept the library's choice off this kernel: 7848x7808x528 86 us, 256x128 104)
@@ -355,6 +360,8 @@ double streaming_bound_us(const tb_problem& pr, const tb_hw& hw) {
   return 13.0 + weight / (hw.hbm_gbps * (esz > 1.0 ? 0.425 : 0.575) * 1e3) + a_reread / (hw.hbm_gbps * 2.125 * 1e3);
 }
 
+bool narrow_tile(const TileInfo& v) { return v.bn == 32 && v.dt != TB_F32; }
+
 int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, int ntiles, tb_selection* out) {
   int best = -1;
   double best_t = 0, best_c = 0, best_m = 0;
@@ -364,8 +371,10 @@ int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, in
     if (v.lds_bytes > hw.lds_bytes) continue;
     // decode-like problems (a handful of rows): tiles taller than twice the row count only add
     // LDS traffic and idle MFMA rows when a shorter tile exists
+    // (the small tiles of few-tile problems, see family(): whole tiles only, and not where the streaming kernel is at home, which is weighed against the others)
+    if (narrow_tile(v) && (pr.streamk || pr.num_groups > 0 || (pr.m <= 64 && pr.n >= 1024 && pr.a_k_contiguous && pr.b_k_contiguous))) continue;
     bool shorter_exists = false;
-    for (int q = 0; q < ntiles; ++q) shorter_exists |= tiles[q].fast && tiles[q].bm < v.bm && tiles[q].bm >= pr.m;
+    for (int q = 0; q < ntiles; ++q) shorter_exists |= tiles[q].fast && !narrow_tile(tiles[q]) && tiles[q].bm < v.bm && tiles[q].bm >= pr.m;
     if (shorter_exists && pr.num_groups == 0) continue;
     if (pr.num_groups > 0) {
       // grouped, with a tail that is cut into K ranges or short last blocks left to a second launch (other launches: estimate_grouped_us): the row counts live on the

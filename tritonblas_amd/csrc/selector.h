@@ -20,6 +20,8 @@ void hierarchical_split(int64_t total_tiles, int hw_cus, int num_xcds, int64_t* 
 bool rest_of_k_pays(int64_t m, int64_t n, int64_t k, int bk, int c_bits, int n_cu);
 int variant_occupancy(const TileInfo& v, const tb_hw& hw);
 int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, int ntiles, tb_selection* out);
+// 32x32 and 64x32 tiles of the 16- and 8-bit types
+bool narrow_tile(const TileInfo& v);
 // model time (us) of one tile variant on a problem, and of the streaming small-M kernel
 double estimate_tile_us(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bool streamk);
 // ... of a grouped launch whose row counts only the device knows (FP8; 0: no figures for this variant)

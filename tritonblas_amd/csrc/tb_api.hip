@@ -381,7 +381,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
       // the model's order, and of that the first tile whose queue counters and partial tiles fit (see fitting_plan)
       std::vector<std::pair<double, const TileInfo*>> order;
       for (auto& t : infos)
-        if (t.fast) order.emplace_back(estimate_tile_us(pr, hw, t, pr.streamk != 0), &t);
+        if (t.fast && !narrow_tile(t)) order.emplace_back(estimate_tile_us(pr, hw, t, pr.streamk != 0), &t);
       std::sort(order.begin(), order.end());
       Job named = j;
       named.room = 0;
