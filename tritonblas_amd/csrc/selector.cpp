@@ -308,10 +308,11 @@ double estimate_tile_us(const tb_problem& pr, const tb_hw& hw, const TileInfo& v
   return score(pr, hw, v, streamk, &c, &m);
 }
 
-// A grouped FP8 launch.  The rows of an expert are taken as spread around their mean, by chance and by a tenth of it, which gives the row blocks to expect; per variant:
+// A grouped FP8 launch.  The rows of an expert are taken as spread around their mean, by chance and by 7 % of it, which gives the row blocks to expect; per variant:
 // us a 128-byte K step and tile keeps a CU busy, the least a step takes, us a tile costs beside its steps, us per MB of operands and results, and
-// how much of a last round that is not full is waited for.  The two times are those of different units and add up as squares do.  Fitted on 1298 random launches
-// (4, 8 and 16 experts, 16..16384 rows, n 1024..14336, k 1024..8192) per variant: 8 to 17 % off at one sigma; the variant it picks takes 1.037 times the best
+// how much of a last round that is not full is waited for (a hundredth of a round more than whole ones is an expectation that chance makes, not a round: 16 experts of
+// 1984x3584, 6786 rows, 256.2 tiles of 256x256 to expect).  The two times are those of different units and add up as squares do.  Fitted on 1298 random launches
+// (4, 8 and 16 experts, 16..16384 rows, n 1024..14336, k 1024..8192) per variant: 8 to 17 % off at one sigma; the variant it picks takes 1.032 times (on 420 others, as built, 1.025) the best
 // one's time in the geometric mean, one picked by the rows per expert alone (256x256 from 192, 128x128 from 96, else 64x64) 1.214 times.
 // 4 experts of 1536x7168, 1000 rows: 89 us that way, 29 now; 16 of 1024x8192, 600 rows: 54 and 34.
 double estimate_grouped_us(const tb_problem& pr, const tb_hw& hw, const TileInfo& v) {
@@ -325,16 +326,19 @@ double estimate_grouped_us(const tb_problem& pr, const tb_hw& hw, const TileInfo
   for (auto& x : fits) if (x.bm == v.bm && x.bn == v.bn && x.waves == v.threads / 64 && x.stages == v.stages) f = &x;
   if (!f || pr.num_groups <= 0 || pr.m <= 0) return 0.0;
   const double e = pr.num_groups, rows = (double)pr.m, mean = rows / e;
-  const double spread = std::max({std::sqrt(mean * (1.0 - 1.0 / e)), 0.1 * mean, 1e-6});
+  const double spread = std::max({std::sqrt(mean * (1.0 - 1.0 / e)), 0.07 * mean, 1e-6});
   const double used = e * (1.0 - std::pow(1.0 - 1.0 / e, rows));      // experts with rows at all
   double blocks = used;
   for (int64_t at = v.bm; (double)at < mean + 5.0 * spread; at += v.bm) blocks += e * 0.5 * std::erfc(((double)at + 0.5 - mean) / (spread * std::sqrt(2.0)));
   const double tiles = blocks * (double)cdiv(pr.n, v.bn), steps = (double)cdiv(pr.k, 128);
   const int occ = variant_occupancy(v, hw);
-  const double rounds = tiles / hw.n_cu / occ;
+  const double rounds = tiles / hw.n_cu / occ, slack = 0.01;
   double us;
-  if (rounds <= 1.0) us = steps * std::max(std::ceil(tiles / hw.n_cu) * f->step, f->least) + f->tile;
-  else us = (f->round * std::ceil(rounds) + (1.0 - f->round) * rounds) * (steps * std::max(occ * f->step, f->least) + f->tile);
+  if (rounds <= 1.0 + slack) us = steps * std::max(std::ceil(tiles / hw.n_cu - slack) * f->step, f->least) + f->tile;
+  else us = (f->round * std::ceil(rounds - slack) + (1.0 - f->round) * rounds) * (steps * std::max(occ * f->step, f->least) + f->tile);
+  // (in several rounds the four-wave kernel stores a tile under the next one's K loop, 4 us of its cost, and 256x128 tiles fall out of step: 16 experts of 4096x2048, 16384 rows
+  // 157 us and 186 where one round of both is priced alike)
+  if (rounds > 1.0 + slack && v.bm == 256) us = v.bn == 128 ? us * 1.05 : v.threads == 256 ? us - 4.0 * (rounds - 1.0) : us;
   const double mb = (used * pr.n * pr.k + rows * pr.k + rows * pr.n * type_bits(pr.c_type) / 8.0) * 1e-6;
   return 3.0 + std::hypot(us, mb * f->mb);
 }
