@@ -83,6 +83,17 @@ bool rest_of_k_pays(int64_t m, int64_t n, int64_t k, int bk, int c_bits, int n_c
   return steps >= (whole ? (ragged ? 36 : 24) : (ragged ? 20 : 10));
 }
 
+// Whether they are the faster ones for an even number of K steps.  They store a tile under the next one's K loop, which one round of tiles has no use for, and
+// the eight-wave kernel starts sooner (one tile to a workgroup).  Hand-scheduled by eight-wave time, 256x256 tiles: one round, 16-bit 1.28 at 4 steps, 1.16 at 8, 1.10 at 12, 1.03 at 16,
+// 0.98 at 24, 0.92 at 40; int8 1.41, 1.22, 1.13, 1.09, 1.01 at 24, 0.98 at 36; FP8 1.54, 1.41, 1.25, 1.19, 1.05 at 24, 1.01 at 32, 0.97 at 40.  Two rounds: 1.08 to 1.10 at 4, 1.01 at 12, 0.92 to
+// 0.97 at 16.  More: 0.91 to 1.0 (8 bits 1.01 to 1.13 at 4).
+bool even_k_pays(int64_t m, int64_t n, int64_t k, int bk, int type, int n_cu) {
+  const int64_t steps = k / bk, tiles = cdiv(m, 256) * cdiv(n, 256);
+  if (type == TB_FP4_E2M1 || tiles > 2 * (int64_t)n_cu) return true;
+  if (tiles > n_cu) return steps >= 12;
+  return steps >= (type == TB_FP8_E4M3 || type == TB_FP8_E5M2 ? 32 : 24);
+}
+
 // Measured behaviour of the built kernels on MI355X that the model is anchored to:
 //   * a CU that is kept busy by `occ` resident workgroups finishes one K step of one tile every
 //     ideal_step / eff: eff = fraction of the MFMA peak the kernel family sustains for that tile;
@@ -226,7 +237,7 @@ static double score(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bo
   const int64_t whole_k = pr.k / v.bk;
   const bool rest = pr.k % (2 * (int64_t)v.bk) != 0;
   const bool w4 = v.threads == 256 && area >= 256 * 256 && whole_k >= 4 &&
-                  (!rest || (pr.a_type != TB_FP4_E2M1 && pr.c_type != TB_I8 && pr.a_k_contiguous && pr.b_k_contiguous &&
+                  (!rest ? streamk || pr.num_groups > 0 || even_k_pays(pr.m, pr.n, pr.k, v.bk, pr.a_type, hw.n_cu) : (pr.a_type != TB_FP4_E2M1 && pr.c_type != TB_I8 && pr.a_k_contiguous && pr.b_k_contiguous &&
                              rest_of_k_pays(pr.m, pr.n, pr.k, v.bk, type_bits(pr.c_type), hw.n_cu)));
   int64_t k_steps = k_iters;
   double rest_us = 0.0;

@@ -18,6 +18,7 @@ int ws_counters_per_xcd(int64_t total_tiles);
 void hierarchical_split(int64_t total_tiles, int hw_cus, int num_xcds, int64_t* local_per_xcd, int64_t* global_tiles);
 // whether the hand-scheduled 256x256 kernels are the faster ones for a K that is no even number of K steps
 bool rest_of_k_pays(int64_t m, int64_t n, int64_t k, int bk, int c_bits, int n_cu);
+bool even_k_pays(int64_t m, int64_t n, int64_t k, int bk, int type, int n_cu);     // ... that is one (type: a public element type)
 int variant_occupancy(const TileInfo& v, const tb_hw& hw);
 int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, int ntiles, tb_selection* out);
 // 32x32 and 64x32 tiles of the 16- and 8-bit types

@@ -185,7 +185,7 @@ const std::vector<TileInfo>& tile_infos(int dt) {
 // FP8 36 us with two workgroups of four waves, 42 with one of eight at a time.)  The 256x128 tile, three stages and eight waves, is for what 256x256 leaves
 // half empty (2048x4096x4096 FP8 35, 256x256 40), 128x64 with four for a tile per CU at half the rows (512x4096x14336 FP8 51, 64x64 60).
 const Variant* find_variant(int dt, int bm, int bn, int bk, int alay, int blay, int fast, int64_t total_tiles = 0,
-                            const tb_hw* hw = nullptr, bool need_sk = false, int64_t k = 0, int out8 = 0, bool rest_pays = true) {
+                            const tb_hw* hw = nullptr, bool need_sk = false, int64_t k = 0, int out8 = 0, bool rest_pays = true, bool even_pays = true) {
   const Variant* v; int n;
   variant_table(dt, &v, &n);
   // the hand-scheduled 4-wave kernels run K steps in pairs (the pieces of a Stream-K tail in blocks of four) and take what is left behind them
@@ -205,7 +205,7 @@ const Variant* find_variant(int dt, int bm, int bn, int bk, int alay, int blay, 
         return &v[i];
   const Variant* best = nullptr;
   for (int i = 0; i < n; ++i) {
-    if (v[i].k_step_pairs && !rest_pays && k % (2 * (int64_t)v[i].bk) != 0) continue;    // (the eight-wave kernel of the tile)
+    if (v[i].k_step_pairs && !(k % (2 * (int64_t)v[i].bk) != 0 ? rest_pays : even_pays)) continue;    // (the eight-wave kernel of the tile)
     if (!(usable(v[i]) && v[i].fast == fast && v[i].alay == alay && v[i].blay == blay && (fast == 0 || (v[i].bm == bm && v[i].bn == bn && v[i].bk == bk))))
       continue;
     if (!best) { best = &v[i]; if (!hw || total_tiles <= 0 || !fast) return best; continue; }   // (listed first: the default depth)
@@ -440,7 +440,8 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
     const bool by_model = j.num_groups > 0 && j.bm == 0 && !j.grp_sk && j.grp_phase == 0;
     if (by_model) { bm = bn = 256; bk = 128; }
     v = find_variant(j.dt, bm, bn, bk, alay, blay, 1, at_once, &hw, is_streamk(j.schedule) && j.num_groups == 0, j.K,
-                     j.c_type == TB_I8 ? 2 : (is_f8_type(j.c_type) ? 1 : 0), rest_pays());
+                     j.c_type == TB_I8 ? 2 : (is_f8_type(j.c_type) ? 1 : 0), rest_pays(),
+                     is_streamk(j.schedule) || j.num_groups > 0 || even_k_pays(j.M, j.N, j.K, 128 / usz * epu, model_type(j.dt), hw.n_cu));
     if (by_model) v = grouped_variant(j, hw, v);
     if (!v) return TB_ERR_BAD_TILE;
   } else {
