@@ -764,6 +764,20 @@ def test_few_k_steps_and_a_rest_go_to_the_eight_wave_kernel(a_type):
                 assert info.waves == (4 if info.four_wave else 8)
 
 
+@pytest.mark.parametrize("a_type", ["TB_FP8_E4M3", "TB_FP8_E5M2", "TB_I8", "TB_BF16", "TB_F16"])
+def test_few_even_k_steps_go_to_the_eight_wave_kernel(a_type):
+    """... and for an even number of K steps, by how many rounds of tiles there are; Stream-K launches keep the hand-scheduled kernel."""
+    from tritonblas_amd import _lib
+    code = getattr(_lib, a_type)
+    width = 128 if a_type in ("TB_FP8_E4M3", "TB_FP8_E5M2", "TB_I8") else 64
+    one_round = 32 if a_type.startswith("TB_FP8") else 24
+    for m, n, start in [(4096, 4096, one_round), (500, 300, one_round), (4096, 4352, 12), (4096, 8192, 12), (4096, 8448, 4), (7000, 9000, 4)]:
+        for steps in range(4, 42, 2):
+            info = _launch_of(_job(code, m, n, steps * width, tile=(256, 256, width)))
+            assert (info.four_wave == 1) == (steps >= start), (m, n, steps)
+            assert info.waves == (4 if info.four_wave else 8)
+
+
 def test_tiles_of_the_register_loading_kernels():
     """Rows off 16 bytes run in 128x128 or 64x64 tiles: 128 where the chosen tile has it on both sides, and where fp32 fills the CUs with them once."""
     from tritonblas_amd import _lib

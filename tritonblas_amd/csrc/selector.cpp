@@ -85,12 +85,13 @@ bool rest_of_k_pays(int64_t m, int64_t n, int64_t k, int bk, int c_bits, int n_c
 
 // Whether they are the faster ones for an even number of K steps.  They store a tile under the next one's K loop, which one round of tiles has no use for, and
 // the eight-wave kernel starts sooner (one tile to a workgroup).  Hand-scheduled by eight-wave time, 256x256 tiles: one round, 16-bit 1.28 at 4 steps, 1.16 at 8, 1.10 at 12, 1.03 at 16,
-// 0.98 at 24, 0.92 at 40; int8 1.41, 1.22, 1.13, 1.09, 1.01 at 24, 0.98 at 36; FP8 1.54, 1.41, 1.25, 1.19, 1.05 at 24, 1.01 at 32, 0.97 at 40.  Two rounds: 1.08 to 1.10 at 4, 1.01 at 12, 0.92 to
-// 0.97 at 16.  More: 0.91 to 1.0 (8 bits 1.01 to 1.13 at 4).
+// 0.98 at 24, 0.92 at 40; int8 1.41, 1.22, 1.13, 1.09, 1.01 at 24, 0.98 at 36; FP8 1.54, 1.41, 1.25, 1.19, 1.05 at 24, 1.01 at 32, 0.97 at 40; MXFP4 1.55, 1.30, 1.20, 1.15,
+// 0.97 at 24, 0.94 at 32 (7860x1552x1536 28.3 us and 19.5).  Two rounds: 1.08 to 1.10 at 4, 1.01 at 12, 0.92 to
+// 0.97 at 16 (MXFP4 1.28, 1.10, 1.05 at 14).  More: 0.91 to 1.0 (8 bits 1.01 to 1.13 at 4).
 bool even_k_pays(int64_t m, int64_t n, int64_t k, int bk, int type, int n_cu) {
   const int64_t steps = k / bk, tiles = cdiv(m, 256) * cdiv(n, 256);
-  if (type == TB_FP4_E2M1 || tiles > 2 * (int64_t)n_cu) return true;
-  if (tiles > n_cu) return steps >= 12;
+  if (tiles > 2 * (int64_t)n_cu) return true;
+  if (tiles > n_cu) return steps >= (type == TB_FP4_E2M1 ? 16 : 12);
   return steps >= (type == TB_FP8_E4M3 || type == TB_FP8_E5M2 ? 32 : 24);
 }
 
@@ -123,14 +124,16 @@ static Family family(int dt, const TileInfo& v, bool w4, int64_t tiles, int n_cu
     // taken was 1.029 times the best one's time in the geometric mean, 1.57 at most; with these three figures 1.003 and 1.19.  Stream-K launches cut such tiles
     // instead and keep their own.)
     static const double f32[6] = {0.92, 0.77, 0.77, 0.86, 0.82, 0.70}, f32_sk[6] = {0.92, 0.77, 0.77, 0.86, 0.86, 0.65};
-    const double tile_us = cls == 0 ? (w4 ? 8.0 : 12.0) : (cls <= 2 ? 4.0 : 3.0);
+    // (MXFP4 256x256 with eight waves, a round of one tile to a workgroup: 2 to 16 K steps 13.9 to 34.1 us, within 1.5 of the hand-scheduled kernel's figures)
+    const bool w8_one = cls == 0 && dt == TB_FP4_E2M1 && !streamk && !grouped && tiles <= n_cu;
+    const double tile_us = cls == 0 ? (w4 || w8_one ? 8.0 : 12.0) : (cls <= 2 ? 4.0 : 3.0);
     double lat = dt != TB_F32 ? 1.0 : cls == 5 ? (streamk ? 0.6 : 0.4) : cls == 4 && !streamk ? 1.7 : 1.0;
     if (dt == TB_FP4_E2M1 && !grouped) {      // (three copy stages: see find_variant)
       if (cls == 2 && tiles <= n_cu && v.bk == 256) lat = 0.88;
       if (cls == 3) lat = 0.85;
       if (cls == 4 && tiles <= 2 * (int64_t)n_cu) lat = 0.66;
     }
-    return {dt == TB_F32 ? (streamk ? f32_sk : f32)[cls] : (w4 && cls == 0 ? 0.56 : f4[cls]), tile_us, lat};
+    return {dt == TB_F32 ? (streamk ? f32_sk : f32)[cls] : ((w4 && cls == 0) || w8_one ? 0.56 : f4[cls]), tile_us, lat};
   }
   //                                     256x256  256x128 128x128 128x64 64x64  32x128
   static const double eff16[6] = {0.69, 0.506, 0.388, 0.357, 0.246, 0.12}, us16[6] = {9.5, 5.0, 3.8, 2.8, 3.0, 3.0};
