@@ -778,6 +778,24 @@ def test_few_even_k_steps_go_to_the_eight_wave_kernel(a_type):
             assert info.waves == (4 if info.four_wave else 8)
 
 
+@pytest.mark.parametrize("dtype,m,n,k", [(torch.bfloat16, 4096, 4096, 1280), (torch.bfloat16, 4096, 4096, 512), (torch.float8_e4m3fn, 4096, 4096, 3840),
+                                         (torch.int8, 4096, 4096, 1024)])
+def test_few_even_k_steps_in_launches_that_loop_over_tiles(dtype, m, n, k):
+    """... but only where a workgroup has one tile: launches that loop, from a caller's grid or the work-stealing queues, keep the hand-scheduled kernel."""
+    import tritonblas_amd as tb
+    from tritonblas_amd import _lib
+    code, tile = _lib.tb_dtype(dtype), (256, 256, 128 // dtype.itemsize)
+    assert _launch_of(_job(code, m, n, k, tile=tile)).four_wave == 0
+    for schedule in (_lib.TB_SCHED_PERSISTENT, _lib.TB_SCHED_WORK_STEALING):
+        for cus in (32, 64, 128, 255):
+            assert _launch_of(_job(code, m, n, k, schedule, cus, tile=tile)).four_wave == 1
+            sel = tb.OrigamiMatmulSelector(m, n, k, dtype, dtype, torch.bfloat16, None, total_cus=cus)
+            info = _launch_of(_job(code, m, n, k, schedule, cus * sel.waves_per_eu, tile=(sel.block_m, sel.block_n, sel.block_k)))
+            assert info.four_wave == (sel.block_m == sel.block_n == 256)
+    assert _launch_of(_job(code, m, n, k, _lib.TB_SCHED_WORK_STEALING, tile=tile)).four_wave == 1
+    assert _launch_of(_job(code, m, n, k, _lib.TB_SCHED_WORK_STEALING, tile=tile, cu_mask=256, cu_mask_len=64)).four_wave == 1      # (an address that nobody reads)
+
+
 def test_tiles_of_the_register_loading_kernels():
     """Rows off 16 bytes run in 128x128 or 64x64 tiles: 128 where the chosen tile has it on both sides, and where fp32 fills the CUs with them once."""
     from tritonblas_amd import _lib

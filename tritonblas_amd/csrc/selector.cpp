@@ -87,7 +87,9 @@ bool rest_of_k_pays(int64_t m, int64_t n, int64_t k, int bk, int c_bits, int n_c
 // the eight-wave kernel starts sooner (one tile to a workgroup).  Hand-scheduled by eight-wave time, 256x256 tiles: one round, 16-bit 1.28 at 4 steps, 1.16 at 8, 1.10 at 12, 1.03 at 16,
 // 0.98 at 24, 0.92 at 40; int8 1.41, 1.22, 1.13, 1.09, 1.01 at 24, 0.98 at 36; FP8 1.54, 1.41, 1.25, 1.19, 1.05 at 24, 1.01 at 32, 0.97 at 40; MXFP4 1.55, 1.30, 1.20, 1.15,
 // 0.97 at 24, 0.94 at 32 (7860x1552x1536 28.3 us and 19.5).  Two rounds: 1.08 to 1.10 at 4, 1.01 at 12, 0.92 to
-// 0.97 at 16 (MXFP4 1.28, 1.10, 1.05 at 14).  More: 0.91 to 1.0 (8 bits 1.01 to 1.13 at 4).
+// 0.97 at 16 (MXFP4 1.28, 1.10, 1.05 at 14).  More: 0.91 to 1.0 (8 bits 1.01 to 1.13 at 4).  Launches of one tile to a workgroup only: from a caller's grid or the
+// work-stealing queues the eight-wave kernel loops too, without either advantage.  Hand-scheduled and eight-wave, us: bf16 4096x4096x1280 on 64 workgroups 96.6 and 122.5, from the
+// queues 105 and 125, from those of the whole device 42.2 and 43.5; FP8 4096x4096x3840 on 128 70 and 83; int8 2048x4096x1536 on 128, a tile each, 22.3 and 25.6.
 bool even_k_pays(int64_t m, int64_t n, int64_t k, int bk, int type, int n_cu) {
   const int64_t steps = k / bk, tiles = cdiv(m, 256) * cdiv(n, 256);
   if (tiles > 2 * (int64_t)n_cu) return true;
@@ -223,7 +225,7 @@ int streamk_grid(int64_t total, int64_t k_iters, int slots, int n_cu, double ste
 }
 
 static double score(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bool streamk, double* comp_us,
-                    double* mem_us, int* sk_grid_out = nullptr) {
+                    double* mem_us, int* sk_grid_out = nullptr, bool looped = false) {
   const double clk = hw.clock_khz * 1e3;
   const int bits = type_bits(pr.a_type);
   const double esz = bits / 8.0;
@@ -240,7 +242,7 @@ static double score(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bo
   const int64_t whole_k = pr.k / v.bk;
   const bool rest = pr.k % (2 * (int64_t)v.bk) != 0;
   const bool w4 = v.threads == 256 && area >= 256 * 256 && whole_k >= 4 &&
-                  (!rest ? streamk || pr.num_groups > 0 || even_k_pays(pr.m, pr.n, pr.k, v.bk, pr.a_type, hw.n_cu) : (pr.a_type != TB_FP4_E2M1 && pr.c_type != TB_I8 && pr.a_k_contiguous && pr.b_k_contiguous &&
+                  (!rest ? streamk || looped || pr.num_groups > 0 || even_k_pays(pr.m, pr.n, pr.k, v.bk, pr.a_type, hw.n_cu) : (pr.a_type != TB_FP4_E2M1 && pr.c_type != TB_I8 && pr.a_k_contiguous && pr.b_k_contiguous &&
                              rest_of_k_pays(pr.m, pr.n, pr.k, v.bk, type_bits(pr.c_type), hw.n_cu)));
   int64_t k_steps = k_iters;
   double rest_us = 0.0;
@@ -380,9 +382,10 @@ double streaming_bound_us(const tb_problem& pr, const tb_hw& hw) {
 
 bool narrow_tile(const TileInfo& v) { return v.bn == 32 && v.dt != TB_F32; }
 
-int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, int ntiles, tb_selection* out) {
+int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, int ntiles, tb_selection* out, TileUse use) {
   int best = -1;
   double best_t = 0, best_c = 0, best_m = 0;
+  const bool part = hw.n_cu < hw.num_xcd * hw.cu_per_xcd;      // (a selector for some of the CUs, whose launches carry a grid)
   for (int i = 0; i < ntiles; ++i) {
     const TileInfo& v = tiles[i];
     if (!v.fast) continue;  // the gather kernels are a fallback, never a choice of the model
@@ -402,7 +405,7 @@ int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, in
       if (v.bm != want || v.bn != want) continue;
     }
     double c, m;
-    double t = score(pr, hw, v, pr.streamk != 0, &c, &m);
+    double t = score(pr, hw, v, pr.streamk != 0, &c, &m, nullptr, use.looped || part);
     // prefer the larger tile on ties (less L2 traffic than the model resolves)
     if (best < 0 || t < best_t * 0.995 || (t <= best_t * 1.005 && (int64_t)v.bm * v.bn > (int64_t)tiles[best].bm * tiles[best].bn)) {
       best = i; best_t = t; best_c = c; best_m = m;

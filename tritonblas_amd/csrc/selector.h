@@ -20,7 +20,12 @@ void hierarchical_split(int64_t total_tiles, int hw_cus, int num_xcds, int64_t* 
 bool rest_of_k_pays(int64_t m, int64_t n, int64_t k, int bk, int c_bits, int n_cu);
 bool even_k_pays(int64_t m, int64_t n, int64_t k, int bk, int type, int n_cu);     // ... that is one (type: a public element type)
 int variant_occupancy(const TileInfo& v, const tb_hw& hw);
-int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, int ntiles, tb_selection* out);
+// How a launch goes over its tiles.  looped: workgroups that take tile after tile, from a caller's grid or the work-stealing queues, and not one workgroup to a
+// tile.
+struct TileUse {
+  bool looped = false;
+};
+int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, int ntiles, tb_selection* out, TileUse use = {});
 // 32x32 and 64x32 tiles of the 16- and 8-bit types
 bool narrow_tile(const TileInfo& v);
 // model time (us) of one tile variant on a problem, and of the streaming small-M kernel

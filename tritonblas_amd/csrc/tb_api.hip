@@ -366,6 +366,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
   if (k_major_ok(j.B, j.b_sr, j.b_sk, j.N)) blay = LAY_K; else if (m_major_ok(j.B, j.b_sr, j.b_sk, j.N)) blay = LAY_M;
 
   // tile
+  const bool one_tile = j.schedule == TB_SCHED_PERSISTENT && j.grid <= 0;      // (to a workgroup, where the kernel has that form)
   int bm = j.bm, bn = j.bn, bk = j.bk;
   tb_selection sel;
   std::memset(&sel, 0, sizeof(sel));
@@ -391,7 +392,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
       }
       return TB_ERR_WORKSPACE;
     }
-    int st = select_tile(pr, hw, infos.data(), (int)infos.size(), &sel);
+    int st = select_tile(pr, hw, infos.data(), (int)infos.size(), &sel, TileUse{!one_tile});
     if (st != TB_OK) return st;
     bm = sel.block_m; bn = sel.block_n; bk = sel.block_k;
   }
@@ -441,7 +442,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
     if (by_model) { bm = bn = 256; bk = 128; }
     v = find_variant(j.dt, bm, bn, bk, alay, blay, 1, at_once, &hw, is_streamk(j.schedule) && j.num_groups == 0, j.K,
                      j.c_type == TB_I8 ? 2 : (is_f8_type(j.c_type) ? 1 : 0), rest_pays(),
-                     is_streamk(j.schedule) || j.num_groups > 0 || even_k_pays(j.M, j.N, j.K, 128 / usz * epu, model_type(j.dt), hw.n_cu));
+                     !one_tile || j.num_groups > 0 || even_k_pays(j.M, j.N, j.K, 128 / usz * epu, model_type(j.dt), hw.n_cu));
     if (by_model) v = grouped_variant(j, hw, v);
     if (!v) return TB_ERR_BAD_TILE;
   } else {
