@@ -211,6 +211,10 @@ typedef struct tb_launch_info {
 } tb_launch_info;
 int tb_gemm_launch_info(const tb_gemm_desc* desc, tb_launch_info* out);
 
+/* The same for a persistent call, which may run as two launches (column_split): the columns that the first one computes, all of them where it is the only one,
+ * and what both launch (launches: two of them; the second stays zero where there is none). */
+int tb_gemm_split_info(const tb_gemm_desc* desc, int64_t* first_columns, tb_launch_info* launches);
+
 /* Reads the status word of the current GPU's static workspace into *status (1: a Stream-K launch through
  * tb_gemm_static_workspace ran into spin_limit and stored NaN tiles) and, with clear != 0, sets it back to 0.
  * Waits for the device's earlier work; allocates nothing.  A caller-owned workspace carries the same word at

@@ -796,6 +796,30 @@ def test_few_even_k_steps_in_launches_that_loop_over_tiles(dtype, m, n, k):
     assert _launch_of(_job(code, m, n, k, _lib.TB_SCHED_WORK_STEALING, tile=tile, cu_mask=256, cu_mask_len=64)).four_wave == 1      # (an address that nobody reads)
 
 
+def _split_of(d):
+    """The columns of a persistent call's first launch, and what its one or two launches are."""
+    import ctypes as C
+    from tritonblas_amd import _lib
+    columns, launches = C.c_int64(), (_lib.tb_launch_info * 2)()
+    assert _lib.load().tb_gemm_split_info(d, columns, launches) == _lib.TB_OK
+    return columns.value, launches
+
+
+@pytest.mark.parametrize("a_type", ["TB_BF16", "TB_F16", "TB_FP8_E4M3", "TB_FP8_E5M2", "TB_I8", "TB_F32"])
+def test_both_parts_of_a_column_split_add_up_k_alike(a_type):
+    """The columns behind the whole rounds run a tile of the same K step as the others, and no streaming kernel: every column of C sums K in the same order."""
+    from tritonblas_amd import _lib
+    code, splits = getattr(_lib, a_type), 0
+    for m in (64, 512, 1024, 1280, 1792, 2048, 4096):
+        for n in (6656, 6912, 8448, 8704, 9472, 13312, 70000):
+            for k in (256, 512, 640, 1024, 2304, 3072):
+                first, (a, b) = _split_of(_job(code, m, n, k, c_type=_lib.TB_F32 if a_type == "TB_F32" else None))
+                if first < n:
+                    splits += 1
+                    assert a.block_k == b.block_k and not a.skinny and not b.skinny, (m, n, k)
+    assert splits >= 10
+
+
 def test_tiles_of_the_register_loading_kernels():
     """Rows off 16 bytes run in 128x128 or 64x64 tiles: 128 where the chosen tile has it on both sides, and where fp32 fills the CUs with them once."""
     from tritonblas_amd import _lib

@@ -12,7 +12,7 @@ TYPES = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32, "fp
 REL = {"bf16": 2.0 ** -8, "f16": 2.0 ** -11, "f32": 0.0, "fp8": 2.0 ** -8, "i8": 2.0 ** -8}
 
 
-def _product(a, b, c, tile, grid):
+def _product(a, b, c, tile, grid, column_split=-1):
     from tritonblas_amd import _lib
     d = _lib.tb_gemm_desc()
     d.struct_bytes = C.sizeof(_lib.tb_gemm_desc)
@@ -25,7 +25,7 @@ def _product(a, b, c, tile, grid):
     d.c_stride_m, d.c_stride_n = c.stride()
     d.a, d.b, d.c = a.data_ptr(), b.data_ptr(), c.data_ptr()
     d.block_m, d.block_n, d.block_k = tile
-    d.grid, d.column_split = grid, -1
+    d.grid, d.column_split = grid, column_split
     assert _lib.load().tb_gemm(d, _lib.stream_handle()) == _lib.TB_OK
     return c
 
@@ -98,3 +98,20 @@ def test_few_tiles(m, n, k, kind):
     for tile in ((0, 0, 0), (32, 32, step), (64, 32, step)):
         got = _product(a, b, torch.full((m, n), float("nan"), device="cuda", dtype=out), tile, 0)
         assert ((got.double() - want).abs() <= REL[kind] * want.abs()).all(), tile       # (whole numbers below 2**24: the sums are exact)
+
+
+def _split_and_whole(kind, m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    if kind == "i8":
+        a, b = (torch.randint(-127, 128, s, device="cuda", generator=g).to(torch.int8) for s in ((m, k), (n, k)))
+    else:
+        a, b = (torch.randn(s, device="cuda", generator=g).to(TYPES[kind]) for s in ((m, k), (n, k)))
+    out = TYPES[kind] if kind in ("bf16", "f16") else torch.float32
+    return [_product(a, b.T, torch.full((m, n), float("nan"), device="cuda", dtype=out), (0, 0, 0), 0, column_split=c) for c in (0, -1)]
+
+
+@pytest.mark.parametrize("kind,m,n,k", [("bf16", 1792, 9472, 2304), ("f16", 1024, 8448, 256), ("fp8", 1024, 8448, 640), ("i8", 1024, 8448, 640)])
+def test_column_split_with_a_rest_of_few_tiles(kind, m, n, k):
+    """The columns behind the whole rounds, few enough for tiles of another K step, have the bits that one launch gives them."""
+    split, whole = _split_and_whole(kind, m, n, k)
+    assert torch.equal(split, whole)

@@ -31,7 +31,7 @@ EXPORTED_SYMBOLS = [
     "tb_column_sum",
     "tb_column_sum_bytes",
     "tb_tile_coords", "tb_default_panel", "tb_ws_queue_tile", "tb_hierarchical_split",
-    "tb_workspace_layout", "tb_debug_option", "tb_gemm_static_workspace", "tb_static_workspace_status", "tb_gemm_launch_info",
+    "tb_workspace_layout", "tb_debug_option", "tb_gemm_static_workspace", "tb_static_workspace_status", "tb_gemm_launch_info", "tb_gemm_split_info",
 ]
 
 
@@ -175,6 +175,7 @@ def load():
     lib.tb_hierarchical_split.argtypes = [C.c_int64, C.c_int32, C.c_int32, C.POINTER(C.c_int32), C.POINTER(C.c_int32)]
     lib.tb_gemm_static_workspace.argtypes = [C.POINTER(tb_gemm_desc), C.c_void_p]
     lib.tb_gemm_launch_info.argtypes = [C.POINTER(tb_gemm_desc), C.POINTER(tb_launch_info)]
+    lib.tb_gemm_split_info.argtypes = [C.POINTER(tb_gemm_desc), C.POINTER(C.c_int64), C.POINTER(tb_launch_info)]
     lib.tb_static_workspace_status.argtypes = [C.POINTER(C.c_int), C.c_int]
     lib.tb_static_workspace_status.restype = C.c_int
     lib.tb_workspace_layout.argtypes = [C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]

@@ -390,6 +390,7 @@ int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, in
     const TileInfo& v = tiles[i];
     if (!v.fast) continue;  // the gather kernels are a fallback, never a choice of the model
     if (v.lds_bytes > hw.lds_bytes) continue;
+    if (use.block_k > 0 && v.bk != use.block_k) continue;
     // decode-like problems (a handful of rows): tiles taller than twice the row count only add
     // LDS traffic and idle MFMA rows when a shorter tile exists
     // (the small tiles of few-tile problems, see family(): whole tiles only, and not where the streaming kernel is at home, which is weighed against the others)

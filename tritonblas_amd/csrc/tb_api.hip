@@ -267,6 +267,7 @@ struct Job {
   int grp_sk = 0;          // grouped: cut the tiles that do not fill whole rounds of the grid into K ranges (needs a workspace)
   int column_split = 0;
   int tiles_only = 0;      // 1: never the streaming kernel
+  int only_bk = 0;         // > 0: the library chooses among the tiles of this K step
 };
 
 // Workspace layout (bytes): [0, 256) control words | work-stealing queue counters, one 256-byte line
@@ -392,7 +393,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
       }
       return TB_ERR_WORKSPACE;
     }
-    int st = select_tile(pr, hw, infos.data(), (int)infos.size(), &sel, TileUse{!one_tile});
+    int st = select_tile(pr, hw, infos.data(), (int)infos.size(), &sel, TileUse{!one_tile, j.only_bk});
     if (st != TB_OK) return st;
     bm = sel.block_m; bn = sel.block_n; bk = sel.block_k;
   }
@@ -712,7 +713,7 @@ PlanKey plan_key(const Job& j, int dev) {
       j.mxa_sr, j.mxa_sk, j.mxb_sr, j.mxb_sk, j.bias_stride, j.bm, j.bn, j.bk, j.group_m, j.num_xcds, j.grid,
       j.counters_per_xcd, j.ws_mode, j.ws_local, j.cu_mask_len, j.ws_global, j.num_groups, j.grp_phase, j.grp_big,
       j.grp_thr, j.grp_sk, j.b_group_stride, j.sb_group_stride, al(j.A), al(j.B), al(j.C), al(j.mxa), al(j.mxb),
-      al(j.bias), j.sa ? 1 : 0, j.sb ? 1 : 0, j.cu_mask ? 1 : 0, j.group_offsets ? 1 : 0, j.column_split, j.retreat, j.tiles_only, (int64_t)j.room,
+      al(j.bias), j.sa ? 1 : 0, j.sb ? 1 : 0, j.cu_mask ? 1 : 0, j.group_offsets ? 1 : 0, j.column_split, j.retreat, j.tiles_only, j.only_bk, (int64_t)j.room,
       (int64_t)g_hooks_version};
   static_assert(sizeof(f) <= sizeof(k.v), "PlanKey too small");
   for (int64_t x : f) k.v[i++] = x;
@@ -841,6 +842,10 @@ struct SplitChoice { PlanKey key; int64_t n1; uint64_t stamp; };   // n1 = 0: on
 SplitChoice g_splits[PLAN_CACHE];
 int g_splits_used = 0;
 
+bool may_split(const Job& j) {
+  return j.schedule == TB_SCHED_PERSISTENT && j.column_split == 0 && j.grid <= 0 && j.num_groups == 0 && !hooks().no_column_split;
+}
+
 // columns [0, n1) keep the planned tile, the rest becomes a problem of its own; 0 = do not split
 int64_t column_split_point(const Job& j, const tb_hw& hw, const Plan& whole) {
   const Variant* v = whole.v;
@@ -860,10 +865,30 @@ int64_t column_split_point(const Job& j, const tb_hw& hw, const Plan& whole) {
   pr.n = n2;
   tb_selection rest;
   const auto& infos = tile_infos(j.dt);
-  if (select_tile(pr, hw, infos.data(), (int)infos.size(), &rest) != TB_OK) return 0;
+  if (select_tile(pr, hw, infos.data(), (int)infos.size(), &rest, TileUse{false, v->bk}) != TB_OK) return 0;
   // (testing hook: TB_FORCE_COLUMN_SPLIT=1 splits whatever the model says)
   if (!hooks().force_column_split && t_first + rest.est_total_us > 0.97 * t_whole) return 0;
   return n1;
+}
+
+// The two launches of a split behind column n1, and whether it is one: the first runs what the whole would.  The second takes a tile of the same K step: one of another
+// groups the products of a step differently, 16 bits, or has a longer remainder of K, which comes first, and a column's bits would depend on where the split lies.
+// make: job -> plan.
+template <class F>
+bool split_plans(const Job& j, const Plan& whole, int64_t n1, F&& make, Job* a, Job* b, Plan* pa, Plan* pb) {
+  const Variant* v = whole.v;
+  *a = *b = j;
+  a->N = n1; a->bm = v->bm; a->bn = v->bn; a->bk = v->bk;
+  b->N = j.N - n1; b->bm = b->bn = b->bk = 0; b->group_m = 0;
+  b->only_bk = v->bk;
+  a->tiles_only = b->tiles_only = 1;
+  b->B = (const uint8_t*)j.B + n1 * j.b_sr * unit_bytes(j.dt);
+  b->C = (uint8_t*)j.C + n1 * j.c_sn * c_bytes(j.c_type);
+  if (j.sb) b->sb = j.sb + n1;
+  if (j.bias) b->bias = (const uint8_t*)j.bias + n1 * j.bias_stride * (j.bias_type == TB_F32 ? 4 : 2);
+  if (j.mxb) b->mxb = (const uint8_t*)j.mxb + n1 * j.mxb_sr;
+  if (make(*a, pa) != TB_OK || make(*b, pb) != TB_OK) return false;
+  return pa->v == v;      // (the split must not change what the main part runs)
 }
 
 int launch_columns(const Job& j, hipStream_t stream) {
@@ -885,8 +910,7 @@ int launch_columns(const Job& j, hipStream_t stream) {
     whole.workspace = nullptr; whole.workspace_bytes = 0;
     return launch_columns(whole, stream);
   }
-  if (j.schedule != TB_SCHED_PERSISTENT || j.column_split != 0 || j.grid > 0 || j.num_groups > 0 || hooks().no_column_split)
-    return launch(j, stream);
+  if (!may_split(j)) return launch(j, stream);
   tb_hw hw;
   int st = current_hw(&hw);
   if (st != TB_OK) return st;
@@ -913,20 +937,9 @@ int launch_columns(const Job& j, hipStream_t stream) {
     }
   }
   if (n1 <= 0) return run_plan(j, whole, stream);
-  const Variant* v = whole.v;
-  const int usz = unit_bytes(j.dt);
-  Job a = j, b = j;
-  a.N = n1; a.bm = v->bm; a.bn = v->bn; a.bk = v->bk;
-  b.N = j.N - n1; b.bm = b.bn = b.bk = 0; b.group_m = 0;
-  b.B = (const uint8_t*)j.B + n1 * j.b_sr * usz;
-  b.C = (uint8_t*)j.C + n1 * j.c_sn * c_bytes(j.c_type);
-  if (j.sb) b.sb = j.sb + n1;
-  if (j.bias) b.bias = (const uint8_t*)j.bias + n1 * j.bias_stride * (j.bias_type == TB_F32 ? 4 : 2);
-  if (j.mxb) b.mxb = (const uint8_t*)j.mxb + n1 * j.mxb_sr;
+  Job a, b;
   Plan pa, pb;
-  st = cached_plan(a, hw, &pa);
-  if (st == TB_OK) st = cached_plan(b, hw, &pb);
-  if (st != TB_OK || pa.v != v) return run_plan(j, whole, stream);   // (the split must not change what the main part runs)
+  if (!split_plans(j, whole, n1, [&](const Job& x, Plan* p) { return cached_plan(x, hw, p); }, &a, &b, &pa, &pb)) return run_plan(j, whole, stream);
   st = run_plan(a, pa, stream);
   if (st != TB_OK) return st;
   return run_plan(b, pb, stream);
@@ -1147,6 +1160,16 @@ int tb_static_workspace_status(int* status, int clear) {
   return TB_OK;
 }
 
+static void fill_launch_info(const Plan& plan, tb_launch_info* out) {
+  std::memset(out, 0, sizeof(*out));
+  out->block_m = plan.v->bm; out->block_n = plan.v->bn; out->block_k = plan.v->bk;
+  out->waves = plan.v->threads / 64; out->four_wave = plan.v->k_step_pairs ? 1 : 0;
+  out->mode = plan.p.mode; out->grid = plan.grid; out->total_tiles = plan.p.total_tiles;
+  out->sk_tiles = plan.p.mode == MODE_SK ? plan.p.sk_tiles : 0;
+  out->sk_unit = plan.p.mode == MODE_SK ? std::max(1, plan.p.sk_unit) : 0;
+  out->sk_ws = plan.p.sk_ws; out->skinny = plan.skinny ? 1 : 0;
+}
+
 int tb_gemm_launch_info(const tb_gemm_desc* desc, tb_launch_info* out) {
   if (!out) return TB_ERR_NULL_POINTER;
   Job j;
@@ -1159,13 +1182,32 @@ int tb_gemm_launch_info(const tb_gemm_desc* desc, tb_launch_info* out) {
   auto make = [&](const Job& x, Plan* p) { return make_plan(x, hw, have_dev, p); };
   st = j.workspace ? fitting_plan(j, make, &plan) : make(j, &plan);
   if (st != TB_OK) return st;
-  std::memset(out, 0, sizeof(*out));
-  out->block_m = plan.v->bm; out->block_n = plan.v->bn; out->block_k = plan.v->bk;
-  out->waves = plan.v->threads / 64; out->four_wave = plan.v->k_step_pairs ? 1 : 0;
-  out->mode = plan.p.mode; out->grid = plan.grid; out->total_tiles = plan.p.total_tiles;
-  out->sk_tiles = plan.p.mode == MODE_SK ? plan.p.sk_tiles : 0;
-  out->sk_unit = plan.p.mode == MODE_SK ? std::max(1, plan.p.sk_unit) : 0;
-  out->sk_ws = plan.p.sk_ws; out->skinny = plan.skinny ? 1 : 0;
+  fill_launch_info(plan, out);
+  return TB_OK;
+}
+
+int tb_gemm_split_info(const tb_gemm_desc* desc, int64_t* first_columns, tb_launch_info* launches) {
+  if (!first_columns || !launches) return TB_ERR_NULL_POINTER;
+  Job j, a, b;
+  int st = job_from_gemm(desc, &j);
+  if (st != TB_OK) return st;
+  tb_hw hw;
+  const bool have_dev = current_hw(&hw) == TB_OK;
+  if (!have_dev) default_hw(&hw);
+  auto make = [&](const Job& x, Plan* p) { return make_plan(x, hw, have_dev, p); };
+  Plan whole, pa, pb;
+  st = make(j, &whole);
+  if (st != TB_OK) return st;
+  *first_columns = j.N;
+  std::memset(launches, 0, 2 * sizeof(*launches));
+  const int64_t n1 = may_split(j) ? column_split_point(j, hw, whole) : 0;
+  if (n1 <= 0 || !split_plans(j, whole, n1, make, &a, &b, &pa, &pb)) {
+    fill_launch_info(whole, launches);
+    return TB_OK;
+  }
+  *first_columns = n1;
+  fill_launch_info(pa, launches);
+  fill_launch_info(pb, launches + 1);
   return TB_OK;
 }
 
