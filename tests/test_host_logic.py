@@ -820,6 +820,31 @@ def test_both_parts_of_a_column_split_add_up_k_alike(a_type):
     assert splits >= 10
 
 
+@pytest.mark.parametrize("a_type,m,n,steps,columns", [
+    ("TB_BF16", 1280, 13312, 16, 13056), ("TB_F16", 1280, 13312, 22, 13056), ("TB_BF16", 4096, 4352, 16, 4096), ("TB_BF16", 8192, 5120, 8, 4096),
+    ("TB_FP8_E4M3", 1280, 13312, 16, 13056), ("TB_FP8_E5M2", 1280, 13312, 18, 13056), ("TB_FP8_E4M3", 4096, 4352, 24, 4096), ("TB_FP8_E4M3", 8192, 2560, 30, 2048),
+    ("TB_I8", 1280, 13312, 16, 13056)])
+def test_a_column_split_whose_parts_run_either_kernel_of_the_tile(a_type, m, n, steps, columns):
+    """Just over one or two rounds of 256x256 tiles: the whole would run the hand-scheduled kernel, the columns that fill the rounds the eight-wave one, and the
+    launch is split all the same.  A K with a rest, which the two add up in another order, is split only where both run one kernel."""
+    from tritonblas_amd import _lib
+    code = getattr(_lib, a_type)
+    step = 64 if a_type in ("TB_BF16", "TB_F16") else 128
+    d = _job(code, m, n, steps * step)
+    whole = _launch_of(d)
+    first, (a, b) = _split_of(d)
+    assert (whole.block_m, whole.block_n, whole.four_wave) == (256, 256, 1)
+    assert first == columns and (a.block_m, a.block_n, a.four_wave) == (256, 256, 0) and b.total_tiles > 0
+    for k in range(steps * step - 7 * step, steps * step, 16):
+        d = _job(code, m, n, k)
+        first, (a, _) = _split_of(d)
+        if first < n and k % (2 * a.block_k):
+            whole = _launch_of(d)
+            assert (a.block_m, a.block_n, a.waves, a.four_wave) == (whole.block_m, whole.block_n, whole.waves, whole.four_wave)
+    d.column_split = -1
+    assert _split_of(d)[0] == n
+
+
 def test_tiles_of_the_register_loading_kernels():
     """Rows off 16 bytes run in 128x128 or 64x64 tiles: 128 where the chosen tile has it on both sides, and where fp32 fills the CUs with them once."""
     from tritonblas_amd import _lib

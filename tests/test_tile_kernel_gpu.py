@@ -115,3 +115,10 @@ def test_column_split_with_a_rest_of_few_tiles(kind, m, n, k):
     """The columns behind the whole rounds, few enough for tiles of another K step, have the bits that one launch gives them."""
     split, whole = _split_and_whole(kind, m, n, k)
     assert torch.equal(split, whole)
+
+
+@pytest.mark.parametrize("kind,m,n,k", [("bf16", 1280, 13312, 1024), ("f16", 4096, 4360, 1024), ("fp8", 1280, 13312, 2048), ("i8", 1280, 13312, 2048)])
+def test_column_split_over_both_kernels_of_the_tile(kind, m, n, k):
+    """A split whose columns in whole rounds run the eight-wave kernel where the whole would run the hand-scheduled one (see the host test of the route): the same bits."""
+    split, whole = _split_and_whole(kind, m, n, k)
+    assert torch.equal(split, whole)

@@ -319,9 +319,9 @@ int streamk_grid_for(const tb_problem& pr, const tb_hw& hw, const TileInfo& v) {
   return grid;
 }
 
-double estimate_tile_us(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bool streamk) {
+double estimate_tile_us(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bool streamk, TileUse use) {
   double c, m;
-  return score(pr, hw, v, streamk, &c, &m);
+  return score(pr, hw, v, streamk, &c, &m, nullptr, use.looped);
 }
 
 // A grouped FP8 launch.  The rows of an expert are taken as spread around their mean, by chance and by 7 % of it, which gives the row blocks to expect; per variant:

@@ -30,7 +30,7 @@ int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, in
 // 32x32 and 64x32 tiles of the 16- and 8-bit types
 bool narrow_tile(const TileInfo& v);
 // model time (us) of one tile variant on a problem, and of the streaming small-M kernel
-double estimate_tile_us(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bool streamk);
+double estimate_tile_us(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bool streamk, TileUse use = {});
 // ... of a grouped launch whose row counts only the device knows (FP8; 0: no figures for this variant)
 double estimate_grouped_us(const tb_problem& pr, const tb_hw& hw, const TileInfo& v);
 double estimate_streaming_us(const tb_problem& pr, const tb_hw& hw, int cols);

@@ -861,7 +861,8 @@ int64_t column_split_point(const Job& j, const tb_hw& hw, const Plan& whole) {
   const TileInfo ti{v->dt, v->bm, v->bn, v->bk, v->threads, v->lds_bytes, v->minb, v->fast, v->stages};
   const double t_whole = estimate_tile_us(pr, hw, ti, false);
   pr.n = n1;
-  const double t_first = estimate_tile_us(pr, hw, ti, false);
+  // (by the whole's kernel also where the other one is ahead for fewer tiles, which the model has no better price for: FP8 1280x13312x2048 38 us split, 47 whole)
+  const double t_first = estimate_tile_us(pr, hw, ti, false, TileUse{whole.v->k_step_pairs != 0});
   pr.n = n2;
   tb_selection rest;
   const auto& infos = tile_infos(j.dt);
@@ -871,9 +872,10 @@ int64_t column_split_point(const Job& j, const tb_hw& hw, const Plan& whole) {
   return n1;
 }
 
-// The two launches of a split behind column n1, and whether it is one: the first runs what the whole would.  The second takes a tile of the same K step: one of another
-// groups the products of a step differently, 16 bits, or has a longer remainder of K, which comes first, and a column's bits would depend on where the split lies.
-// make: job -> plan.
+// The two launches of a split behind column n1, and whether it is one: the first runs the tile of the whole, by the same kernel or, where K is whole pairs of K
+// steps, by the other one of the 256x256 tile.  (Which of the two is ahead goes by the number of tiles and the first launch has fewer: bf16 1280x13312x1024, 260 tiles by
+// hand-scheduled kernel or 255 by eight waves.  Both add up whole K steps in the same order.)  The second takes a tile of the same K step: one of another groups the products of a
+// step differently, 16 bits, or has a longer remainder of K, which comes first, and a column's bits would depend on where the split lies.  make: job -> plan.
 template <class F>
 bool split_plans(const Job& j, const Plan& whole, int64_t n1, F&& make, Job* a, Job* b, Plan* pa, Plan* pb) {
   const Variant* v = whole.v;
@@ -888,7 +890,7 @@ bool split_plans(const Job& j, const Plan& whole, int64_t n1, F&& make, Job* a, 
   if (j.bias) b->bias = (const uint8_t*)j.bias + n1 * j.bias_stride * (j.bias_type == TB_F32 ? 4 : 2);
   if (j.mxb) b->mxb = (const uint8_t*)j.mxb + n1 * j.mxb_sr;
   if (make(*a, pa) != TB_OK || make(*b, pb) != TB_OK) return false;
-  return pa->v == v;      // (the split must not change what the main part runs)
+  return pa->v == v || (pa->v->fast == LOAD_DIRECT && pa->v->bm == v->bm && pa->v->bn == v->bn && pa->v->bk == v->bk && j.K % (2 * (int64_t)v->bk) == 0);
 }
 
 int launch_columns(const Job& j, hipStream_t stream) {
