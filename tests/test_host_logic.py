@@ -845,6 +845,39 @@ def test_a_column_split_whose_parts_run_either_kernel_of_the_tile(a_type, m, n, 
     assert _split_of(d)[0] == n
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float8_e4m3fn, torch.int8])
+@pytest.mark.parametrize("m,n,k", [(512, 512, 8192), (256, 256, 7904), (200, 1000, 2000)])
+def test_small_tiles_are_for_cus_that_would_be_idle(dtype, m, n, k):
+    """32x32 and 64x32 tiles split what leaves CUs idle in 64x64: a launch that its caller keeps to fewer workgroups than it would have of them has none idle,
+    and one that draws its tiles from the work-stealing queues takes 64x32 alone."""
+    import tritonblas_amd as tb
+    from tritonblas_amd import _lib
+    from tritonblas_amd.matmul import _tile_of
+    code, queues = _lib.tb_dtype(dtype), _lib.TB_SCHED_WORK_STEALING
+    own = _launch_of(_job(code, m, n, k))
+    assert own.block_n == 32
+    for grid in (8, 16, 32, 64, 128, 256):
+        for info in (_launch_of(_job(code, m, n, k, grid=grid)), _launch_of(_job(code, m, n, k, queues, grid)),
+                     _launch_of(_job(code, m, n, k, queues, cu_mask=256, cu_mask_len=grid))):       # (an address that nobody reads)
+            assert info.block_n > 32 or info.total_tiles <= grid
+            assert info.block_n > 32 or info.mode != 1 or info.block_m == 64
+        assert grid > 16 or (info.block_m, info.block_n) == (64, 64)
+    info = _launch_of(_job(code, m, n, k, queues))
+    assert (info.block_m, info.block_n) == (64, 32) and info.total_tiles <= 256
+    sel = tb.OrigamiMatmulSelector(m, n, k, dtype, dtype, torch.bfloat16, None)
+    assert (sel.block_m, sel.block_n) == (own.block_m, own.block_n)
+    model = sel.block_m, sel.block_n, sel.block_k
+    assert _tile_of(sel, queues, k, dtype, True) == (0, 0, 0) and _tile_of(sel, _lib.TB_SCHED_PERSISTENT, k, dtype, True) == model == _tile_of(sel, _lib.TB_SCHED_STREAMK, k, dtype, True)
+    for cus in (8, 16, 64):
+        sel = tb.OrigamiMatmulSelector(m, n, k, dtype, dtype, torch.bfloat16, None, total_cus=cus)
+        tiles = -(-m // sel.block_m) * -(-n // sel.block_n)
+        assert sel.block_n > 32 or tiles <= cus * sel.waves_per_eu
+        model = sel.block_m, sel.block_n, sel.block_k
+        assert _tile_of(sel, queues, k, dtype, True) == ((64, 32, model[2]) if model[1] == 32 else model) and _tile_of(sel, _lib.TB_SCHED_PERSISTENT, k, dtype, False) == model
+        sel._sel.block_m = sel._sel.block_n = 32      # (a tile that the caller put into the selector stays)
+        assert model[:2] == (32, 32) or _tile_of(sel, queues, k, dtype, True) == (32, 32, model[2])
+
+
 def test_tiles_of_the_register_loading_kernels():
     """Rows off 16 bytes run in 128x128 or 64x64 tiles: 128 where the chosen tile has it on both sides, and where fp32 fills the CUs with them once."""
     from tritonblas_amd import _lib

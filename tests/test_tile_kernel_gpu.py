@@ -12,7 +12,7 @@ TYPES = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32, "fp
 REL = {"bf16": 2.0 ** -8, "f16": 2.0 ** -11, "f32": 0.0, "fp8": 2.0 ** -8, "i8": 2.0 ** -8}
 
 
-def _product(a, b, c, tile, grid, column_split=-1):
+def _product(a, b, c, tile, grid, column_split=-1, schedule=0, workspace=None):
     from tritonblas_amd import _lib
     d = _lib.tb_gemm_desc()
     d.struct_bytes = C.sizeof(_lib.tb_gemm_desc)
@@ -25,7 +25,9 @@ def _product(a, b, c, tile, grid, column_split=-1):
     d.c_stride_m, d.c_stride_n = c.stride()
     d.a, d.b, d.c = a.data_ptr(), b.data_ptr(), c.data_ptr()
     d.block_m, d.block_n, d.block_k = tile
-    d.grid, d.column_split = grid, column_split
+    d.grid, d.column_split, d.schedule = grid, column_split, schedule
+    if workspace is not None:
+        d.workspace, d.workspace_bytes, d.epoch = workspace.data_ptr(), workspace.numel(), _lib.TB_EPOCH_ON_DEVICE
     assert _lib.load().tb_gemm(d, _lib.stream_handle()) == _lib.TB_OK
     return c
 
@@ -98,6 +100,33 @@ def test_few_tiles(m, n, k, kind):
     for tile in ((0, 0, 0), (32, 32, step), (64, 32, step)):
         got = _product(a, b, torch.full((m, n), float("nan"), device="cuda", dtype=out), tile, 0)
         assert ((got.double() - want).abs() <= REL[kind] * want.abs()).all(), tile       # (whole numbers below 2**24: the sums are exact)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "f16", "fp8", "i8"])
+@pytest.mark.parametrize("m,n,k", [(33, 40, 4096), (200, 1000, 2000), (256, 256, 7904), (31, 33, 272), (353, 1264, 1552)])
+def test_small_tiles_under_the_other_schedules(m, n, k, kind):
+    """32x32 and 64x32 tiles from the work-stealing queues and with a Stream-K tail, named and as the library chooses, on the whole device and on 24 workgroups; one
+    workspace for all launches.  Then through a selector, which has a small tile for each of these."""
+    import tritonblas_amd as tb
+    from tritonblas_amd import _lib
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randint(-2, 3, (m, k), device="cuda", generator=g).to(TYPES[kind])
+    b = torch.randint(-2, 3, (n, k), device="cuda", generator=g).to(TYPES[kind]).T
+    want = a.double() @ b.double()
+    out = TYPES[kind] if kind in ("bf16", "f16") else torch.bfloat16
+    step = 128 if kind in ("bf16", "f16") else 256
+    workspace = torch.zeros(64 << 20, dtype=torch.uint8, device="cuda")
+    for schedule in (_lib.TB_SCHED_WORK_STEALING, _lib.TB_SCHED_STREAMK, _lib.TB_SCHED_STREAMK_WS):
+        for grid in (0, 24):
+            for tile in ((0, 0, 0), (32, 32, step), (64, 32, step)):
+                got = _product(a, b, torch.full((m, n), float("nan"), device="cuda", dtype=out), tile, grid, schedule=schedule, workspace=workspace)
+                assert ((got.double() - want).abs() <= REL[kind] * want.abs()).all(), (schedule, grid, tile)
+    selector = tb.OrigamiMatmulSelector(m, n, k, a.dtype, b.dtype, out, a.device)
+    config = tb.matmul_preamble(selector, a.device)
+    for streamk in (False, True):
+        got = torch.full((m, n), float("nan"), device="cuda", dtype=out)
+        tb.matmul_lt(a, b, got, selector, config, enable_streamk=streamk, work_stealing=True)
+        assert ((got.double() - want).abs() <= REL[kind] * want.abs()).all(), streamk
 
 
 def _split_and_whole(kind, m, n, k):

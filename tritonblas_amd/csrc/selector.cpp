@@ -224,8 +224,12 @@ int streamk_grid(int64_t total, int64_t k_iters, int slots, int n_cu, double ste
   return (int)(total * best_s);
 }
 
+// A selector for some of the CUs: its launches carry a grid, which is what these CUs hold of the tile.
+static bool of_the_cus(const tb_hw& hw) { return hw.n_cu < hw.num_xcd * hw.cu_per_xcd; }
+static int64_t workgroups_of(const TileInfo& v, const tb_hw& hw, TileUse use) { return use.workgroups > 0 ? use.workgroups : (int64_t)hw.n_cu * variant_occupancy(v, hw); }
+
 static double score(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bool streamk, double* comp_us,
-                    double* mem_us, int* sk_grid_out = nullptr, bool looped = false) {
+                    double* mem_us, int* sk_grid_out = nullptr, TileUse use = {}) {
   const double clk = hw.clock_khz * 1e3;
   const int bits = type_bits(pr.a_type);
   const double esz = bits / 8.0;
@@ -239,10 +243,11 @@ static double score(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bo
   // (an even number of whole K steps; what is behind them, up to two steps at about 3.5 us each and 2 more, only from K-contiguous operands, not MXFP4, and
   // without an int8 result: the kernels that find_variant has.  Of the Stream-K launches those that share no tile have them too; the others are
   // priced alike: with the eight-wave kernel's figures for both FP8 1556x10016x1840 goes from 48 to 56 us, and 44 bf16 problems come out level)
+  const bool part = of_the_cus(hw);
   const int64_t whole_k = pr.k / v.bk;
   const bool rest = pr.k % (2 * (int64_t)v.bk) != 0;
   const bool w4 = v.threads == 256 && area >= 256 * 256 && whole_k >= 4 &&
-                  (!rest ? streamk || looped || pr.num_groups > 0 || even_k_pays(pr.m, pr.n, pr.k, v.bk, pr.a_type, hw.n_cu) : (pr.a_type != TB_FP4_E2M1 && pr.c_type != TB_I8 && pr.a_k_contiguous && pr.b_k_contiguous &&
+                  (!rest ? streamk || use.looped || part || pr.num_groups > 0 || even_k_pays(pr.m, pr.n, pr.k, v.bk, pr.a_type, hw.n_cu) : (pr.a_type != TB_FP4_E2M1 && pr.c_type != TB_I8 && pr.a_k_contiguous && pr.b_k_contiguous &&
                              rest_of_k_pays(pr.m, pr.n, pr.k, v.bk, type_bits(pr.c_type), hw.n_cu)));
   int64_t k_steps = k_iters;
   double rest_us = 0.0;
@@ -321,7 +326,7 @@ int streamk_grid_for(const tb_problem& pr, const tb_hw& hw, const TileInfo& v) {
 
 double estimate_tile_us(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bool streamk, TileUse use) {
   double c, m;
-  return score(pr, hw, v, streamk, &c, &m, nullptr, use.looped);
+  return score(pr, hw, v, streamk, &c, &m, nullptr, use);
 }
 
 // A grouped FP8 launch.  The rows of an expert are taken as spread around their mean, by chance and by 7 % of it, which gives the row blocks to expect; per variant:
@@ -385,7 +390,6 @@ bool narrow_tile(const TileInfo& v) { return v.bn == 32 && v.dt != TB_F32; }
 int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, int ntiles, tb_selection* out, TileUse use) {
   int best = -1;
   double best_t = 0, best_c = 0, best_m = 0;
-  const bool part = hw.n_cu < hw.num_xcd * hw.cu_per_xcd;      // (a selector for some of the CUs, whose launches carry a grid)
   for (int i = 0; i < ntiles; ++i) {
     const TileInfo& v = tiles[i];
     if (!v.fast) continue;  // the gather kernels are a fallback, never a choice of the model
@@ -395,6 +399,10 @@ int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, in
     // LDS traffic and idle MFMA rows when a shorter tile exists
     // (the small tiles of few-tile problems, see family(): whole tiles only, and not where the streaming kernel is at home, which is weighed against the others)
     if (narrow_tile(v) && (pr.streamk || pr.num_groups > 0 || (pr.m <= 64 && pr.n >= 1024 && pr.a_k_contiguous && pr.b_k_contiguous))) continue;
+    // (they are for CUs that would be idle: a launch kept to some workgroups takes them where each has one tile at most.  bf16 512x512x8192 on 16 workgroups 125 us in 64x64,
+    // 277 in 32x32; 256x256x7904 on 32 32 and 36, on 64 32 and 20.  From the work-stealing queues, where each workgroup more costs a walk over the counters, 64x32
+    // alone, where every CU has a tile at most: 0.58 to 0.98 of the time of 64x64 on 14 such shapes in bf16, 0.45 to 1.02 in FP8; 32x32 up to 1.31, 64x32 with 304 tiles 1.27.)
+    if (narrow_tile(v) && (use.queues || use.workgroups > 0 || of_the_cus(hw)) && (cdiv(pr.m, v.bm) * cdiv(pr.n, v.bn) > workgroups_of(v, hw, use) || (use.queues && v.bm == 32))) continue;
     bool shorter_exists = false;
     for (int q = 0; q < ntiles; ++q) shorter_exists |= tiles[q].fast && !narrow_tile(tiles[q]) && tiles[q].bm < v.bm && tiles[q].bm >= pr.m;
     if (shorter_exists && pr.num_groups == 0) continue;
@@ -406,7 +414,7 @@ int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, in
       if (v.bm != want || v.bn != want) continue;
     }
     double c, m;
-    double t = score(pr, hw, v, pr.streamk != 0, &c, &m, nullptr, use.looped || part);
+    double t = score(pr, hw, v, pr.streamk != 0, &c, &m, nullptr, use);
     // prefer the larger tile on ties (less L2 traffic than the model resolves)
     if (best < 0 || t < best_t * 0.995 || (t <= best_t * 1.005 && (int64_t)v.bm * v.bn > (int64_t)tiles[best].bm * tiles[best].bn)) {
       best = i; best_t = t; best_c = c; best_m = m;

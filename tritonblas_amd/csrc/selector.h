@@ -21,10 +21,13 @@ bool rest_of_k_pays(int64_t m, int64_t n, int64_t k, int bk, int c_bits, int n_c
 bool even_k_pays(int64_t m, int64_t n, int64_t k, int bk, int type, int n_cu);     // ... that is one (type: a public element type)
 int variant_occupancy(const TileInfo& v, const tb_hw& hw);
 // How a launch goes over its tiles.  looped: workgroups that take tile after tile, from a caller's grid or the work-stealing queues, and not one workgroup to a
-// tile.  block_k: tiles of this K step only (0: any).
+// tile.  block_k: tiles of this K step only (0: any).  queues: they come from the work-stealing queues.  workgroups: as many as the caller keeps the launch to (0: as
+// many as the device holds).
 struct TileUse {
   bool looped = false;
   int block_k = 0;
+  bool queues = false;
+  int workgroups = 0;
 };
 int select_tile(const tb_problem& pr, const tb_hw& hw, const TileInfo* tiles, int ntiles, tb_selection* out, TileUse use = {});
 // 32x32 and 64x32 tiles of the 16- and 8-bit types

@@ -393,7 +393,9 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
       }
       return TB_ERR_WORKSPACE;
     }
-    int st = select_tile(pr, hw, infos.data(), (int)infos.size(), &sel, TileUse{!one_tile, j.only_bk});
+    const bool queues = j.schedule == TB_SCHED_WORK_STEALING;
+    const TileUse use{!one_tile, j.only_bk, queues, queues && j.cu_mask && j.grid <= 0 ? std::max(1, j.cu_mask_len) : std::max(0, j.grid)};
+    int st = select_tile(pr, hw, infos.data(), (int)infos.size(), &sel, use);
     if (st != TB_OK) return st;
     bm = sel.block_m; bn = sel.block_n; bk = sel.block_k;
   }

@@ -85,7 +85,8 @@ class OrigamiMatmulSelector:
         _lib.check(_lib.load().tb_select(prob, self._hardware._c, sel), "tb_select")
         self._sel = sel
         # (a launch whose operands ask for another tile may leave the choice to the library: not a partition's)
-        self._model_tile = (sel.block_m, sel.block_n, sel.block_k) if total_cus is None else None
+        tile = sel.block_m, sel.block_n, sel.block_k
+        self._model_tile, self._part_tile = (tile, None) if total_cus is None else (None, tile)
         self._num_stages = sel.num_stages
         self._grid = sel.sk_grid if self.streamk else self._N_CU
         self._workgroup_mapping = sel.group_m
