@@ -878,6 +878,24 @@ def test_small_tiles_are_for_cus_that_would_be_idle(dtype, m, n, k):
         assert model[:2] == (32, 32) or _tile_of(sel, queues, k, dtype, True) == (32, 32, model[2])
 
 
+def test_fp32_and_int8_tiles_of_launches_kept_to_some_workgroups():
+    """The tiles that pay where the whole device would be idle else are not for a part of it, but for fp32 tiles that all run at once."""
+    import tritonblas_amd as tb
+    from tritonblas_amd import _lib
+
+    def side(a_type, m, n, k, **kw):
+        info = _launch_of(_job(a_type, m, n, k, c_type=_lib.TB_F32 if a_type == _lib.TB_F32 else None, **kw))
+        return info.block_m, info.block_n
+    for m, n, k in [(1664, 480, 5568), (512, 2048, 2848), (240, 3552, 4672)]:
+        assert side(_lib.TB_F32, m, n, k) == (32, 32)
+        assert side(_lib.TB_F32, m, n, k, grid=64) == (64, 64) == side(_lib.TB_F32, m, n, k, grid=128, schedule=_lib.TB_SCHED_WORK_STEALING)
+        assert tb.OrigamiMatmulSelector(m, n, k, torch.float32, torch.float32, torch.float32, None, total_cus=64).block_m == 64
+    assert tb.OrigamiMatmulSelector(256, 512, 2048, torch.float32, torch.float32, torch.float32, None, total_cus=32).block_m == 32
+    assert side(_lib.TB_F32, 20, 4000, 512, grid=16) == (32, 32)          # (few rows: the shortest tile there is)
+    sel = tb.OrigamiMatmulSelector(640, 1024, 3072, torch.int8, torch.int8, torch.bfloat16, None, total_cus=32)
+    assert (sel.block_m, sel.block_n) == (128, 128)
+
+
 def test_tiles_of_the_register_loading_kernels():
     """Rows off 16 bytes run in 128x128 or 64x64 tiles: 128 where the chosen tile has it on both sides, and where fp32 fills the CUs with them once."""
     from tritonblas_amd import _lib

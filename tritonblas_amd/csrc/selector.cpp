@@ -115,7 +115,7 @@ struct Family {
 };
 // lat: the deeper variants of the 64x64 tile run while at most two (three) tiles per CU exist, the eight-wave 128x128 tile while every tile has
 // a CU of its own (find_variant)
-static Family family(int dt, const TileInfo& v, bool w4, int64_t tiles, int n_cu, bool grouped, bool streamk) {
+static Family family(int dt, const TileInfo& v, bool w4, int64_t tiles, int n_cu, bool grouped, bool older) {
   const int area = v.bm * v.bn;
   const int cls = (v.bm < 64 || v.bn < 64) ? 5 : area >= 256 * 256 ? 0 : area >= 256 * 128 ? 1 : area >= 128 * 128 ? 2 : area >= 128 * 64 ? 3 : 4;
   if (dt == TB_FP4_E2M1 || dt == TB_F32) {
@@ -124,18 +124,18 @@ static Family family(int dt, const TileInfo& v, bool w4, int64_t tiles, int n_cu
     // 2048^3 130 us against 147, 1000x3000x1504 79 and 108.  One 64x64 workgroup to a CU hides nothing, its step takes twice the MFMAs' time: 32x32 tiles
     // fill the CUs better there, 1664x480x5568 164 us and 105, 512x2048x2848 86 and 59, 240x3552x4672 140 and 91.  Of 894 problems, 100..8192 a side, four orders, the tile
     // taken was 1.029 times the best one's time in the geometric mean, 1.57 at most; with these three figures 1.003 and 1.19.  Stream-K launches cut such tiles
-    // instead and keep their own.)
+    // instead and keep their own: `older`.)
     static const double f32[6] = {0.92, 0.77, 0.77, 0.86, 0.82, 0.70}, f32_sk[6] = {0.92, 0.77, 0.77, 0.86, 0.86, 0.65};
     // (MXFP4 256x256 with eight waves, a round of one tile to a workgroup: 2 to 16 K steps 13.9 to 34.1 us, within 1.5 of the hand-scheduled kernel's figures)
-    const bool w8_one = cls == 0 && dt == TB_FP4_E2M1 && !streamk && !grouped && tiles <= n_cu;
+    const bool w8_one = cls == 0 && dt == TB_FP4_E2M1 && !older && !grouped && tiles <= n_cu;
     const double tile_us = cls == 0 ? (w4 || w8_one ? 8.0 : 12.0) : (cls <= 2 ? 4.0 : 3.0);
-    double lat = dt != TB_F32 ? 1.0 : cls == 5 ? (streamk ? 0.6 : 0.4) : cls == 4 && !streamk ? 1.7 : 1.0;
+    double lat = dt != TB_F32 ? 1.0 : cls == 5 ? (older ? 0.6 : 0.4) : cls == 4 && !older ? 1.7 : 1.0;
     if (dt == TB_FP4_E2M1 && !grouped) {      // (three copy stages: see find_variant)
       if (cls == 2 && tiles <= n_cu && v.bk == 256) lat = 0.88;
       if (cls == 3) lat = 0.85;
       if (cls == 4 && tiles <= 2 * (int64_t)n_cu) lat = 0.66;
     }
-    return {dt == TB_F32 ? (streamk ? f32_sk : f32)[cls] : ((w4 && cls == 0) || w8_one ? 0.56 : f4[cls]), tile_us, lat};
+    return {dt == TB_F32 ? (older ? f32_sk : f32)[cls] : ((w4 && cls == 0) || w8_one ? 0.56 : f4[cls]), tile_us, lat};
   }
   //                                     256x256  256x128 128x128 128x64 64x64  32x128
   static const double eff16[6] = {0.69, 0.506, 0.388, 0.357, 0.246, 0.12}, us16[6] = {9.5, 5.0, 3.8, 2.8, 3.0, 3.0};
@@ -150,15 +150,15 @@ static Family family(int dt, const TileInfo& v, bool w4, int64_t tiles, int n_cu
   // 200x1000x2000 11.4 and 6.9; FP8 256x256x7904 19.9 and 9.9, 130x520x3008 8.6 and 5.7.  64x32: bf16 128x4096x4096 21.6 and 16.6.  On 1500 problems of at most 768 tiles of 64x64 each in
   // bf16 and FP8 the choice among the three takes 1.003 and 1.015 times the best one's time, 1/1.35 and 1/1.26 of what 64x64 takes.
   if (v.bn == 32) return half ? (v.bm == 32 ? Family{0.10, 1.2, 0.33} : Family{0.12, 1.2, 0.36}) : v.bm == 32 ? Family{0.10, 1.2, 0.36} : Family{0.15, 1.5, 0.55};
-  Family f = half ? Family{eff16[cls], us16[cls], 1.0} : dt == TB_I8 ? (streamk ? Family{effi_sk[cls], usi_sk[cls], 1.0} : Family{effi[cls], usi[cls], 1.0}) : Family{eff8[cls], us8[cls], 1.0};
+  Family f = half ? Family{eff16[cls], us16[cls], 1.0} : dt == TB_I8 ? (older ? Family{effi_sk[cls], usi_sk[cls], 1.0} : Family{effi[cls], usi[cls], 1.0}) : Family{eff8[cls], us8[cls], 1.0};
   // (the eight-wave 256x256 kernel.  16-bit, M-contiguous operands and a rest of K, 44 problems of 256..8192 in three orders: the model's tile 1.013 times the
   // fastest one's time; 1.021 with 0.89 and 4 us more a tile, which kept the library's choice off this kernel: 7848x7808x528 86 us, 256x128 104)
-  if (cls == 0 && !w4) { f.eff *= half ? 0.97 : dt == TB_I8 && !streamk ? 0.91 : 0.86; f.tile_us += half ? 0.0 : 4.0; }
+  if (cls == 0 && !w4) { f.eff *= half ? 0.97 : dt == TB_I8 && !older ? 0.91 : 0.86; f.tile_us += half ? 0.0 : 4.0; }
   if (grouped) return f;
   if (cls == 1 && !half && dt != TB_I8) f.lat = 1.19;
   if (cls == 2 && tiles <= n_cu) f.lat = 0.825;
   if (cls == 3) f.lat = half ? 0.61 : 0.645;
-  if (cls == 4) f.lat = tiles <= 2 * (int64_t)n_cu ? 0.47 : tiles <= 3 * (int64_t)n_cu ? 0.85 : dt == TB_I8 && !streamk ? 0.8 : 1.0;
+  if (cls == 4) f.lat = tiles <= 2 * (int64_t)n_cu ? 0.47 : tiles <= 3 * (int64_t)n_cu ? 0.85 : dt == TB_I8 && !older ? 0.8 : 1.0;
   return f;
 }
 
@@ -255,7 +255,11 @@ static double score(const tb_problem& pr, const tb_hw& hw, const TileInfo& v, bo
     k_steps = whole_k & ~1ll;
     rest_us = 2.0 + 3.5 * (double)(k_iters - k_steps);
   }
-  const Family fam = family(pr.a_type, v, w4, cdiv(pr.m, v.bm) * cdiv(pr.n, v.bn), hw.n_cu, pr.num_groups > 0, streamk);
+  // (the figures of int8 and fp32 were fitted on launches of the whole device.  On 64 workgroups fp32 1664x480x5568 takes 418 us by the older ones, in 64x64 tiles, 563 by these in
+  // 32x32, which are ahead there only where all of them run at once: 256x512x2048 on 128 42 and 20.  int8 640x1024x3072 on 32 CUs 16.8 us in 128x128, 24.6 in 256x128.)
+  const bool kept = part || use.workgroups > 0;
+  const bool at_once = pr.a_type == TB_F32 && cdiv(pr.m, 32) * cdiv(pr.n, 32) <= workgroups_of(v, hw, use);
+  const Family fam = family(pr.a_type, v, w4, cdiv(pr.m, v.bm) * cdiv(pr.n, v.bn), hw.n_cu, pr.num_groups > 0, streamk || (kept && !at_once));
   const double t_thru = ideal_step_us / fam.eff;   // CU time per tile K step, saturated
   const double t_lat = (0.30 + (v.bm + v.bn) * (v.bk * esz) / 1.0e5) * fam.lat;   // floor per K step of one workgroup
   const double t_tile = fam.tile_us + rest_us;
