@@ -438,12 +438,28 @@ __device__ __forceinline__ void epilogue_w4_owner(const GemmParams& p, const Til
 static __device__ unsigned long long w4_lab_ts[1024 * 32];
 #endif
 
+// A pointer to global memory as a value that the compiler knows no origin of.  (Through its address space: a generic one would be accessed by flat instructions,
+// which count as LDS accesses too, and out of order; the K loops count theirs.)
+template <class X>
+__device__ __forceinline__ void own_value(X*& q) {
+  __attribute__((address_space(1))) X* g;
+  asm("s_mov_b64 %0, %1" : "=s"(g) : "s"((__attribute__((address_space(1))) X*)q));
+  q = (X*)g;
+}
+
 // SK: the schedule may end in a Stream-K tail (pieces of a tile's K range, cut at multiples of four K steps:
 // GemmParams::sk_unit = 4), with the partial-tile exchange of gemm_kernel<T, true>.
 // REST: K is more than the K loop's steps (GemmParams::k_rest).  A kernel of its own: the code between two K loop statements is fetched anew for every tile,
 // and the rest's cost all others 0.3 to 0.5 % (8192x28672x8192 FP8 1203 -> 1206 us with its code behind the loop, 1214 -> 1220 in between).
 template <class T, bool SK = false, bool REST = false>
-__global__ __launch_bounds__(256, 1) void gemm_kernel_w4(const GemmParams p) {
+__global__ __launch_bounds__(256, 1) void gemm_kernel_w4(const GemmParams args) {
+  GemmParams p = args;
+  // The eight pointers at the head of the parameters may be loaded as one tuple of 16 registers.  MXFP4, which spills the most, spilled that tuple, and each of 217 uses of a
+  // pointer in the stores of tiles that end inside C brought all 16 back: 5260 v_readlane in the kernel, 1470 where each pointer is a value of its own.
+  // 1425x8992x9216, one tile to a workgroup and the last ones ending there, 73.0 us and 70.2; 3000x7000x8192 125 and 122.  (The other types have 1390 to 2720 either way.)
+  if constexpr (T::DT == DT_FP4) {
+    own_value(p.A); own_value(p.B); own_value(p.C); own_value(p.sa); own_value(p.sb); own_value(p.bias); own_value(p.mxa); own_value(p.mxb);
+  }
   static_assert(T::BM == 256 && T::BN == 256 && T::BKB == 128 && T::WM == 2 && T::WN == 2 && T::STAGES == 2, "fixed shape");
   static_assert(is_f8(T::DT) || T::DT == DT_FP4 || T::DT == DT_BF16 || T::DT == DT_F16 || T::DT == DT_I8, "element types with a generated K loop");
   static_assert((T::ALAY == LAY_K && T::BLAY == LAY_K) || (T::USZ == 2 && !SK), "M-contiguous operands: 16-bit types, whole tiles");
