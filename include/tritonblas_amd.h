@@ -249,6 +249,7 @@ typedef struct tb_gemm_fp4_desc {
 } tb_gemm_fp4_desc;
 
 int tb_gemm_fp4(const tb_gemm_fp4_desc* desc, void* stream);
+int tb_gemm_fp4_launch_info(const tb_gemm_fp4_desc* desc, tb_launch_info* out);   /* as tb_gemm_launch_info */
 
 /* ---- grouped (MoE) FP8 GEMM — no counterpart in the reference -------------------------------- */
 typedef struct tb_grouped_gemm_desc {
@@ -268,7 +269,10 @@ typedef struct tb_grouped_gemm_desc {
   int32_t group_m, num_xcds;
   int32_t small_rows;         /* > 0: an expert's last, partial row block of at most this many rows is
                                  left to a second launch with a short (32-row) tile instead of costing
-                                 a whole tall tile per column block.  0 and -1: one launch.
+                                 a whole tall tile per column block.  -1: one launch.  0: one launch, too, but
+                                 with streamk, no tile named, a long K and a table that last blocks of up to 64
+                                 rows may take past its first or second round: the kernels price both plans from
+                                 the row counts on the device and split where that is cheaper.
                                  The split needs k % 256 == 0 and a tall (>= 128-row) tile.            */
   int32_t streamk;            /* 1: the tiles that do not fill whole rounds of the grid are cut into K ranges
                                  (Stream-K, as kernels/streamk_gemm.py:160-384 does for one matrix) whenever the
@@ -283,6 +287,9 @@ typedef struct tb_grouped_gemm_desc {
 } tb_grouped_gemm_desc;
 
 int tb_grouped_gemm_fp8(const tb_grouped_gemm_desc* desc, void* stream);
+/* As tb_gemm_launch_info, for the one or two launches of a grouped call (launches: two of them; the second stays zero where there is none).  total_tiles is the most
+ * entries that the tile table can have; the row counts are only known on the device. */
+int tb_grouped_launch_info(const tb_grouped_gemm_desc* desc, tb_launch_info* launches);
 /* Workspace a streamk = 1 call with this descriptor needs (0: none, the launch runs whole tiles only). */
 size_t tb_grouped_workspace_bytes(const tb_grouped_gemm_desc* desc);
 /* Host-side evaluation of the rule the grouped kernel applies on the device: of a table of total_tiles tiles

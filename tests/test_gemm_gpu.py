@@ -942,8 +942,7 @@ def test_grouped_streamk_tail(counts, grid, fix, tb_option):
 
 
 def test_grouped_streamk_default_two_launch_plan(tb_option):
-    """Default plan (the device chooses between one and two launches) with the Stream-K tail on (the workspace is the
-    package's per-stream one): oracle values in every row."""
+    """No tile named, with the Stream-K tail on (the workspace is the package's per-stream one): oracle values in every row."""
     import tritonblas_amd as tb
     _say("grouped streamk tail, default plan")
     tb_option("grid", 6)
@@ -954,6 +953,27 @@ def test_grouped_streamk_default_two_launch_plan(tb_option):
     for _ in range(2):
         tb.grouped_matmul_a8w8(aq.cuda(), wq.cuda(), sa.cuda(), sw.cuda(), c, offsets.cuda(), enable_streamk=True)
     _check(c.cpu(), OG.ref_grouped_gemm_fp8(aq, wq, sa, sw, offsets, return_fp32=True), torch.bfloat16, TOL_Q)
+
+
+@pytest.mark.parametrize("counts,split", [([520, 1040, 514, 0], True), ([700, 700, 700, 0], False), ([2071, 1, 1, 1], True)])
+def test_grouped_streamk_verdict(counts, split, tb_option):
+    """A Stream-K call whose short row blocks take the table past its first round on 16 workgroups, by row counts for which they are left to a second launch and for which they
+    are not (the oracle's verdict): the oracle's values in every row, in the workspace of an earlier call and in one of its own."""
+    import tritonblas_amd as tb
+    from oracle import schedule as S
+    from tritonblas_amd.config import MatmulConfig
+    _say(f"grouped streamk verdict counts={counts}")
+    n, k = 512, 6144
+    tb_option("grid", 16)
+    offsets, aq, wq, sa, sw = _grouped_problem(counts, n, k, 27)
+    assert S.grouped_split_pays(offsets.tolist(), 256, 64, 32, n // 256, n // 128, 16, 16) == split
+    want = OG.ref_grouped_gemm_fp8(aq, wq, sa, sw, offsets, return_fp32=True)
+    config = MatmulConfig(device=torch.device("cuda"), workspace=None)
+    for cfg in (None, config, config):
+        c = torch.full((sum(counts), n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        tb.grouped_matmul_a8w8(aq.cuda(), wq.cuda(), sa.cuda(), sw.cuda(), c, offsets.cuda(), enable_streamk=True, config=cfg)
+        _check(c.cpu(), want, torch.bfloat16, TOL_Q)
+    assert config.status() == 0
 
 
 def test_results_with_a_further_dimension_of_one():

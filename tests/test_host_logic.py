@@ -896,6 +896,45 @@ def test_fp32_and_int8_tiles_of_launches_kept_to_some_workgroups():
     assert (sel.block_m, sel.block_n) == (128, 128)
 
 
+def _grouped_job(rows, experts, n, k, **fields):
+    from tritonblas_amd import _lib
+    g = _lib.tb_grouped_gemm_desc()
+    g.struct_bytes, g.c_type = C.sizeof(_lib.tb_grouped_gemm_desc), _lib.TB_BF16
+    g.m_total, g.n, g.k, g.num_groups = rows, n, k, experts
+    g.a_stride_m, g.w_stride_g, g.w_stride_n, g.c_stride_m, g.c_stride_n = k, n * k, k, n, 1
+    for name, value in fields.items():
+        setattr(g, name, value)
+    return g
+
+
+def _grouped_launches(*args, tile=None, **fields):
+    from tritonblas_amd import _lib
+    if tile:
+        fields.update(block_m=tile[0], block_n=tile[1], block_k=tile[2])
+    launches = (_lib.tb_launch_info * 2)()
+    assert _lib.load().tb_grouped_launch_info(_grouped_job(*args, **fields), launches) == _lib.TB_OK
+    return launches
+
+
+def test_which_grouped_calls_plan_two_launches():
+    """A verdict on the device about a second launch is for calls with a Stream-K tail (the 256x256 hand-scheduled kernel on K in blocks of four steps) whose short row
+    blocks may take the table past its first or second round."""
+    two_by_verdict = [(4096, 8, 4096, 14336), (4096, 4, 4096, 6144), (8192, 8, 4096, 8192)]
+    for case in two_by_verdict:
+        first, second = _grouped_launches(*case, streamk=1)
+        assert (first.block_m, first.block_n, first.four_wave) == (256, 256, 1) and (second.block_m, second.block_n, second.block_k) == (32, 128, 256)
+    for rows, experts, n, k in [(8192, 8, 14336, 4096), (4096, 8, 4096, 14336), (1000, 4, 1536, 7168), (1024, 16, 4096, 2048), (8192, 8, 14336, 4096 + 256)]:
+        for small in (-1, 0):
+            assert _grouped_launches(rows, experts, n, k, small_rows=small)[1].total_tiles == 0
+        assert _grouped_launches(rows, experts, n, k, streamk=1, small_rows=-1)[1].total_tiles == 0
+        assert (_grouped_launches(rows, experts, n, k, streamk=1)[1].total_tiles > 0) == ((rows, experts, n, k) in two_by_verdict)
+        assert _grouped_launches(rows, experts, n, k, streamk=1, tile=(256, 256, 128))[1].total_tiles == 0       # (a tile that the caller names)
+        assert _grouped_launches(rows, experts, n, k, small_rows=40, tile=(256, 256, 128))[1].total_tiles > 0
+    # a short K; no tail; no round that short blocks could end; rounds enough to share one more among
+    for case in [(4096, 8, 4096, 4096), (4096, 8, 4096, 14336 + 128), (6144, 8, 4096, 14336), (2048, 8, 4096, 14336), (16384, 8, 4096, 14336)]:
+        assert _grouped_launches(*case, streamk=1)[1].total_tiles == 0
+
+
 def test_tiles_of_the_register_loading_kernels():
     """Rows off 16 bytes run in 128x128 or 64x64 tiles: 128 where the chosen tile has it on both sides, and where fp32 fills the CUs with them once."""
     from tritonblas_amd import _lib

@@ -31,7 +31,7 @@ EXPORTED_SYMBOLS = [
     "tb_column_sum",
     "tb_column_sum_bytes",
     "tb_tile_coords", "tb_default_panel", "tb_ws_queue_tile", "tb_hierarchical_split",
-    "tb_workspace_layout", "tb_debug_option", "tb_gemm_static_workspace", "tb_static_workspace_status", "tb_gemm_launch_info", "tb_gemm_split_info",
+    "tb_workspace_layout", "tb_debug_option", "tb_gemm_static_workspace", "tb_static_workspace_status", "tb_gemm_launch_info", "tb_gemm_split_info", "tb_grouped_launch_info", "tb_gemm_fp4_launch_info",
 ]
 
 
@@ -163,6 +163,8 @@ def load():
     lib.tb_grouped_gemm_fp8.argtypes = [C.POINTER(tb_grouped_gemm_desc), C.c_void_p]
     lib.tb_grouped_workspace_bytes.argtypes = [C.POINTER(tb_grouped_gemm_desc)]
     lib.tb_grouped_workspace_bytes.restype = C.c_size_t
+    lib.tb_gemm_fp4_launch_info.argtypes = [C.POINTER(tb_gemm_fp4_desc), C.POINTER(tb_launch_info)]
+    lib.tb_grouped_launch_info.argtypes = [C.POINTER(tb_grouped_gemm_desc), C.POINTER(tb_launch_info)]
     lib.tb_streamk_tail_tiles.argtypes = [C.c_int32] * 5
     lib.tb_hadamard_mxfp4_quant.argtypes = [C.POINTER(tb_quant_desc), C.c_void_p]
     lib.tb_quantize_rows.argtypes = [C.POINTER(tb_row_quant_desc), C.c_void_p]

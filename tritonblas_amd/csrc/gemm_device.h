@@ -100,7 +100,12 @@ struct GemmParams {
   // grouped, two launches: phase 1 tiles every expert's rows with grp_big-row blocks but leaves a last
   // partial block of at most grp_thr rows to phase 2, which tiles just those rows with a short tile
   // (a handful of rows would otherwise cost a whole tall tile per column block).  Phase 0: one launch.
+  // With grp_auto (launches with a Stream-K tail) every workgroup of both launches first prices the two plans from the row counts
+  // (rounds of tall tiles cost 4, rounds of short tiles 3) and both launches act on the same verdict:
+  // either the first runs the one-launch table and the second does nothing, or they split the rows.
   int32_t grp_phase, grp_big, grp_thr;
+  int32_t grp_auto, grp_small_bm;
+  int32_t grp_other_tn, grp_other_grid;   // column tiles and grid of the other launch
   // grouped with a Stream-K tail (4-wave kernels): the tiles that do not fill whole rounds of the grid are cut into
   // K ranges as in MODE_SK; how many that is follows from the row counts, so every workgroup works it out
   // itself (sk_tail_tiles).  grp_sk_fix: what one extra piece of a tile costs its owner, in K steps.
@@ -1454,6 +1459,28 @@ __device__ __forceinline__ void plain_tile(const GemmParams& p, int tile, int BM
 }
 
 // Grouped table: experts in order, expert e owns (its row blocks in this phase) * tiles_n tiles, m-block fastest.
+// The phase that a launch with grp_auto runs: 0 one-launch table, 1 / 2 the split tables, -1 nothing.  Only kernels with a Stream-K tail know of it, and only where the host
+// sees a round that short blocks could end (make_plan): 8 experts of 4096x14336, 4096 rows, by the verdict and in one launch always, 260 us and 331 with 457 to 554 rows
+// each, 279 and 318 with 4089 and single rows; where it is one launch the empty second one costs 7 to 14.
+__device__ __forceinline__ int grouped_verdict(const GemmParams& p, int grid) {
+  int b0 = 0, b1 = 0, b2 = 0;
+  for (int e = 0; e < p.num_groups; ++e) {
+    const int rows = max(p.group_offsets[e + 1] - p.group_offsets[e], 0);
+    const int full = rows / p.grp_big, rem = rows - full * p.grp_big;
+    const bool small = rem > 0 && rem <= p.grp_thr;
+    b0 += full + (rem > 0 ? 1 : 0);
+    b1 += full + ((rem > 0 && !small) ? 1 : 0);
+    b2 += small ? (rem + p.grp_small_bm - 1) / p.grp_small_bm : 0;
+  }
+  const int tn_big = p.grp_phase == 1 ? p.tiles_n : p.grp_other_tn, tn_small = p.grp_phase == 1 ? p.grp_other_tn : p.tiles_n;
+  const int g_big = p.grp_phase == 1 ? grid : p.grp_other_grid, g_small = p.grp_phase == 1 ? p.grp_other_grid : grid;
+  const int64_t one = 4 * (((int64_t)b0 * tn_big + g_big - 1) / g_big);
+  const int64_t two = 4 * (((int64_t)b1 * tn_big + g_big - 1) / g_big) + 3 * (((int64_t)b2 * tn_small + g_small - 1) / g_small);
+  const bool split = b2 > 0 && two < one;
+  if (p.grp_phase == 1) return split ? 1 : 0;
+  return split ? 2 : -1;
+}
+
 // the row blocks of expert e in the table of a phase: their number, the first row and the row limit
 __device__ __forceinline__ int grouped_rows(const GemmParams& p, int phase, int e, int BM, int& base, int& lim) {
   const int lo = p.group_offsets[e], hi = p.group_offsets[e + 1];
@@ -1536,12 +1563,15 @@ struct Sched {
   int step;               // work stealing: queue visit index
   int64_t start, last, q, rem;  // Stream-K iteration range of this workgroup
   int dp_tiles;
+  int gphase;             // grouped: which tile table this launch runs
   int gtotal;             // grouped with a Stream-K tail: entries of that table
   bool ws_phase;          // Stream-K with work stealing: still drawing whole tiles from the queues
 
   __device__ __forceinline__ void init(const GemmParams& p) {
     G = gridDim.x;
     gtotal = 0;
+    gphase = p.grp_phase;
+    if constexpr (SK) { if (p.mode == MODE_GROUPED && p.grp_auto) gphase = grouped_verdict(p, G); }
     pid = blockIdx.x;
     sk_id = blockIdx.x;
     if (p.mode != MODE_WS && p.num_xcds > 1) pid = chiplet_transform_chunked(pid, G, p.num_xcds, p.chunk);
@@ -1563,11 +1593,11 @@ struct Sched {
       last = (int64_t)dp_tiles * ipt + (sk_id + 1) * q + min((int64_t)sk_id + 1, rem);
     }
     if constexpr (SK) {
-      if (p.mode == MODE_GROUPED && p.grp_sk) {
+      if (p.mode == MODE_GROUPED && p.grp_sk && gphase >= 0) {
         // the table's real length is only known here; whole rounds first, the rest in K ranges (ordered as in MODE_SK)
         const int unit = max(1, p.sk_unit);
         const int64_t ipt = p.k_iters / unit;
-        gtotal = grouped_total(p, p.grp_phase, T::BM);
+        gtotal = grouped_total(p, gphase, T::BM);
         const int skt = sk_tail_tiles(gtotal, G, (int)ipt, unit, p.grp_sk_fix);
         dp_tiles = gtotal - skt;
         const int64_t total_sk = (int64_t)skt * ipt;
@@ -1644,13 +1674,13 @@ struct Sched {
       bool tail = false;
       if constexpr (SK) tail = p.grp_sk != 0;
       if (!tail) {
-        if (next_tile >= p.total_tiles) return false;
-        bool ok = grouped_tile(p, p.grp_phase, next_tile, T::BM, T::BN, T::USZ, w.tc);
+        if (gphase < 0 || next_tile >= p.total_tiles) return false;
+        bool ok = grouped_tile(p, gphase, next_tile, T::BM, T::BN, T::USZ, w.tc);
         next_tile = ok ? next_tile + G : p.total_tiles;
         return ok;
       }
       if (next_tile < dp_tiles) {
-        grouped_tile(p, p.grp_phase, next_tile, T::BM, T::BN, T::USZ, w.tc);
+        grouped_tile(p, gphase, next_tile, T::BM, T::BN, T::USZ, w.tc);
         next_tile += G;
         return true;
       }
@@ -1728,7 +1758,7 @@ struct Sched {
     const int64_t tile_first = (int64_t)tile * ipt;
     const int64_t tile_end = tile_first + ipt;
     const int64_t begin = max(tile_first, start);
-    if (grouped) grouped_tile(p, p.grp_phase, tile, T::BM, T::BN, T::USZ, w.tc);
+    if (grouped) grouped_tile(p, gphase, tile, T::BM, T::BN, T::USZ, w.tc);
     else plain_tile(p, tile, T::BM, T::BN, w.tc);
     w.it0 = (int)(begin - tile_first) * unit;
     w.it1 = (int)(last - tile_first) * unit;

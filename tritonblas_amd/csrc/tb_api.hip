@@ -263,7 +263,7 @@ struct Job {
   // grouped
   const int32_t* group_offsets = nullptr; int num_groups = 0;
   int64_t b_group_stride = 0, sb_group_stride = 0;
-  int grp_phase = 0, grp_big = 0, grp_thr = 0;   // see GemmParams
+  int grp_phase = 0, grp_big = 0, grp_thr = 0, grp_auto = 0;   // see GemmParams
   int grp_sk = 0;          // grouped: cut the tiles that do not fill whole rounds of the grid into K ranges (needs a workspace)
   int column_split = 0;
   int tiles_only = 0;      // 1: never the streaming kernel
@@ -559,11 +559,26 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
     // the tile table has at most this many entries (every expert may end in a partial row block);
     // a resident grid loops over it
     p.mode = MODE_GROUPED;
-    p.grp_phase = j.grp_phase; p.grp_big = j.grp_big; p.grp_thr = j.grp_thr;
+    // Stream-K tail: only the hand-scheduled 4-wave kernel has the cheap exchange of partial tiles that makes
+    // it pay (K ranges in blocks of four steps), and only the launch of the tall tiles
+    const bool tail = j.grp_sk && j.grp_phase != 2 && v->k_step_pairs && v->kernel_sk && p.k_rest == 0 && p.k_iters % 4 == 0 && p.k_iters >= 8 && occ == 1;
+    p.grp_phase = j.grp_phase; p.grp_big = j.grp_big; p.grp_thr = j.grp_thr; p.grp_auto = j.grp_auto;
     if (p.grp_phase == 1) {
       // only a tall fast tile leaves its short last blocks to a second launch
-      if (v->fast && v->bm >= 128 && j.grp_thr > 0 && j.grp_thr < v->bm) p.grp_big = v->bm;
-      else p.grp_phase = 0;
+      bool two = v->fast && v->bm >= 128 && j.grp_thr > 0 && j.grp_thr < v->bm;
+      if (j.grp_auto) {
+        // A verdict on the device, for launches with a tail, costs 7 to 14 us where it is one launch.  It can only be two where the short blocks may take the table past a round
+        // that the tall ones alone fit, and pays where that is the first or second and long.  Two launches by verdict and one always, us in all over even, halved, single-row and
+        // Zipf counts: 4 and 8 experts, 4096 rows, n 4096: K 14336 0.905 and 0.951, 6144 0.945 and 0.966, 4096 0.979 and 1.013; 8192 rows 0.97 to 1.01.
+        // Fewer rows to an expert: 2048 and 3072 rows of 8 1.02 to 1.07.  No such round: 6144 rows 1.04 to 1.09; seven and more: 8192 rows, n 14336 1.04 to 1.08.
+        const int64_t at_once = hooks().grid > 0 ? hooks().grid : resident;
+        const int64_t least = (std::max<int64_t>(0, j.M - (int64_t)j.grp_thr * j.num_groups) + v->bm - 1) / v->bm * p.tiles_n;
+        const int64_t most = std::min<int64_t>(j.M, (j.M + (int64_t)j.num_groups * (v->bm - 1)) / v->bm) * p.tiles_n;
+        const int64_t round = std::max<int64_t>(1, (least + at_once - 1) / at_once);
+        two = two && tail && j.K >= 6144 && j.M >= 512 * (int64_t)j.num_groups && round <= 2 && most > round * at_once;
+      }
+      if (two) p.grp_big = v->bm;
+      else p.grp_phase = p.grp_auto = 0;
     }
     if (p.grp_phase == 2 && (p.grp_big <= 0 || p.grp_thr <= 0)) return TB_ERR_BAD_ARGUMENT;
     const int64_t bound = p.grp_phase == 2
@@ -574,9 +589,7 @@ int make_plan(const Job& j, const tb_hw& hw, bool need_device, Plan* plan) {
     grid = (int)std::min<int64_t>(bound, resident);
     if (hooks().grid > 0) grid = (int)std::min<int64_t>(bound, hooks().grid);
     plan->one = p.grp_phase == 0 && hooks().grid <= 0 && group_kernel(*v) != nullptr;
-    // Stream-K tail: only the hand-scheduled 4-wave kernel has the cheap exchange of partial tiles that makes
-    // it pay (K ranges in blocks of four steps), and only the launch of the tall tiles
-    if (j.grp_sk && p.grp_phase != 2 && v->k_step_pairs && v->kernel_sk && p.k_rest == 0 && p.k_iters % 4 == 0 && p.k_iters >= 8 && occ == 1) {
+    if (tail) {
       p.grp_sk = 1;
       // (measured with 8 experts, 2072 tiles of 32 K steps on 256 workgroups: the launch that cuts 280 tiles
       // takes 63 us longer than 7 whole rounds and 35 K steps would -- every workgroup writes and reads a
@@ -714,7 +727,7 @@ PlanKey plan_key(const Job& j, int dev) {
       j.dt, j.c_type, j.bias_type, j.schedule, dev, j.M, j.N, j.K, j.a_sr, j.a_sk, j.b_sr, j.b_sk, j.c_sm, j.c_sn,
       j.mxa_sr, j.mxa_sk, j.mxb_sr, j.mxb_sk, j.bias_stride, j.bm, j.bn, j.bk, j.group_m, j.num_xcds, j.grid,
       j.counters_per_xcd, j.ws_mode, j.ws_local, j.cu_mask_len, j.ws_global, j.num_groups, j.grp_phase, j.grp_big,
-      j.grp_thr, j.grp_sk, j.b_group_stride, j.sb_group_stride, al(j.A), al(j.B), al(j.C), al(j.mxa), al(j.mxb),
+      j.grp_thr, j.grp_auto, j.grp_sk, j.b_group_stride, j.sb_group_stride, al(j.A), al(j.B), al(j.C), al(j.mxa), al(j.mxb),
       al(j.bias), j.sa ? 1 : 0, j.sb ? 1 : 0, j.cu_mask ? 1 : 0, j.group_offsets ? 1 : 0, j.column_split, j.retreat, j.tiles_only, j.only_bk, (int64_t)j.room,
       (int64_t)g_hooks_version};
   static_assert(sizeof(f) <= sizeof(k.v), "PlanKey too small");
@@ -829,7 +842,9 @@ int run_plan(const Job& j, Plan& plan, hipStream_t stream) {
     p.B -= v->blay == LAY_K ? step : step * j.b_sk;
   }
   void* args[] = {(void*)&p};
-  const void* kern = (p.mode == MODE_SK || p.grp_sk) ? plan.v->kernel_sk : p.k_rest ? w4_kernel_rest(j.dt) : !plan.one ? v->kernel : p.mode == MODE_GROUPED ? group_kernel(*v) : v->kernel_one;
+  const bool with_tail = p.mode == MODE_SK || p.grp_sk || p.grp_auto;
+  if (with_tail && p.epoch == EPOCH_ON_DEVICE && !p.ctl) return TB_ERR_WORKSPACE;      // (these kernels read the launch's count there)
+  const void* kern = with_tail ? plan.v->kernel_sk : p.k_rest ? w4_kernel_rest(j.dt) : !plan.one ? v->kernel : p.mode == MODE_GROUPED ? group_kernel(*v) : v->kernel_one;
   hipError_t e = hipLaunchKernel(kern, dim3((unsigned)plan.grid), dim3((unsigned)plan.v->threads), args, 0, stream);
   if (e != hipSuccess) { (void)hipGetLastError(); return TB_ERR_LAUNCH; }
   return TB_OK;
@@ -969,6 +984,29 @@ void init_scratch(int dev) {
   if (e != hipSuccess || !ptr) { (void)hipGetLastError(); g_scratch[dev].status = TB_ERR_NO_DEVICE; return; }
   g_scratch[dev].ptr = ptr;
   g_scratch[dev].status = TB_OK;
+}
+
+// the short FP8 tile the second launch of a grouped GEMM runs
+constexpr int kGroupedSmallBM = 32, kGroupedSmallBN = 128, kGroupedSmallBK = 256;
+
+// The plan of the first launch and, where *two stays true, that of the second.  make: job -> plan.
+template <class F>
+int plan_grouped(const Job& j, bool* two, F&& make, Job* j2, Plan* first, Plan* second) {
+  int st = make(j, first);
+  if (st != TB_OK) return st;
+  *two = *two && first->p.grp_phase == 1;
+  if (!*two) return TB_OK;
+  *j2 = j;
+  j2->bm = kGroupedSmallBM; j2->bn = kGroupedSmallBN; j2->bk = kGroupedSmallBK;
+  j2->grp_phase = 2; j2->grp_big = first->p.grp_big;
+  j2->grp_sk = 0; j2->workspace = nullptr; j2->workspace_bytes = 0;
+  j2->epoch = 0;       // (the kernel that knows of the verdict has a Stream-K tail, too, and would look for the launch's count in a workspace)
+  st = make(*j2, second);
+  if (st != TB_OK) return st;
+  first->p.grp_small_bm = second->p.grp_small_bm = second->v->bm;
+  first->p.grp_other_tn = second->p.tiles_n; first->p.grp_other_grid = second->grid;
+  second->p.grp_other_tn = first->p.tiles_n; second->p.grp_other_grid = first->grid;
+  return TB_OK;
 }
 
 int job_from_gemm(const tb_gemm_desc* d, Job* j) {
@@ -1227,10 +1265,9 @@ size_t tb_workspace_bytes(const tb_gemm_desc* desc) {
   return plan.ws_need;
 }
 
-int tb_gemm_fp4(const tb_gemm_fp4_desc* d, void* stream) {
+static int job_from_fp4(const tb_gemm_fp4_desc* d, Job* out) {
   if (!d) return TB_ERR_NULL_POINTER;
   if (d->struct_bytes != sizeof(tb_gemm_fp4_desc)) return TB_ERR_BAD_ARGUMENT;
-  if (!d->a || !d->b || !d->c || !d->a_scales || !d->b_scales) return TB_ERR_NULL_POINTER;
   if (d->k <= 0 || d->k % 32) return TB_ERR_BAD_SHAPE;
   Job j;
   j.dt = TB_FP4_E2M1; j.c_type = d->c_type;
@@ -1242,11 +1279,32 @@ int tb_gemm_fp4(const tb_gemm_fp4_desc* d, void* stream) {
   j.mxa_sr = d->a_scales_stride_m; j.mxa_sk = d->a_scales_stride_k;
   j.mxb_sr = d->b_scales_stride_n; j.mxb_sk = d->b_scales_stride_k;
   j.bm = d->block_m; j.bn = d->block_n; j.bk = d->block_k; j.group_m = d->group_m; j.num_xcds = d->num_xcds;
+  *out = j;
+  return TB_OK;
+}
+
+int tb_gemm_fp4(const tb_gemm_fp4_desc* d, void* stream) {
+  Job j;
+  const int st = job_from_fp4(d, &j);
+  if (d && d->struct_bytes == sizeof(tb_gemm_fp4_desc) && (!d->a || !d->b || !d->c || !d->a_scales || !d->b_scales)) return TB_ERR_NULL_POINTER;
+  if (st != TB_OK) return st;
   return launch(j, (hipStream_t)stream);
 }
 
-// the short FP8 tile the second launch of a grouped GEMM runs
-constexpr int kGroupedSmallBM = 32, kGroupedSmallBN = 128, kGroupedSmallBK = 256;
+int tb_gemm_fp4_launch_info(const tb_gemm_fp4_desc* d, tb_launch_info* out) {
+  if (!out) return TB_ERR_NULL_POINTER;
+  Job j;
+  int st = job_from_fp4(d, &j);
+  if (st != TB_OK) return st;
+  tb_hw hw;
+  const bool have_dev = current_hw(&hw) == TB_OK;
+  if (!have_dev) default_hw(&hw);
+  Plan plan;
+  st = make_plan(j, hw, have_dev, &plan);
+  if (st != TB_OK) return st;
+  fill_launch_info(plan, out);
+  return TB_OK;
+}
 
 // the job of the (first) launch; *two: a second launch with the short tile may follow
 static int job_from_grouped(const tb_grouped_gemm_desc* d, Job* out, bool* two) {
@@ -1272,10 +1330,12 @@ static int job_from_grouped(const tb_grouped_gemm_desc* d, Job* out, bool* two) 
     j.epoch = d->epoch; j.spin_limit = d->spin_limit;
   }
   // Two launches where asked for: tall tiles for whole row blocks and long remainders, then a short streaming tile for the experts whose last
-  // block holds few rows.  (Never by itself: a short tile costs 3/4 of a tall one and covers half its columns, and an empty second launch takes 7 us.)
+  // block holds few rows.  By itself only in front of a Stream-K tail, as the kernels find from the row counts (grouped_verdict): without one
+  // it was level at best with one launch of the right tile on even, skewed and single-row counts, and an empty second launch takes 7 us.
   if (d->small_rows < -1) return TB_ERR_BAD_ARGUMENT;
-  *two = d->small_rows > 0 && d->k % kGroupedSmallBK == 0;
-  if (*two) { j.grp_phase = 1; j.grp_thr = d->small_rows; }
+  const bool by_verdict = d->small_rows == 0 && d->block_m == 0 && d->streamk;
+  *two = (d->small_rows > 0 || by_verdict) && d->k % kGroupedSmallBK == 0;
+  if (*two) { j.grp_phase = 1; j.grp_thr = by_verdict ? 64 : d->small_rows; j.grp_auto = by_verdict; }
   *out = j;
   return TB_OK;
 }
@@ -1309,19 +1369,30 @@ int tb_grouped_gemm_fp8(const tb_grouped_gemm_desc* d, void* stream) {
   tb_hw hw;
   st = current_hw(&hw);
   if (st != TB_OK) return st;
+  Job j2;
   Plan first, second;
-  st = cached_plan(j, hw, &first);
-  if (st != TB_OK) return st;
-  if (first.p.grp_phase != 1) return run_plan(j, first, (hipStream_t)stream);
-  Job j2 = j;
-  j2.bm = kGroupedSmallBM; j2.bn = kGroupedSmallBN; j2.bk = kGroupedSmallBK;
-  j2.grp_phase = 2; j2.grp_big = first.p.grp_big;
-  j2.grp_sk = 0; j2.workspace = nullptr; j2.workspace_bytes = 0;
-  st = cached_plan(j2, hw, &second);
-  if (st != TB_OK) return st;
-  st = run_plan(j, first, (hipStream_t)stream);
-  if (st != TB_OK) return st;
+  st = plan_grouped(j, &two, [&](const Job& x, Plan* p) { return cached_plan(x, hw, p); }, &j2, &first, &second);
+  if (st == TB_OK) st = run_plan(j, first, (hipStream_t)stream);
+  if (st != TB_OK || !two) return st;
   return run_plan(j2, second, (hipStream_t)stream);
+}
+
+int tb_grouped_launch_info(const tb_grouped_gemm_desc* d, tb_launch_info* launches) {
+  if (!launches) return TB_ERR_NULL_POINTER;
+  Job j, j2;
+  bool two = false;
+  int st = job_from_grouped(d, &j, &two);
+  if (st != TB_OK) return st;
+  tb_hw hw;
+  const bool have_dev = current_hw(&hw) == TB_OK;
+  if (!have_dev) default_hw(&hw);
+  Plan first, second;
+  st = plan_grouped(j, &two, [&](const Job& x, Plan* p) { return make_plan(x, hw, have_dev, p); }, &j2, &first, &second);
+  if (st != TB_OK) return st;
+  std::memset(launches, 0, 2 * sizeof(*launches));
+  fill_launch_info(first, launches);
+  if (two) fill_launch_info(second, launches + 1);
+  return TB_OK;
 }
 
 int tb_hadamard_mxfp4_quant(const tb_quant_desc* d, void* stream) {

@@ -528,7 +528,8 @@ def grouped_matmul_a8w8(a, w, a_scale, w_scale, c, group_offsets, block_m: int =
     weight ``w[e]`` (N, K); ``c[rows] = cast((a[rows] @ w[e].T) * a_scale[rows, None] * w_scale[e][None, :])``.
     ``group_offsets`` is an int32 device tensor of E+1 ascending row offsets.  No host sync: the row counts
     are only read on the device, and the tile is sized by what the average expert has of them.  ``small_rows`` > 0: an expert's last partial
-    row block of at most that many rows goes to a second launch with a 32-row tile (0 and -1: one launch).
+    row block of at most that many rows goes to a second launch with a 32-row tile (-1: one launch; 0: one launch, with ``enable_streamk`` and no tile
+    named as many as are cheaper by the row counts, decided on the device).
     ``enable_streamk``: the tiles that do not fill whole rounds of the launch grid are cut into K ranges when the
     row counts make that cheaper than one more round (decided on the device; only those tiles' summation order
     changes).  The flags and partial tiles live in ``config``'s workspace, by default the one this package keeps
