@@ -935,6 +935,93 @@ def test_which_grouped_calls_plan_two_launches():
         assert _grouped_launches(*case, streamk=1)[1].total_tiles == 0
 
 
+GROUPED_VARIANTS = [((256, 128, 128), 423), ((128, 128, 128), 222), ((128, 128, 128), 424), ((128, 64, 128), 424), ((64, 64, 128), 222), ((64, 64, 128), 223),
+                    ((64, 64, 128), 224), ((32, 128, 256), 143)]
+
+
+def test_grouped_kernels_of_one_tile_to_a_workgroup(tb_option):
+    """Each variant that the cost model knows, but for 256x256, has the kernel of one table entry to a workgroup, and every table fits the grid: a launch has as many
+    workgroups as its table can have entries, over experts without rows and more of them than a wave has lanes."""
+    import random
+    from oracle import schedule as S
+    rng = random.Random(11)
+    for tile, waves in GROUPED_VARIANTS:
+        tb_option("waves", waves)
+        for experts in (1, 7, 64, 65, 200):
+            for _ in range(4):
+                counts = [rng.choice([0, 1, rng.randint(1, tile[0]), tile[0] - 1, tile[0], tile[0] + 1, rng.randint(1, 2000)]) for _ in range(experts)]
+                counts[rng.randrange(experts)] += 1
+                info = _grouped_launches(sum(counts), experts, 520, 512, tile=tile)[0]
+                assert (info.block_m, info.block_n) == tile[:2] and info.waves == (waves // 100) * (waves // 10 % 10)
+                table = sum(-(-c // tile[0]) for c in counts) * -(-520 // tile[1])
+                assert info.grid == info.total_tiles >= table, (tile, waves, experts)
+                offsets = [0]
+                for c in counts:
+                    offsets.append(offsets[-1] + c)
+                assert S.grouped_tile_lookup(table - 1, offsets, tile[0], -(-520 // tile[1])) is not None
+                assert S.grouped_tile_lookup(table, offsets, tile[0], -(-520 // tile[1])) is None
+        # the most entries: one row above a whole block for every expert
+        rows = 65 * (tile[0] + 1)
+        assert _grouped_launches(rows, 65, 520, 512, tile=tile)[0].total_tiles == 65 * 2 * -(-520 // tile[1])
+    tb_option("waves", 0)
+    info = _grouped_launches(8192, 8, 14336, 4096, tile=(256, 256, 128))[0]
+    assert info.four_wave == 1 and info.grid == 256 < info.total_tiles
+
+
+@pytest.mark.parametrize("rows,experts,n,k,want", [(8192, 8, 14336, 4096, (256, 256)), (4096, 16, 4096, 2048, (256, 128)), (1024, 8, 14336, 4096, (128, 128)),
+                                                   (1000, 4, 1536, 7168, (128, 64)), (64, 8, 14336, 4096, (64, 64)), (3000, 4, 1536, 7168, (256, 128))])
+def test_the_grouped_models_choice(rows, experts, n, k, want):
+    info = _grouped_launches(rows, experts, n, k)[0]
+    assert (info.block_m, info.block_n) == want
+
+
+@pytest.mark.parametrize("a_type", ["TB_BF16", "TB_F16", "TB_F32", "TB_FP8_E4M3", "TB_FP8_E5M2", "TB_I8"])
+def test_persistent_launches_have_a_workgroup_to_a_tile(a_type):
+    """... whatever the tile, with fewer tiles than the device holds and with more, but for the hand-scheduled kernels; a launch that names a grid loops."""
+    from tritonblas_amd import _lib
+    code = getattr(_lib, a_type)
+    c_type = _lib.TB_F32 if a_type == "TB_F32" else None
+    buf = (C.c_int32 * 60)()
+    for i in range(_lib.load().tb_list_tiles(code, buf, 20)):
+        tile = tuple(buf[3 * i:3 * i + 3])
+        for m, n in [(40, 520), (300, 700), (9000, 9000)]:
+            info = _launch_of(_job(code, m, n, 2 * tile[2], c_type=c_type, tile=tile, column_split=-1))
+            assert info.skinny == 1 or (info.block_m, info.block_n) == tile[:2]
+            assert info.skinny == 1 or info.four_wave == 1 or info.grid == info.total_tiles
+            info = _launch_of(_job(code, m, n, 2 * tile[2], grid=3, c_type=c_type, tile=tile))
+            assert info.skinny == 1 or info.grid == min(3, info.total_tiles)
+
+
+@pytest.mark.parametrize("a_type", ["TB_BF16", "TB_F16", "TB_FP8_E4M3", "TB_I8"])
+def test_which_problems_of_few_tiles_take_small_ones(a_type):
+    """Both sides of the lines: few rows against many columns are the streaming kernel's or a taller tile's."""
+    from tritonblas_amd import _lib
+    for m, n, k, small in [(65, 1024, 256, True), (64, 1024, 512, False), (64, 1000, 528, True), (33, 40, 4096, True), (200, 1000, 2000, True), (256, 256, 7904, True), (31, 33, 272, True),
+                           (1, 1000, 1040, True), (64, 4096, 4096, False), (2048, 2048, 2048, False)]:
+        info = _launch_of(_job(getattr(_lib, a_type), m, n, k))
+        assert (info.block_n == 32) == small, (m, n, k, info.block_m, info.block_n)
+    # Stream-K launches have none
+    assert _launch_of(_job(getattr(_lib, a_type), 256, 256, 7904, _lib.TB_SCHED_STREAMK)).block_n > 32
+
+
+def test_few_even_k_steps_of_mxfp4():
+    """The lines of MXFP4 for the two kernels of the 256x256 tile: 24 K steps of 256 values in one round, 16 in two, none beyond."""
+    from tritonblas_amd import _lib
+    for m, n, start in [(4096, 4096, 24), (7860, 1552, 24), (4096, 8192, 16), (4096, 8448, 4)]:
+        for steps in range(4, 30, 2):
+            g = _lib.tb_gemm_fp4_desc()
+            g.struct_bytes, g.c_type = C.sizeof(_lib.tb_gemm_fp4_desc), _lib.TB_BF16
+            g.m, g.n, g.k = m, n, steps * 256
+            g.a_stride_m = g.b_stride_n = g.k // 2
+            g.c_stride_m, g.c_stride_n = n, 1
+            g.a_scales_stride_m = g.b_scales_stride_n = g.k // 32
+            g.a_scales_stride_k = g.b_scales_stride_k = 1
+            g.block_m, g.block_n, g.block_k = 256, 256, 256
+            info = _lib.tb_launch_info()
+            assert _lib.load().tb_gemm_fp4_launch_info(g, info) == _lib.TB_OK
+            assert (info.four_wave == 1) == (steps >= start) and info.waves == (4 if info.four_wave else 8), (m, n, steps)
+
+
 def test_tiles_of_the_register_loading_kernels():
     """Rows off 16 bytes run in 128x128 or 64x64 tiles: 128 where the chosen tile has it on both sides, and where fp32 fills the CUs with them once."""
     from tritonblas_amd import _lib
