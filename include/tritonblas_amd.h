@@ -203,7 +203,8 @@ int tb_gemm_static_workspace(const tb_gemm_desc* desc, void* stream);
 /* What a tb_gemm call with this descriptor would launch (nothing is launched): the tile, the kernel family
  * (waves per workgroup; four_wave: the hand-scheduled 256x256 kernel), the grid, how many tiles form the Stream-K
  * tail and in units of how many K steps their ranges are cut, whether the whole tiles come from the work-stealing
- * queues, whether the small-M streaming kernel runs instead of a tile kernel.  Without a workspace in the
+ * queues, whether the small-M streaming kernel runs instead of a tile kernel.  (A Stream-K call that shares no tile runs as the
+ * persistent call of its tile, which tb_gemm_split_info knows.)  Without a workspace in the
  * descriptor: what runs with one of tb_workspace_bytes() bytes.  For tests and for callers that log
  * their launches; no counterpart in the reference (its launchers print the same facts when asked to be verbose). */
 typedef struct tb_launch_info {
@@ -211,7 +212,7 @@ typedef struct tb_launch_info {
 } tb_launch_info;
 int tb_gemm_launch_info(const tb_gemm_desc* desc, tb_launch_info* out);
 
-/* The same for a persistent call, which may run as two launches (column_split): the columns that the first one computes, all of them where it is the only one,
+/* The same for a persistent call, or a Stream-K call that shares no tile and is run as one, which may be two launches (column_split): the columns that the first one computes, all of them where it is the only one,
  * and what both launch (launches: two of them; the second stays zero where there is none). */
 int tb_gemm_split_info(const tb_gemm_desc* desc, int64_t* first_columns, tb_launch_info* launches);
 

@@ -1022,6 +1022,18 @@ def test_few_even_k_steps_of_mxfp4():
             assert (info.four_wave == 1) == (steps >= start) and info.waves == (4 if info.four_wave else 8), (m, n, steps)
 
 
+@pytest.mark.parametrize("a_type,m,n,k", [("TB_BF16", 1024, 1024, 1024), ("TB_BF16", 2048, 2048, 2048), ("TB_FP8_E4M3", 4096, 4096, 1024)])
+def test_stream_k_calls_that_share_no_tile_run_as_persistent_ones(a_type, m, n, k):
+    """... of the tile that they have, by a workgroup to a tile where it has that kernel, and by the same line for few even K steps."""
+    from tritonblas_amd import _lib
+    code = getattr(_lib, a_type)
+    plan = _launch_of(_job(code, m, n, k, _lib.TB_SCHED_STREAMK))
+    assert plan.mode == 0
+    first, (a, b) = _split_of(_job(code, m, n, k, _lib.TB_SCHED_STREAMK))
+    own = _launch_of(_job(code, m, n, k, tile=(plan.block_m, plan.block_n, plan.block_k)))
+    assert first == n and (a.block_m, a.block_n, a.waves, a.four_wave, a.grid) == (own.block_m, own.block_n, own.waves, own.four_wave, own.total_tiles) and b.total_tiles == 0
+
+
 def test_tiles_of_the_register_loading_kernels():
     """Rows off 16 bytes run in 128x128 or 64x64 tiles: 128 where the chosen tile has it on both sides, and where fp32 fills the CUs with them once."""
     from tritonblas_amd import _lib

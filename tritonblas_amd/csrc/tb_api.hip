@@ -889,6 +889,19 @@ int64_t column_split_point(const Job& j, const tb_hw& hw, const Plan& whole) {
   return n1;
 }
 
+// A Stream-K launch whose plan shares no tile runs whole tiles on the whole-tile kernel; it is then the
+// persistent launch of the same tile, partial last round and all, and is treated as one.
+bool may_be_persistent(const Job& j) { return j.schedule == TB_SCHED_STREAMK && j.column_split == 0 && j.num_groups == 0 && !hooks().no_column_split; }
+Job persistent_job(const Job& j, const tb_hw& hw, const Plan& plan) {
+  Job whole = j;
+  whole.schedule = TB_SCHED_PERSISTENT;
+  whole.grid = whole_tile_grid(j, hw, plan, plan.grid);
+  whole.tiles_only = plan.kept;
+  whole.bm = plan.v->bm; whole.bn = plan.v->bn; whole.bk = plan.v->bk;
+  whole.workspace = nullptr; whole.workspace_bytes = 0;
+  return whole;
+}
+
 // The two launches of a split behind column n1, and whether it is one: the first runs the tile of the whole, by the same kernel or, where K is whole pairs of K
 // steps, by the other one of the 256x256 tile.  (Which of the two is ahead goes by the number of tiles and the first launch has fewer: bf16 1280x13312x1024, 260 tiles by
 // hand-scheduled kernel or 255 by eight waves.  Both add up whole K steps in the same order.)  The second takes a tile of the same K step: one of another groups the products of a
@@ -911,9 +924,7 @@ bool split_plans(const Job& j, const Plan& whole, int64_t n1, F&& make, Job* a, 
 }
 
 int launch_columns(const Job& j, hipStream_t stream) {
-  if (j.schedule == TB_SCHED_STREAMK && j.column_split == 0 && j.num_groups == 0 && !hooks().no_column_split) {
-    // A Stream-K launch whose plan shares no tile runs whole tiles on the whole-tile kernel; it is then the
-    // persistent launch of the same tile, partial last round and all, and is treated as one.
+  if (may_be_persistent(j)) {
     tb_hw hw;
     int st = current_hw(&hw);
     if (st != TB_OK) return st;
@@ -921,13 +932,7 @@ int launch_columns(const Job& j, hipStream_t stream) {
     st = launch_plan(j, hw, &plan);
     if (st != TB_OK) return st;
     if (plan.skinny || plan.p.mode != MODE_STATIC) return run_plan(j, plan, stream);
-    Job whole = j;
-    whole.schedule = TB_SCHED_PERSISTENT;
-    whole.grid = whole_tile_grid(j, hw, plan, plan.grid);
-    whole.tiles_only = plan.kept;
-    whole.bm = plan.v->bm; whole.bn = plan.v->bn; whole.bk = plan.v->bk;
-    whole.workspace = nullptr; whole.workspace_bytes = 0;
-    return launch_columns(whole, stream);
+    return launch_columns(persistent_job(j, hw, plan), stream);
   }
   if (!may_split(j)) return launch(j, stream);
   tb_hw hw;
@@ -1238,7 +1243,11 @@ int tb_gemm_split_info(const tb_gemm_desc* desc, int64_t* first_columns, tb_laun
   if (!have_dev) default_hw(&hw);
   auto make = [&](const Job& x, Plan* p) { return make_plan(x, hw, have_dev, p); };
   Plan whole, pa, pb;
-  st = make(j, &whole);
+  st = j.workspace ? fitting_plan(j, make, &whole) : make(j, &whole);
+  if (st == TB_OK && may_be_persistent(j) && !whole.skinny && whole.p.mode == MODE_STATIC) {
+    j = persistent_job(j, hw, whole);
+    st = make(j, &whole);
+  }
   if (st != TB_OK) return st;
   *first_columns = j.N;
   std::memset(launches, 0, 2 * sizeof(*launches));
