@@ -160,7 +160,7 @@ def grouped_two_launch_blocks(offsets, phase, big_m, small_rows, block_m):
 
 
 def grouped_split_pays(offsets, big_m, small_rows, small_m, tiles_n_big, tiles_n_small, grid_big, grid_small):
-    """The verdict both launches of a grouped GEMM reach on the device from the row counts: split when
+    """The verdict both launches of a grouped GEMM with a Stream-K tail, where the host plans two, reach on the device from the row counts: split when
     4 * rounds(tall tiles of the split plan) + 3 * rounds(short tiles) < 4 * rounds(tall tiles of the
     one-launch plan) and there is a short block at all (a round of short tiles streams half a tall
     round's weight bytes but is bound by that stream: measured at three quarters of a tall round).

@@ -135,7 +135,7 @@ def _grouped_cases(n, seed):
     for i in range(n):
         experts = rng.randint(1, 9)
         counts = [rng.choice([0, 1, rng.randint(1, 70), rng.randint(100, 600), 256, 257]) for _ in range(experts)]
-        # plan: the library's own (0: one or two launches, priced on the device), one launch (-1), or the
+        # plan: the library's own (0), one launch (-1), or the
         # tall tile forced and last row blocks of at most that many rows left to the second launch
         out.append(dict(idx=i, counts=counts, n=rng.choice([64, 200, 384, 1000]), k=rng.choice([128, 512, 1152, 1024]),
                         seed=rng.randint(0, 1 << 30), small_rows=rng.choice([0, 0, -1, 16, 32, 64, 100, 200])))

@@ -102,6 +102,20 @@ def test_few_tiles(m, n, k, kind):
         assert ((got.double() - want).abs() <= REL[kind] * want.abs()).all(), tile       # (whole numbers below 2**24: the sums are exact)
 
 
+@pytest.mark.parametrize("kind", ["bf16", "f16", "fp8"])
+@pytest.mark.parametrize("k", [640, 1152, 1200, 2432])
+def test_order_of_k_in_small_tiles(kind, k):
+    """Values that fp32 sums round.  The remainder of K is added first, and tiles whose K steps are twice as long have another one where it holds half a step: each tile
+    adds up K in an order of its own, and all are within the rounding of k fp32 sums (2**-24 each of at most the sum of the magnitudes) of the product in 64 bits."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    a, b = (torch.randn(s, device="cuda", generator=g).to(TYPES[kind]) for s in ((200, k), (1000, k)))
+    want, size = a.double() @ b.double().T, a.double().abs() @ b.double().abs().T
+    unit = 64 if kind in ("bf16", "f16") else 128
+    for tile in ((0, 0, 0), (32, 32, 2 * unit), (64, 32, 2 * unit), (32, 128, 2 * unit), (64, 64, unit)):
+        got = _product(a, b.T, torch.full((200, 1000), float("nan"), device="cuda"), tile, 0)
+        assert ((got.double() - want).abs() <= k * 2.0 ** -24 * size).all(), tile
+
+
 @pytest.mark.parametrize("kind", ["bf16", "f16", "fp8", "i8"])
 @pytest.mark.parametrize("m,n,k", [(33, 40, 4096), (200, 1000, 2000), (256, 256, 7904), (31, 33, 272), (353, 1264, 1552)])
 def test_small_tiles_under_the_other_schedules(m, n, k, kind):

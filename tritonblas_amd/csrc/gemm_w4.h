@@ -455,7 +455,7 @@ template <class T, bool SK = false, bool REST = false>
 __global__ __launch_bounds__(256, 1) void gemm_kernel_w4(const GemmParams args) {
   GemmParams p = args;
   // The eight pointers at the head of the parameters may be loaded as one tuple of 16 registers.  MXFP4, which spills the most, spilled that tuple, and each of 217 uses of a
-  // pointer in the stores of tiles that end inside C brought all 16 back: 5260 v_readlane in the kernel, 1470 where each pointer is a value of its own.
+  // pointer in the stores of tiles that end inside C brought all 16 back: 5260 v_readlane in the kernel, 1500 where each pointer is a value of its own.
   // 1425x8992x9216, one tile to a workgroup and the last ones ending there, 73.0 us and 70.2; 3000x7000x8192 125 and 122.  (The other types have 1390 to 2720 either way.)
   if constexpr (T::DT == DT_FP4) {
     own_value(p.A); own_value(p.B); own_value(p.C); own_value(p.sa); own_value(p.sb); own_value(p.bias); own_value(p.mxa); own_value(p.mxb);
