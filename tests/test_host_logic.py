@@ -852,7 +852,7 @@ def test_small_tiles_are_for_cus_that_would_be_idle(dtype, m, n, k):
     and one that draws its tiles from the work-stealing queues takes 64x32 alone."""
     import tritonblas_amd as tb
     from tritonblas_amd import _lib
-    from tritonblas_amd.matmul import _tile_of
+    from tritonblas_amd.matmul import _queue_tile
     code, queues = _lib.tb_dtype(dtype), _lib.TB_SCHED_WORK_STEALING
     own = _launch_of(_job(code, m, n, k))
     assert own.block_n == 32
@@ -866,16 +866,15 @@ def test_small_tiles_are_for_cus_that_would_be_idle(dtype, m, n, k):
     assert (info.block_m, info.block_n) == (64, 32) and info.total_tiles <= 256
     sel = tb.OrigamiMatmulSelector(m, n, k, dtype, dtype, torch.bfloat16, None)
     assert (sel.block_m, sel.block_n) == (own.block_m, own.block_n)
-    model = sel.block_m, sel.block_n, sel.block_k
-    assert _tile_of(sel, queues, k, dtype, True) == (0, 0, 0) and _tile_of(sel, _lib.TB_SCHED_PERSISTENT, k, dtype, True) == model == _tile_of(sel, _lib.TB_SCHED_STREAMK, k, dtype, True)
+    assert _queue_tile(sel, dtype) == (0, 0, 0)
     for cus in (8, 16, 64):
         sel = tb.OrigamiMatmulSelector(m, n, k, dtype, dtype, torch.bfloat16, None, total_cus=cus)
         tiles = -(-m // sel.block_m) * -(-n // sel.block_n)
         assert sel.block_n > 32 or tiles <= cus * sel.waves_per_eu
         model = sel.block_m, sel.block_n, sel.block_k
-        assert _tile_of(sel, queues, k, dtype, True) == ((64, 32, model[2]) if model[1] == 32 else model) and _tile_of(sel, _lib.TB_SCHED_PERSISTENT, k, dtype, False) == model
+        assert _queue_tile(sel, dtype) == ((64, 32, model[2]) if model[1] == 32 else model)
         sel._sel.block_m = sel._sel.block_n = 32      # (a tile that the caller put into the selector stays)
-        assert model[:2] == (32, 32) or _tile_of(sel, queues, k, dtype, True) == (32, 32, model[2])
+        assert model[:2] == (32, 32) or _queue_tile(sel, dtype) == (32, 32, model[2])
 
 
 def test_fp32_and_int8_tiles_of_launches_kept_to_some_workgroups():

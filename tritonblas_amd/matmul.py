@@ -120,21 +120,17 @@ def _flat_scales(a_scale, b_scale, M, N):
     return a_scale, b_scale
 
 
-def _tile_of(selector, schedule, K, dtype, k_contiguous):
-    """The tile that a launch names, (0, 0, 0) where it leaves the choice to the library: where the selector's is the model's as well, and the model did not know all.
+def _queue_tile(selector, dtype):
+    """The tile that a work-stealing launch names, (0, 0, 0) where it leaves the choice to the library.
 
-    A selector knows sizes and types, not how the operands are stored.  That matters to the tile model only where K is no even number of K
-    steps: the hand-scheduled kernels take what is left behind them from K-contiguous operands whose rows start on 16 bytes, for others the model
-    has the eight-wave kernel's figures (bf16 3232x6880x2272 with a row-major b: 256x128 for a selector, 113 us, and 256x256 once the layout is told, 102).
-    Nor does it know that the tiles come from the work-stealing queues, which 32x32 tiles do not suit (FP8 256x256x7904 31.5 us, in 64x32 19; of a selector
-    for 64 CUs 28.6 and 19)."""
+    The model that chose a selector's tile did not know that the tiles come from the queues, which 32x32 tiles of the 16- and 8-bit types do not suit (FP8
+    256x256x7904 31.5 us, in 64x32 19; with a selector for 64 CUs 28.6 and 19)."""
     tile = selector.block_m, selector.block_n, selector.block_k
-    if schedule in (_lib.TB_SCHED_STREAMK, _lib.TB_SCHED_STREAMK_WS):
+    if tile[1] != 32 or dtype == torch.float32:
         return tile
-    small = schedule == _lib.TB_SCHED_WORK_STEALING and tile[1] == 32 and dtype != torch.float32
     if tile == getattr(selector, "_model_tile", None):
-        return (0, 0, 0) if small or (K % (2 * tile[2]) != 0 and not k_contiguous) else tile
-    return (64, *tile[1:]) if small and tile == getattr(selector, "_part_tile", None) else tile
+        return 0, 0, 0
+    return (64, *tile[1:]) if tile == getattr(selector, "_part_tile", None) else tile
 
 
 def _launch_gemm(a, b, c, selector, config, schedule, bias=None, a_scale=None, b_scale=None, sk_grid=None):
@@ -161,11 +157,18 @@ def _launch_gemm(a, b, c, selector, config, schedule, bias=None, a_scale=None, b
     block_m = block_n = block_k = group_m = num_xcds = counters = 0
     if selector is not None:
         block_m, block_n, block_k = selector.block_m, selector.block_n, selector.block_k
-        if schedule or K % (2 * block_k):
-            block_m, block_n, block_k = _tile_of(selector, schedule, K, a.dtype, a_sk == 1 == b_sk and (a_sm | b_sn) % 16 == 0)
         group_m, num_xcds, counters = selector.group_m, selector.num_sms, selector.COUNTERS_PER_XCD
-        if block_m == 0:
-            group_m = counters = 0
+        # A selector knows sizes and types, not how the operands are stored.  That matters to the tile model only where K is no even number of K
+        # steps: the hand-scheduled kernels take what is left behind them from K-contiguous operands whose rows start on 16 bytes, for others the model
+        # has the eight-wave kernel's figures.  Then the library's own choice, the same model with the operands at hand, takes the place of a choice that is
+        # the model's as well (bf16 3232x6880x2272 with a row-major b: 256x128 for a selector, 113 us, and 256x256 once the layout is told, 102).
+        if (K % (2 * block_k) and not (a_sk == 1 == b_sk and (a_sm | b_sn) % 16 == 0) and not streamk
+                and (block_m, block_n, block_k) == getattr(selector, "_model_tile", None)):
+            block_m = block_n = block_k = group_m = 0
+        elif schedule and not streamk:      # (work stealing)
+            block_m, block_n, block_k = _queue_tile(selector, a.dtype)
+            if block_m == 0:
+                group_m = counters = 0
     grid = 0
     if selector is not None and not streamk and getattr(selector, "_total_cus", None) is not None:
         # a selector built for a CU partition sizes the launch (reference matmul.py:113: grid = N_CU):
