@@ -733,7 +733,7 @@ __device__ __forceinline__ void mainloop(const GemmParams& p, const TileCtx& tc,
     int stage = 0;
     constexpr int READS = T::KSUB * (RPFA * T::TM + RPFB * T::TN), MFMAS = T::KSUB * T::TM * T::TN;
     // AMONG: the copies of step it + S between shares of the reads and MFMAs.  Issued in one go behind the barrier they hold every wave up together, a copy
-    // keeps the address path of the CU for 16 cycles, and only then its MFMAs begin.  Each in front of its share; behind it they start too late where the copies
+    // keeps the address path of the CU busy for 18 to 23 cycles, and only then its MFMAs begin.  Each in front of its share; behind it they start too late where the copies
     // bound the step (128x128 below 46.6 -> 47.5, 47.8 -> 52).  In one go and among, 128x128, us: bf16 512x1024x4096 32.7 and 26.0, 2048^3 23.7 and 23.1,
     // 1871x1728x12544 105.5 and 101.5, 2048x4096x4096 81.7 and 74.8, 584x4624x3688 46.0 and 46.6, 584x4608x3688 51.3 and 47.8; FP8 512x1024x4096 18.1 and 15.7, 2048^3 14.4 and
     // 13.6; 128x64: bf16 512x1024x4096 23.0 and 19.4, 1536x1536x4096 48.9 and 45.3, 512x4096x14336 96.2 and 95.7; 256x128: bf16 2048x4096x4096 62.1
